@@ -1,16 +1,17 @@
-// C = op(A) op(B) (+ bias) (+ residual), activation epilogue.
+// C = op(A) op(B) (+ bias) (+ residual), activation epilogue: the dispatch, and
 //
-//   gemm_mfma_nt_kernel   bf16 / f16, A [M,K] and B [N,K] both K-contiguous (the
-//                         nn::Linear case x W^T): v_mfma_f32_32x32x16, workgroup
-//                         tile 128x128x64 or 64x128x64, 4 waves, A/B tiles staged
-//                         through LDS with up to three k-tiles in flight, fp32
-//                         accumulation.
-//   gemm_generic_kernel   any dtype / any transpose combination, 16x16 LDS tiles,
-//                         fp32 FMA.
+//   gemm_mfma_nt_256_kernel    large bf16 / f16 x W^T: 256 x 256 tiles
+//   gemm_mfma_f32_ring_kernel  fp32 x W^T on the fp32 matrix instruction
+//   gemm_generic_kernel        any dtype / any transpose combination, 16x16 LDS tiles, fp32 FMA
+//
+// The other 16-bit kernels are in gemm_tile_*.hip (middle-sized products), gemm_small.hip (few rows or few output
+// tiles) and gemm_skinny.hip (at most eight rows).
 #include "common.hpp"
+#include "gemm_small.hpp"
 #include "gemm_skinny.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <mutex>
 #include <set>
@@ -52,10 +53,6 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs g) {
     }
 }
 
-// Epilogue of the MFMA kernels: accumulator element e of 32x32 tile (i, j) is
-// C[m_base + 32 i + 8 (e/4) + 4 g2 + e%4][n_base + 32 j + l32].  bias, residual and
-// the activation are applied in fp32 before the one rounding to the output type.
-// The activation is resolved outside the element loops.
 template <bool BF16>
 __device__ __forceinline__ float load16(const void *p, int64_t i) {
     const uint16_t b = static_cast<const uint16_t *>(p)[i];
@@ -66,177 +63,7 @@ __device__ __forceinline__ void store16(void *p, int64_t i, float x) {
     static_cast<uint16_t *>(p)[i] = BF16 ? f32_to_bf16_bits(x) : f32_to_f16_bits(x);
 }
 
-// C and the residual are addressed through buffer descriptors that cover exactly the valid
-// rows of the block, so a row past the end of C is dropped by the hardware bounds check;
-// columns past the end are masked per lane.  When all MI*32 rows are valid (FULL_ROWS)
-// the row offset travels in the scalar offset of the instruction, otherwise it is added
-// to the lane's offset, which is what the bounds check looks at.
-// (Column tiles outside, rows inside: on the ring kernels' products the other nesting measured 3 - 5 % slower.)
-// Requires MI*32 * ldc * 2 < 2^31.
-template <bool BF16, int RESIDUAL_T, bool FULL_ROWS, int OP, int MI, int NJ> // RESIDUAL_T: 0 no, 1 yes, 2 decided at run time
-__device__ __forceinline__ void gemm_store_tiles_as(const GemmArgs &g, const float16_t (&acc)[MI][NJ], int64_t m_base, int64_t n_base, int64_t coff, int l32, int g2) {
-    const bool RESIDUAL = RESIDUAL_T == 1 || (RESIDUAL_T == 2 && g.residual != nullptr);
-    const int ldc2 = static_cast<int>(g.ldc) * 2;
-    const int cols_valid = static_cast<int>(min<int64_t>(32 * NJ, g.N - n_base));
-    const int rows_valid = static_cast<int>(min<int64_t>(32 * MI, g.M - m_base));
-    const int extent = (rows_valid - 1) * ldc2 + cols_valid * 2;
-    const int64_t origin = coff + m_base * g.ldc + n_base;
-    const __amdgpu_buffer_rsrc_t crsrc = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint16_t *>(g.c) + origin, 0, extent, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(static_cast<const uint16_t *>(RESIDUAL ? g.residual : g.c)) + origin, 0, extent, 0x00020000);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int col = 32 * j + l32;
-        if (col >= cols_valid) continue;
-        const float bias = g.bias ? load16<BF16>(g.bias, n_base + col) : 0.0f;
-        const int voff = 4 * g2 * ldc2 + col * 2;
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            float x[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                x[e] = acc[i][j][e] + bias;
-                if (RESIDUAL) {
-                    const int roff = (32 * i + 8 * (e / 4) + e % 4) * ldc2;
-                    const uint16_t r = __builtin_amdgcn_raw_buffer_load_b16(rrsrc, FULL_ROWS ? voff : voff + roff, FULL_ROWS ? roff : 0, 0);
-                    x[e] += BF16 ? bf16_bits_to_f32(r) : f16_bits_to_f32(r);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 16; e += 2) {
-                const float y0 = gemm_epilogue16(OP, x[e]), y1 = gemm_epilogue16(OP, x[e + 1]);
-                const uint32_t w = BF16 ? pack_bf16x2(y0, y1) : pack_f16x2(y0, y1);
-                const int roff = (32 * i + 8 * (e / 4) + e % 4) * ldc2;
-                __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(w & 0xFFFFu), crsrc, FULL_ROWS ? voff : voff + roff, FULL_ROWS ? roff : 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(w >> 16), crsrc, FULL_ROWS ? voff : voff + roff + ldc2, FULL_ROWS ? roff + ldc2 : 0, 0);
-            }
-        }
-    }
-}
-
-template <bool BF16, int MI, int NJ>
-__device__ __forceinline__ void gemm_store_tiles(const GemmArgs &g, const float16_t (&acc)[MI][NJ], int64_t m_base, int64_t n_base, int64_t coff, int l32, int g2) {
-    if (m_base >= g.M || n_base >= g.N) return;
-    const bool full_rows = m_base + MI * 32 <= g.M;
-    // the cheap epilogues get a specialisation per (residual, full rows); the transcendental
-    // ones are large when unrolled 128 times, and one general instance each is enough
-#define AXHIP_GEMM_EPI_FAST(OP)                                                                                         \
-    if (full_rows) {                                                                                                    \
-        if (g.residual) gemm_store_tiles_as<BF16, 1, true, OP, MI, NJ>(g, acc, m_base, n_base, coff, l32, g2);          \
-        else gemm_store_tiles_as<BF16, 0, true, OP, MI, NJ>(g, acc, m_base, n_base, coff, l32, g2);                     \
-    } else {                                                                                                            \
-        if (g.residual) gemm_store_tiles_as<BF16, 1, false, OP, MI, NJ>(g, acc, m_base, n_base, coff, l32, g2);         \
-        else gemm_store_tiles_as<BF16, 0, false, OP, MI, NJ>(g, acc, m_base, n_base, coff, l32, g2);                    \
-    }
-#define AXHIP_GEMM_EPI_GENERAL(OP) gemm_store_tiles_as<BF16, 2, false, OP, MI, NJ>(g, acc, m_base, n_base, coff, l32, g2);
-    switch (g.epilogue) {
-    case AXHIP_OP_RELU: AXHIP_GEMM_EPI_FAST(AXHIP_OP_RELU) break;
-    case AXHIP_OP_GELU: AXHIP_GEMM_EPI_GENERAL(AXHIP_OP_GELU) break;
-    case AXHIP_OP_SILU: AXHIP_GEMM_EPI_GENERAL(AXHIP_OP_SILU) break;
-    case AXHIP_OP_SIGMOID: AXHIP_GEMM_EPI_GENERAL(AXHIP_OP_SIGMOID) break;
-    case AXHIP_OP_TANH: AXHIP_GEMM_EPI_GENERAL(AXHIP_OP_TANH) break;
-    default: AXHIP_GEMM_EPI_FAST(0) break;
-    }
-#undef AXHIP_GEMM_EPI_FAST
-#undef AXHIP_GEMM_EPI_GENERAL
-}
-
-
-// ------------------------------------------------------------------- MFMA NT
-// Work-group tile BM x 128 x 64 (BM = 128 or 64), 4 waves in a 2 x 2 layout, each
-// owning a (BM/2) x 64 block of C as 32x32 MFMA tiles.  A and B k-tiles travel
-// HBM/L2 -> registers -> LDS; NPRE k-tiles are in flight in registers at any
-// time, which is what hides the load latency when a small problem leaves one
-// work-group per CU (the nn::Linear shapes of a single sequence).  The k loop is
-// unrolled NPRE times so that each in-flight tile has its own registers.
-constexpr int TN = 128, TK = 64;
-constexpr int LDS_STRIDE = TK + 8; // 144 B rows: consecutive rows shift by 4 banks (+32)
-
-template <bool BF16, int BM, int NPRE>
-__global__ __launch_bounds__(256, BM == 128 ? 2 : 1) void gemm_mfma_nt_kernel(const GemmArgs g) {
-    constexpr int MI = BM / 64;  // 32-row MFMA tiles per wave in M
-    constexpr int NA = BM / 32;  // 16-byte chunks of A per thread per k-tile (BM rows x 8 chunks / 256 threads)
-    __shared__ __attribute__((aligned(16))) uint16_t As[BM * LDS_STRIDE];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[TN * LDS_STRIDE];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
-    const int l32 = lane % 32, g2 = lane / 32;
-    const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * 64;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BM, n0 = static_cast<int64_t>(blockIdx.x) * TN;
-    const int64_t bz = blockIdx.z;
-    const uint16_t *A = static_cast<const uint16_t *>(g.a) + bz * g.sa;
-    const uint16_t *B = static_cast<const uint16_t *>(g.b) + bz * g.sb;
-
-    float16_t acc[MI][2];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    uint4_t ra[NPRE][NA], rb[NPRE][4];
-    auto load_tiles = [&](int s, int64_t k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int id = tid + 256 * i;
-            const int row = id / 8, cc = id % 8;
-            const int64_t k = k0 + 8 * cc;
-            if (i < NA) {
-                ra[s][i < NA ? i : 0] = uint4_t{0, 0, 0, 0};
-                if (m0 + row < g.M && k < g.K) ra[s][i < NA ? i : 0] = *reinterpret_cast<const uint4_t *>(A + (m0 + row) * g.a_rs + k);
-            }
-            rb[s][i] = uint4_t{0, 0, 0, 0};
-            if (n0 + row < g.N && k < g.K) rb[s][i] = *reinterpret_cast<const uint4_t *>(B + (n0 + row) * g.b_cs + k);
-        }
-    };
-    auto stage_tiles = [&](int s) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int id = tid + 256 * i;
-            const int row = id / 8, cc = id % 8;
-            if (i < NA) *reinterpret_cast<uint4_t *>(&As[row * LDS_STRIDE + 8 * cc]) = ra[s][i < NA ? i : 0];
-            *reinterpret_cast<uint4_t *>(&Bs[row * LDS_STRIDE + 8 * cc]) = rb[s][i];
-        }
-    };
-    auto multiply_tile = [&]() {
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ++ks) {
-            uint4_t af[MI], bf[2];
-#pragma unroll
-            for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<const uint4_t *>(&As[(wm + 32 * i + l32) * LDS_STRIDE + 16 * ks + 8 * g2]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bf[j] = *reinterpret_cast<const uint4_t *>(&Bs[(wn + 32 * j + l32) * LDS_STRIDE + 16 * ks + 8 * g2]);
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if constexpr (BF16)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, af[i]), __builtin_bit_cast(bf16x8_t, bf[j]), acc[i][j], 0, 0, 0);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, af[i]), __builtin_bit_cast(half8_t, bf[j]), acc[i][j], 0, 0, 0);
-                }
-        }
-    };
-
-#pragma unroll
-    for (int s = 0; s < NPRE; ++s)
-        if (static_cast<int64_t>(s) * TK < g.K) load_tiles(s, static_cast<int64_t>(s) * TK);
-    for (int64_t k0 = 0; k0 < g.K; k0 += NPRE * TK) {
-#pragma unroll
-        for (int s = 0; s < NPRE; ++s) {
-            const int64_t k = k0 + static_cast<int64_t>(s) * TK;
-            if (k < g.K) {
-                __syncthreads(); // every wave is done reading the previous tile
-                stage_tiles(s);
-                __syncthreads();
-                if (k + NPRE * TK < g.K) load_tiles(s, k + NPRE * TK);
-                multiply_tile();
-            }
-        }
-    }
-
-    gemm_store_tiles<BF16, MI, 2>(g, acc, m0 + wm, n0 + wn, bz * g.sc, l32, g2);
-}
+constexpr int TK = 64; // k-tile of the 256 x 256 kernel
 
 // ----------------------------------------------------------- MFMA NT, 256x256
 // Large products: work-group tile 256 x 256 x 64, 8 waves in a 2 x 4 layout, each owning 128 x 64 of C as 8 x 4
@@ -541,133 +368,6 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
     gemm_store_tiles16<BF16>(g, acc, m0 + wm, n0 + wn, bz * g.sc, l16, g4, big_lds + wave * 16384);
 }
 
-// --------------------------------------------------- MFMA NT, multi-stage ring
-// Mid-size products (too few 256 x 256 tiles to fill the chip): work-group tile TM x TN x 64,
-// 4 waves in a 2 x 2 layout, and an S-stage ring of k-tiles in LDS filled by buffer_load ... lds.
-// One work-group per CU cannot hide the L2 latency (about 1 us under load) behind a k-tile's
-// 0.15 - 0.3 us of MFMA work by occupancy, so S - 1 k-tiles are kept in flight instead and the
-// wait before a k-tile is a counted vmcnt that only covers the oldest one.  The k loop is unrolled
-// by S so that every stage address is an immediate.  Same LDS row layout and XOR swizzle, same
-// tile order over the XCDs and same epilogue as the 256 x 256 kernel.
-// Requires K % 64 == 0 and max(TM, TN) * max(lda, ldb) * 2 < 2^31 (checked by the launcher).
-template <bool BF16, int TM, int TNR, int S>
-__global__ __launch_bounds__(256, 1) void gemm_mfma_nt_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
-    constexpr int MI = TM / 64, NJ = TNR / 64;       // 32x32 MFMA tiles per wave
-    constexpr int NLA = TM / 32, NLB = TNR / 32;      // wave-wide loads (8 rows each) per wave per k-tile
-    constexpr int STAGEB = (TM + TNR) * BIG_ROWB;     // bytes per ring stage: A rows, then B rows
-    extern __shared__ __attribute__((aligned(1024))) unsigned char big_lds[];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
-    const int l32 = lane % 32, g2 = lane / 32;
-
-    const int per_xcd = gridDim.x / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles_m * tiles_n) return;
-    constexpr int GR = 4;
-    const int group = t / (GR * tiles_n), first_m = group * GR;
-    const int gsz = min(GR, tiles_m - first_m);
-    const int rem = t - group * GR * tiles_n;
-    const int tm = first_m + rem % gsz, tn = rem / gsz;
-    const int64_t m0 = static_cast<int64_t>(tm) * TM, n0 = static_cast<int64_t>(tn) * TNR;
-    const int64_t bz = blockIdx.y;
-    const uint16_t *A = static_cast<const uint16_t *>(g.a) + bz * g.sa + m0 * g.a_rs;
-    const uint16_t *B = static_cast<const uint16_t *>(g.b) + bz * g.sb + n0 * g.b_cs;
-    const int arow_bytes = static_cast<int>(g.a_rs) * 2, brow_bytes = static_cast<int>(g.b_cs) * 2;
-    const int rows_a = static_cast<int>(min<int64_t>(TM, g.M - m0)), rows_b = static_cast<int>(min<int64_t>(TNR, g.N - n0));
-    const int4_t arsrc = gemm_rsrc(A, (rows_a - 1) * arow_bytes + static_cast<int>(g.K) * 2);
-    const int4_t brsrc = gemm_rsrc(B, (rows_b - 1) * brow_bytes + static_cast<int>(g.K) * 2);
-
-    // load n of wave w covers tile rows 32 n + 8 w + (lane >> 3)
-    const int ld_r = 8 * wave + (lane >> 3);
-    const int ld_c = (lane & 7) ^ ((ld_r >> 1) & 7);
-    int a_voff[NLA], b_voff[NLB];
-#pragma unroll
-    for (int n = 0; n < NLA; ++n) a_voff[n] = (32 * n + ld_r) * arow_bytes + ld_c * 16;
-#pragma unroll
-    for (int n = 0; n < NLB; ++n) b_voff[n] = (32 * n + ld_r) * brow_bytes + ld_c * 16;
-    const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(big_lds));
-    const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + 8 * wave * BIG_ROWB);
-    auto load_tile = [&](int kt, int stage) {
-        const int soff = kt * BIG_ROWB;
-#pragma unroll
-        for (int n = 0; n < NLA; ++n) gemm_load_to_lds(arsrc, lds_wave + stage * STAGEB + n * 32 * BIG_ROWB, a_voff[n], soff);
-#pragma unroll
-        for (int n = 0; n < NLB; ++n) gemm_load_to_lds(brsrc, lds_wave + stage * STAGEB + TM * BIG_ROWB + n * 32 * BIG_ROWB, b_voff[n], soff);
-    };
-
-    const int wm = (wave / 2) * (TM / 2), wn = (wave % 2) * (TNR / 2);
-    int f_off[TK / 16];
-#pragma unroll
-    for (int ks = 0; ks < TK / 16; ++ks) f_off[ks] = l32 * BIG_ROWB + (((2 * ks + g2) ^ ((l32 >> 1) & 7)) * 16);
-
-    float16_t acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    uint4_t fa[2][MI], fb[2][NJ];
-    auto read_frags = [&](int slot, int stage, int ks) {
-        const unsigned char *As = big_lds + stage * STAGEB + wm * BIG_ROWB;
-        const unsigned char *Bs = big_lds + stage * STAGEB + (TM + wn) * BIG_ROWB;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) fb[slot][j] = *reinterpret_cast<const uint4_t *>(Bs + 32 * j * BIG_ROWB + f_off[ks]);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) fa[slot][i] = *reinterpret_cast<const uint4_t *>(As + 32 * i * BIG_ROWB + f_off[ks]);
-    };
-    auto multiply = [&](int slot) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                if constexpr (BF16)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fa[slot][i]), __builtin_bit_cast(bf16x8_t, fb[slot][j]), acc[i][j], 0, 0, 0);
-                else
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, fa[slot][i]), __builtin_bit_cast(half8_t, fb[slot][j]), acc[i][j], 0, 0, 0);
-            }
-    };
-
-    const int nk = static_cast<int>(g.K / TK);
-    // s_waitcnt vmcnt(N) with the other counters left alone: N = loads of the S - 2 k-tiles that may still be in flight
-    constexpr int INFLIGHT = (NLA + NLB) * (S - 2);
-    static_assert(INFLIGHT < 64, "vmcnt is a 6-bit counter");
-    constexpr int WAIT_OLDEST = (INFLIGHT & 0xF) | 0x0F70 | ((INFLIGHT >> 4) << 14);
-#pragma unroll
-    for (int st = 0; st < S - 1; ++st)
-        if (st < nk) load_tile(st, st);
-
-    // k-tile kt lives in ring stage ST (= kt % S, a compile-time value in the unrolled loop)
-    auto step = [&](auto stage_tag, int kt) {
-        constexpr int ST = decltype(stage_tag)::value;
-        if (kt + S - 2 < nk) __builtin_amdgcn_s_waitcnt(WAIT_OLDEST); // everything older than the S - 2 newest k-tiles has landed
-        else __builtin_amdgcn_s_waitcnt(0x0F70);                      // tail: fewer loads behind this one, wait for all
-        __syncthreads(); // k-tile kt is complete for every wave, and k-tile kt - 1 (whose stage is refilled next) is no longer read
-        if (kt + S - 1 < nk) load_tile(kt + S - 1, (ST + S - 1) % S);
-        read_frags(0, ST, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ++ks) {
-            if (ks + 1 < TK / 16) read_frags((ks + 1) & 1, ST, ks + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(ks & 1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    auto steps = [&](auto self, auto stage_tag, int kt0) -> void { // step<0>(kt0), step<1>(kt0 + 1), ... step<S-1>
-        constexpr int ST = decltype(stage_tag)::value;
-        if constexpr (ST < S) {
-            if (kt0 + ST < nk) {
-                step(stage_tag, kt0 + ST);
-                self(self, std::integral_constant<int, ST + 1>{}, kt0);
-            }
-        }
-    };
-    for (int kt0 = 0; kt0 < nk; kt0 += S) steps(steps, std::integral_constant<int, 0>{}, kt0);
-
-    gemm_store_tiles<BF16, MI, NJ>(g, acc, m0 + wm, n0 + wn, bz * g.sc, l32, g2);
-}
-
 // ------------------------------------------------------------------ fp32, MFMA
 // C = A B^T in fp32 on v_mfma_f32_32x32x2_f32 (fp32 products, fp32 accumulation: no precision is given up against
 // the FMA kernel), A [M,K] and B [N,K] both K-contiguous.  Same skeleton as the 16-bit ring kernel: a k-tile is 32
@@ -811,12 +511,6 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
 
 using namespace axhip;
 
-// AXHIP_GEMM_RING=0 routes mid-size products to the register-staged kernels (for A/B timing)
-static bool ring_enabled() {
-    static const bool on = [] { const char *e = std::getenv("AXHIP_GEMM_RING"); return !(e && e[0] == '0'); }();
-    return on;
-}
-
 // AXHIP_GEMM_F32_MFMA=0 routes fp32 products to the FMA kernel (for A/B timing)
 static bool f32_mfma_enabled() {
     static const bool on = [] { const char *e = std::getenv("AXHIP_GEMM_F32_MFMA"); return !(e && e[0] == '0'); }();
@@ -829,14 +523,10 @@ static bool skinny_enabled() {
     return on;
 }
 
-// AXHIP_GEMM_RING_TILE=0..2 forces one ring tile shape (128x128, 64x128, 128x192) for A/B timing
-static int ring_tile_override() {
-    static const int v = [] { const char *e = std::getenv("AXHIP_GEMM_RING_TILE"); return (e && e[0] >= '0' && e[0] <= '2') ? e[0] - '0' : -1; }();
-    return v;
-}
-
 namespace {
-// whether (and into how many padded columns) a product is repacked before it runs on the k-contiguous kernels
+// whether (and into how many padded columns) a product is repacked before it runs on the k-contiguous kernels: fp32, and
+// 16-bit ones with A stored [k, m]; the workspace that axhip_gemm_workspace_bytes asks for does not depend on the type,
+// so that a program's figures stay what they were when every such product was repacked
 struct Repack { bool on, a, b; int64_t kp; };
 Repack repack_plan(const AxhipGemmParams &p) {
     const int64_t kvec = p.dtype == AXHIP_DTYPE_F32 ? 4 : 8;
@@ -879,6 +569,98 @@ extern "C" int axhip_gemm_ws(const void *a, const void *b, void *c, const AxhipG
 }
 
 namespace {
+// ---- 16-bit products: which kernel
+// A stored along k, and everything within the 32-bit offsets the kernels address with.
+bool takes_half_kernels(const AxhipGemmParams &p) {
+    constexpr int64_t LD = int64_t(1) << 21, SIDE = int64_t(1) << 30;
+    return !p.trans_a && p.k >= 8 && (p.trans_b || p.n >= 8) && p.m < SIDE && p.n < SIDE && p.k < SIDE && p.lda < LD && p.ldb < LD &&
+           p.ldc < (int64_t(1) << 31) && (p.trans_b || (p.k + 64) * p.ldb < SIDE);
+}
+// rows of both operands on 16-byte boundaries and in whole 16-byte vectors
+bool half_aligned(const AxhipGemmParams &p, const void *a, const void *b) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0 && (p.k | p.lda | p.ldb | p.stride_a | p.stride_b | (p.trans_b ? 0 : p.n)) % 8 == 0;
+}
+
+// The candidates with the time each takes, in us: start + k (per_k + per_k_full u) r + per_round (r - 1), r being the
+// rounds its work-groups take on the 256 CUs (whole rounds of the tile kernels, of which a CU holds one; the small ones
+// share a CU, and a part of a round costs about half of what is missing from a whole one) and u how full the first is.
+// The coefficients are fitted to 300 products of m 16 .. 3000, n 128 .. 5120, k 128 .. 4096, bf16, operands from the
+// caches: mean error 3 - 9 %, and the kernel picked is on average 1 % slower than the fastest of all.  Rows off the
+// 16-byte grid cost the small kernels 1.9 times per element of k (odd k of 842 .. 2045).
+struct HalfKernel {
+    enum Kind { BIG256, TILE, SMALL } kind;
+    int shape, waves;
+    float start, per_k, per_k_full, per_round;
+    bool nt, nn, ragged;
+};
+constexpr HalfKernel HALF_KERNELS[] = {
+    {HalfKernel::BIG256, 0, 8, 7.0f, 0.0160f, 0.0057f, 4.0f, true, false, false},
+    {HalfKernel::TILE, TILE_256x128, 8, 6.5f, 0.0080f, 0.0034f, 6.4f, true, true, false},
+    {HalfKernel::TILE, TILE_192x128, 8, 5.7f, 0.0063f, 0.0024f, 4.9f, true, true, false},
+    {HalfKernel::TILE, TILE_128x128, 8, 4.9f, 0.0048f, 0.0014f, 4.1f, true, true, false},
+    {HalfKernel::TILE, TILE_64x128, 8, 4.9f, 0.0032f, 0.0009f, 3.7f, true, true, false},
+    {HalfKernel::TILE, TILE_128x128, 8, 9.5f, 0.0095f, 0.0f, 5.0f, true, true, true}, // (through registers)
+    {HalfKernel::SMALL, SMALL_64x64, 8, 4.35f, 0.00245f, 0.00148f, 3.6f, true, true, false},
+    {HalfKernel::SMALL, SMALL_64x64, 4, 4.15f, 0.00324f, 0.00047f, 1.65f, true, true, false},
+    {HalfKernel::SMALL, SMALL_32x64, 8, 3.50f, 0.00170f, 0.00085f, 2.3f, true, true, false},
+    {HalfKernel::SMALL, SMALL_32x64, 4, 3.30f, 0.00210f, 0.00030f, 0.6f, true, true, false},
+    {HalfKernel::SMALL, SMALL_16x64, 8, 3.19f, 0.00150f, 0.00035f, 0.77f, false, true, false},
+    {HalfKernel::SMALL, SMALL_16x64, 4, 3.04f, 0.00183f, 0.00008f, 0.27f, false, true, false},
+    {HalfKernel::SMALL, SMALL_32x32, 8, 3.07f, 0.00105f, 0.00045f, 0.76f, true, false, false},
+    {HalfKernel::SMALL, SMALL_32x32, 4, 2.95f, 0.00148f, 0.00005f, 0.26f, true, false, false},
+    {HalfKernel::SMALL, SMALL_32x16, 8, 2.92f, 0.00074f, 0.00032f, 0.33f, true, false, false},
+    {HalfKernel::SMALL, SMALL_32x16, 4, 2.91f, 0.00102f, 0.00004f, 0.10f, true, false, false},
+    {HalfKernel::SMALL, SMALL_16x16, 8, 2.95f, 0.00045f, 0.00024f, 0.19f, true, false, false},
+    {HalfKernel::SMALL, SMALL_16x16, 4, 2.94f, 0.00069f, 0.00004f, 0.02f, true, false, false},
+};
+
+const HalfKernel &choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
+    const HalfKernel *best = nullptr;
+    float best_cost = 0.0f;
+    const uint32_t m = static_cast<uint32_t>(p.m), n = static_cast<uint32_t>(p.n);
+    const float k = static_cast<float>((p.k + 63) / 64 * 64), batch = static_cast<float>(p.batch);
+    for (const HalfKernel &h : HALF_KERNELS) {
+        if (p.trans_b ? !h.nt : !h.nn) continue;
+        if (h.kind != HalfKernel::SMALL && h.ragged == aligned) continue;
+        if (h.kind == HalfKernel::BIG256 && (p.k % TK != 0 || p.m < BIG || p.n < BIG || p.ldc >= (1 << 21))) continue;
+        const uint32_t tm = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tm : SMALL_GEOMETRY[h.shape].tm;
+        const uint32_t tn = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tn : SMALL_GEOMETRY[h.shape].tn;
+        const float full = batch * static_cast<float>((m + tm - 1) / tm) * static_cast<float>((n + tn - 1) / tn) * (1.0f / 256.0f);
+        const float whole = std::ceil(full), r = full <= 1.0f ? 1.0f : h.kind == HalfKernel::SMALL ? 0.5f * (whole + full) : whole;
+        const float per_k = (h.per_k + h.per_k_full * std::min(full, 1.0f)) * (h.kind == HalfKernel::SMALL && !aligned ? 1.9f : 1.0f);
+        const float cost = h.start + k * per_k * r + h.per_round * (r - 1.0f);
+        if (!best || cost < best_cost) { best_cost = cost; best = &h; }
+    }
+    return *best;
+}
+
+int launch_big(const GemmArgs &g, bool bf, int batch, hipStream_t s) {
+    const int tiles_m = static_cast<int>((g.M + BIG - 1) / BIG), tiles_n = static_cast<int>((g.N + BIG - 1) / BIG);
+    const dim3 grid(static_cast<unsigned>(8 * ((tiles_m * tiles_n + 7) / 8)), static_cast<unsigned>(batch));
+    constexpr size_t lds_bytes = 4 * BIG_TILEB;
+    static const bool configured = [] {
+        bool ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_nt_256_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
+        ok = ok && hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_nt_256_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
+        return ok;
+    }();
+    AXHIP_REQUIRE(configured, AXHIP_ERR_UNSUPPORTED, "axhip_gemm: cannot reserve %zu bytes of LDS", lds_bytes);
+    if (bf) hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<true>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
+    else hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<false>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
+    return AXHIP_OK;
+}
+
+int launch_half(const AxhipGemmParams &p, const void *a, const void *b, void *c, const HalfKernel &k, bool aligned, bool bf, hipStream_t s) {
+    TileArgs t{};
+    t.a = a; t.b = b; t.c = c; t.bias = p.bias; t.residual = p.residual;
+    t.sa = p.stride_a; t.sb = p.stride_b; t.sc = p.stride_c;
+    t.M = static_cast<int>(p.m); t.N = static_cast<int>(p.n); t.K = static_cast<int>(p.k);
+    t.lda = static_cast<int>(p.lda); t.ldb = static_cast<int>(p.ldb); t.ldc = static_cast<int>(p.ldc);
+    t.epilogue = p.epilogue_op;
+    const int batch = static_cast<int>(p.batch);
+    if (k.kind == HalfKernel::SMALL) return launch_small(t, bf, !p.trans_b, k.shape, k.waves, batch, s);
+    return p.trans_b ? launch_tile_nt(t, bf, k.shape, aligned, batch, s) : launch_tile_nn(t, bf, k.shape, aligned, batch, s);
+}
+
 int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *params, CallScratch *scratch_in, void *workspace, size_t workspace_bytes, void *stream) {
     AXHIP_REQUIRE(params != nullptr, AXHIP_ERR_INVALID_ARG, "axhip_gemm: params is NULL");
     const AxhipGemmParams &p = *params;
@@ -907,13 +689,17 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     if (rc) return rc;
     hipStream_t s = resolve_stream(stream);
 
-    // The matrix-core kernels read both operands along k, in 16-byte vectors.  An operand stored the other way (A as
+    // The fp32 matrix kernel reads both operands along k, in 16-byte vectors (the 16-bit ones read A along k).  An operand stored the other way (A as
     // [k, m], B as [k, n]: matmul(a, b) with a plain [k, n] right-hand side), or a reduction length that is not a whole
     // number of vectors, leaves only the FMA kernel below, a hundred times slower on a large product.  Such a product
     // is repacked first, into stream-ordered temporary memory (freed in stream order behind the product): the operand
     // that lies the other way is transposed; an unaligned k is zero-padded to the next multiple of 64 in both operands.
     const Repack rp = repack_plan(p);
-    if (rp.on && !scratch_in) {
+    if (workspace) {
+        const size_t need = repack_bytes(p);
+        AXHIP_REQUIRE(workspace_bytes >= need, AXHIP_ERR_WORKSPACE, "axhip_gemm: the workspace holds %zu bytes, the call needs %zu (ask axhip_gemm_workspace_bytes)", workspace_bytes, need);
+    }
+    if (rp.on && !scratch_in && !(p.dtype != AXHIP_DTYPE_F32 && takes_half_kernels(p))) {
         const bool pad_k = rp.kp != p.k;
         const int64_t es = p.dtype == AXHIP_DTYPE_F32 ? 4 : 2, kp = rp.kp;
         AxhipGemmParams q = p;
@@ -982,79 +768,11 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const int rows_per_wave = forced_rows == 1 || forced_rows == 2 || forced_rows == 4 ? forced_rows : (p.m >= 2 && w_elems >= (int64_t(64) << 20)) ? 2 : 1;
         const unsigned blocks = static_cast<unsigned>((p.n + 4 * rows_per_wave - 1) / (4 * rows_per_wave));
         launch_skinny(k, static_cast<int>(p.m), rows_per_wave, blocks, s);
-    } else if (half && nt && p.k > 0 && p.k % TK == 0 && p.m >= BIG && p.n >= BIG && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.batch < 65536 &&
-        ((p.m + BIG - 1) / BIG) * ((p.n + BIG - 1) / BIG) * p.batch >= 128) {
-        // 256 x 256 tiles once they give at least half the CUs a work-group
-        const int tiles_m = static_cast<int>((p.m + BIG - 1) / BIG), tiles_n = static_cast<int>((p.n + BIG - 1) / BIG);
-        const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-        const dim3 grid(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch));
-        constexpr size_t lds_bytes = 4 * BIG_TILEB;
-        static const bool configured = [] {
-            bool ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_nt_256_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
-            ok = ok && hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_nt_256_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
-            return ok;
-        }();
-        AXHIP_REQUIRE(configured, AXHIP_ERR_UNSUPPORTED, "axhip_gemm: cannot reserve %zu bytes of LDS", lds_bytes);
-        if (p.dtype == AXHIP_DTYPE_BF16) hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<true>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
-        else hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<false>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
-    } else if (half && nt && p.k > 0 && p.k % TK == 0 && p.k >= 4 * TK && p.lda < (1 << 22) && p.ldb < (1 << 22) && p.batch < 65536 &&
-               ring_enabled()) {
-        // mid-size: the ring kernels
-        const bool bf = p.dtype == AXHIP_DTYPE_BF16;
-        auto launch = [&](auto kernel, int tm_rows, int tn_cols, size_t lds_bytes) -> int {
-            static std::mutex mu;
-            static std::set<const void *> configured;
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                if (!configured.count(reinterpret_cast<const void *>(kernel))) {
-                    AXHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-                    configured.insert(reinterpret_cast<const void *>(kernel));
-                }
-            }
-            const int tiles_m = static_cast<int>((p.m + tm_rows - 1) / tm_rows), tiles_n = static_cast<int>((p.n + tn_cols - 1) / tn_cols);
-            const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(256), lds_bytes, s, g, tiles_m, tiles_n);
-            return AXHIP_OK;
-        };
-        // Tile shape by modelled time: rounds of work-groups over the 256 CUs x (ring fill and epilogue + the tile's
-        // k loop).  The k-loop cost per tile element is calibrated on the Whisper projections (64 x 128 tiles pay 1.4x
-        // per element for their lower reuse of the LDS fragments, 128 x 192 tiles 1.13x for their shorter ring).  The
-        // wide tile exists because a product such as 1500 x 3840 x 1280 makes 360 tiles of 128 x 128 (two rounds, the
-        // second 40 % full) but 240 of 128 x 192.
-        struct RingTile { int tm, tn; double per_elem; };
-        static const RingTile candidates[] = {{128, 128, 1.0}, {64, 128, 1.42}, {128, 192, 1.13}};
-        int best = 0;
-        double best_cost = 0.0;
-        for (int c = 0; c < 3; ++c) {
-            const RingTile &rt = candidates[c];
-            if (ring_tile_override() >= 0 && c != ring_tile_override()) continue;
-            const int64_t tiles = ((p.m + rt.tm - 1) / rt.tm) * ((p.n + rt.tn - 1) / rt.tn) * p.batch;
-            const double rounds = static_cast<double>((tiles + 255) / 256);
-            // fixed part: 3 us, in units where a 128 x 128 x 1280 k loop costs 12.25 us
-            const double cost = rounds * (3.0 + 12.25 * rt.per_elem * (rt.tm * rt.tn / 16384.0) * (static_cast<double>(p.k) / 1280.0));
-            if (best_cost == 0.0 || cost < best_cost) { best_cost = cost; best = c; }
-        }
-        int rc2;
-        switch (best) {
-        case 0: rc2 = bf ? launch(gemm_mfma_nt_ring_kernel<true, 128, 128, 4>, 128, 128, 4 * 256 * BIG_ROWB) : launch(gemm_mfma_nt_ring_kernel<false, 128, 128, 4>, 128, 128, 4 * 256 * BIG_ROWB); break;
-        case 1: rc2 = bf ? launch(gemm_mfma_nt_ring_kernel<true, 64, 128, 6>, 64, 128, 6 * 192 * BIG_ROWB) : launch(gemm_mfma_nt_ring_kernel<false, 64, 128, 6>, 64, 128, 6 * 192 * BIG_ROWB); break;
-        default: rc2 = bf ? launch(gemm_mfma_nt_ring_kernel<true, 128, 192, 4>, 128, 192, 4 * 320 * BIG_ROWB) : launch(gemm_mfma_nt_ring_kernel<false, 128, 192, 4>, 128, 192, 4 * 320 * BIG_ROWB); break; // all 160 KiB of LDS
-        }
-        if (rc2) return rc2;
-    } else if (half && nt && p.k > 0) {
-        // Tall tiles (two work-groups per CU, one k-tile in flight) once they fill the chip;
-        // otherwise 64-row tiles, one work-group per CU with three k-tiles in flight.
-        const int64_t tiles128 = ((p.n + TN - 1) / TN) * ((p.m + 127) / 128) * p.batch;
-        const bool bf = p.dtype == AXHIP_DTYPE_BF16;
-        if (tiles128 >= 512) {
-            dim3 grid(static_cast<unsigned>((p.n + TN - 1) / TN), static_cast<unsigned>((p.m + 127) / 128), static_cast<unsigned>(p.batch));
-            if (bf) hipLaunchKernelGGL((gemm_mfma_nt_kernel<true, 128, 1>), grid, dim3(256), 0, s, g);
-            else hipLaunchKernelGGL((gemm_mfma_nt_kernel<false, 128, 1>), grid, dim3(256), 0, s, g);
-        } else {
-            dim3 grid(static_cast<unsigned>((p.n + TN - 1) / TN), static_cast<unsigned>((p.m + 63) / 64), static_cast<unsigned>(p.batch));
-            if (bf) hipLaunchKernelGGL((gemm_mfma_nt_kernel<true, 64, 3>), grid, dim3(256), 0, s, g);
-            else hipLaunchKernelGGL((gemm_mfma_nt_kernel<false, 64, 3>), grid, dim3(256), 0, s, g);
-        }
+    } else if (half && takes_half_kernels(p)) {
+        const bool aligned = half_aligned(p, a, b), bf = p.dtype == AXHIP_DTYPE_BF16;
+        const HalfKernel &k = choose_half_kernel(p, aligned);
+        rc = k.kind == HalfKernel::BIG256 ? launch_big(g, bf, static_cast<int>(p.batch), s) : launch_half(p, a, b, c, k, aligned, bf, s);
+        if (rc) return rc;
     } else if (p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
                p.stride_a % 4 == 0 && p.stride_b % 4 == 0 && al16(a) && al16(b) && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
                p.batch < 65536 && p.m * p.n * p.batch >= 64 * 64 * 16 && f32_mfma_enabled()) {

@@ -26,6 +26,23 @@ __device__ __forceinline__ float gemm_epilogue16(int op, float x) {
     }
 }
 
+// ... of N values: one branch for all of them
+template <int N> __device__ __forceinline__ void gemm_epilogue16_all(int op, float (&x)[N]) {
+#define AXHIP_EPILOGUE_CASE(OP)                                                   \
+    case OP:                                                                      \
+        _Pragma("unroll") for (int e = 0; e < N; ++e) x[e] = gemm_epilogue16(OP, x[e]); \
+        break;
+    switch (op) {
+        AXHIP_EPILOGUE_CASE(AXHIP_OP_RELU)
+        AXHIP_EPILOGUE_CASE(AXHIP_OP_GELU)
+        AXHIP_EPILOGUE_CASE(AXHIP_OP_SILU)
+        AXHIP_EPILOGUE_CASE(AXHIP_OP_SIGMOID)
+        AXHIP_EPILOGUE_CASE(AXHIP_OP_TANH)
+    default: break;
+    }
+#undef AXHIP_EPILOGUE_CASE
+}
+
 // x W^T with at most 8 rows of x (a decoding step: one token, or a handful, against a weight matrix), both operands
 // along k.  The product is bound by reading W once, and a tiling by output tiles would give the chip N / 128
 // work-groups.  Here a wavefront owns R rows of W (R = 1, 2 or 4: enough wavefronts for every SIMD) and walks k with

@@ -1,0 +1,17 @@
+// x W^T: see gemm_tile_kernel.hpp.
+#include "gemm_tile_kernel.hpp"
+
+namespace axhip {
+template <bool BF16> static int launch_nt(const TileArgs &g, int shape, bool aligned, int batch, hipStream_t s) {
+    if (!aligned) return launch_tile_kernel<BF16, false, false, 4, 2, 2, 2, 64, 2>(g, batch, s);
+    switch (shape) {
+    case TILE_256x128: return launch_tile_kernel<BF16, false, true, 8, 2, 2, 2, 64, 3>(g, batch, s);
+    case TILE_192x128: return launch_tile_kernel<BF16, false, true, 6, 2, 2, 2, 64, 3>(g, batch, s);
+    case TILE_128x128: return launch_tile_kernel<BF16, false, true, 4, 2, 2, 2, 64, 4>(g, batch, s);
+    default: return launch_tile_kernel<BF16, false, true, 4, 1, 2, 4, 128, 3>(g, batch, s);
+    }
+}
+int launch_tile_nt(const TileArgs &g, bool bf16, int shape, bool aligned, int batch, hipStream_t s) {
+    return bf16 ? launch_nt<true>(g, shape, aligned, batch, s) : launch_nt<false>(g, shape, aligned, batch, s);
+}
+} // namespace axhip

@@ -248,3 +248,28 @@ def test_seeded_random_shapes_match_fp64(dt):
         tol = 1e-4 * (1 + np.abs(want)) if dt == F32 else 2e-2 + 2.0**-8 * np.abs(want)
         assert got.shape == (batch, M, N)
         assert np.all(np.abs(got - want) <= tol), (case, M, N, K, batch, shared_w, epi, float(np.max(np.abs(got - want))))
+
+
+@pytest.mark.parametrize("dt", [BF16, F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", [
+    (1, 9, 8, 1), (17, 33, 65, 3), (33, 64, 71, 1), (16, 63, 64, 2), (65, 72, 200, 1), (40, 2056, 1032, 1), (129, 1000, 511, 1),  # few rows or few tiles
+    (300, 2104, 200, 2), (385, 5128, 264, 1), (1025, 3848, 136, 1), (1537, 5000, 72, 1),  # 64 .. 256 x 128 tiles, k not whole k-tiles
+    (1500, 2001, 203, 1), (1100, 1999, 1001, 1)])  # 128 x 128 tiles through registers: rows off the 16-byte grid
+def test_half_products_at_the_edges_of_tiles(dt, nn, M, N, K, batch):
+    """x W^T and a b of every 16-bit kernel: one element more and fewer than tiles, pieces of k and 16-byte vectors,
+    rows shorter than a tile (n of 9 and 63), bias + residual + activation.  Against float64 of the same 16-bit inputs:
+    the result is rounded once (half an ulp: 2^-8 of it at most with bf16's 8 significant bits, 2^-11 with f16's 11), the sum is fp32 (K ulps of the sum of magnitudes at most)."""
+    g = axo.PCG64(3 * M + 5 * N + K)
+    x = axo.to_bits(g.normal((batch, M, K)), dt)
+    W = axo.to_bits(g.normal((batch, K, N) if nn else (batch, N, K)) / np.sqrt(K), dt)
+    bias, res = axo.to_bits(g.normal((N,)) * 0.1, dt), axo.to_bits(g.normal((batch, M, N)), dt)
+    got = axo.to_f32(gh.gemm(x, W, dt, trans_b=not nn, bias=bias, residual=res, epilogue="relu"), dt).astype(np.float64)
+    x64, w64 = axo.to_f32(x, dt).astype(np.float64), axo.to_f32(W, dt).astype(np.float64)
+    w64 = w64 if nn else np.swapaxes(w64, -1, -2)
+    b64, r64 = axo.to_f32(bias, dt).astype(np.float64), axo.to_f32(res, dt).astype(np.float64)
+    want = np.maximum(x64 @ w64 + b64 + r64, 0.0)
+    magnitude = np.abs(x64) @ np.abs(w64) + np.abs(b64) + np.abs(r64)
+    tol = (2.0**-8 if dt == BF16 else 2.0**-11) * np.abs(want) + (K + 2) * 2.0**-24 * magnitude + (0.0 if dt == BF16 else 2.0**-25)
+    assert got.shape == want.shape
+    assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
