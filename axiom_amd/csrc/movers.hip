@@ -793,58 +793,108 @@ __global__ __launch_bounds__(256) void argreduce_merge_kernel(const float *part_
 }
 
 // ------------------------------------------------ reductions along an inner axis
-// Sum / max / min along the middle extent of a contiguous (outer, axis, inner) view, inner > 1: the layout of
-// argreduce_strided_vec_kernel (a thread owns the V inner positions of one 16-byte vector, TX threads side by side,
-// the TY = 256 / TX thread rows of a work-group share the axis and merge through LDS); fp32 accumulation, the result
-// scaled (mean) and rounded to the output type.
+// Sum / max / min along the middle extent of a contiguous (outer, axis, inner) view, inner >= V: a thread owns the V
+// inner positions of one 16-byte vector, TX threads lie side by side and the TY = THREADS / TX thread rows of a
+// work-group share the axis (shuffles between the lanes of a wavefront that share a column, LDS between wavefronts);
+// fp32 accumulation, the result scaled (mean) and rounded to the output type.  Rows need no alignment: the loads are
+// unaligned ones, and the last vector of a row that is no whole number of them is moved left to end with the row (the
+// columns it shares with its neighbour are worked out twice, the same way).  With a scalar walk per result such rows took
+// 85 us for the sum over axis 1 of f16 [345, 256, 52], which this reads in 5.
+// FLAT: a thread per vector walks a short axis alone, nothing to merge.
 template <int RED> __device__ __forceinline__ float red_identity() { return RED == AXHIP_RED_MAX ? -INFINITY : RED == AXHIP_RED_MIN ? INFINITY : RED == AXHIP_RED_PROD ? 1.0f : 0.0f; }
 template <int RED> __device__ __forceinline__ float red_combine(float a, float b) { return RED == AXHIP_RED_MAX ? fmaxf(a, b) : RED == AXHIP_RED_MIN ? fminf(a, b) : RED == AXHIP_RED_PROD ? a * b : a + b; }
 
-template <int RED, int DT, int TX>
-__global__ __launch_bounds__(256) void reduce_strided_vec_kernel(const void *src, int64_t outer, int64_t axis, int64_t inner, float scale, void *dst, int dst_dt) {
-    constexpr int TY = 256 / TX, U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8;
-    __shared__ float sv[TY == 1 ? 1 : TY][TY == 1 ? 1 : TX][V + 1];
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    const int64_t ivecs = inner / V, groups = (ivecs + TX - 1) / TX, total = outer * groups;
-    const int n = static_cast<int>(axis);
-    for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
-        const int64_t o = g / groups, iv = (g - o * groups) * TX + tx;
-        const bool there = iv < ivecs;
-        const uint4_t *first = reinterpret_cast<const uint4_t *>(src) + o * axis * ivecs + iv;
+// All-reduce over the lanes of a wavefront that share lane % TX: register swaps between half wavefronts and rows of 16
+// lanes, rotations within a row (a shuffle per step and value through LDS took as long as a short axis' loads).
+template <int V, typename F> __device__ __forceinline__ void across_lanes(float (&x)[V], int TX, F combine) {
+    typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
+    auto halves = [&](auto swap) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const pair_t r = swap(__float_as_uint(x[e]));
+            x[e] = combine(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        }
+    };
+    if (TX <= 32) halves([](uint32_t v) { return __builtin_bit_cast(pair_t, __builtin_amdgcn_permlane32_swap(v, v, false, false)); });
+    if (TX <= 16) halves([](uint32_t v) { return __builtin_bit_cast(pair_t, __builtin_amdgcn_permlane16_swap(v, v, false, false)); });
+#define AXHIP_ROW_ROR(N)                                                                                                                   \
+    if (TX <= N) {                                                                                                                         \
+        _Pragma("unroll") for (int e = 0; e < V; ++e)                                                                                      \
+            x[e] = combine(x[e], __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x[e]), 0x120 + N, 0xF, 0xF, false)));      \
+    }
+    AXHIP_ROW_ROR(8)
+    AXHIP_ROW_ROR(4)
+    AXHIP_ROW_ROR(2)
+    AXHIP_ROW_ROR(1)
+#undef AXHIP_ROW_ROR
+}
+// work-groups that a launch of `total` takes where 2^share neighbours go to one XCD
+__host__ __device__ __forceinline__ int64_t round_up8(int64_t total, int share) { return share == 0 ? total : (total + (8 << share) - 1) & ~static_cast<int64_t>((8 << share) - 1); }
+__device__ __forceinline__ uint4_t axis_load(const char *at) { return reinterpret_cast<const uint4_unaligned_t *>(at)->v; }
+
+template <int RED, int DT, int THREADS, bool FLAT>
+__global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int dst_dt, float scale, int tx_log2) {
+    constexpr int U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V, NW = THREADS / WAVE;
+    __shared__ float red[FLAT ? 1 : NW][FLAT ? 1 : WAVE][V + 1];
+    const int TX = 1 << tx_log2, TY = THREADS >> tx_log2;
+    const int tid = threadIdx.x, tx = tid & (TX - 1), ty = tid >> tx_log2;
+    const int64_t groups = ((inner + V - 1) / V + TX - 1) >> tx_log2, total = outer * groups, pitch = inner * ES, step = TY * pitch;
+    // (groups narrower than a cache line that share one run on the same XCD: work-group b lands on XCD b % 8)
+    const int share = tx_log2 < 3 ? 3 - tx_log2 : 0; // log2 of the groups per line
+    const int64_t last = round_up8(total, share);
+    for (int64_t b = blockIdx.x; b < last; b += gridDim.x) {
+        const int64_t g = (((b >> (3 + share)) * 8 + (b & 7)) << share) + ((b >> 3) & ((1 << share) - 1));
+        if (g >= total) continue; // (whole work-groups)
+        const int64_t o = g / groups, col0 = ((g - o * groups) << tx_log2) * V;
+        const bool there = col0 + tx * V < inner;
+        const int64_t col = there && col0 + tx * V < inner - V ? col0 + tx * V : inner - V;
+        const char *first = static_cast<const char *>(src) + o * n * pitch + col * ES, *at = first + ty * pitch;
         float acc[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) acc[e] = red_identity<RED>();
         if (there)
-            for (int k = ty; k < n; k += TY * U) {
+            for (int k = ty; k < n; k += TY * U, at += U * step) {
                 uint4_t raw[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) raw[u] = first[static_cast<int64_t>(min(k + u * TY, n - 1)) * ivecs];
+                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? at + u * step : first);
+                __builtin_amdgcn_sched_barrier(0); // (all U loads before the first wait)
+                // (past the axis: row 0 again, which changes no maximum or minimum, and adds zeros to a sum -- no branch, into
+                // which the compiler would move the loads)
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (k + u * TY < n) {
-                        float v[V];
-                        arg_unpack<DT>(raw[u], v);
+                for (int u = 0; u < U; ++u) {
+                    if (RED == AXHIP_RED_SUM) raw[u] = k + u * TY < n ? raw[u] : uint4_t{0, 0, 0, 0};
+                    float v[V];
+                    arg_unpack<DT>(raw[u], v);
 #pragma unroll
-                        for (int e = 0; e < V; ++e) acc[e] = red_combine<RED>(acc[e], v[e]);
-                    }
+                    for (int e = 0; e < V; ++e) acc[e] = red_combine<RED>(acc[e], v[e]);
+                }
             }
-        if constexpr (TY == 1) { // a thread walked the whole (short) axis: nothing to merge, one vector store
+        if constexpr (FLAT) { // one vector store, or element stores where the row of results is off the 16-byte grid
             if (there) {
 #pragma unroll
                 for (int e = 0; e < V; ++e) acc[e] *= scale;
-                store_vec<V>(dst, dst_dt, o * inner + iv * V, acc);
+                if (((inner | col) & (V - 1)) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+                    store_vec<V>(dst, dst_dt, o * inner + col, acc);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < V; ++e) store_any(dst, dst_dt, o * inner + col + e, acc[e]);
+                }
             }
         } else {
+            across_lanes(acc, TX, [](float p, float q) { return red_combine<RED>(p, q); });
             __syncthreads(); // the previous group's partials have been read
+            if (tid % WAVE < TX) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) sv[ty][tx][e] = acc[e];
+                for (int e = 0; e < V; ++e) red[tid / WAVE][tid % WAVE][e] = acc[e];
+            }
             __syncthreads();
-            if (there)
-                for (int e = ty; e < V; e += TY) {
-                    float r = sv[0][tx][e];
-                    for (int y = 1; y < TY; ++y) r = red_combine<RED>(r, sv[y][tx][e]);
-                    store_any(dst, dst_dt, o * inner + iv * V + e, r * scale);
-                }
+            for (int x = tid; x < TX * V; x += THREADS) { // (TX <= WAVE)
+                const int c = x / V, e = x % V;
+                float r = red[0][c][e];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) r = red_combine<RED>(r, red[w][c][e]);
+                if (col0 + c * V < inner) store_any(dst, dst_dt, o * inner + min(col0 + c * V, inner - V) + e, r * scale);
+            }
         }
     }
 }
@@ -874,8 +924,8 @@ __global__ __launch_bounds__(256) void reduce_strided_kernel(const void *src, in
 
 namespace axhip {
 // ----------------------------------------------- softmax along an inner axis
-// softmax / log-softmax along the middle extent of a contiguous (outer, axis, inner) view, inner > 1, in the layout of
-// reduce_strided_vec_kernel.  One sweep gathers a running maximum and the sum of 2^(x log2(e) - maximum) per inner
+// softmax / log-softmax along the middle extent of a contiguous (outer, axis, inner) view, inner >= V, in the layout of
+// reduce_axis_kernel (any alignment, the last vector of a row moved left to end with it).  One sweep gathers a running maximum and the sum of 2^(x log2(e) - maximum) per inner
 // position (rescaled once per four elements), the thread rows merge their pairs through LDS, a second sweep over the
 // same elements writes the result: two reads of the input (the second mostly from the caches) and one write.
 // HOLD > 0 (with TX = 256, a thread per vector walking the axis alone): the axis has at most HOLD elements and the thread
@@ -887,12 +937,14 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
     constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
     __shared__ float sm[TY][TX][V + 1], sl[TY][TX][V + 1];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    const int64_t ivecs = inner / V, groups = (ivecs + TX - 1) / TX, total = outer * groups;
+    constexpr int ES = 16 / V;
+    const int64_t groups = ((inner + V - 1) / V + TX - 1) / TX, total = outer * groups, pitch = inner * ES;
     const int n = static_cast<int>(axis);
     for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
-        const int64_t o = g / groups, iv = (g - o * groups) * TX + tx;
-        const bool there = iv < ivecs;
-        const uint4_t *first = reinterpret_cast<const uint4_t *>(src) + o * axis * ivecs + iv;
+        const int64_t o = g / groups, at = ((g - o * groups) * TX + tx) * V, col = at < inner - V ? at : inner - V;
+        const bool there = at < inner;
+        const char *first = static_cast<const char *>(src) + o * axis * pitch + col * ES;
+        const int64_t step = TY * pitch;
         float m[V], l[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) {
@@ -903,7 +955,7 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
         if constexpr (HOLD > 0) {
             if (there) {
 #pragma unroll
-                for (int k = 0; k < HOLD; ++k) keep[k] = first[static_cast<int64_t>(min(k, n - 1)) * ivecs];
+                for (int k = 0; k < HOLD; ++k) keep[k] = axis_load(first + min(k, n - 1) * pitch);
             }
         }
         auto gather = [&](int k, const uint4_t (&raw)[U]) { // running maximum and rescaled sum over U axis elements
@@ -934,10 +986,11 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                         gather(k, raw);
                     }
             } else {
-                for (int k = ty; k < n; k += TY * U) {
+                const char *from = first + ty * pitch;
+                for (int k = ty; k < n; k += TY * U, from += U * step) {
                     uint4_t raw[U];
 #pragma unroll
-                    for (int u = 0; u < U; ++u) raw[u] = first[static_cast<int64_t>(min(k + u * TY, n - 1)) * ivecs];
+                    for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
                     gather(k, raw);
                 }
             }
@@ -968,7 +1021,7 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                         arg_unpack<DT>(raw[u], v);
 #pragma unroll
                         for (int e = 0; e < V; ++e) v[e] = LOG ? (v[e] * LOG2E - shift[e]) * LN2 : __builtin_amdgcn_exp2f(v[e] * LOG2E - shift[e]) * inv[e];
-                        store_vec<V>(dst, DT, (o * axis + k + u * TY) * inner + iv * V, v);
+                        store_vec<V, true>(dst, DT, (o * axis + k + u * TY) * inner + col, v);
                     }
         };
         if (there) {
@@ -980,10 +1033,11 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                         emit(k, raw);
                     }
             } else {
-                for (int k = ty; k < n; k += TY * U) {
+                const char *from = first + ty * pitch;
+                for (int k = ty; k < n; k += TY * U, from += U * step) {
                     uint4_t raw[U];
 #pragma unroll
-                    for (int u = 0; u < U; ++u) raw[u] = first[static_cast<int64_t>(min(k + u * TY, n - 1)) * ivecs];
+                    for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
                     emit(k, raw);
                 }
             }
@@ -991,54 +1045,52 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
     }
 }
 
-// A long axis read ONCE: a 1024-thread block holds an [axis, TX vectors] tile of the input in registers, as the raw
-// 16-byte vectors it was loaded as -- thread (ty, tx) the rows ty, ty + TY, ... (RPT of them, TY = 1024 / TX) of
-// vector column tx, so TX neighbouring lanes read TX * 16 consecutive bytes of a row --, works out the columns'
-// maxima and sums across its threads (shuffles between the lanes of a wave that share a column, LDS between the
-// waves) and writes the results from the same registers.  TX = 16, 8 or 4 for axes of up to 1024, 2048 or 4096
-// elements (16 rows per thread at most: 64 registers of raw words).  With TX = 4 a row's 64 bytes are half a cache
-// line: the two blocks that share the lines run on the same XCD (block b lands on XCD b % 8), so the second one finds
-// them in that L2.
-template <bool LOG, int DT, int RPT>
-__global__ __launch_bounds__(1024) void softmax_axis_tile_kernel(const void *src, int64_t outer, int64_t axis, int64_t inner, int tx_log2, void *dst) {
-    constexpr int V = DT == AXHIP_DTYPE_F32 ? 4 : 8;
+// An axis read ONCE: a block holds an [axis, TX vectors] tile of the input in registers, as the raw 16-byte vectors it
+// was loaded as -- thread (ty, tx) the rows ty, ty + TY, ... (RPT of them, TY = THREADS / TX) of vector column tx, so TX
+// neighbouring lanes read TX * 16 consecutive bytes of a row --, works out the columns' maxima and sums across its
+// threads (shuffles between the lanes of a wave that share a column, LDS between the waves) and writes the results from
+// the same registers.  At most 16 rows per thread (64 registers of raw words).  Where TX is below 8 a row's piece is less
+// than a cache line: the blocks that share the lines run on the same XCD (block b lands on XCD b % 8), so the second one
+// finds them in that L2.
+template <bool LOG, int DT, int RPT, int THREADS>
+__global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int tx_log2) {
+    constexpr int V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V, NW = THREADS / WAVE;
     constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
-    __shared__ float red[16][16][V + 1];
-    const int TX = 1 << tx_log2, TY = 1024 >> tx_log2;
+    __shared__ float red[NW][WAVE][V + 1];
+    const int TX = 1 << tx_log2, TY = THREADS >> tx_log2;
     const int tid = threadIdx.x, tx = tid & (TX - 1), ty = tid >> tx_log2, wave = tid / WAVE;
-    const int64_t ivecs = inner / V, ctiles = (ivecs + TX - 1) / TX, tiles = outer * ctiles;
-    const int share = TX >= 8 ? 1 : 8 / TX; // blocks per cache line of a row
-    const int n = static_cast<int>(axis);
-    const int64_t slot = blockIdx.x / 8, xcd = blockIdx.x % 8;
-    const int64_t tile = ((slot / share) * 8 + xcd) * share + slot % share;
+    const int64_t ctiles = ((inner + V - 1) / V + TX - 1) >> tx_log2, tiles = outer * ctiles, pitch = inner * ES;
+    const int share = tx_log2 < 3 ? 3 - tx_log2 : 0; // log2 of the blocks per cache line of a row
+    const uint32_t slot = blockIdx.x / 8, xcd = blockIdx.x % 8;
+    const int64_t tile = (static_cast<int64_t>((slot >> share) * 8 + xcd) << share) + (slot & ((1 << share) - 1));
     if (tile >= tiles) return; // (whole block)
-    const int64_t o = tile / ctiles, iv = (tile - o * ctiles) * TX + tx;
-    const bool there = iv < ivecs;
-    const uint4_t *first = reinterpret_cast<const uint4_t *>(src) + o * axis * ivecs + (there ? iv : 0);
+    const int64_t o = tile / ctiles, at = (((tile - o * ctiles) << tx_log2) + tx) * V, col = at < inner - V ? at : inner - V;
+    const bool there = at < inner;
+    const char *first = static_cast<const char *>(src) + o * n * pitch + col * ES;
     uint4_t raw[RPT];
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) raw[r] = first[static_cast<int64_t>(min(ty + r * TY, n - 1)) * ivecs];
-    // column statistic over the block: lanes of a wave that share tx, then the 16 waves
-    auto across = [&](float (&x)[V], bool is_max) {
-        for (int d = TX; d < WAVE; d <<= 1) {
-#pragma unroll
-            for (int e = 0; e < V; ++e) {
-                const float y = __shfl_xor(x[e], d, WAVE);
-                x[e] = is_max ? fmaxf(x[e], y) : x[e] + y;
-            }
-        }
+    for (int r = 0; r < RPT; ++r) raw[r] = axis_load(ty + r * TY < n ? first + ty * pitch + r * (TY * pitch) : first);
+    // column statistic over the block: lanes of a wave that share tx, then the waves -- a thread per value merges them and
+    // hands the result to all (every thread merging its V columns itself is 16 V LDS reads of straight-line code, twice)
+    auto across = [&](float (&x)[V], bool is_max) { // (TX <= WAVE)
+        if (is_max) across_lanes(x, TX, [](float p, float q) { return fmaxf(p, q); });
+        else across_lanes(x, TX, [](float p, float q) { return p + q; });
         __syncthreads(); // the previous statistic has been read
-        if ((tid % WAVE) < TX) {
+        if (tid % WAVE < TX) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) red[wave][tx][e] = x[e];
+            for (int e = 0; e < V; ++e) red[wave][tid % WAVE][e] = x[e];
+        }
+        __syncthreads();
+        for (int q = tid; q < TX * V; q += THREADS) { // (nobody else reads these values: red[0] takes the merged ones)
+            const int c = q / V, e = q % V;
+            float a = red[0][c][e];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) a = is_max ? fmaxf(a, red[w][c][e]) : a + red[w][c][e];
+            red[0][c][e] = a;
         }
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            float a = red[0][tx][e];
-            for (int w = 1; w < 16; ++w) a = is_max ? fmaxf(a, red[w][tx][e]) : a + red[w][tx][e];
-            x[e] = a;
-        }
+        for (int e = 0; e < V; ++e) x[e] = red[0][tx][e];
     };
     float m[V], l[V];
 #pragma unroll
@@ -1081,7 +1133,7 @@ __global__ __launch_bounds__(1024) void softmax_axis_tile_kernel(const void *src
             arg_unpack<DT>(raw[r], v);
 #pragma unroll
             for (int e = 0; e < V; ++e) v[e] = LOG ? (v[e] * LOG2E - shift[e]) * LN2 : __builtin_amdgcn_exp2f(v[e] * LOG2E - shift[e]) * inv[e];
-            store_vec<V>(dst, DT, (o * axis + ty + r * TY) * inner + iv * V, v);
+            store_vec<V, true>(dst, DT, (o * n + ty + r * TY) * inner + col, v);
         }
 }
 
@@ -1108,34 +1160,43 @@ __global__ __launch_bounds__(256) void softmax_strided_kernel(const void *src, i
 int launch_reduce_axis(const void *src, int dtype, int64_t outer, int64_t axis, int64_t inner, int red, float scale, void *dst, int dst_dtype, hipStream_t s) {
     const int es = dtype == AXHIP_DTYPE_F32 ? 4 : 2;
     const bool bytes = dtype == AXHIP_DTYPE_U8 || dst_dtype == AXHIP_DTYPE_U8;
-    if (red != AXHIP_RED_PROD && !bytes && inner % (16 / es) == 0 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) { // (products, truth values: the element-wise kernel)
-        const int64_t ivecs = inner / (16 / es);
+    if (red != AXHIP_RED_PROD && !bytes && inner >= 16 / es) { // (products, truth values, rows shorter than a vector: the element-wise kernel)
+        const int64_t vecs = (inner + 16 / es - 1) / (16 / es);
         // a short axis with plenty of results: a thread per vector walks it alone (no merge through LDS)
-        const bool flat = axis <= 32 && outer * ((ivecs + 255) / 256) >= 1024 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0;
-        // (32-vector column groups from 512 of them on: sum over axis 1 of bf16 [256, 1024, 512] 44.5 -> 38.2 us, 75 -> 88 %
-        // of the HBM peak; AXHIP_REDUCE_AXIS_WIDE_FROM=<n>, read once, moves the threshold)
+        const bool flat = axis <= 32 && outer * ((vecs + 255) / 256) >= 1024;
+        // 32-vector column groups from 512 of them on (sum over axis 1 of bf16 [256, 1024, 512] 44.5 -> 38.2 us, 75 -> 88 %
+        // of the HBM peak against 8-vector ones; AXHIP_REDUCE_AXIS_WIDE_FROM=<n>, read once, moves the threshold), never
+        // wider than the row, and no more thread rows than the axis gives four elements each
         static const int wide_from = [] { const char *e = getenv("AXHIP_REDUCE_AXIS_WIDE_FROM"); return e ? atoi(e) : 512; }();
-        const bool wide = outer * ((ivecs + 31) / 32) >= wide_from;
-        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(outer * (flat ? (ivecs + 255) / 256 : wide ? (ivecs + 31) / 32 : (ivecs + 7) / 8), 256 * 64));
-#define AXHIP_RED_VEC_TX(RED, DT, TX) hipLaunchKernelGGL((reduce_strided_vec_kernel<RED, DT, TX>), dim3(blocks), dim3(256), 0, s, src, outer, axis, inner, scale, dst, dst_dtype)
-#define AXHIP_RED_VEC_DT(RED, DT)                                                                                                          \
+        int tx_log2 = outer * ((vecs + 31) / 32) >= wide_from ? 5 : 3;
+        while (tx_log2 > 3 && ((vecs + (1 << tx_log2) - 1) >> tx_log2 << tx_log2) * 8 > vecs * 9) --tx_log2; // (an eighth of the lanes idle at most)
+        while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= vecs) --tx_log2;
+        while (tx_log2 < 6 && (256 >> tx_log2) * 4 > axis && (int64_t(1) << tx_log2) < vecs) ++tx_log2;
+        if (flat) tx_log2 = 8;
+        auto groups_of = [&](int log2) { return outer * ((vecs + (int64_t(1) << log2) - 1) >> log2); };
+        // fewer work-groups than CUs: larger ones, as far as the axis has elements for them, and narrower ones, as far as
+        // a thread still has more than eight
+        const bool large = !flat && groups_of(tx_log2) <= 256 && axis >= (256 >> tx_log2) * 4;
+        while (large && tx_log2 > 1 && groups_of(tx_log2) <= 128 && axis > (1024 >> tx_log2) * 8) --tx_log2;
+        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(round_up8(groups_of(tx_log2), tx_log2 < 3 ? 3 - tx_log2 : 0), 256 * 64));
+        const int n = static_cast<int>(axis);
+#define AXHIP_RED_AXIS(RED, DT)                                                                                                            \
     do {                                                                                                                                   \
-        if (flat) AXHIP_RED_VEC_TX(RED, DT, 256);                                                                                          \
-        else if (wide) AXHIP_RED_VEC_TX(RED, DT, 32);                                                                                      \
-        else AXHIP_RED_VEC_TX(RED, DT, 8);                                                                                                 \
+        if (flat) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, true>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2);        \
+        else if (large) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 1024, false>), dim3(blocks), dim3(1024), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2); \
+        else hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, false>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2);             \
     } while (0)
 #define AXHIP_RED_VEC(RED)                                                                                                                 \
     do {                                                                                                                                   \
-        if (dtype == AXHIP_DTYPE_F32) AXHIP_RED_VEC_DT(RED, AXHIP_DTYPE_F32);                                                              \
-        else if (dtype == AXHIP_DTYPE_F16) AXHIP_RED_VEC_DT(RED, AXHIP_DTYPE_F16);                                                         \
-        else AXHIP_RED_VEC_DT(RED, AXHIP_DTYPE_BF16);                                                                                      \
+        if (dtype == AXHIP_DTYPE_F32) AXHIP_RED_AXIS(RED, AXHIP_DTYPE_F32);                                                                \
+        else if (dtype == AXHIP_DTYPE_F16) AXHIP_RED_AXIS(RED, AXHIP_DTYPE_F16);                                                           \
+        else AXHIP_RED_AXIS(RED, AXHIP_DTYPE_BF16);                                                                                        \
     } while (0)
         if (red == AXHIP_RED_SUM) AXHIP_RED_VEC(AXHIP_RED_SUM);
         else if (red == AXHIP_RED_MAX) AXHIP_RED_VEC(AXHIP_RED_MAX);
         else AXHIP_RED_VEC(AXHIP_RED_MIN);
 #undef AXHIP_RED_VEC
-#undef AXHIP_RED_VEC_DT
-#undef AXHIP_RED_VEC_TX
+#undef AXHIP_RED_AXIS
     } else {
         const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((outer * inner + 255) / 256, 256 * 32));
         if (red == AXHIP_RED_SUM) hipLaunchKernelGGL(reduce_strided_kernel<AXHIP_RED_SUM>, dim3(blocks), dim3(256), 0, s, src, dtype, outer, axis, inner, scale, dst, dst_dtype);
@@ -1783,26 +1844,37 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
     if (rc) return rc;
     hipStream_t s = resolve_stream(stream);
     const int es = dtype == AXHIP_DTYPE_F32 ? 4 : 2;
-    if (inner % (16 / es) == 0 && ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15u) == 0) {
-        const int64_t ivecs = inner / (16 / es);
-        // a long axis that a block can hold: one read.  Where it pays against the two-sweep kernel (one 1024-thread block per
-        // CU, whose load, arithmetic and store phases do not overlap): fp32 axes of 512 to 2048 elements (126 against 179 us
-        // on [16, 2048, 2048]), 16-bit axes of 1024 to 4096 (274 against 348 us on [64, 2048, 2048]); shorter axes and
-        // fp32 axes of 4096 (64-byte row pieces) stay on the two-sweep kernel
-        const bool tile_pays = dtype == AXHIP_DTYPE_F32 ? axis >= 512 && axis <= 2048 : axis >= 1024 && axis <= 4096;
+    if (inner >= 16 / es) {
+        const int64_t ivecs = (inner + 16 / es - 1) / (16 / es), bytes = outer * axis * inner * es;
+        // An axis that a block can hold is read once.  Up to 512 elements: four rows per thread (256 threads up to 256
+        // elements, so that several blocks share a CU), as wide as that allows; bf16 [64, 256, 2048] 72 -> 40 us, fp32
+        // [256, 128, 1024] 76 -> 58 us against the two-sweep kernel.  Longer axes of large arrays take 1024-thread blocks of
+        // sixteen rows per thread, where they pay (one block per CU, whose load, arithmetic and store phases do not overlap):
+        // fp32 axes of up to 2048 elements (126 against 179 us on [16, 2048, 2048]), 16-bit axes of 1024 to 4096 (274 against
+        // 348 us on [64, 2048, 2048]), TX = 16, 8 or 4 vectors for axes of up to 1024, 2048 or 4096; fp32 axes of more than 2048
+        // only where the two-sweep kernel would leave the chip short of work-groups.  Small arrays, whose two
+        // sweeps are two trips to memory and little else, take four rows per thread whatever the axis: the code of sixteen
+        // takes longer to arrive than the array.
+        const bool small = bytes <= (int64_t(24) << 20);
+        const bool tile_pays = axis <= 512 || (axis <= 4096 && (small || (dtype == AXHIP_DTYPE_F32 ? axis <= 2048 || outer * ((ivecs + 7) / 8) < 512 : axis >= 1024)));
         if (tile_pays && softmax_axis_tile_enabled()) {
-            const int tx_log2 = axis <= 1024 ? 4 : axis <= 2048 ? 3 : 2;
-            const int TXv = 1 << tx_log2, TYv = 1024 >> tx_log2;
+            const bool narrow = axis <= 256;
+            int tx_log2 = axis <= 1024 ? 4 : axis <= 2048 ? 3 : 2;
+            if (small || axis <= 512)
+                for (tx_log2 = narrow ? 4 : 3; tx_log2 > 0 && ((narrow ? 1024 : 4096) >> tx_log2) < axis; --tx_log2) {}
+            while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= ivecs) --tx_log2;
+            const int TXv = 1 << tx_log2, TYv = (narrow ? 256 : 1024) >> tx_log2;
             const int64_t tiles = outer * ((ivecs + TXv - 1) / TXv);
-            const int share = TXv >= 8 ? 1 : 8 / TXv;
-            const int64_t nblocks = (tiles + 8 * share - 1) / (8 * share) * (8 * share);
+            const int64_t nblocks = round_up8(tiles, tx_log2 < 3 ? 3 - tx_log2 : 0);
             if (nblocks < (int64_t(1) << 31)) {
                 const bool few = (axis + TYv - 1) / TYv <= 4; // rows per thread
-#define AXHIP_SMT_R(LOG, DT, R) hipLaunchKernelGGL((softmax_axis_tile_kernel<LOG, DT, R>), dim3(static_cast<unsigned>(nblocks)), dim3(1024), 0, s, src, outer, axis, inner, tx_log2, dst)
+                const int n = static_cast<int>(axis);
+#define AXHIP_SMT_R(LOG, DT, R, T) hipLaunchKernelGGL((softmax_axis_tile_kernel<LOG, DT, R, T>), dim3(static_cast<unsigned>(nblocks)), dim3(T), 0, s, src, dst, outer, inner, n, tx_log2)
 #define AXHIP_SMT_DT(LOG, DT)                                                                                                              \
     do {                                                                                                                                   \
-        if (few) AXHIP_SMT_R(LOG, DT, 4);                                                                                                  \
-        else AXHIP_SMT_R(LOG, DT, 16);                                                                                                     \
+        if (narrow) AXHIP_SMT_R(LOG, DT, 4, 256);                                                                                          \
+        else if (few) AXHIP_SMT_R(LOG, DT, 4, 1024);                                                                                       \
+        else AXHIP_SMT_R(LOG, DT, 16, 1024);                                                                                               \
     } while (0)
 #define AXHIP_SMT(LOG)                                                                                                                     \
     do {                                                                                                                                   \

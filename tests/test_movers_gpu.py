@@ -486,3 +486,31 @@ def test_mover_argument_errors():
     assert L.axhip_pad(None, None, F32, 9, i64([1]), i64([1]), i64([0]), i64([0]), 0.0, None) == capi.ERR_INVALID_ARG
     assert L.axhip_gather_rows(None, F32, 4, 4, None, 2, 1, None, None) == capi.ERR_INVALID_ARG
     assert L.axhip_masked_fill(None, F32, None, None, 1, i64([4]), i64([-1]), i64([1]), 0.0, None) == capi.ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,axis,inner", [(3, 1, 9), (2, 33, 8), (40, 100, 17), (7, 257, 33), (300, 54, 381), (1, 1500, 131), (5, 64, 2049), (600, 3, 2055), (1, 4096, 9), (1, 3301, 2044)])
+def test_axis_reductions_and_softmax_over_rows_off_the_vector_grid(dt, outer, axis, inner):
+    """Rows that are no whole number of 16-byte vectors (and rows of one vector): the last vector of a row is moved left,
+    narrow and wide groups, few groups over a long axis, a short axis walked by one thread.  Max: exact.  Sum: fp32
+    accumulation, `axis` ulps of the sum of magnitudes at most, rounded once.  Softmax: six fp32 roundings (argument,
+    exponential, sum, reciprocal, product) of relative size 2^-23 x (1 + |argument| <= 16) and the sum's, rounded once."""
+    rng = np.random.default_rng(axis + inner)
+    bits = axo.to_bits((rng.normal(size=(outer, axis, inner)) * 2).astype(np.float32), dt)
+    x = axo.to_f32(bits, dt).astype(np.float64)
+    d, half = gh.to_dev(bits), {F32: 0.0, F16: 2.0**-11, BF16: 2.0**-8}[dt]
+    for red, want, acc in (("max", x.max(1), 0.0), ("sum", x.sum(1), axis * 2.0**-24 * np.abs(x).sum(1))):
+        out = gh.empty_dev((outer, inner), dt)
+        gh.sync()
+        capi.check(capi.lib().axhip_reduce_axis(d.data_ptr(), dt, outer, axis, inner, capi.RED[red], out.data_ptr(), dt, None))
+        gh.sync()
+        got = axo.to_f32(gh.to_host(out, gh.np_store_dtype(dt)), dt).reshape(outer, inner)
+        assert np.all(np.abs(got - want) <= acc + (half * np.abs(want) * (1 + 2.0**-10) if red == "sum" else 0.0)), red
+    out = gh.empty_dev((outer, axis, inner), dt)
+    gh.sync()
+    capi.check(capi.lib().axhip_softmax_axis(d.data_ptr(), dt, outer, axis, inner, 0, out.data_ptr(), None))
+    gh.sync()
+    got = axo.to_f32(gh.to_host(out, gh.np_store_dtype(dt)), dt).reshape(outer, axis, inner)
+    want = np.exp(x - x.max(1, keepdims=True))
+    want /= want.sum(1, keepdims=True)
+    assert np.all(np.abs(got - want) <= want * (half + (6 * 17 + axis) * 2.0**-23) + (2.0**-25 if dt == F16 else 1e-37))
