@@ -17,6 +17,9 @@
 //                       softmax in the exp2 domain; fp32 accumulators.
 //   sdpa_mfma_kernel    bf16 / f16, head_dim 32: same arithmetic, K and V tiles
 //                       staged through registers into LDS.
+//   sdpa_direct16_kernel, sdpa_direct_f32_kernel (sdpa_direct.hip)  a few query
+//                       rows against many keys; short fp32 sequences: no LDS
+//                       tiles, K and V from memory into the MFMA operands.
 //   sdpa_generic_kernel any dtype, head_dim <= 256, fp32 FMA arithmetic; used
 //                       for fp32 inputs and for head sizes the MFMA kernels do
 //                       not cover.
@@ -27,7 +30,7 @@
 // single exchange with lane ^ 32, and the exponentiated tile is already laid out
 // as the B operand of the second product O^T += V^T * P^T: no trip through LDS
 // for P.
-#include "common.hpp"
+#include "sdpa.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -37,62 +40,16 @@
 
 namespace axhip {
 
-struct SdpaArgs {
-    const void *q, *k, *v;
-    void *o;
-    const uint8_t *mask;
-    int B, H, Sq, Skv, D;
-    float scale;       // softmax scale
-    float scale_log2e; // scale * log2(e)
-    int causal;
-    int nqb; // query blocks per (batch, head)
-    int dtype;
-    int64_t qs[3], ks[3], vs[3], os[3], ms[2];
-    // key split of sdpa_mfma_kernel (decoding: few query rows, few heads, a long key sequence): `ksplit` work-groups
-    // per (batch, head) take `kchunk` keys each and leave normalised fp32 partial outputs and the base-2 logarithm of
-    // their softmax denominators (reference maximum included) for sdpa_splitk_merge_kernel
-    int ksplit, kchunk;
-    float *opart, *lse;
-};
-
-constexpr float NEG_INF_F = -__builtin_huge_valf();
-
 // ---------------------------------------------------------------- MFMA kernel
 
 constexpr int BM = 128; // query rows per workgroup (4 waves x 32)
 constexpr int BN = 64;  // keys per LDS tile
-// Growth of the running row maximum (log2 domain) that is tolerated before the
-// accumulators are rescaled: exponentials stay below 2^8, far inside fp32/bf16/f16 range.
-constexpr float RESCALE_THRESHOLD = 8.0f;
-
 template <bool BF16>
 __device__ __forceinline__ float16_t mfma_32x32x16(uint4_t a, uint4_t b, float16_t c) {
     if constexpr (BF16)
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
-}
-
-template <bool BF16> __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    if constexpr (BF16) {
-        typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-        typedef float float2_t __attribute__((ext_vector_type(2)));
-        float2_t f = {lo, hi};
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t)); // v_cvt_pk_bf16_f32, RNE
-    } else {
-        return pack_f16x2(lo, hi); // v_cvt_pk_f16_f32, RNE
-    }
-}
-
-// acc + lo + hi of a packed pair, one v_dot2c instruction
-template <bool BF16> __device__ __forceinline__ float add_pair(uint32_t packed, float acc) {
-    if constexpr (BF16) {
-        typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, packed), __builtin_bit_cast(bf16x2_t, 0x3F803F80u), acc, false);
-    } else {
-        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, packed), __builtin_bit_cast(half2_t, 0x3C003C00u), acc, false);
-    }
 }
 
 // LDS transpose read (ds_read_b64_tr_b16).  Within each group of 16 lanes, lane i
@@ -391,36 +348,6 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_mfma_kernel(const S
                              pack2<BF16>(oacc[dt][4 * i4 + 2] * inv, oacc[dt][4 * i4 + 3] * inv)};
                 if (d < dv) *reinterpret_cast<uint2_t *>(orow + d) = w;
             }
-    }
-}
-
-// out = sum_s 2^(lse_s - max lse) O_s / sum_s 2^(lse_s - max lse) over the `ksplit` partial results of a (batch, head,
-// query row); a thread per (row, four dims)
-template <bool BF16>
-__global__ __launch_bounds__(256) void sdpa_splitk_merge_kernel(const SdpaArgs a, int D) {
-    const int64_t quads = D / 4, total = static_cast<int64_t>(a.B) * a.H * a.Sq * quads;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
-        const int64_t row = i / quads; // (batch, head, query row)
-        const int d = static_cast<int>(i - row * quads) * 4;
-        const int64_t bh = row / a.Sq;
-        const int q = static_cast<int>(row - bh * a.Sq);
-        float top = NEG_INF_F;
-        for (int s = 0; s < a.ksplit; ++s) top = fmaxf(top, a.lse[(bh * a.ksplit + s) * a.Sq + q]);
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, den = 0.0f;
-        if (top != NEG_INF_F)
-            for (int s = 0; s < a.ksplit; ++s) {
-                const int64_t slot = (bh * a.ksplit + s) * a.Sq + q;
-                const float w = __builtin_amdgcn_exp2f(a.lse[slot] - top);
-                const float4_t o = *reinterpret_cast<const float4_t *>(a.opart + slot * D + d);
-                acc[0] += w * o[0]; acc[1] += w * o[1]; acc[2] += w * o[2]; acc[3] += w * o[3];
-                den += w;
-            }
-        const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-        if (d < a.D) {
-            uint16_t *orow = static_cast<uint16_t *>(a.o) + (bh / a.H) * a.os[0] + (bh % a.H) * a.os[1] + static_cast<int64_t>(q) * a.os[2];
-            const uint2_t w = {pack2<BF16>(acc[0] * inv, acc[1] * inv), pack2<BF16>(acc[2] * inv, acc[3] * inv)};
-            *reinterpret_cast<uint2_t *>(orow + d) = w;
-        }
     }
 }
 
@@ -1768,6 +1695,39 @@ DecodeSplit decode_split_plan(const AxhipSdpaParams &p, bool has_mask) {
     return d;
 }
 
+// The few-row kernel of sdpa_direct.hip: up to DIRECT_ROWS query rows, no mask.  One work-group per (batch, head), or one
+// per chunk of keys.  `required`: the workspace is asked for as for any decoding step; otherwise the problem ran without
+// one before there was this kernel, and a caller that brings none, or too little, gets the undivided form.
+//
+// Splitting pays where one work-group's keys take longer than the whole read at the rate of the chip plus the second
+// kernel.  Fitted to 17 problems of 6 .. 1024 slices and 161 .. 16384 keys: a work-group takes 12 ns a key of 128 dims
+// (6 ns of 64), the chip reads 5.8 TB/s, merging costs 3.5 us.  20 slices of 1152 keys of 128: 13.6 us undivided, 8.9 in
+// 9; 128 of 16384: 219 and 179; but 240 of 1102 of 64 14.7 and 17.6, 256 of 4096 of 128 90 and 95.  The work-groups of
+// one round: one per CU at 128 dims (204 registers), two at 64; two rounds where the chunks stay long.
+struct DirectPlan { bool on, required; DecodeSplit split; };
+DirectPlan direct_plan(const AxhipSdpaParams &p, bool has_mask) {
+    DirectPlan d{false, false, {0, 0, 0, 0}};
+    const bool half = p.dtype == AXHIP_DTYPE_BF16 || p.dtype == AXHIP_DTYPE_F16;
+    const int64_t slices = static_cast<int64_t>(p.batch) * p.heads;
+    if (!half || has_mask || p.is_causal || p.seq_q <= 0 || p.seq_q > DIRECT_ROWS || p.seq_kv <= 0 || p.head_dim <= 0 || p.head_dim > 128 ||
+        p.head_dim % 8 != 0 || slices <= 0 || slices >= (int64_t(1) << 24) || !sdpa_decode_split)
+        return d;
+    d.on = true;
+    const int D = p.head_dim <= 64 ? 64 : 128;
+    const DecodeSplit before = decode_split_plan(p, has_mask);
+    const double whole = static_cast<double>(slices) * p.seq_kv * p.head_dim * 4 / 5.8e6, key = D == 64 ? 6e-3 : 12e-3; // us
+    int64_t parts = (D == 64 ? 512 : 256) / slices;
+    if (p.seq_kv / std::max<int64_t>(parts, 1) >= 4096) parts *= 2;
+    parts = std::min<int64_t>({parts, p.seq_kv / 128, before.ksplit > 0 ? before.ksplit : 64});
+    if (parts < 2 || std::max(p.seq_kv * key, whole) <= std::max(p.seq_kv * key / static_cast<double>(parts), whole) + 3.5) return d;
+    d.required = before.ksplit > 0;
+    d.split.DD = D;
+    d.split.kchunk = static_cast<int>(((p.seq_kv + parts - 1) / parts + BN - 1) / BN * BN);
+    d.split.ksplit = (p.seq_kv + d.split.kchunk - 1) / d.split.kchunk;
+    d.split.bytes = static_cast<size_t>(slices) * d.split.ksplit * p.seq_q * (D + 1) * sizeof(float);
+    return d;
+}
+
 template <bool BF16, int D> int launch_mfma(const SdpaArgs &a, hipStream_t s) {
     const unsigned grid = static_cast<unsigned>(a.nqb) * static_cast<unsigned>(a.B * a.H);
     constexpr size_t lds = D > 128 ? sdpa_mfma_lds_bytes<D>() : 0;
@@ -1840,7 +1800,8 @@ const char *axhip_sdpa_kernel_name(const AxhipSdpaParams *p) {
 size_t axhip_sdpa_workspace_bytes(const AxhipSdpaParams *params, int has_mask) {
     if (!params || validate(*params) != AXHIP_OK) return 0;
     if (pick_kernel(*params, nullptr, nullptr, nullptr, nullptr) != SdpaKind::MFMA) return 0;
-    return CallScratch::rounded(decode_split_plan(*params, has_mask != 0).bytes);
+    const DirectPlan direct = direct_plan(*params, has_mask != 0);
+    return CallScratch::rounded(direct.on ? direct.split.bytes : decode_split_plan(*params, has_mask != 0).bytes);
 }
 
 int axhip_sdpa_fwd(const void *q, const void *k, const void *v, void *o, const uint8_t *mask,
@@ -1895,7 +1856,12 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         // chip a work-group per slice: the keys are split between work-groups instead (flash decoding), partial
         // results in stream-ordered temporary memory, merged by a second kernel.
         const int64_t slices = static_cast<int64_t>(p.batch) * p.heads;
-        const DecodeSplit ds = decode_split_plan(p, mask != nullptr);
+        const DirectPlan direct = direct_plan(p, mask != nullptr);
+        const DecodeSplit ds = direct.on ? direct.split : decode_split_plan(p, mask != nullptr);
+        if (direct.on && (ds.ksplit == 0 || (!direct.required && (!workspace || workspace_bytes < CallScratch::rounded(ds.bytes))))) {
+            last_schedule = "direct";
+            return launch_sdpa_direct16(a, bf, s);
+        }
         if (ds.ksplit > 0) {
             last_schedule = "decode_split";
             const int DD = ds.DD;
@@ -1910,7 +1876,10 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
             a.lse = a.opart + rows * DD;
             a.nqb = 1;
             const unsigned grid = static_cast<unsigned>(slices * a.ksplit);
-            if (DD == 64) {
+            if (direct.on) {
+                rc = launch_sdpa_direct16(a, bf, s);
+                if (rc) return rc;
+            } else if (DD == 64) {
                 if (bf) hipLaunchKernelGGL((sdpa_mfma_kernel<true, 64, false, true>), dim3(grid), dim3(256), 0, s, a);
                 else hipLaunchKernelGGL((sdpa_mfma_kernel<false, 64, false, true>), dim3(grid), dim3(256), 0, s, a);
             } else {
@@ -1923,10 +1892,7 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
                 if (bf) hipLaunchKernelGGL((sdpa_mfma_kernel<true, 128, false, true>), dim3(grid), dim3(256), lds, s, a);
                 else hipLaunchKernelGGL((sdpa_mfma_kernel<false, 128, false, true>), dim3(grid), dim3(256), lds, s, a);
             }
-            const int64_t items = slices * p.seq_q * (DD / 4);
-            const unsigned mgrid = static_cast<unsigned>(std::min<int64_t>((items + 255) / 256, 4096));
-            if (bf) hipLaunchKernelGGL(sdpa_splitk_merge_kernel<true>, dim3(mgrid), dim3(256), 0, s, a, DD);
-            else hipLaunchKernelGGL(sdpa_splitk_merge_kernel<false>, dim3(mgrid), dim3(256), 0, s, a, DD);
+            launch_sdpa_merge(a, bf, DD, s);
             rc = scratch.release();
             if (rc) return rc;
             AXHIP_CHECK_HIP(hipGetLastError());
@@ -1999,6 +1965,15 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         last_schedule = "mfma_f32";
         // waves per 32-row query block, by how many such blocks there are for the 1024 SIMDs (thresholds from timings
         // of 128 .. 1024 blocks: below 0.75 blocks per SIMD the four-way split wins by up to 2.7x, above 1.5 none is needed)
+        // Up to one 16-row block per CU the kernel without LDS tiles is the faster one (8 heads of 512 rows of 64: 16.3 ->
+        // 10.6 us, causal 16.2 -> 10.4, masked 17.9 -> 14.6; 8 of 333 x 1000 of 128: 51.5 -> 26.2); with 512 blocks its reads
+        // of K and V by every block cost more than the idle CUs did (16 heads of 512: 16.6 and 19.6 us).
+        const int64_t blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * p.batch * p.heads;
+        if (blocks16 <= 256 && p.head_dim > 32 && sdpa_f32_split == 0) {
+            last_schedule = "direct";
+            a.nqb = (p.seq_q + 15) / 16;
+            return launch_sdpa_direct_f32(a, s);
+        }
         const int64_t blocks32 = static_cast<int64_t>((p.seq_q + 31) / 32) * p.batch * p.heads;
         int split = blocks32 >= 1536 ? 1 : blocks32 >= 768 ? 2 : 4;
         if (sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4) split = sdpa_f32_split;

@@ -114,7 +114,9 @@ int axhip_sdpa_fwd(const void *q, const void *k, const void *v, void *o,
  * caller (the role of the reference's caller-owned command buffers,
  * src/backends/metal/metal_common.hpp:53-123: the backend allocates nothing
  * behind the caller's back).  axhip_sdpa_workspace_bytes answers 0 for every
- * problem that needs none; has_mask: whether a mask will be passed. */
+ * problem that needs none; has_mask: whether a mask will be passed.  Steps of
+ * fewer than 8 M key elements (slices x keys x dims) only run faster with it:
+ * without one, or with less, they run undivided and allocate nothing. */
 size_t axhip_sdpa_workspace_bytes(const AxhipSdpaParams *params_host, int has_mask);
 int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o,
                       const uint8_t *mask, const AxhipSdpaParams *params_host,
@@ -124,7 +126,7 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o,
  * the process. */
 const char *axhip_sdpa_kernel_name(const AxhipSdpaParams *params_host);
 /* diagnostic: the schedule the calling thread's last axhip_sdpa_fwd launched ("pingpong", "pipelined8",
- * "pipelined4", "key_split", "decode_split", "register_staged", "mfma_f32", "generic", "empty"); several
+ * "pipelined4", "key_split", "decode_split", "direct", "register_staged", "mfma_f32", "generic", "empty"); several
  * schedules share one kernel name.  AXHIP_SDPA_PINGPONG=0 in the environment (read when the library loads)
  * sends "pingpong" problems to "pipelined8". */
 const char *axhip_sdpa_last_schedule(void);

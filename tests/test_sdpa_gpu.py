@@ -429,3 +429,58 @@ def test_ping_pong_schedule_on_head_split_views_and_a_row_dominated_by_a_late_ke
         want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), False, None)
         err = np.max(np.abs(gotf[b:b + 1, h:h + 1] - want))
         assert err < 2e-2, ((b, h), err)
+
+
+@pytest.mark.parametrize("Sq,Skv", [(1, 1), (1, 31), (3, 33), (8, 256), (1, 257), (5, 1300), (8, 2049)])
+@pytest.mark.parametrize("dt,D", [(BF16, 64), (F16, 128), (BF16, 40), (F16, 72), (BF16, 8)], ids=["bf16-64", "f16-128", "bf16-40", "f16-72", "bf16-8"])
+def test_few_query_rows(dt, D, Sq, Skv):
+    """A decoding step: undivided and with its keys divided by a workspace, on rows of a [batch, position, heads x dim]
+    cache whose further positions (and the output's further columns) are none of its business.  One rounding of the
+    probabilities and one of the result: 2^-8 + 2^-9 of values below 4 in bf16, held to the 2e-2 of this file."""
+    import ctypes as C
+
+    import torch
+
+    from axiom_amd import capi
+
+    lib, B, H = capi.lib(), 2, 3
+    g = axo.PCG64(91 + Sq + Skv)
+    q, k, v = (axo.to_bits(g.normal(s), dt) for s in ((B, Sq, H, D), (B, Skv, H, D), (B, Skv, H, D)))
+    extra = 40
+    cache = [np.full((B, Skv + extra, H, D), axo.to_bits(np.full(1, np.nan, np.float32), dt)[0], k.dtype) for _ in range(2)]
+    cache[0][:, :Skv], cache[1][:, :Skv] = k, v
+    dq, dk, dv = (gh.to_dev(np.ascontiguousarray(t)) for t in (q, *cache))
+    p = capi.SdpaParams()
+    p.dtype, p.batch, p.heads, p.seq_q, p.seq_kv, p.head_dim, p.scale, p.is_causal = dt, B, H, Sq, Skv, D, -1.0, 0
+    p.q_strides[:] = p.o_strides[:] = (Sq * H * D, D, H * D)
+    p.k_strides[:] = p.v_strides[:] = ((Skv + extra) * H * D, D, H * D)
+    wide = [axo.to_f32(t, dt).transpose(0, 2, 1, 3).astype(np.float64) for t in (q, k, v)]
+    want = naive_attention64(*wide, 1 / math.sqrt(D), False, None).transpose(0, 2, 1, 3)
+    need = lib.axhip_sdpa_workspace_bytes(C.byref(p), 0)
+    assert (need > 0) == (Skv >= 1300)
+    for given in sorted({0, max(0, need - 256), need}):
+        o = gh.empty_dev((B * Sq * H * D + 64,), dt)
+        o.fill_(0x5A5A)
+        ws = torch.zeros(max(given, 1), dtype=torch.uint8, device="cuda")
+        gh.sync()
+        capi.check(lib.axhip_sdpa_fwd_ws(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), o.data_ptr(), None, C.byref(p), ws.data_ptr() if given else None, given, None))
+        gh.sync()
+        assert lib.axhip_sdpa_last_schedule() == (b"decode_split" if given == need and need else b"direct")
+        got = gh.to_host(o, gh.np_store_dtype(dt))
+        assert (got[-64:] == 0x5A5A).all()
+        assert np.max(np.abs(axo.to_f32(got[:-64], dt).reshape(want.shape) - want)) < 2e-2
+
+
+@pytest.mark.parametrize("case", [(1, 2, 1, 1, 64, False, None), (1, 2, 17, 33, 64, True, None), (2, 4, 15, 300, 128, False, "mod3"), (1, 8, 200, 129, 36, True, None),
+                                  (1, 3, 33, 1000, 100, False, None), (2, 8, 250, 257, 64, False, "mod3"), (1, 1, 16, 15, 128, True, None)], ids=lambda c: "x".join(str(x) for x in c))
+def test_f32_short_sequences(case):
+    """At most one 16-row block per CU: keys in whole and broken 32-key steps, rows past the end, dims below the size."""
+    from axiom_amd import capi
+
+    B, H, Sq, Skv, D, causal, mk = case
+    q, k, v = inputs(B, H, Sq, Skv, D, F32, seed=5)
+    mask = make_mask(mk, Sq, Skv)
+    got, _ = gh.sdpa(q, k, v, F32, -1.0, causal, mask)
+    assert capi.lib().axhip_sdpa_last_schedule() == b"direct"
+    want = naive_attention64(q, k, v, 1 / math.sqrt(D), causal, mask)
+    assert np.allclose(got, want, rtol=1e-4, atol=1e-4), np.max(np.abs(got - want))
