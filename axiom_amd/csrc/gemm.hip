@@ -7,6 +7,7 @@
 // The other 16-bit kernels are in gemm_tile_*.hip (middle-sized products), gemm_small.hip (few rows or few output
 // tiles) and gemm_skinny.hip (at most eight rows).
 #include "common.hpp"
+#include "gemm_f32.hpp"
 #include "gemm_small.hpp"
 #include "gemm_skinny.hpp"
 
@@ -634,6 +635,66 @@ const HalfKernel &choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
     return *best;
 }
 
+// ---- fp32 products: which kernel
+// The tile of the ring kernel, by rounds of work-groups x tile area (it is bound by the matrix pipe), and that product.
+constexpr int F32_RING_TILES[4][2] = {{128, 128}, {64, 128}, {128, 192}, {64, 64}};
+struct F32Ring { int tile; float area; }; // area: rounds x tile, in tiles of 128 x 128
+F32Ring f32_ring_tile(const AxhipGemmParams &p) {
+    F32Ring best{0, 0.0f};
+    float best_cost = 0.0f;
+    for (int c = 0; c < 4; ++c) {
+        const int tm = F32_RING_TILES[c][0], tn = F32_RING_TILES[c][1];
+        const int64_t tiles = ((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) * p.batch;
+        const float rounds = static_cast<float>((tiles + 255) / 256), area = static_cast<float>(tm * tn) / 16384.0f, cost = rounds * (0.05f + area);
+        if (c == 0 || cost < best_cost) { best_cost = cost; best = {c, rounds * area}; }
+    }
+    return best;
+}
+// both operands along k, whole 16-byte vectors, offsets of 32 bits
+bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
+    return !p.trans_a && p.trans_b && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && p.stride_a % 4 == 0 && p.stride_b % 4 == 0 &&
+           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0 && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
+           p.m * p.n * p.batch >= 64 * 64 * 16 && f32_mfma_enabled();
+}
+// The time of the kernels of gemm_f32.hip in us, as for the 16-bit ones above: start + k (per_k + (per_k_full +
+// per_k_odd) u) r + per_round (r - 1), per_k_odd for rows off the 16-byte grid.  Fitted with the ring kernel's to 220
+// products of m 9 .. 8192, n 64 .. 4096, k 64 .. 4096 (mean error 5 - 8 %); on average the one picked is
+// 2 % slower than the fastest, and 2.3 times as fast as the ring and FMA kernels, which had these products to themselves:
+// 99 x 1024 x 5120 104 -> 18 us, 186 x 640 x 958 35 -> 8, 48 x 384 x 2048 77 -> 6.3.  Large products with both operands
+// along k stay on the ring: 2048^3 157 us against 188.
+struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
+constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
+    {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f},
+    {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f}, {4.59f, 0.00939f, 0.00112f, 3.91f, 0.00138f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}};
+
+// An F32Shape, or -1: the kernel that this product had otherwise (`ring`: the ring kernel, after `repacked` bytes were
+// written and read if there are any; else the FMA kernel).
+int choose_f32_kernel(const AxhipGemmParams &p, bool ring, double repacked) {
+    constexpr int64_t SIDE = int64_t(1) << 30, LD = int64_t(1) << 31;
+    // (below 64 K multiplications the FMA kernel is as fast: 17 x 70 x 33 3.5 us on either)
+    if (p.trans_a || p.k < 32 || p.n < 4 || p.m >= SIDE || p.n >= SIDE || p.k >= SIDE || p.lda >= LD || p.ldb >= LD || p.ldc >= LD ||
+        p.m * p.n * p.batch < 65536 / p.k || !f32_mfma_enabled())
+        return -1;
+    const float k = static_cast<float>(p.k), u = p.k % 4 != 0 || (!p.trans_b && p.n % 4 != 0) ? 1.0f : 0.0f;
+    int best = -1;
+    float best_cost = 0.0f;
+    if (ring) {
+        // (less than fitted: where the two are close, the ring is no slower than before)
+        const float padded = static_cast<float>((p.k + 31) / 32 * 32);
+        best_cost = 0.85f * (3.7f + (0.0718f * padded + 9.4f) * f32_ring_tile(p).area + (repacked > 0.0 ? 4.7f + 2.1e-7f * static_cast<float>(repacked) : 0.0f));
+    }
+    for (int i = 0; i < F32_SHAPES; ++i) {
+        const F32Kernel &h = F32_KERNELS[i];
+        const float full = static_cast<float>(p.batch) * static_cast<float>((p.m + F32_GEOMETRY[i].tm - 1) / F32_GEOMETRY[i].tm) *
+                           static_cast<float>((p.n + F32_GEOMETRY[i].tn - 1) / F32_GEOMETRY[i].tn) * (1.0f / 256.0f);
+        if (full > 65536.0f) continue; // (tiles are counted in 32 bits)
+        const float r = full <= 1.0f ? 1.0f : 0.5f * (std::ceil(full) + full);
+        const float cost = h.start + k * (h.per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
+        if ((best < 0 && !ring) || cost < best_cost) { best_cost = cost; best = i; }
+    }
+    return best;
+}
+
 int launch_big(const GemmArgs &g, bool bf, int batch, hipStream_t s) {
     const int tiles_m = static_cast<int>((g.M + BIG - 1) / BIG), tiles_n = static_cast<int>((g.N + BIG - 1) / BIG);
     const dim3 grid(static_cast<unsigned>(8 * ((tiles_m * tiles_n + 7) / 8)), static_cast<unsigned>(batch));
@@ -649,13 +710,18 @@ int launch_big(const GemmArgs &g, bool bf, int batch, hipStream_t s) {
     return AXHIP_OK;
 }
 
-int launch_half(const AxhipGemmParams &p, const void *a, const void *b, void *c, const HalfKernel &k, bool aligned, bool bf, hipStream_t s) {
+TileArgs tile_args(const AxhipGemmParams &p, const void *a, const void *b, void *c) {
     TileArgs t{};
     t.a = a; t.b = b; t.c = c; t.bias = p.bias; t.residual = p.residual;
     t.sa = p.stride_a; t.sb = p.stride_b; t.sc = p.stride_c;
     t.M = static_cast<int>(p.m); t.N = static_cast<int>(p.n); t.K = static_cast<int>(p.k);
     t.lda = static_cast<int>(p.lda); t.ldb = static_cast<int>(p.ldb); t.ldc = static_cast<int>(p.ldc);
     t.epilogue = p.epilogue_op;
+    return t;
+}
+
+int launch_half(const AxhipGemmParams &p, const void *a, const void *b, void *c, const HalfKernel &k, bool aligned, bool bf, hipStream_t s) {
+    const TileArgs t = tile_args(p, a, b, c);
     const int batch = static_cast<int>(p.batch);
     if (k.kind == HalfKernel::SMALL) return launch_small(t, bf, !p.trans_b, k.shape, k.waves, batch, s);
     return p.trans_b ? launch_tile_nt(t, bf, k.shape, aligned, batch, s) : launch_tile_nn(t, bf, k.shape, aligned, batch, s);
@@ -699,7 +765,10 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const size_t need = repack_bytes(p);
         AXHIP_REQUIRE(workspace_bytes >= need, AXHIP_ERR_WORKSPACE, "axhip_gemm: the workspace holds %zu bytes, the call needs %zu (ask axhip_gemm_workspace_bytes)", workspace_bytes, need);
     }
-    if (rp.on && !scratch_in && !(p.dtype != AXHIP_DTYPE_F32 && takes_half_kernels(p))) {
+    const bool f32 = p.dtype == AXHIP_DTYPE_F32, repack = rp.on && !scratch_in;
+    const double repacked = repack ? 8.0 * static_cast<double>(p.batch) * static_cast<double>((rp.a ? p.m : 0) + (rp.b ? p.n : 0)) * static_cast<double>(p.k) : 0.0;
+    const int f32_shape = f32 ? choose_f32_kernel(p, repack || takes_f32_ring(p, a, b), repacked) : -1;
+    if (repack && f32_shape < 0 && (f32 || !takes_half_kernels(p))) {
         const bool pad_k = rp.kp != p.k;
         const int64_t es = p.dtype == AXHIP_DTYPE_F32 ? 4 : 2, kp = rp.kp;
         AxhipGemmParams q = p;
@@ -773,10 +842,11 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const HalfKernel &k = choose_half_kernel(p, aligned);
         rc = k.kind == HalfKernel::BIG256 ? launch_big(g, bf, static_cast<int>(p.batch), s) : launch_half(p, a, b, c, k, aligned, bf, s);
         if (rc) return rc;
-    } else if (p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
-               p.stride_a % 4 == 0 && p.stride_b % 4 == 0 && al16(a) && al16(b) && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
-               p.batch < 65536 && p.m * p.n * p.batch >= 64 * 64 * 16 && f32_mfma_enabled()) {
-        // fp32 x W^T on the fp32 MFMA; tile shape by rounds of work-groups x tile area (the kernel is bound by the matrix pipe)
+    } else if (f32_shape >= 0) {
+        rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, static_cast<int>(p.batch), s);
+        if (rc) return rc;
+    } else if (f32 && takes_f32_ring(p, a, b)) {
+        // fp32 x W^T on the fp32 MFMA
         auto launch = [&](auto kernel, int tm_rows, int tn_cols, size_t lds_bytes) -> int {
             static std::mutex mu;
             static std::set<const void *> configured;
@@ -792,16 +862,8 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
             hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(256), lds_bytes, s, g, tiles_m, tiles_n);
             return AXHIP_OK;
         };
-        static const int shapes[4][2] = {{128, 128}, {64, 128}, {128, 192}, {64, 64}};
-        int best = 0;
-        double best_cost = 0.0;
-        for (int c = 0; c < 4; ++c) {
-            const int64_t tiles = ((p.m + shapes[c][0] - 1) / shapes[c][0]) * ((p.n + shapes[c][1] - 1) / shapes[c][1]) * p.batch;
-            const double cost = static_cast<double>((tiles + 255) / 256) * (0.05 + shapes[c][0] * shapes[c][1] / 16384.0);
-            if (best_cost == 0.0 || cost < best_cost) { best_cost = cost; best = c; }
-        }
         int rc2;
-        switch (best) {
+        switch (f32_ring_tile(p).tile) {
         case 0: rc2 = launch(gemm_mfma_f32_ring_kernel<128, 128, 3>, 128, 128, 3 * 256 * BIG_ROWB); break;
         case 1: rc2 = launch(gemm_mfma_f32_ring_kernel<64, 128, 3>, 64, 128, 3 * 192 * BIG_ROWB); break;
         case 3: rc2 = launch(gemm_mfma_f32_ring_kernel<64, 64, 3>, 64, 64, 3 * 128 * BIG_ROWB); break;

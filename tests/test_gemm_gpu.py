@@ -273,3 +273,22 @@ def test_half_products_at_the_edges_of_tiles(dt, nn, M, N, K, batch):
     tol = (2.0**-8 if dt == BF16 else 2.0**-11) * np.abs(want) + (K + 2) * 2.0**-24 * magnitude + (0.0 if dt == BF16 else 2.0**-25)
     assert got.shape == want.shape
     assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", [
+    (90, 37, 33, 1), (17, 261, 32, 3), (16, 1041, 95, 1), (65, 50, 1024, 2), (9, 700, 2049, 1),  # 16 rows: pieces of 64 and 32 k, whole and broken
+    (33, 515, 64, 9), (513, 129, 100, 4), (31, 4, 600, 1), (200, 2047, 257, 1),                  # 32 rows; n of one lane's columns
+    (1000, 1030, 70, 1), (385, 67, 130, 32), (1023, 961, 513, 1)])                               # 64 x 64
+def test_f32_products_at_the_edges_of_tiles(nn, M, N, K, batch):
+    """x W^T and a b in fp32 without shared tiles: rows, columns and k that end inside a tile, a lane's columns and a
+    piece, with bias, residual and activation.  Against float64: K + 2 roundings of the sum of magnitudes at most."""
+    g = axo.PCG64(7 * M + 3 * N + K)
+    x, W = g.normal((batch, M, K)).astype(np.float32), (g.normal((batch, K, N) if nn else (batch, N, K)) / np.sqrt(K)).astype(np.float32)
+    bias, res = (g.normal((N,)) * 0.1).astype(np.float32), g.normal((batch, M, N)).astype(np.float32)
+    got = gh.gemm(x, W, F32, trans_b=not nn, bias=bias, residual=res, epilogue="relu").astype(np.float64)
+    x64, w64 = x.astype(np.float64), W.astype(np.float64) if nn else np.swapaxes(W.astype(np.float64), -1, -2)
+    want = np.maximum(x64 @ w64 + bias + res, 0.0)
+    magnitude = np.abs(x64) @ np.abs(w64) + np.abs(bias) + np.abs(res)
+    assert got.shape == want.shape
+    assert np.all(np.abs(got - want) <= (K + 2) * 2.0**-24 * magnitude)
