@@ -108,36 +108,46 @@ struct TransposeArgs {
     int src_dtype, dst_dtype, n_other;
     int64_t nJ, nL, src_stride_l, dst_stride_j; // the source stride of J and the destination stride of L are 1
     int64_t tiles_j, tiles_l;
+    uint32_t blocks, per_xcd; // tiles in all; of each of the eight XCDs, if each is to take neighbouring ones
     int64_t oshape[AXHIP_MAX_DIMS], osrc[AXHIP_MAX_DIMS], odst[AXHIP_MAX_DIMS];
 };
 
-// The same for views that move whole 16-byte vectors on both sides (equal 2- or 4-byte element types; extents, strides
-// and bases multiples of a vector -- or of half a vector on a side, LG / SG = 8: that side moves 8-byte pieces, e.g. the
-// 3000-byte rows of a [.., 1500] 16-bit array): tiles of 16 x 16 vectors -- 128 x 128 16-bit or 64 x 64 32-bit
-// elements, 256-byte runs on the read and on the write side.  A thread reads vectors along J, scatters their elements as 32-bit words into
-// a tile that is stored transposed (16-bit: two neighbouring rows of L packed into one word first), and the tile
-// leaves as 16-byte LDS reads along L.  Tile rows are 256 bytes = 16 chunks; chunk c of row j sits at c ^ (j / V mod 16),
-// which spreads the words of one scatter over all 64 banks and keeps the 16 reads of a row apart.
-template <int ES, int LG, int SG>
+// The same for equal 2- or 4-byte element types, in whole 16-byte vectors on both sides (LG / SG = 16: extents, strides
+// and bases are multiples of a vector; 8: of half a vector, e.g. the 3000-byte rows of a [.., 1500] 16-bit array; ES: of
+// nothing -- vectors are unaligned, the last one of a row is fetched as the 16 bytes that end with it and shifted into
+// place, and leaves in pieces).  Tiles of NV x NV vectors: 128 x 128 16-bit or 64 x 64 32-bit elements with NV = 16,
+// 256-byte runs on the read and on the write side.  A thread reads vectors along J, scatters their elements as 32-bit
+// words into a tile that is stored transposed (16-bit: two neighbouring rows of L packed into one word first), and the
+// tile leaves as 16-byte LDS reads along L.  Chunk c of tile row j sits at c ^ (j / V mod NV), which spreads the words of
+// one scatter over the banks and keeps the reads of a row apart.
+template <int ES, int LG, int SG, int NV>
 __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs a) {
-    constexpr int V = 16 / ES, T = 16 * V; // elements per vector, tile edge
-    // 16 bytes at `at`, of which the elements below `n` exist (whole pieces of LG bytes)
+    constexpr int V = 16 / ES, T = NV * V, PASS = 256 / NV; // elements per vector, tile edge, rows per pass of the work-group
+    // 16 bytes at `at`, of which the elements below `n` exist (whole pieces of LG bytes; LG = ES: of a row of V or more)
     auto load16 = [](const char *at, int64_t n) {
         if constexpr (LG == 16) {
             return n > 0 ? *reinterpret_cast<const uint4_t *>(at) : uint4_t{0, 0, 0, 0};
-        } else {
+        } else if constexpr (LG == 8) {
             const uint2_t lo = n > 0 ? *reinterpret_cast<const uint2_t *>(at) : uint2_t{0, 0};
             const uint2_t hi = n > V / 2 ? *reinterpret_cast<const uint2_t *>(at + 8) : uint2_t{0, 0};
             return uint4_t{lo.x, lo.y, hi.x, hi.y};
+        } else {
+            if (n <= 0) return uint4_t{0, 0, 0, 0};
+            const int drop = n >= V ? 0 : V - static_cast<int>(n);
+            const uint4_t v = vec_load<true>(reinterpret_cast<const uint4_t *>(at - drop * ES));
+            return drop == 0 ? v : __builtin_bit_cast(uint4_t, __builtin_bit_cast(unsigned __int128, v) >> (8 * ES * drop));
         }
     };
-    __shared__ __attribute__((aligned(16))) uint32_t tile[T * 64];
-    int64_t b = blockIdx.x;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[T * NV * 4];
+    const uint32_t t = a.per_xcd ? blockIdx.x % 8 * a.per_xcd + blockIdx.x / 8 : blockIdx.x;
+    if (t >= a.blocks) return;
+    int64_t b = t;
     const int64_t tl = b % a.tiles_l;
     b /= a.tiles_l;
     // (work-groups that run side by side take tiles along a diagonal: with a power of two as row length, tiles of one
-    // tile row or column start a multiple of 2 MiB apart on one of the two sides and would queue on the same channels)
-    const int64_t tj = (b % a.tiles_j + tl) % a.tiles_j;
+    // tile row or column start a multiple of 2 MiB apart on one of the two sides and would queue on the same channels.
+    // Neighbours of one XCD are to share the lines of the rows they write, and keep to a tile row.)
+    const int64_t tj = a.per_xcd ? b % a.tiles_j : (b % a.tiles_j + tl) % a.tiles_j;
     int64_t o = b / a.tiles_j;
     int64_t src_base = 0, dst_base = 0;
     for (int d = a.n_other - 1; d >= 0; --d) {
@@ -146,60 +156,78 @@ __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs 
         src_base += c * a.osrc[d];
         dst_base += c * a.odst[d];
     }
-    const int tid = threadIdx.x, jv = tid % 16, hi = tid / 16;
+    const int tid = threadIdx.x, jv = tid % NV, hi = tid / NV;
     const int64_t j0 = tj * T, l0 = tl * T;
     const char *src = static_cast<const char *>(a.src);
     char *dst = static_cast<char *>(a.dst);
     const int64_t j_left = a.nJ - (j0 + jv * V); // elements of this thread's vectors that exist (whole pieces)
     if constexpr (ES == 2) {
-        // pairs of rows: pair p = rows 2p, 2p + 1 of the tile; four per thread
-        uint4_t r0[4], r1[4];
+        // pairs of rows: pair p = rows 2p, 2p + 1 of the tile
+        constexpr int N = T / 2 / PASS;
+        uint4_t r0[N], r1[N];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int64_t l = l0 + 2 * (hi + 16 * it);
+        for (int it = 0; it < N; ++it) {
+            const int64_t l = l0 + 2 * (hi + PASS * it);
             const int64_t at = (src_base + l * a.src_stride_l + j0 + jv * V) * ES;
             r0[it] = load16(src + at, l < a.nL ? j_left : 0);
             r1[it] = load16(src + at + a.src_stride_l * ES, l + 1 < a.nL ? j_left : 0);
         }
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int p = hi + 16 * it; // the pair's word: chunk p / 4, word p % 4 of row j
+        for (int it = 0; it < N; ++it) {
+            const int p = hi + PASS * it; // the pair's word: chunk p / 4, word p % 4 of row j
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 const uint32_t w0 = r0[it][e / 2], w1 = r1[it][e / 2];
                 const uint32_t word = e % 2 ? __builtin_amdgcn_perm(w1, w0, 0x07060302u) : __builtin_amdgcn_perm(w1, w0, 0x05040100u);
-                tile[(jv * V + e) * 64 + (((p / 4) ^ jv) * 4) + p % 4] = word;
+                tile[(jv * V + e) * NV * 4 + (((p / 4) ^ jv) * 4) + p % 4] = word;
             }
         }
     } else {
-        uint4_t r[4];
+        constexpr int N = T / PASS;
+        uint4_t r[N];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int64_t l = l0 + hi + 16 * it;
+        for (int it = 0; it < N; ++it) {
+            const int64_t l = l0 + hi + PASS * it;
             r[it] = load16(src + (src_base + l * a.src_stride_l + j0 + jv * V) * ES, l < a.nL ? j_left : 0);
         }
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int l = hi + 16 * it;
+        for (int it = 0; it < N; ++it) {
+            const int l = hi + PASS * it;
 #pragma unroll
-            for (int e = 0; e < V; ++e) tile[(jv * V + e) * 64 + (((l / 4) ^ jv) * 4) + l % 4] = r[it][e];
+            for (int e = 0; e < V; ++e) tile[(jv * V + e) * NV * 4 + (((l / 4) ^ jv) * 4) + l % 4] = r[it][e];
         }
     }
     __syncthreads();
-    // rows j of the transposed tile, 16 vectors along L each
-    const int lv = tid % 16;
+    // rows j of the transposed tile, NV vectors along L each
+    const int lv = tid % NV;
     const int64_t l_left = a.nL - (l0 + lv * V);
 #pragma unroll
-    for (int it = 0; it < T / 16; ++it) {
-        const int j = hi + 16 * it;
-        const uint4_t t = *reinterpret_cast<const uint4_t *>(&tile[j * 64 + ((lv ^ ((j / V) & 15)) * 4)]);
+    for (int it = 0; it < T / PASS; ++it) {
+        const int j = hi + PASS * it;
+        uint4_t v = *reinterpret_cast<const uint4_t *>(&tile[j * NV * 4 + ((lv ^ ((j / V) & (NV - 1))) * 4)]);
         char *to = dst + (dst_base + (j0 + j) * a.dst_stride_j + l0 + lv * V) * ES;
         if (j0 + j >= a.nJ) continue;
         if constexpr (SG == 16) {
-            if (l_left > 0) *reinterpret_cast<uint4_t *>(to) = t;
-        } else {
-            if (l_left > 0) *reinterpret_cast<uint2_t *>(to) = uint2_t{t.x, t.y};
-            if (l_left > V / 2) *reinterpret_cast<uint2_t *>(to + 8) = uint2_t{t.z, t.w};
+            if (l_left > 0) *reinterpret_cast<uint4_t *>(to) = v;
+        } else if constexpr (SG == 8) {
+            if (l_left > 0) *reinterpret_cast<uint2_t *>(to) = uint2_t{v.x, v.y};
+            if (l_left > V / 2) *reinterpret_cast<uint2_t *>(to + 8) = uint2_t{v.z, v.w};
+        } else if (l_left >= V) {
+            vec_store<true>(reinterpret_cast<uint4_t *>(to), v);
+        } else if (l_left > 0) { // 8, 4 and 2 bytes
+            const int bytes = static_cast<int>(l_left) * ES;
+            if (bytes & 8) {
+                vec_store<true>(reinterpret_cast<uint2_t *>(to), uint2_t{v.x, v.y});
+                v.x = v.z;
+                v.y = v.w;
+                to += 8;
+            }
+            if (bytes & 4) {
+                reinterpret_cast<uint32_unaligned_t *>(to)->v = v.x;
+                v.x = v.y;
+                to += 4;
+            }
+            if (ES == 2 && (bytes & 2)) *reinterpret_cast<uint16_t *>(to) = static_cast<uint16_t>(v.x);
         }
     }
 }
@@ -1367,24 +1395,43 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
             return 0;
         };
         const int lg = side(t.nJ, t.src_stride_l, t.osrc, src), sg = side(t.nL, t.dst_stride_j, t.odst, dst);
-        const bool whole = src_dtype == dst_dtype && src_dtype != AXHIP_DTYPE_U8 && lg > 0 && sg > 0;
+        const bool whole = src_dtype == dst_dtype && src_dtype != AXHIP_DTYPE_U8;
         static const bool vec_tiles = [] { const char *e = getenv("AXHIP_TRANSPOSE_VEC"); return !(e && e[0] == '0'); }();
         if (whole && vec_tiles) {
-            const int64_t edge = 16 * (16 / es);
+            // Rows of the output that start inside a 128-byte line make neighbouring tiles write parts of the same lines:
+            // such tiles go to one XCD, whose L2 puts the parts together, and are smaller, so that it still holds them
+            // (bf16 [32, 1500, 1280] 70.8 us in the other order, 60.9 with large tiles, 59.3 with small ones; fp32 130,
+            // 113, 98).  Rows of whole lines take large tiles along a diagonal over all XCDs (bf16 [8, 4096, 4096] 96 us
+            // against 117).  Extents of one large tile or less: small ones waste fewer lanes (bf16 [2000, 64, 130] 25 ->
+            // 17 us), except that fp32's 32 elements are too few (fp32 [5000, 33, 65] 29 us against 40).
+            const bool lines = t.dst_stride_j * es % 128 == 0;
+            const int64_t narrow = std::min(t.nJ, t.nL);
+            const bool together = !lines || (es == 2 && narrow <= 128);
+            const int nv = es == 2 ? (together ? 8 : 16) : (!lines && narrow > 64 ? 8 : 16);
+            const int64_t edge = nv * (16 / es);
             t.tiles_j = (t.nJ + edge - 1) / edge; t.tiles_l = (t.nL + edge - 1) / edge;
             blocks = blocks / (((t.nJ + 63) / 64) * ((t.nL + 63) / 64)) * t.tiles_j * t.tiles_l;
-            AXHIP_REQUIRE(blocks < (int64_t(1) << 31), AXHIP_ERR_UNSUPPORTED, "axhip_strided_copy: view too large");
-            const dim3 grid(static_cast<unsigned>(blocks));
+            AXHIP_REQUIRE(blocks < (int64_t(1) << 31) - 8, AXHIP_ERR_UNSUPPORTED, "axhip_strided_copy: view too large");
+            t.blocks = static_cast<uint32_t>(blocks);
+            t.per_xcd = together ? (t.blocks + 7) / 8 : 0;
+            const dim3 grid(t.per_xcd ? 8 * t.per_xcd : t.blocks);
+#define AXHIP_TRANSPOSE_NV(ES, LG, SG)                                                                                   \
+    do {                                                                                                                 \
+        if (nv == 16) hipLaunchKernelGGL((transpose_vec_kernel<ES, LG, SG, 16>), grid, dim3(256), 0, s, t);              \
+        else hipLaunchKernelGGL((transpose_vec_kernel<ES, LG, SG, 8>), grid, dim3(256), 0, s, t);                        \
+    } while (0)
 #define AXHIP_TRANSPOSE(ES)                                                                                              \
     do {                                                                                                                 \
-        if (lg == 16 && sg == 16) hipLaunchKernelGGL((transpose_vec_kernel<ES, 16, 16>), grid, dim3(256), 0, s, t);      \
-        else if (lg == 16) hipLaunchKernelGGL((transpose_vec_kernel<ES, 16, 8>), grid, dim3(256), 0, s, t);              \
-        else if (sg == 16) hipLaunchKernelGGL((transpose_vec_kernel<ES, 8, 16>), grid, dim3(256), 0, s, t);              \
-        else hipLaunchKernelGGL((transpose_vec_kernel<ES, 8, 8>), grid, dim3(256), 0, s, t);                             \
+        if (lg == 0 || sg == 0) AXHIP_TRANSPOSE_NV(ES, ES, ES);                                                          \
+        else if (lg == 16 && sg == 16) AXHIP_TRANSPOSE_NV(ES, 16, 16);                                                   \
+        else if (lg == 16) AXHIP_TRANSPOSE_NV(ES, 16, 8);                                                                \
+        else if (sg == 16) AXHIP_TRANSPOSE_NV(ES, 8, 16);                                                                \
+        else AXHIP_TRANSPOSE_NV(ES, 8, 8);                                                                               \
     } while (0)
             if (es == 2) AXHIP_TRANSPOSE(2);
             else AXHIP_TRANSPOSE(4);
 #undef AXHIP_TRANSPOSE
+#undef AXHIP_TRANSPOSE_NV
             AXHIP_CHECK_HIP(hipGetLastError());
             return AXHIP_OK;
         }

@@ -514,3 +514,23 @@ def test_axis_reductions_and_softmax_over_rows_off_the_vector_grid(dt, outer, ax
     want = np.exp(x - x.max(1, keepdims=True))
     want /= want.sum(1, keepdims=True)
     assert np.all(np.abs(got - want) <= want * (half + (6 * 17 + axis) * 2.0**-23) + (2.0**-25 if dt == F16 else 1e-37))
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,cols,others,skip", [(16, 16, 3, 0), (17, 64, 2, 1), (65, 129, 2, 0), (64, 127, 40, 3), (127, 61, 1, 0), (129, 200, 2, 5), (333, 66, 9, 0), (257, 1030, 1, 1)])
+def test_transposes_off_the_vector_grid_are_bit_exact(dt, rows, cols, others, skip):
+    """Rows that start anywhere and end inside a vector, on either side: every remainder, one tile and several, a view that
+    starts `skip` elements into its array's rows; the result is followed by elements that are not its own."""
+    base = sample((others, rows, cols + skip), dt, rows + cols)
+    d = gh.to_dev(base)
+    view = base[:, :, skip:].transpose(0, 2, 1)
+    n = view.size
+    out = gh.empty_dev((n + 32,), dt)
+    mark = sample((32,), dt, 4)
+    out[n:].copy_(gh.to_dev(mark))
+    gh.sync()
+    capi.check(capi.lib().axhip_strided_copy(d.data_ptr() + skip * base.itemsize, dt, out.data_ptr(), dt, 3, i64(view.shape), i64(elem_strides(view)), None))
+    gh.sync()
+    got = gh.to_host(out, base.dtype)
+    assert np.array_equal(got[:n].reshape(view.shape), np.ascontiguousarray(view))
+    assert np.array_equal(got[n:], mark)
