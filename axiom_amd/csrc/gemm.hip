@@ -377,7 +377,10 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // agree).  K only has to be a multiple of 4: the chunks of the last k-tile that lie past K are sent out of the
 // descriptor's range and arrive as zeros.  At 1/16 of the 16-bit MFMA rate the kernel is bound by the matrix pipe,
 // not by the ring.
-template <int TM, int TNR, int S>
+// NN: B is [K,N].  Its k-tile then is 32 rows of TNR floats, which the same loads bring in (N a multiple of 4), and a
+// lane's four k values of its column are four 4-byte reads -- as many LDS cycles as the one of 16 bytes, and no pass that
+// transposes B first.
+template <int TM, int TNR, int S, bool NN>
 __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
     constexpr int MI = TM / 64, NJ = TNR / 64;
     constexpr int NLA = TM / 32, NLB = TNR / 32;
@@ -398,30 +401,37 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const int64_t m0 = static_cast<int64_t>(tm) * TM, n0 = static_cast<int64_t>(tn) * TNR;
     const int64_t bz = blockIdx.y;
     const float *A = static_cast<const float *>(g.a) + bz * g.sa + m0 * g.a_rs;
-    const float *B = static_cast<const float *>(g.b) + bz * g.sb + n0 * g.b_cs;
-    const int arow_bytes = static_cast<int>(g.a_rs) * 4, brow_bytes = static_cast<int>(g.b_cs) * 4;
+    const float *B = static_cast<const float *>(g.b) + bz * g.sb + n0 * (NN ? 1 : g.b_cs);
+    const int arow_bytes = static_cast<int>(g.a_rs) * 4, brow_bytes = static_cast<int>(NN ? g.b_rs : g.b_cs) * 4;
     const int rows_a = static_cast<int>(min<int64_t>(TM, g.M - m0)), rows_b = static_cast<int>(min<int64_t>(TNR, g.N - n0));
     const int K = static_cast<int>(g.K);
     const int4_t arsrc = gemm_rsrc(A, (rows_a - 1) * arow_bytes + K * 4);
-    const int4_t brsrc = gemm_rsrc(B, (rows_b - 1) * brow_bytes + K * 4);
+    const int4_t brsrc = gemm_rsrc(B, NN ? (K - 1) * brow_bytes + rows_b * 4 : (rows_b - 1) * brow_bytes + K * 4);
 
     const int ld_r = 8 * wave + (lane >> 3);
     const int ld_c = (lane & 7) ^ ((ld_r >> 1) & 7); // source chunk of this lane: floats 4 ld_c .. 4 ld_c + 3 of the k-tile
+    constexpr int OUT_OF_RANGE = 0x7FFFFFF0;
     int a_voff[NLA], b_voff[NLB];
 #pragma unroll
     for (int n = 0; n < NLA; ++n) a_voff[n] = (32 * n + ld_r) * arow_bytes + ld_c * 16;
 #pragma unroll
-    for (int n = 0; n < NLB; ++n) b_voff[n] = (32 * n + ld_r) * brow_bytes + ld_c * 16;
+    for (int n = 0; n < NLB; ++n) {
+        const int at = (4 * n + wave) * 1024 + lane * 16; // of the tile
+        if (NN) b_voff[n] = at % (TNR * 4) < rows_b * 4 ? at / (TNR * 4) * brow_bytes + at % (TNR * 4) : OUT_OF_RANGE;
+        else b_voff[n] = (32 * n + ld_r) * brow_bytes + ld_c * 16;
+    }
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(big_lds));
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + 8 * wave * BIG_ROWB);
-    constexpr int OUT_OF_RANGE = 0x7FFFFFF0;
     auto load_tile = [&](int kt, int stage) {
         const int soff = kt * BIG_ROWB;
         const bool k_ok = kt * KF + ld_c * 4 < K; // false only for the trailing chunks of a ragged last k-tile
 #pragma unroll
         for (int n = 0; n < NLA; ++n) gemm_load_to_lds(arsrc, lds_wave + stage * STAGEB + n * 32 * BIG_ROWB, k_ok ? a_voff[n] : OUT_OF_RANGE, soff);
 #pragma unroll
-        for (int n = 0; n < NLB; ++n) gemm_load_to_lds(brsrc, lds_wave + stage * STAGEB + TM * BIG_ROWB + n * 32 * BIG_ROWB, k_ok ? b_voff[n] : OUT_OF_RANGE, soff);
+        for (int n = 0; n < NLB; ++n) {
+            const bool ok = NN ? kt * KF + ((4 * n + wave) * 1024 + lane * 16) / (TNR * 4) < K : k_ok;
+            gemm_load_to_lds(brsrc, lds_wave + stage * STAGEB + TM * BIG_ROWB + n * 32 * BIG_ROWB, ok ? b_voff[n] : OUT_OF_RANGE, NN ? kt * KF * brow_bytes : soff);
+        }
     };
 
     const int wm = (wave / 2) * (TM / 2), wn = (wave % 2) * (TNR / 2);
@@ -440,9 +450,16 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     float4_t fa[2][MI], fb[2][NJ];
     auto read_frags = [&](int slot, int stage, int ks) {
         const unsigned char *As = big_lds + stage * STAGEB + wm * BIG_ROWB;
-        const unsigned char *Bs = big_lds + stage * STAGEB + (TM + wn) * BIG_ROWB;
+        const unsigned char *Bs = big_lds + stage * STAGEB + (NN ? TM : TM + wn) * BIG_ROWB;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) fb[slot][j] = *reinterpret_cast<const float4_t *>(Bs + 32 * j * BIG_ROWB + f_off[ks]);
+        for (int j = 0; j < NJ; ++j) {
+            if constexpr (NN) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) fb[slot][j][c] = reinterpret_cast<const float *>(Bs)[(8 * ks + 4 * g2 + c) * TNR + wn + 32 * j + l32];
+            } else {
+                fb[slot][j] = *reinterpret_cast<const float4_t *>(Bs + 32 * j * BIG_ROWB + f_off[ks]);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < MI; ++i) fa[slot][i] = *reinterpret_cast<const float4_t *>(As + 32 * i * BIG_ROWB + f_off[ks]);
     };
@@ -650,9 +667,9 @@ F32Ring f32_ring_tile(const AxhipGemmParams &p) {
     }
     return best;
 }
-// both operands along k, whole 16-byte vectors, offsets of 32 bits
+// A along k, whole 16-byte vectors, offsets of 32 bits
 bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
-    return !p.trans_a && p.trans_b && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && p.stride_a % 4 == 0 && p.stride_b % 4 == 0 &&
+    return !p.trans_a && (p.trans_b || (p.n % 4 == 0 && p.n < (1 << 24) && (p.k + 64) * p.ldb < (int64_t(1) << 29))) && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && p.stride_a % 4 == 0 && p.stride_b % 4 == 0 &&
            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0 && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
            p.m * p.n * p.batch >= 64 * 64 * 16 && f32_mfma_enabled();
 }
@@ -755,8 +772,8 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     if (rc) return rc;
     hipStream_t s = resolve_stream(stream);
 
-    // The fp32 matrix kernel reads both operands along k, in 16-byte vectors (the 16-bit ones read A along k).  An operand stored the other way (A as
-    // [k, m], B as [k, n]: matmul(a, b) with a plain [k, n] right-hand side), or a reduction length that is not a whole
+    // The matrix kernels read A along k, the fp32 ring kernel in 16-byte vectors.  An operand stored the other way (A as
+    // [k, m]; B as [k, n] where its rows are no whole vectors), or a reduction length that is not a whole
     // number of vectors, leaves only the FMA kernel below, a hundred times slower on a large product.  Such a product
     // is repacked first, into stream-ordered temporary memory (freed in stream order behind the product): the operand
     // that lies the other way is transposed; an unaligned k is zero-padded to the next multiple of 64 in both operands.
@@ -765,10 +782,10 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const size_t need = repack_bytes(p);
         AXHIP_REQUIRE(workspace_bytes >= need, AXHIP_ERR_WORKSPACE, "axhip_gemm: the workspace holds %zu bytes, the call needs %zu (ask axhip_gemm_workspace_bytes)", workspace_bytes, need);
     }
-    const bool f32 = p.dtype == AXHIP_DTYPE_F32, repack = rp.on && !scratch_in;
+    const bool f32 = p.dtype == AXHIP_DTYPE_F32, repack = rp.on && !scratch_in && !(f32 ? takes_f32_ring(p, a, b) : takes_half_kernels(p));
     const double repacked = repack ? 8.0 * static_cast<double>(p.batch) * static_cast<double>((rp.a ? p.m : 0) + (rp.b ? p.n : 0)) * static_cast<double>(p.k) : 0.0;
     const int f32_shape = f32 ? choose_f32_kernel(p, repack || takes_f32_ring(p, a, b), repacked) : -1;
-    if (repack && f32_shape < 0 && (f32 || !takes_half_kernels(p))) {
+    if (repack && f32_shape < 0) {
         const bool pad_k = rp.kp != p.k;
         const int64_t es = p.dtype == AXHIP_DTYPE_F32 ? 4 : 2, kp = rp.kp;
         AxhipGemmParams q = p;
@@ -864,10 +881,13 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         };
         int rc2;
         switch (f32_ring_tile(p).tile) {
-        case 0: rc2 = launch(gemm_mfma_f32_ring_kernel<128, 128, 3>, 128, 128, 3 * 256 * BIG_ROWB); break;
-        case 1: rc2 = launch(gemm_mfma_f32_ring_kernel<64, 128, 3>, 64, 128, 3 * 192 * BIG_ROWB); break;
-        case 3: rc2 = launch(gemm_mfma_f32_ring_kernel<64, 64, 3>, 64, 64, 3 * 128 * BIG_ROWB); break;
-        default: rc2 = launch(gemm_mfma_f32_ring_kernel<128, 192, 3>, 128, 192, 3 * 320 * BIG_ROWB); break;
+#define AXHIP_RING(TM, TN) \
+    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, 3, false>, TM, TN, 3 * (TM + TN) * BIG_ROWB) : launch(gemm_mfma_f32_ring_kernel<TM, TN, 3, true>, TM, TN, 3 * (TM + TN) * BIG_ROWB)
+        case 0: AXHIP_RING(128, 128); break;
+        case 1: AXHIP_RING(64, 128); break;
+        case 3: AXHIP_RING(64, 64); break;
+        default: AXHIP_RING(128, 192); break;
+#undef AXHIP_RING
         }
         if (rc2) return rc2;
     } else {

@@ -1403,11 +1403,11 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
             // (bf16 [32, 1500, 1280] 70.8 us in the other order, 60.9 with large tiles, 59.3 with small ones; fp32 130,
             // 113, 98).  Rows of whole lines take large tiles along a diagonal over all XCDs (bf16 [8, 4096, 4096] 96 us
             // against 117).  Extents of one large tile or less: small ones waste fewer lanes (bf16 [2000, 64, 130] 25 ->
-            // 17 us), except that fp32's 32 elements are too few (fp32 [5000, 33, 65] 29 us against 40).
+            // 17 us), except that fp32's 32 elements are too few (fp32 [5000, 33, 65] 30 us against 40).
             const bool lines = t.dst_stride_j * es % 128 == 0;
             const int64_t narrow = std::min(t.nJ, t.nL);
-            const bool together = !lines || (es == 2 && narrow <= 128);
-            const int nv = es == 2 ? (together ? 8 : 16) : (!lines && narrow > 64 ? 8 : 16);
+            const bool together = es == 2 ? !lines || narrow <= 128 : !lines && narrow > 64;
+            const int nv = together ? 8 : 16;
             const int64_t edge = nv * (16 / es);
             t.tiles_j = (t.nJ + edge - 1) / edge; t.tiles_l = (t.nL + edge - 1) / edge;
             blocks = blocks / (((t.nJ + 63) / 64) * ((t.nL + 63) / 64)) * t.tiles_j * t.tiles_l;

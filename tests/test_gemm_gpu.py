@@ -292,3 +292,29 @@ def test_f32_products_at_the_edges_of_tiles(nn, M, N, K, batch):
     magnitude = np.abs(x64) @ np.abs(w64) + np.abs(bias) + np.abs(res)
     assert got.shape == want.shape
     assert np.all(np.abs(got - want) <= (K + 2) * 2.0**-24 * magnitude)
+
+
+@pytest.mark.parametrize("M,N,K,batch", [(2048, 2044, 132, 1), (1000, 1100, 260, 8), (1024, 1024, 1024, 1), (1300, 4000, 44, 3), (700, 2500, 1000, 1)])
+def test_f32_products_of_plain_matrices_on_the_ring(M, N, K, batch):
+    """a b with b stored [k, n] in whole vectors, sizes of the ring kernel's four tiles: k that ends inside a k-tile, rows
+    and columns inside a tile; b lies in front of NaNs.  The same bound as above."""
+    import ctypes as C
+
+    import torch
+
+    from axiom_amd import capi
+
+    g = axo.PCG64(M + N + K)
+    x, W = g.normal((batch, M, K)).astype(np.float32), (g.normal((batch, K, N)) / np.sqrt(K)).astype(np.float32)
+    da, db = gh.to_dev(x), torch.full((batch * K * N + 64 * N,), float("nan"), device="cuda")
+    db[: batch * K * N] = gh.to_dev(W).flatten()
+    c = gh.empty_dev((batch, M, N), F32)
+    p = capi.GemmParams()
+    p.dtype, p.m, p.n, p.k, p.batch, p.lda, p.ldb, p.ldc = F32, M, N, K, batch, K, N, N
+    p.stride_a, p.stride_b, p.stride_c = M * K, K * N, M * N
+    gh.sync()
+    capi.check(capi.lib().axhip_gemm(da.data_ptr(), db.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    got = c.double()
+    x64, w64 = da.double(), gh.to_dev(W).double()
+    assert bool(((got - x64 @ w64).abs() <= (K + 2) * 2.0**-24 * (x64.abs() @ w64.abs())).all())
