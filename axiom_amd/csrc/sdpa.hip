@@ -18,8 +18,8 @@
 //   sdpa_mfma_kernel    bf16 / f16, head_dim 32: same arithmetic, K and V tiles
 //                       staged through registers into LDS.
 //   sdpa_direct16_kernel, sdpa_direct_f32_kernel (sdpa_direct.hip)  a few query
-//                       rows against many keys; short fp32 sequences: no LDS
-//                       tiles, K and V from memory into the MFMA operands.
+//                       rows against many keys; short fp32 sequences: no
+//                       shared LDS tiles, a barrier only at the end.
 //   sdpa_generic_kernel any dtype, head_dim <= 256, fp32 FMA arithmetic; used
 //                       for fp32 inputs and for head sizes the MFMA kernels do
 //                       not cover.
@@ -1965,8 +1965,8 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         last_schedule = "mfma_f32";
         // waves per 32-row query block, by how many such blocks there are for the 1024 SIMDs (thresholds from timings
         // of 128 .. 1024 blocks: below 0.75 blocks per SIMD the four-way split wins by up to 2.7x, above 1.5 none is needed)
-        // Up to one 16-row block per CU the kernel without LDS tiles is the faster one (8 heads of 512 rows of 64: 16.3 ->
-        // 10.6 us, causal 16.2 -> 10.4, masked 17.9 -> 14.6; 8 of 333 x 1000 of 128: 51.5 -> 26.2); with 512 blocks its reads
+        // Up to one 16-row block per CU the kernel without shared tiles is the faster one (8 heads of 512 rows of 64: 16.3 ->
+        // 9.5 us, causal 16.2 -> 9.6, masked 17.9 -> 13.0; 8 of 333 x 1000 of 128: 51.5 -> 25.1); with 512 blocks its reads
         // of K and V by every block cost more than the idle CUs did (16 heads of 512: 16.6 and 19.6 us).
         const int64_t blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * p.batch * p.heads;
         if (blocks16 <= 256 && p.head_dim > 32 && sdpa_f32_split == 0) {

@@ -51,7 +51,7 @@ template <bool BF16> __device__ __forceinline__ float add_pair(uint32_t packed, 
     }
 }
 
-// sdpa_direct.hip: a few query rows against many keys, K and V straight from memory into the matrix operands
+// sdpa_direct.hip: a few query rows against many keys, short fp32 sequences
 constexpr int DIRECT_WAVES = 8;      // per work-group
 constexpr int DIRECT_ROWS = 8;       // query rows of the 16-bit kernel, at most
 constexpr int DIRECT_KEYS = 32;      // keys of one step of a wave; a.kchunk is a multiple of it

@@ -1,18 +1,30 @@
-// Attention without LDS tiles: K and V go from memory straight into the operands of the matrix instructions.
+// Attention without shared LDS tiles, for few query rows and short sequences.
 //
 // A work-group owns one block of query rows; its eight waves take 32-key steps of the keys in turn and meet once, at
-// the end, through LDS.  What makes the detour through LDS unnecessary is that the order in which keys and head
-// dimensions run through an MFMA is free as long as both operands agree on it:
+// the end, through LDS.  V goes from memory straight into the operands of the matrix instructions.  What makes a detour
+// through LDS unnecessary is that the order in which keys and head dimensions run through an MFMA is free as long as
+// both operands agree on it:
 //   S^T = K Q^T    leaves lane (l16, g) with query l16 and keys 4 g + i of a 16-key sub-tile;
 //   O^T = V^T P^T  then takes these keys as k-slots (the probabilities are the B operand as they stand), and lane
 //                  (l16, g) needs, of V, the rows of ITS keys and, for output tile t, dimension l16 * (D / 16) + t --
 //                  so its whole share of V is a few rows of 16-byte runs that it loads itself, and the transpose is
 //                  byte permutes between its own registers.
 #include "sdpa.hpp"
+#include "gemm_tile_device.hpp" // wave_lds_fence
 
 namespace axhip {
 
 namespace {
+
+// K can be loaded as fragments -- 16 bytes of each of 16 rows side by side, four times the lines of an instruction that
+// loads whole rows -- or as rows, through 8 KiB of LDS that are the wave's own.  The rows are the faster ones where a
+// work-group's latency counts (fp32 B1 H8 S512 10.3 -> 9.5 us, 96 slices of 700 keys 7.1 -> 6.2, 12 of 300 of 128 dims 6.4 ->
+// 5.5), the fragments by 1 - 4 % where the chip streams (128 slices of 16384 keys of 128 178 against 180 us, 256 of 4096
+// 89.7 against 93.0).
+// 16-byte chunk c of row r of a stage, CH chunks a row, spread so that neither the rows written nor the 16 rows of a
+// fragment read meet on a bank:
+constexpr int DIRECT_STAGE = 8192;
+template <int CH> __device__ __forceinline__ int stage_at(int r, int c) { return (r * CH + (c ^ (CH == 8 ? (r >> 1) & 7 : r & 15))) * 16; }
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -58,10 +70,10 @@ template <int D> __device__ __forceinline__ Merged direct_merge(const float *lds
 
 // ------------------------------------------------------------- 16-bit, decoding
 // Up to DIRECT_ROWS query rows against a long run of keys: bound by one read of K and V.  A step of a wave is 32 keys,
-// 16 loads of 16 bytes (D = 64: 8), requested one step ahead, so a work-group has 128 KiB on the way or in use
+// 16 loads of 16 bytes (D = 64: 4, and 8 of 8), requested one step ahead, so a work-group has 128 KiB on the way or in use
 // (D = 128) and needs no barrier to keep it so.  Of the 16 query columns of the MFMAs most are empty; they cost nothing
 // that the loads would not cost anyway (16 MFMAs of 16 cycles for 16 KiB).
-template <bool BF16, int D, bool SPLIT>
+template <bool BF16, int D, bool SPLIT, bool STAGED>
 __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(const SdpaArgs a) {
     constexpr int KJ = D / 32; // 32-dim fragments of a K row
     constexpr int NT = D / 16; // output tiles; elements of V a lane holds per key
@@ -80,9 +92,16 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(con
     const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(K), 0, (a.Skv - 1) * krow + dv * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(V), 0, (a.Skv - 1) * vrow + dv * 2, 0x00020000);
     constexpr int OUTSIDE = static_cast<int>(0x80000000u);
-    int koff[KJ];
+    constexpr int CH = D / 8, RL = WAVE / CH, KL = DIRECT_KEYS / RL; // chunks of a row, rows of a load, loads of a step
+    const int k_row = lane / CH, k_ch = lane % CH;
+    static_assert(KL == 2 * KJ, "the fragments of a step");
+    int koff[STAGED ? 1 : KJ]; // of the row; of the fragments of a row
 #pragma unroll
-    for (int j = 0; j < KJ; ++j) koff[j] = 32 * j + 8 * g < dv ? l16 * krow + (32 * j + 8 * g) * 2 : OUTSIDE;
+    for (int j = 0; j < (STAGED ? 1 : KJ); ++j) {
+        const int d = STAGED ? k_ch * 8 : 32 * j + 8 * g;
+        koff[j] = d < dv ? (STAGED ? k_row : l16) * krow + d * 2 : OUTSIDE;
+    }
+    unsigned char *stage = reinterpret_cast<unsigned char *>(lds) + wave * DIRECT_STAGE;
     const int voff = l16 * NT < dv ? 4 * g * vrow + l16 * NT * 2 : OUTSIDE;
 
     uint4_t qf[KJ];
@@ -91,13 +110,12 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(con
         qf[j] = l16 < rows && 32 * j + 8 * g < dv ? *reinterpret_cast<const uint4_t *>(Q + l16 * a.qs[2] + 32 * j + 8 * g) : uint4_t{0, 0, 0, 0};
 
     const int k_first = SPLIT ? split * a.kchunk : 0, k_end = SPLIT ? min(a.Skv, k_first + a.kchunk) : a.Skv;
-    uint4_t kf[2][KJ];
+    uint4_t kf[KL];
     uint32_t vf[8][NT / 2];
     auto load = [&](int at) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int j = 0; j < KJ; ++j) kf[u][j] = __builtin_amdgcn_raw_buffer_load_b128(kr, koff[j] + (at + 16 * u) * krow, 0, 0);
+        for (int n = 0; n < KL; ++n)
+            kf[n] = __builtin_amdgcn_raw_buffer_load_b128(kr, koff[STAGED ? 0 : n % KJ] + (at + (STAGED ? RL * n : 16 * (n / KJ))) * krow, 0, 0);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int off = voff + (at + 16 * (e / 4) + e % 4) * vrow;
@@ -119,12 +137,13 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(con
     int at = k_first + DIRECT_KEYS * wave;
     if (at < k_end) load(at);
     while (at < k_end) {
-        uint4_t kc[2][KJ];
+        uint4_t kc[STAGED ? 1 : KL];
         uint32_t vc[8][NT / 2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int j = 0; j < KJ; ++j) kc[u][j] = kf[u][j];
+        for (int n = 0; n < KL; ++n) {
+            if constexpr (STAGED) *reinterpret_cast<uint4_t *>(stage + stage_at<CH>(RL * n + k_row, k_ch)) = kf[n];
+            else kc[n] = kf[n];
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -134,12 +153,19 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(con
         if (at < k_end) load(at);
 
         f32x4_t s[2];
+        if constexpr (STAGED) wave_lds_fence();
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             s[u] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < KJ; ++j) s[u] = mfma_16x16x32<BF16>(kc[u][j], qf[j], s[u]);
+            for (int j = 0; j < KJ; ++j) {
+                uint4_t k;
+                if constexpr (STAGED) k = *reinterpret_cast<const uint4_t *>(stage + stage_at<CH>(16 * u + l16, 4 * j + g));
+                else k = kc[u * KJ + j];
+                s[u] = mfma_16x16x32<BF16>(k, qf[j], s[u]);
+            }
         }
+        if constexpr (STAGED) wave_lds_fence();
         if (now + DIRECT_KEYS > a.Skv) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -180,6 +206,7 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct16_kernel(con
 
     // tile t, element i of lane (l16, g): query l16, dim (4 g + i) * NT + t
     const float l_tot = group_sum(l_run);
+    if constexpr (STAGED) __syncthreads(); // the stages become the states
     if (l16 < rows) {
         float *row = &lds[(wave * rows + l16) * (D + 4)];
 #pragma unroll
@@ -212,11 +239,18 @@ int launch_sdpa_direct16(const SdpaArgs &a, bool bf16, hipStream_t s) {
     const bool split = a.ksplit > 0;
     const unsigned grid = static_cast<unsigned>(a.B * a.H * (split ? a.ksplit : 1));
     const bool narrow = a.D <= 64;
-    const int lds = narrow ? direct_lds_bytes<64>(a.Sq) : direct_lds_bytes<128>(a.Sq);
+    // (from 200 slices on the chip streams: 240 slices of 1102 keys of 64 14.6 us by fragments, 14.8 by rows; 4096 of 16 keys
+    // 20.6 and 22.2)
+    const bool staged = !split && a.B * a.H < 200;
+    constexpr int stages = DIRECT_WAVES * DIRECT_STAGE;
+    static_assert(direct_lds_bytes<128>(DIRECT_ROWS) <= stages && stages <= 65536, "the states take the place of the stages");
+    const int lds = staged ? stages : narrow ? direct_lds_bytes<64>(a.Sq) : direct_lds_bytes<128>(a.Sq);
 #define AXHIP_DIRECT(BF, DD)                                                                                              \
     do {                                                                                                                  \
-        if (split) hipLaunchKernelGGL((sdpa_direct16_kernel<BF, DD, true>), dim3(grid), dim3(64 * DIRECT_WAVES), lds, s, a);  \
-        else hipLaunchKernelGGL((sdpa_direct16_kernel<BF, DD, false>), dim3(grid), dim3(64 * DIRECT_WAVES), lds, s, a);       \
+        const dim3 threads(64 * DIRECT_WAVES);                                                                            \
+        if (split) hipLaunchKernelGGL((sdpa_direct16_kernel<BF, DD, true, false>), dim3(grid), threads, lds, s, a);       \
+        else if (staged) hipLaunchKernelGGL((sdpa_direct16_kernel<BF, DD, false, true>), dim3(grid), threads, lds, s, a); \
+        else hipLaunchKernelGGL((sdpa_direct16_kernel<BF, DD, false, false>), dim3(grid), threads, lds, s, a);            \
     } while (0)
     if (bf16 && narrow) AXHIP_DIRECT(true, 64);
     else if (bf16) AXHIP_DIRECT(true, 128);
@@ -314,9 +348,12 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
     const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(K), 0, (a.Skv - 1) * krow + dv * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(V), 0, (a.Skv - 1) * vrow + dv * 4, 0x00020000);
     constexpr int OUTSIDE = static_cast<int>(0x80000000u);
-    int koff[KJ], voff[VH];
-#pragma unroll
-    for (int j = 0; j < KJ; ++j) koff[j] = 16 * j + 4 * g < dv ? l16 * krow + (16 * j + 4 * g) * 4 : OUTSIDE;
+    constexpr int CH = D / 4, RL = WAVE / CH, KL = KEYS / RL; // chunks of a row, rows of a load, loads of a step
+    static_assert(KEYS * CH * 16 == DIRECT_STAGE, "a step of K");
+    const int k_row = lane / CH, k_ch = lane % CH;
+    const int koff = k_ch * 4 < dv ? k_row * krow + k_ch * 16 : OUTSIDE;
+    unsigned char *stage = reinterpret_cast<unsigned char *>(lds) + wave * DIRECT_STAGE;
+    int voff[VH];
 #pragma unroll
     for (int v = 0; v < VH; ++v) voff[v] = 64 * v + 4 * l16 < dv ? 4 * g * vrow + (64 * v + 4 * l16) * 4 : OUTSIDE;
 
@@ -326,13 +363,14 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
         qf[j] = q_ok && 16 * j + 4 * g < dv ? *reinterpret_cast<const f32x4_t *>(Q + q * a.qs[2] + 16 * j + 4 * g) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     const int k_end = a.causal ? min(a.Skv, q0 + ROWS) : a.Skv;
-    f32x4_t kf[SUB][KJ], vf[SUB][4][VH];
+    uint4_t kf[KL];
+    f32x4_t vf[SUB][4][VH];
     uint32_t mf[SUB]; // the mask bytes of this lane's four keys
     auto load = [&](int at) {
 #pragma unroll
-        for (int u = 0; u < SUB; ++u) {
+        for (int n = 0; n < KL; ++n) kf[n] = __builtin_amdgcn_raw_buffer_load_b128(kr, koff + (at + RL * n) * krow, 0, 0);
 #pragma unroll
-            for (int j = 0; j < KJ; ++j) kf[u][j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(kr, koff[j] + (at + 16 * u) * krow, 0, 0));
+        for (int u = 0; u < SUB; ++u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -358,12 +396,12 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
     int at = KEYS * wave;
     if (at < k_end) load(at);
     while (at < k_end) {
-        f32x4_t kc[SUB][KJ], vc[SUB][4][VH];
+        f32x4_t vc[SUB][4][VH];
         uint32_t mc[SUB];
 #pragma unroll
-        for (int u = 0; u < SUB; ++u) {
+        for (int n = 0; n < KL; ++n) *reinterpret_cast<uint4_t *>(stage + stage_at<CH>(RL * n + k_row, k_ch)) = kf[n];
 #pragma unroll
-            for (int j = 0; j < KJ; ++j) kc[u][j] = kf[u][j];
+        for (int u = 0; u < SUB; ++u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -377,12 +415,18 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
         f32x4_t s[SUB];
 #pragma unroll
         for (int u = 0; u < SUB; ++u) s[u] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        wave_lds_fence();
 #pragma unroll
-        for (int j = 0; j < KJ; ++j)
+        for (int j = 0; j < KJ; ++j) {
+            f32x4_t kc[SUB];
+#pragma unroll
+            for (int u = 0; u < SUB; ++u) kc[u] = *reinterpret_cast<const f32x4_t *>(stage + stage_at<CH>(16 * u + l16, 4 * j + g));
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int u = 0; u < SUB; ++u) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[u][j][c], qf[j][c], s[u], 0, 0, 0);
+                for (int u = 0; u < SUB; ++u) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[u][c], qf[j][c], s[u], 0, 0, 0);
+        }
+        wave_lds_fence();
         if (HAS_MASK || now + KEYS > a.Skv || (a.causal && now + KEYS - 1 > q0)) {
             const int last = a.causal ? min(a.Skv - 1, q) : a.Skv - 1;
 #pragma unroll
@@ -424,6 +468,7 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
 
     // tile (v, c), element i of lane (l16, g): query l16, dim 64 v + 4 (4 g + i) + c
     const float l_tot = group_sum(l_run);
+    __syncthreads(); // the stages become the states
     float *row = &lds[(wave * ROWS + l16) * (D + 4)];
 #pragma unroll
     for (int v = 0; v < VH; ++v)
@@ -444,7 +489,7 @@ __global__ __launch_bounds__(64 * DIRECT_WAVES, 2) void sdpa_direct_f32_kernel(c
 }
 
 template <int D> static int launch_direct_f32(const SdpaArgs &a, hipStream_t s) {
-    constexpr int lds = direct_lds_bytes<D>(16);
+    constexpr int stages = DIRECT_WAVES * DIRECT_STAGE, states = direct_lds_bytes<D>(16), lds = stages > states ? stages : states;
     static const hipError_t attr = [] {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&sdpa_direct_f32_kernel<D, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         return e != hipSuccess ? e : hipFuncSetAttribute(reinterpret_cast<const void *>(&sdpa_direct_f32_kernel<D, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);

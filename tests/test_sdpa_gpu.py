@@ -432,8 +432,8 @@ def test_ping_pong_schedule_on_head_split_views_and_a_row_dominated_by_a_late_ke
 
 
 @pytest.mark.parametrize("Sq,Skv", [(1, 1), (1, 31), (3, 33), (8, 256), (1, 257), (5, 1300), (8, 2049)])
-@pytest.mark.parametrize("dt,D", [(BF16, 64), (F16, 128), (BF16, 40), (F16, 72), (BF16, 8)], ids=["bf16-64", "f16-128", "bf16-40", "f16-72", "bf16-8"])
-def test_few_query_rows(dt, D, Sq, Skv):
+@pytest.mark.parametrize("dt,D,B", [(BF16, 64, 2), (F16, 128, 2), (BF16, 40, 2), (F16, 72, 2), (BF16, 8, 2), (F16, 56, 67), (BF16, 128, 67)])
+def test_few_query_rows(dt, D, B, Sq, Skv):
     """A decoding step: undivided and with its keys divided by a workspace, on rows of a [batch, position, heads x dim]
     cache whose further positions (and the output's further columns) are none of its business.  One rounding of the
     probabilities and one of the result: 2^-8 + 2^-9 of values below 4 in bf16, held to the 2e-2 of this file."""
@@ -443,7 +443,9 @@ def test_few_query_rows(dt, D, Sq, Skv):
 
     from axiom_amd import capi
 
-    lib, B, H = capi.lib(), 2, 3
+    if B > 2 and Skv > 300:
+        pytest.skip("long rows run with the few slices")
+    lib, H = capi.lib(), 3
     g = axo.PCG64(91 + Sq + Skv)
     q, k, v = (axo.to_bits(g.normal(s), dt) for s in ((B, Sq, H, D), (B, Skv, H, D), (B, Skv, H, D)))
     extra = 40
