@@ -952,17 +952,22 @@ __global__ __launch_bounds__(256) void reduce_strided_kernel(const void *src, in
 
 namespace axhip {
 // ----------------------------------------------- softmax along an inner axis
+__device__ __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f); } // (v_exp_f32, v_log_f32: base 2)
+__device__ __forceinline__ float log_of(float x) { return __builtin_amdgcn_logf(x) * 0.69314718055994530942f; }
+
 // softmax / log-softmax along the middle extent of a contiguous (outer, axis, inner) view, inner >= V, in the layout of
-// reduce_axis_kernel (any alignment, the last vector of a row moved left to end with it).  One sweep gathers a running maximum and the sum of 2^(x log2(e) - maximum) per inner
-// position (rescaled once per four elements), the thread rows merge their pairs through LDS, a second sweep over the
-// same elements writes the result: two reads of the input (the second mostly from the caches) and one write.
+// reduce_axis_kernel (any alignment, the last vector of a row moved left to end with it).  One sweep gathers a running
+// maximum and the sum of e^(x - maximum) per inner position (rescaled once per four elements), the thread rows merge
+// their pairs through LDS, a second sweep over the same elements writes the result: two reads of the input (the second
+// mostly from the caches) and one write.  x - maximum is formed before the factor log2(e): it is exact to one rounding of
+// the difference whatever the magnitude of x, where x log2(e) is off by 6e-5 for x around 1000, and it stays finite for
+// every finite x (a column that holds nothing but the type's lowest value is uniform).
 // HOLD > 0 (with TX = 256, a thread per vector walking the axis alone): the axis has at most HOLD elements and the thread
 // keeps them in registers between the two sweeps -- one read of the input.
 template <bool LOG, int DT, int TX, int HOLD = 0>
 __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *src, int64_t outer, int64_t axis, int64_t inner, void *dst) {
     constexpr int TY = 256 / TX, U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8;
     static_assert(HOLD == 0 || (TX == 256 && HOLD % U == 0), "rows held in registers: one thread per vector");
-    constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
     __shared__ float sm[TY][TX][V + 1], sl[TY][TX][V + 1];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
     constexpr int ES = 16 / V;
@@ -992,16 +997,16 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                 for (int u = 0; u < U; ++u) {
                     arg_unpack<DT>(raw[u], t[u]);
 #pragma unroll
-                    for (int e = 0; e < V; ++e) t[u][e] = k + u * TY < n ? t[u][e] * LOG2E : -INFINITY;
+                    for (int e = 0; e < V; ++e) t[u][e] = k + u * TY < n ? t[u][e] : -INFINITY;
                 }
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
                     const float mx = fmaxf(fmaxf(fmaxf(t[0][e], t[1][e]), fmaxf(t[2][e], t[3][e])), m[e]);
-                    const float ref = mx == -INFINITY ? 0.0f : mx; // (nothing finite yet: every term below is 2^-inf = 0)
+                    const float ref = mx == -INFINITY ? 0.0f : mx; // (nothing finite yet: every term below is e^-inf = 0)
                     float add = 0.0f;
 #pragma unroll
-                    for (int u = 0; u < U; ++u) add += __builtin_amdgcn_exp2f(t[u][e] - ref);
-                    l[e] = l[e] * __builtin_amdgcn_exp2f(m[e] - ref) + add;
+                    for (int u = 0; u < U; ++u) add += exp_of(t[u][e] - ref);
+                    l[e] = l[e] * exp_of(m[e] - ref) + add;
                     m[e] = mx;
                 }
         };
@@ -1030,16 +1035,16 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
             sl[ty][tx][e] = l[e];
         }
         __syncthreads();
-        float shift[V], inv[V]; // result = 2^(t - shift) * inv, or (t - shift) * ln 2 with the logarithm of the sum inside shift
+        float shift[V], inv[V]; // result = e^(x - shift) * inv, or x - shift - inv with the logarithm of the sum as inv
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             float M = sm[0][tx][e];
             for (int y = 1; y < TY; ++y) M = fmaxf(M, sm[y][tx][e]);
             const float ref = M == -INFINITY ? 0.0f : M;
             float L = 0.0f;
-            for (int y = 0; y < TY; ++y) L += sl[y][tx][e] * __builtin_amdgcn_exp2f(sm[y][tx][e] - ref);
-            shift[e] = LOG ? M + __builtin_amdgcn_logf(L) : M; // (v_log_f32 is the base-2 logarithm)
-            inv[e] = 1.0f / L;
+            for (int y = 0; y < TY; ++y) L += sl[y][tx][e] * exp_of(sm[y][tx][e] - ref);
+            shift[e] = M;
+            inv[e] = LOG ? log_of(L) : 1.0f / L;
         }
         auto emit = [&](int k, const uint4_t (&raw)[U]) {
 #pragma unroll
@@ -1048,7 +1053,7 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                         float v[V];
                         arg_unpack<DT>(raw[u], v);
 #pragma unroll
-                        for (int e = 0; e < V; ++e) v[e] = LOG ? (v[e] * LOG2E - shift[e]) * LN2 : __builtin_amdgcn_exp2f(v[e] * LOG2E - shift[e]) * inv[e];
+                        for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : exp_of(v[e] - shift[e]) * inv[e];
                         store_vec<V, true>(dst, DT, (o * axis + k + u * TY) * inner + col, v);
                     }
         };
@@ -1083,7 +1088,6 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
 template <bool LOG, int DT, int RPT, int THREADS>
 __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int tx_log2) {
     constexpr int V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V, NW = THREADS / WAVE;
-    constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
     __shared__ float red[NW][WAVE][V + 1];
     const int TX = 1 << tx_log2, TY = THREADS >> tx_log2;
     const int tid = threadIdx.x, tx = tid & (TX - 1), ty = tid >> tx_log2, wave = tid / WAVE;
@@ -1132,26 +1136,26 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
             float t[V];
             arg_unpack<DT>(raw[r], t);
 #pragma unroll
-            for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e] * LOG2E);
+            for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
         }
     across(m, true);
     float ref[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) ref[e] = m[e] == -INFINITY ? 0.0f : m[e]; // (nothing finite: every term is 2^-inf = 0)
+    for (int e = 0; e < V; ++e) ref[e] = m[e] == -INFINITY ? 0.0f : m[e]; // (nothing finite: every term is e^-inf = 0)
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float t[V];
             arg_unpack<DT>(raw[r], t);
 #pragma unroll
-            for (int e = 0; e < V; ++e) l[e] += __builtin_amdgcn_exp2f(t[e] * LOG2E - ref[e]);
+            for (int e = 0; e < V; ++e) l[e] += exp_of(t[e] - ref[e]);
         }
     across(l, false);
-    float shift[V], inv[V]; // result = 2^(t - shift) * inv, or (t - shift) * ln 2 with the logarithm of the sum inside shift
+    float shift[V], inv[V]; // result = e^(x - shift) * inv, or x - shift - inv with the logarithm of the sum as inv
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-        shift[e] = LOG ? m[e] + __builtin_amdgcn_logf(l[e]) : ref[e]; // (v_log_f32 is the base-2 logarithm)
-        inv[e] = 1.0f / l[e];
+        shift[e] = LOG ? m[e] : ref[e];
+        inv[e] = LOG ? log_of(l[e]) : 1.0f / l[e];
     }
     if (!there) return;
 #pragma unroll
@@ -1160,7 +1164,7 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
             float v[V];
             arg_unpack<DT>(raw[r], v);
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[e] = LOG ? (v[e] * LOG2E - shift[e]) * LN2 : __builtin_amdgcn_exp2f(v[e] * LOG2E - shift[e]) * inv[e];
+            for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : exp_of(v[e] - shift[e]) * inv[e];
             store_vec<V, true>(dst, DT, (o * n + ty + r * TY) * inner + col, v);
         }
 }

@@ -534,3 +534,36 @@ def test_transposes_off_the_vector_grid_are_bit_exact(dt, rows, cols, others, sk
     got = gh.to_host(out, base.dtype)
     assert np.array_equal(got[:n].reshape(view.shape), np.ascontiguousarray(view))
     assert np.array_equal(got[n:], mark)
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,axis,inner", [(3, 40, 9), (2, 100, 64), (4, 300, 33), (1, 1030, 24), (1, 4097, 17), (2, 4100, 8), (1100, 5, 512), (1100, 24, 516), (1030, 16, 35), (40, 30, 3)])
+def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner):
+    """Values around +-1000, a column of the type's lowest value alone (uniform: every result is 1 / axis) and one that it
+    masks in part, in every kernel and on both kinds of rows.  x - max is one rounding, 2^-24 |x - max|, however large x is;
+    the exponentials add 2^-22 per unit of an argument that matters (up to 17: below e^-17 a term is under the sum's own
+    rounding) and the sum `axis` roundings, which a logarithm turns into absolute error; then the result's own rounding."""
+    rng = np.random.default_rng(axis * inner + dt)
+    x = (rng.normal(size=(outer, axis, inner)) * 3 + np.where(rng.random((outer, 1, inner)) < 0.5, 1000.0, -1000.0)).astype(np.float32)
+    lowest = {F32: np.finfo(np.float32).min, F16: -65504.0, BF16: axo.to_f32(np.array([0xFF7F], np.uint16), BF16)[0]}[dt]
+    x[:, :, 0] = lowest
+    x[:, 1::2, 1] = lowest
+    bits = axo.to_bits(x, dt)
+    xf, half = axo.to_f32(bits, dt).astype(np.float64), {F32: 2.0**-24, F16: 2.0**-11, BF16: 2.0**-8}[dt]
+    z = xf - xf.max(1, keepdims=True)
+    total = np.exp(z).sum(1, keepdims=True)
+    d, arith = gh.to_dev(bits), (17 * 4 + axis + 8) * 2.0**-24
+    for log, want, tol in ((1, z - np.log(total), arith), (0, np.exp(z) / total, 0.0)):
+        out = gh.empty_dev((outer, axis, inner), dt)
+        gh.sync()
+        capi.check(capi.lib().axhip_softmax_axis(d.data_ptr(), dt, outer, axis, inner, log, out.data_ptr(), None))
+        gh.sync()
+        got = axo.to_f32(gh.to_host(out, gh.np_store_dtype(dt)), dt).reshape(outer, axis, inner)
+        with np.errstate(invalid="ignore"):  # (log: the masked values lie past the type's range in 16 bits and are infinite there)
+            off = np.where(got == want.astype(np.float32), 0.0, np.abs(got - want))
+        if log:
+            fine = np.abs(want) < -float(lowest) * (1 - 2.0**-8)
+            assert np.all(off[fine] <= (tol + (2.0**-24 + half) * np.abs(want) + 2.0**-24 * np.abs(z))[fine])
+            assert np.all(got[~fine] <= -0.99 * -float(lowest))
+        else:
+            assert np.all(off <= want * (half * (1 + 2.0**-10) + 2 * arith) + (2.0**-25 if dt == F16 else 1e-37))
