@@ -1896,7 +1896,10 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
     if (rc) return rc;
     hipStream_t s = resolve_stream(stream);
     const int es = dtype == AXHIP_DTYPE_F32 ? 4 : 2;
-    if (inner >= 16 / es) {
+    // In place, rows that are no whole number of vectors go element by element: the vector kernels work the columns that a
+    // row's last two vectors share out twice, and the second of them may find the first one's results there.
+    const bool shared_columns = src == dst && inner % (16 / es) != 0;
+    if (inner >= 16 / es && !shared_columns) {
         const int64_t ivecs = (inner + 16 / es - 1) / (16 / es), bytes = outer * axis * inner * es;
         // An axis that a block can hold is read once.  Up to 512 elements: four rows per thread (256 threads up to 256
         // elements, so that several blocks share a CU), as wide as that allows; bf16 [64, 256, 2048] 72 -> 40 us, fp32

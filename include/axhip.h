@@ -406,7 +406,8 @@ int axhip_reduce_axis_ws(const void *src, int32_t dtype, int64_t outer, int64_t 
                          int32_t reduce, void *dst, int32_t dst_dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 /* softmax (is_log = 0) / log-softmax along the middle extent of a contiguous
- * (outer, axis, inner) view, dst of the same shape and dtype: Softmax /
+ * (outer, axis, inner) view, dst of the same shape and dtype (src itself, or
+ * memory that does not overlap it): Softmax /
  * LogSoftmax nodes over an axis other than the last one
  * (src/backends/metal/mpsgraph_graph_compiler.mm:287-300 takes any axis),
  * without the two transposing copies.  inner == 1 goes to the fused row

@@ -567,3 +567,21 @@ def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner):
             assert np.all(got[~fine] <= -0.99 * -float(lowest))
         else:
             assert np.all(off <= want * (half * (1 + 2.0**-10) + 2 * arith) + (2.0**-25 if dt == F16 else 1e-37))
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,axis,inner", [(3, 50, 129), (2, 300, 9), (1100, 5, 515), (1100, 24, 520), (40, 7, 64), (1, 4097, 17), (2, 4100, 24)])
+def test_softmax_along_inner_axes_in_place(dt, outer, axis, inner):
+    """dst == src, with rows that are whole vectors and rows whose last vector is moved left over its neighbour's columns
+    (the neighbour in the same work-group and in another one): the reference and tolerance of rows off the vector grid."""
+    rng = np.random.default_rng(axis + 7 * inner)
+    bits = axo.to_bits((rng.normal(size=(outer, axis, inner)) * 2).astype(np.float32), dt)
+    x, half = axo.to_f32(bits, dt).astype(np.float64), {F32: 0.0, F16: 2.0**-11, BF16: 2.0**-8}[dt]
+    d = gh.to_dev(bits)
+    gh.sync()
+    capi.check(capi.lib().axhip_softmax_axis(d.data_ptr(), dt, outer, axis, inner, 0, d.data_ptr(), None))
+    gh.sync()
+    got = axo.to_f32(gh.to_host(d, gh.np_store_dtype(dt)), dt).reshape(outer, axis, inner)
+    want = np.exp(x - x.max(1, keepdims=True))
+    want /= want.sum(1, keepdims=True)
+    assert np.all(np.abs(got - want) <= want * (half + (6 * 17 + axis) * 2.0**-23) + (2.0**-25 if dt == F16 else 1e-37))
