@@ -35,6 +35,10 @@ int rows_setup_device(); // per-device set-up of the fused-row kernels (rows.hip
         }                                             \
     } while (0)
 
+// A launch of 2^32 threads or more along a dimension of its grid is outside HIP's limits: not all of it runs, and no error
+// tells so.
+constexpr bool launch_fits(int64_t blocks, int64_t threads) { return blocks < (int64_t(1) << 31) && blocks * threads < (int64_t(1) << 32); }
+
 // Temporary device memory of ONE call.  With a caller's workspace (the *_ws entry points) it hands out 256-byte
 // aligned slices of that and allocates nothing; without one (workspace == NULL) every request is a stream-ordered
 // allocation that is returned in stream order when the call ends.

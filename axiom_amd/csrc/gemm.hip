@@ -632,7 +632,8 @@ constexpr HalfKernel HALF_KERNELS[] = {
     {HalfKernel::SMALL, SMALL_16x16, 4, 2.94f, 0.00069f, 0.00004f, 0.02f, true, false, false},
 };
 
-const HalfKernel &choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
+// (NULL: no kernel whose work-groups, as many as the product has tiles, can be launched at once)
+const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
     const HalfKernel *best = nullptr;
     float best_cost = 0.0f;
     const uint32_t m = static_cast<uint32_t>(p.m), n = static_cast<uint32_t>(p.n);
@@ -643,13 +644,15 @@ const HalfKernel &choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
         if (h.kind == HalfKernel::BIG256 && (p.k % TK != 0 || p.m < BIG || p.n < BIG || p.ldc >= (1 << 21))) continue;
         const uint32_t tm = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tm : SMALL_GEOMETRY[h.shape].tm;
         const uint32_t tn = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tn : SMALL_GEOMETRY[h.shape].tn;
-        const float full = batch * static_cast<float>((m + tm - 1) / tm) * static_cast<float>((n + tn - 1) / tn) * (1.0f / 256.0f);
+        const uint32_t rows = (m + tm - 1) / tm, cols = (n + tn - 1) / tn;
+        if (!launch_fits(static_cast<int64_t>(rows) * cols + 7, 64 * h.waves)) continue;
+        const float full = batch * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
         const float whole = std::ceil(full), r = full <= 1.0f ? 1.0f : h.kind == HalfKernel::SMALL ? 0.5f * (whole + full) : whole;
         const float per_k = (h.per_k + h.per_k_full * std::min(full, 1.0f)) * (h.kind == HalfKernel::SMALL && !aligned ? 1.9f : 1.0f);
         const float cost = h.start + k * per_k * r + h.per_round * (r - 1.0f);
         if (!best || cost < best_cost) { best_cost = cost; best = &h; }
     }
-    return *best;
+    return best;
 }
 
 // ---- fp32 products: which kernel
@@ -702,9 +705,9 @@ int choose_f32_kernel(const AxhipGemmParams &p, bool ring, double repacked) {
     }
     for (int i = 0; i < F32_SHAPES; ++i) {
         const F32Kernel &h = F32_KERNELS[i];
-        const float full = static_cast<float>(p.batch) * static_cast<float>((p.m + F32_GEOMETRY[i].tm - 1) / F32_GEOMETRY[i].tm) *
-                           static_cast<float>((p.n + F32_GEOMETRY[i].tn - 1) / F32_GEOMETRY[i].tn) * (1.0f / 256.0f);
-        if (full > 65536.0f) continue; // (tiles are counted in 32 bits)
+        const int64_t rows = (p.m + F32_GEOMETRY[i].tm - 1) / F32_GEOMETRY[i].tm, cols = (p.n + F32_GEOMETRY[i].tn - 1) / F32_GEOMETRY[i].tn;
+        if (!launch_fits(rows * cols + 7, 512)) continue; // (eight wavefronts a tile)
+        const float full = static_cast<float>(p.batch) * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
         const float r = full <= 1.0f ? 1.0f : 0.5f * (std::ceil(full) + full);
         const float cost = h.start + k * (h.per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
         if ((best < 0 && !ring) || cost < best_cost) { best_cost = cost; best = i; }
@@ -782,7 +785,9 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const size_t need = repack_bytes(p);
         AXHIP_REQUIRE(workspace_bytes >= need, AXHIP_ERR_WORKSPACE, "axhip_gemm: the workspace holds %zu bytes, the call needs %zu (ask axhip_gemm_workspace_bytes)", workspace_bytes, need);
     }
-    const bool f32 = p.dtype == AXHIP_DTYPE_F32, repack = rp.on && !scratch_in && !(f32 ? takes_f32_ring(p, a, b) : takes_half_kernels(p));
+    const bool f32 = p.dtype == AXHIP_DTYPE_F32;
+    auto half_kernel = [&] { return !f32 && takes_half_kernels(p) ? choose_half_kernel(p, half_aligned(p, a, b)) : nullptr; };
+    const bool repack = rp.on && !scratch_in && !(f32 ? takes_f32_ring(p, a, b) : half_kernel() != nullptr);
     const double repacked = repack ? 8.0 * static_cast<double>(p.batch) * static_cast<double>((rp.a ? p.m : 0) + (rp.b ? p.n : 0)) * static_cast<double>(p.k) : 0.0;
     const int f32_shape = f32 ? choose_f32_kernel(p, repack || takes_f32_ring(p, a, b), repacked) : -1;
     if (repack && f32_shape < 0) {
@@ -854,10 +859,9 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const int rows_per_wave = forced_rows == 1 || forced_rows == 2 || forced_rows == 4 ? forced_rows : (p.m >= 2 && w_elems >= (int64_t(64) << 20)) ? 2 : 1;
         const unsigned blocks = static_cast<unsigned>((p.n + 4 * rows_per_wave - 1) / (4 * rows_per_wave));
         launch_skinny(k, static_cast<int>(p.m), rows_per_wave, blocks, s);
-    } else if (half && takes_half_kernels(p)) {
+    } else if (const HalfKernel *k = half_kernel()) {
         const bool aligned = half_aligned(p, a, b), bf = p.dtype == AXHIP_DTYPE_BF16;
-        const HalfKernel &k = choose_half_kernel(p, aligned);
-        rc = k.kind == HalfKernel::BIG256 ? launch_big(g, bf, static_cast<int>(p.batch), s) : launch_half(p, a, b, c, k, aligned, bf, s);
+        rc = k->kind == HalfKernel::BIG256 ? launch_big(g, bf, static_cast<int>(p.batch), s) : launch_half(p, a, b, c, *k, aligned, bf, s);
         if (rc) return rc;
     } else if (f32_shape >= 0) {
         rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, static_cast<int>(p.batch), s);

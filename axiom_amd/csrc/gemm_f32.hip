@@ -199,7 +199,7 @@ template <bool NN, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, i
     static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     AXHIP_CHECK_HIP(configured);
     const int64_t tiles = static_cast<int64_t>((g.M + 16 * MI - 1) / (16 * MI)) * ((g.N + 16 * NJ - 1) / (16 * NJ));
-    AXHIP_REQUIRE(tiles < (int64_t(1) << 27), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+    AXHIP_REQUIRE(launch_fits(tiles + 7, 64 * F32_WAVES), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * ((tiles + 7) / 8)), static_cast<unsigned>(batch)), dim3(64 * F32_WAVES), lds, s, g);
     return AXHIP_OK;
 }

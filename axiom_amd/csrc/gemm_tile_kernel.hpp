@@ -419,7 +419,7 @@ int launch_tile_kernel(const TileArgs &g, int batch, hipStream_t s) {
     AXHIP_CHECK_HIP(configured);
     constexpr int TM = 16 * MI * WM, TN = 64 * WN;
     const int64_t tiles = static_cast<int64_t>((g.M + TM - 1) / TM) * ((g.N + TN - 1) / TN);
-    AXHIP_REQUIRE(tiles < (int64_t(1) << 27), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+    AXHIP_REQUIRE(launch_fits(tiles + 7, 64 * WM * WN * WK), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * ((tiles + 7) / 8)), static_cast<unsigned>(batch)), dim3(64 * WM * WN * WK), lds, s, g);
     return AXHIP_OK;
 }

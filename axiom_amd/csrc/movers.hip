@@ -1412,10 +1412,12 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
             const int64_t narrow = std::min(t.nJ, t.nL);
             const bool together = es == 2 ? !lines || narrow <= 128 : !lines && narrow > 64;
             // (output rows that one large tile holds whole keep it: bf16 [134, 104, 2624] 32.5 us against 37.6)
-            const int nv = together && !(es == 2 && t.nL > 64 && t.nL <= 128) ? 8 : 16;
-            const int64_t edge = nv * (16 / es);
-            t.tiles_j = (t.nJ + edge - 1) / edge; t.tiles_l = (t.nL + edge - 1) / edge;
-            blocks = blocks / (((t.nJ + 63) / 64) * ((t.nL + 63) / 64)) * t.tiles_j * t.tiles_l;
+            int nv = together && !(es == 2 && t.nL > 64 && t.nL <= 128) ? 8 : 16;
+            const int64_t others = blocks / (t.tiles_j * t.tiles_l);
+            auto tiles = [&](int64_t extent) { return (extent + nv * (16 / es) - 1) / (nv * (16 / es)); };
+            if (!launch_fits(others * tiles(t.nJ) * tiles(t.nL) + 8, 256)) nv = 16; // (small tiles: four times as many)
+            t.tiles_j = tiles(t.nJ); t.tiles_l = tiles(t.nL);
+            blocks = others * t.tiles_j * t.tiles_l;
             AXHIP_REQUIRE(blocks < (int64_t(1) << 31) - 8, AXHIP_ERR_UNSUPPORTED, "axhip_strided_copy: view too large");
             t.blocks = static_cast<uint32_t>(blocks);
             t.per_xcd = together ? (t.blocks + 7) / 8 : 0;
@@ -1921,7 +1923,7 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
             const int TXv = 1 << tx_log2, TYv = (narrow ? 256 : 1024) >> tx_log2;
             const int64_t tiles = outer * ((ivecs + TXv - 1) / TXv);
             const int64_t nblocks = round_up8(tiles, tx_log2 < 3 ? 3 - tx_log2 : 0);
-            if (nblocks < (int64_t(1) << 31)) {
+            if (launch_fits(nblocks, narrow ? 256 : 1024)) { // (else the two-sweep kernel, whose work-groups take several tiles)
                 const bool few = (axis + TYv - 1) / TYv <= 4; // rows per thread
                 const int n = static_cast<int>(axis);
 #define AXHIP_SMT_R(LOG, DT, R, T) hipLaunchKernelGGL((softmax_axis_tile_kernel<LOG, DT, R, T>), dim3(static_cast<unsigned>(nblocks)), dim3(T), 0, s, src, dst, outer, inner, n, tx_log2)

@@ -1710,7 +1710,7 @@ DirectPlan direct_plan(const AxhipSdpaParams &p, bool has_mask) {
     const bool half = p.dtype == AXHIP_DTYPE_BF16 || p.dtype == AXHIP_DTYPE_F16;
     const int64_t slices = static_cast<int64_t>(p.batch) * p.heads;
     if (!half || has_mask || p.is_causal || p.seq_q <= 0 || p.seq_q > DIRECT_ROWS || p.seq_kv <= 0 || p.head_dim <= 0 || p.head_dim > 128 ||
-        p.head_dim % 8 != 0 || slices <= 0 || slices >= (int64_t(1) << 24) || !sdpa_decode_split)
+        p.head_dim % 8 != 0 || slices <= 0 || !launch_fits(slices, 64 * DIRECT_WAVES) || !sdpa_decode_split)
         return d;
     d.on = true;
     const int D = p.head_dim <= 64 ? 64 : 128;
