@@ -842,7 +842,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     const bool f32_nt = p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && al16(a) && al16(b);
     // (the kernel carries leading dimensions as 32-bit element counts)
     const bool ld32 = p.lda < (int64_t(1) << 31) && p.ldb < (int64_t(1) << 31) && p.ldc < (int64_t(1) << 31);
-    if (((half && nt) || f32_nt) && p.batch == 1 && skinny_pays && p.k >= 256 && p.n < (1 << 30) && p.k < (1 << 30) && ld32 && skinny_enabled()) {
+    if (((half && nt) || f32_nt) && p.batch == 1 && skinny_pays && p.k >= 256 && launch_fits(p.n / 4 + 1, 256) && p.k < (1 << 30) && ld32 && skinny_enabled()) {
         // a decoding step: bound by one read of W
         SkinnyArgs k{};
         k.x = a; k.w = b; k.c = c; k.bias = p.bias; k.residual = p.residual;
@@ -880,6 +880,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
             }
             const int tiles_m = static_cast<int>((p.m + tm_rows - 1) / tm_rows), tiles_n = static_cast<int>((p.n + tn_cols - 1) / tn_cols);
             const int per_xcd = (tiles_m * tiles_n + 7) / 8;
+            AXHIP_REQUIRE(launch_fits(int64_t(8) * per_xcd, 256), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
             hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(256), lds_bytes, s, g, tiles_m, tiles_n);
             return AXHIP_OK;
         };
@@ -897,6 +898,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     } else {
         dim3 grid(static_cast<unsigned>((p.n + 15) / 16), static_cast<unsigned>((p.m + 15) / 16), static_cast<unsigned>(p.batch));
         AXHIP_REQUIRE(grid.y < 65536, AXHIP_ERR_UNSUPPORTED, "axhip_gemm: m too large for the generic kernel");
+        AXHIP_REQUIRE(launch_fits((p.n + 15) / 16, 16 * 16), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: n too large for the generic kernel");
         hipLaunchKernelGGL(gemm_generic_kernel, grid, dim3(256), 0, s, g);
     }
     AXHIP_CHECK_HIP(hipGetLastError());

@@ -108,7 +108,8 @@ struct TransposeArgs {
     int src_dtype, dst_dtype, n_other;
     int64_t nJ, nL, src_stride_l, dst_stride_j; // the source stride of J and the destination stride of L are 1
     int64_t tiles_j, tiles_l;
-    uint32_t blocks, per_xcd; // tiles in all; of each of the eight XCDs, if each is to take neighbouring ones
+    int64_t first;            // tile of this launch (a view of very many tiles takes several)
+    uint32_t blocks, per_xcd; // tiles of this launch; of each of the eight XCDs, if each is to take neighbouring ones
     int64_t oshape[AXHIP_MAX_DIMS], osrc[AXHIP_MAX_DIMS], odst[AXHIP_MAX_DIMS];
 };
 
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs 
     __shared__ __attribute__((aligned(16))) uint32_t tile[T * NV * 4];
     const uint32_t t = a.per_xcd ? blockIdx.x % 8 * a.per_xcd + blockIdx.x / 8 : blockIdx.x;
     if (t >= a.blocks) return;
-    int64_t b = t;
+    int64_t b = a.first + t;
     const int64_t tl = b % a.tiles_l;
     b /= a.tiles_l;
     // (work-groups that run side by side take tiles along a diagonal: with a power of two as row length, tiles of one
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs 
 
 __global__ __launch_bounds__(256) void transpose_copy_kernel(const TransposeArgs a) {
     __shared__ float tile[64][65];
-    int64_t b = blockIdx.x;
+    int64_t b = a.first + blockIdx.x;
     const int64_t tl = b % a.tiles_l;
     b /= a.tiles_l;
     const int64_t tj = b % a.tiles_j;
@@ -1400,6 +1401,8 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
         };
         const int lg = side(t.nJ, t.src_stride_l, t.osrc, src), sg = side(t.nL, t.dst_stride_j, t.odst, dst);
         const bool whole = src_dtype == dst_dtype && src_dtype != AXHIP_DTYPE_U8;
+        constexpr int64_t PER_LAUNCH = int64_t(1) << 23;
+        static_assert(launch_fits(PER_LAUNCH, 256), "tiles of a launch");
         static const bool vec_tiles = [] { const char *e = getenv("AXHIP_TRANSPOSE_VEC"); return !(e && e[0] == '0'); }();
         if (whole && vec_tiles) {
             // Rows of the output that start inside a 128-byte line make neighbouring tiles write parts of the same lines:
@@ -1412,16 +1415,10 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
             const int64_t narrow = std::min(t.nJ, t.nL);
             const bool together = es == 2 ? !lines || narrow <= 128 : !lines && narrow > 64;
             // (output rows that one large tile holds whole keep it: bf16 [134, 104, 2624] 32.5 us against 37.6)
-            int nv = together && !(es == 2 && t.nL > 64 && t.nL <= 128) ? 8 : 16;
-            const int64_t others = blocks / (t.tiles_j * t.tiles_l);
-            auto tiles = [&](int64_t extent) { return (extent + nv * (16 / es) - 1) / (nv * (16 / es)); };
-            if (!launch_fits(others * tiles(t.nJ) * tiles(t.nL) + 8, 256)) nv = 16; // (small tiles: four times as many)
-            t.tiles_j = tiles(t.nJ); t.tiles_l = tiles(t.nL);
-            blocks = others * t.tiles_j * t.tiles_l;
-            AXHIP_REQUIRE(blocks < (int64_t(1) << 31) - 8, AXHIP_ERR_UNSUPPORTED, "axhip_strided_copy: view too large");
-            t.blocks = static_cast<uint32_t>(blocks);
-            t.per_xcd = together ? (t.blocks + 7) / 8 : 0;
-            const dim3 grid(t.per_xcd ? 8 * t.per_xcd : t.blocks);
+            const int nv = together && !(es == 2 && t.nL > 64 && t.nL <= 128) ? 8 : 16;
+            const int64_t edge = nv * (16 / es);
+            t.tiles_j = (t.nJ + edge - 1) / edge; t.tiles_l = (t.nL + edge - 1) / edge;
+            blocks = blocks / (((t.nJ + 63) / 64) * ((t.nL + 63) / 64)) * t.tiles_j * t.tiles_l;
 #define AXHIP_TRANSPOSE_NV(ES, LG, SG)                                                                                   \
     do {                                                                                                                 \
         if (nv == 16) hipLaunchKernelGGL((transpose_vec_kernel<ES, LG, SG, 16>), grid, dim3(256), 0, s, t);              \
@@ -1435,15 +1432,20 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
         else if (sg == 16) AXHIP_TRANSPOSE_NV(ES, 8, 16);                                                                \
         else AXHIP_TRANSPOSE_NV(ES, 8, 8);                                                                               \
     } while (0)
-            if (es == 2) AXHIP_TRANSPOSE(2);
-            else AXHIP_TRANSPOSE(4);
+            for (t.first = 0; t.first < blocks; t.first += PER_LAUNCH) {
+                t.blocks = static_cast<uint32_t>(std::min(PER_LAUNCH, blocks - t.first));
+                t.per_xcd = together ? (t.blocks + 7) / 8 : 0;
+                const dim3 grid(t.per_xcd ? 8 * t.per_xcd : t.blocks);
+                if (es == 2) AXHIP_TRANSPOSE(2);
+                else AXHIP_TRANSPOSE(4);
+            }
 #undef AXHIP_TRANSPOSE
 #undef AXHIP_TRANSPOSE_NV
             AXHIP_CHECK_HIP(hipGetLastError());
             return AXHIP_OK;
         }
-        AXHIP_REQUIRE(blocks < (int64_t(1) << 31), AXHIP_ERR_UNSUPPORTED, "axhip_strided_copy: view too large");
-        hipLaunchKernelGGL(transpose_copy_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, t);
+        for (t.first = 0; t.first < blocks; t.first += PER_LAUNCH)
+            hipLaunchKernelGGL(transpose_copy_kernel, dim3(static_cast<unsigned>(std::min(PER_LAUNCH, blocks - t.first))), dim3(256), 0, s, t);
     } else {
         const int64_t blocks = std::min<int64_t>((a.total + 255) / 256, 256 * 64);
         const dim3 grid(static_cast<unsigned>(blocks));

@@ -390,7 +390,11 @@ int axhip_fused_rows(const AxhipRowsProgram *program, void *stream) {
         AXHIP_CHECK_HIP(hipGetLastError());
         return AXHIP_OK;
     }
-    // ... or the interpreter
+    // ... or the interpreter, a work-group of (at least) 256 threads for 256 / group rows, or of 1024 for a streamed row
+    if (pl.kind == RowsPlan::RESIDENT || pl.kind == RowsPlan::STREAMED) {
+        const int64_t threads = pl.kind == RowsPlan::STREAMED ? 1024 : std::max(256, pl.group), rows = pl.kind == RowsPlan::STREAMED ? 1 : threads / pl.group;
+        AXHIP_REQUIRE(launch_fits((P.rows + rows - 1) / rows, threads), AXHIP_ERR_UNSUPPORTED, "axhip_fused_rows: %lld rows without a compiled kernel", static_cast<long long>(P.rows));
+    }
     rc = pl.e == 8 ? launch_plan_e<8>(P, pl, s) : pl.e == 4 ? launch_plan_e<4>(P, pl, s) : launch_plan_e<1>(P, pl, s);
     if (rc) return rc;
     AXHIP_CHECK_HIP(hipGetLastError());

@@ -1850,7 +1850,7 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
 
     if (kind == SdpaKind::MFMA) {
         a.nqb = (p.seq_q + BM - 1) / BM;
-        AXHIP_REQUIRE(static_cast<int64_t>(a.nqb) * p.batch * p.heads < (int64_t(1) << 31), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");
+        AXHIP_REQUIRE(launch_fits(static_cast<int64_t>(a.nqb) * p.batch * p.heads, 256), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");
         const bool bf = p.dtype == AXHIP_DTYPE_BF16;
         // A decoding step -- one block of query rows, few (batch, head) slices, a long key sequence -- would give the
         // chip a work-group per slice: the keys are split between work-groups instead (flash decoding), partial
@@ -1979,7 +1979,7 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         if (sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4) split = sdpa_f32_split;
         const int bmw = 128 / split;
         a.nqb = (p.seq_q + bmw - 1) / bmw;
-        AXHIP_REQUIRE(static_cast<int64_t>(a.nqb) * p.batch * p.heads < (int64_t(1) << 31), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");
+        AXHIP_REQUIRE(launch_fits(static_cast<int64_t>(a.nqb) * p.batch * p.heads, 256), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");
         rc = p.head_dim <= 32 ? launch_mfma_f32_d<32>(a, split, s) : p.head_dim <= 64 ? launch_mfma_f32_d<64>(a, split, s) : launch_mfma_f32_d<128>(a, split, s);
         if (rc) return rc;
     } else {

@@ -65,9 +65,9 @@ def test_products_of_many_row_tiles(dt, m, n, k):
     assert torch.equal(c[at], want)
 
 
-def test_transposed_copy_of_many_small_slices():
-    """fp32 slices of two or three tiles each way: 63 GiB in and out, as many tiles as fit only when they are large."""
-    outer, a, b = 1 << 21, 65, 65
+@pytest.mark.parametrize("outer,a,b", [(1 << 21, 65, 65), ((1 << 24) + 300, 16, 17)])
+def test_transposed_copy_of_many_small_slices(outer, a, b):
+    """fp32 slices of several tiles (63 GiB in and out) and of one, of which there are more than a launch may have."""
     x = torch.empty(outer, a, b, device="cuda").random_(0, 1 << 20)
     y = torch.empty(outer, b, a, device="cuda")
     gh.sync()
