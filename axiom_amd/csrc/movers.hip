@@ -859,25 +859,48 @@ template <int V, typename F> __device__ __forceinline__ void across_lanes(float 
 }
 // work-groups that a launch of `total` takes where 2^share neighbours go to one XCD
 __host__ __device__ __forceinline__ int64_t round_up8(int64_t total, int share) { return share == 0 ? total : (total + (8 << share) - 1) & ~static_cast<int64_t>((8 << share) - 1); }
+__device__ __forceinline__ int64_t axis_group(int64_t b, int share) { return (((b >> (3 + share)) * 8 + (b & 7)) << share) + ((b >> 3) & ((1 << share) - 1)); }
 __device__ __forceinline__ uint4_t axis_load(const char *at) { return reinterpret_cast<const uint4_unaligned_t *>(at)->v; }
 
+// The (outer, inner) positions as `outer * vecs` columns of one vector each, in groups of `width` (at most 256): `per_slice`
+// groups to a slice, or numbered through (0), the groups running from one slice into the next, so that rows of a few
+// vectors fill them as well as long ones.  2^share neighbours run on the same XCD (work-group b lands on XCD b % 8).
+struct AxisGroups { int64_t count, per_slice; int width, share; };
+struct AxisOrigin { int64_t o, vec; int left; }; // slice and vector of a group's first column, columns it has
+__device__ __forceinline__ AxisOrigin axis_origin(const AxisGroups &groups, int64_t g, int64_t outer, int64_t vecs) {
+    const int64_t num = groups.per_slice ? g : g * groups.width, per = groups.per_slice ? groups.per_slice : vecs;
+    const int64_t o = static_cast<int64_t>(static_cast<uint64_t>(num) / static_cast<uint64_t>(per)), rest = num - o * per;
+    const int64_t vec = groups.per_slice ? rest * groups.width : rest, left = groups.per_slice ? vecs - vec : outer * vecs - num;
+    return {o, vec, static_cast<int>(left < groups.width ? left : groups.width)};
+}
+// Kernel arguments that the first branch does not need would be fetched behind it, one latency later: all at once.
+#define AXHIP_ARGS_NOW(n) asm volatile("" ::"s"(src), "s"(dst), "s"(outer), "s"(inner), "s"(n), "s"(groups.count), "s"(groups.per_slice), "s"(groups.width))
+// Elements from the start of that slice to column c of the group (past the last one: to that one), slices `slice` apart.
+template <int V> __device__ __forceinline__ int64_t axis_column(const AxisOrigin &at, int c, int64_t vecs, int64_t inner, int64_t slice) {
+    int64_t iv = at.vec + min(c, at.left - 1), skipped = 0;
+    if (iv >= vecs) {
+        const uint32_t on = vecs >= 256 ? 1 : static_cast<uint32_t>(iv) / static_cast<uint32_t>(vecs);
+        iv -= on * vecs;
+        skipped = on * slice;
+    }
+    return skipped + (iv * V < inner - V ? iv * V : inner - V);
+}
+
 template <int RED, int DT, int THREADS, bool FLAT>
-__global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int dst_dt, float scale, int tx_log2) {
+__global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int dst_dt, float scale, int tx_log2, AxisGroups groups) {
     constexpr int U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V, NW = THREADS / WAVE;
     __shared__ float red[FLAT ? 1 : NW][FLAT ? 1 : WAVE][V + 1];
     const int TX = 1 << tx_log2, TY = THREADS >> tx_log2;
     const int tid = threadIdx.x, tx = tid & (TX - 1), ty = tid >> tx_log2;
-    const int64_t groups = ((inner + V - 1) / V + TX - 1) >> tx_log2, total = outer * groups, pitch = inner * ES, step = TY * pitch;
-    // (groups narrower than a cache line that share one run on the same XCD: work-group b lands on XCD b % 8)
-    const int share = tx_log2 < 3 ? 3 - tx_log2 : 0; // log2 of the groups per line
-    const int64_t last = round_up8(total, share);
+    const int64_t vecs = (inner + V - 1) / V, pitch = inner * ES, step = TY * pitch;
+    AXHIP_ARGS_NOW(n);
+    const int64_t last = round_up8(groups.count, groups.share);
     for (int64_t b = blockIdx.x; b < last; b += gridDim.x) {
-        const int64_t g = (((b >> (3 + share)) * 8 + (b & 7)) << share) + ((b >> 3) & ((1 << share) - 1));
-        if (g >= total) continue; // (whole work-groups)
-        const int64_t o = g / groups, col0 = ((g - o * groups) << tx_log2) * V;
-        const bool there = col0 + tx * V < inner;
-        const int64_t col = there && col0 + tx * V < inner - V ? col0 + tx * V : inner - V;
-        const char *first = static_cast<const char *>(src) + o * n * pitch + col * ES, *at = first + ty * pitch;
+        const int64_t g = axis_group(b, groups.share);
+        if (g >= groups.count) continue; // (whole work-groups)
+        const AxisOrigin origin = axis_origin(groups, g, outer, vecs);
+        const bool there = tx < origin.left;
+        const char *first = static_cast<const char *>(src) + origin.o * n * pitch + axis_column<V>(origin, tx, vecs, inner, n * inner) * ES, *at = first + ty * pitch;
         float acc[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) acc[e] = red_identity<RED>();
@@ -887,11 +910,12 @@ __global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, v
 #pragma unroll
                 for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? at + u * step : first);
                 __builtin_amdgcn_sched_barrier(0); // (all U loads before the first wait)
-                // (past the axis: row 0 again, which changes no maximum or minimum, and adds zeros to a sum -- no branch, into
+                // (past the axis: row 0 again, one line for all, which changes no maximum or minimum, and adds zeros to a sum -- no branch, into
                 // which the compiler would move the loads)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (RED == AXHIP_RED_SUM) raw[u] = k + u * TY < n ? raw[u] : uint4_t{0, 0, 0, 0};
+                    if (FLAT && k + u >= n) break; // (the same for all threads)
+                    if (!FLAT && RED == AXHIP_RED_SUM) raw[u] = k + u * TY < n ? raw[u] : uint4_t{0, 0, 0, 0};
                     float v[V];
                     arg_unpack<DT>(raw[u], v);
 #pragma unroll
@@ -902,11 +926,12 @@ __global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, v
             if (there) {
 #pragma unroll
                 for (int e = 0; e < V; ++e) acc[e] *= scale;
-                if (((inner | col) & (V - 1)) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-                    store_vec<V>(dst, dst_dt, o * inner + col, acc);
+                const int64_t to = origin.o * inner + axis_column<V>(origin, tx, vecs, inner, inner);
+                if (inner % V == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+                    store_vec<V>(dst, dst_dt, to, acc);
                 } else {
 #pragma unroll
-                    for (int e = 0; e < V; ++e) store_any(dst, dst_dt, o * inner + col + e, acc[e]);
+                    for (int e = 0; e < V; ++e) store_any(dst, dst_dt, to + e, acc[e]);
                 }
             }
         } else {
@@ -922,7 +947,7 @@ __global__ __launch_bounds__(THREADS) void reduce_axis_kernel(const void *src, v
                 float r = red[0][c][e];
 #pragma unroll
                 for (int w = 1; w < NW; ++w) r = red_combine<RED>(r, red[w][c][e]);
-                if (col0 + c * V < inner) store_any(dst, dst_dt, o * inner + min(col0 + c * V, inner - V) + e, r * scale);
+                if (c < origin.left) store_any(dst, dst_dt, origin.o * inner + axis_column<V>(origin, c, vecs, inner, inner) + e, r * scale);
             }
         }
     }
@@ -963,34 +988,26 @@ __device__ __forceinline__ float log_of(float x) { return __builtin_amdgcn_logf(
 // mostly from the caches) and one write.  x - maximum is formed before the factor log2(e): it is exact to one rounding of
 // the difference whatever the magnitude of x, where x log2(e) is off by 6e-5 for x around 1000, and it stays finite for
 // every finite x (a column that holds nothing but the type's lowest value is uniform).
-// HOLD > 0 (with TX = 256, a thread per vector walking the axis alone): the axis has at most HOLD elements and the thread
-// keeps them in registers between the two sweeps -- one read of the input.
-template <bool LOG, int DT, int TX, int HOLD = 0>
+template <bool LOG, int DT, int TX>
 __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *src, int64_t outer, int64_t axis, int64_t inner, void *dst) {
     constexpr int TY = 256 / TX, U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8;
-    static_assert(HOLD == 0 || (TX == 256 && HOLD % U == 0), "rows held in registers: one thread per vector");
     __shared__ float sm[TY][TX][V + 1], sl[TY][TX][V + 1];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
     constexpr int ES = 16 / V;
-    const int64_t groups = ((inner + V - 1) / V + TX - 1) / TX, total = outer * groups, pitch = inner * ES;
+    const int64_t vecs = (inner + V - 1) / V, pitch = inner * ES;
+    const AxisGroups groups{(outer * vecs + TX - 1) / TX, 0, TX, 0};
     const int n = static_cast<int>(axis);
-    for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
-        const int64_t o = g / groups, at = ((g - o * groups) * TX + tx) * V, col = at < inner - V ? at : inner - V;
-        const bool there = at < inner;
-        const char *first = static_cast<const char *>(src) + o * axis * pitch + col * ES;
+    for (int64_t g = blockIdx.x; g < groups.count; g += gridDim.x) {
+        const AxisOrigin origin = axis_origin(groups, g, outer, vecs);
+        const int64_t at = origin.o * axis * inner + axis_column<V>(origin, tx, vecs, inner, axis * inner);
+        const bool there = tx < origin.left;
+        const char *first = static_cast<const char *>(src) + at * ES;
         const int64_t step = TY * pitch;
         float m[V], l[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             m[e] = -INFINITY;
             l[e] = 0.0f;
-        }
-        uint4_t keep[HOLD > 0 ? HOLD : 1];
-        if constexpr (HOLD > 0) {
-            if (there) {
-#pragma unroll
-                for (int k = 0; k < HOLD; ++k) keep[k] = axis_load(first + min(k, n - 1) * pitch);
-            }
         }
         auto gather = [&](int k, const uint4_t (&raw)[U]) { // running maximum and rescaled sum over U axis elements
                 float t[U][V];
@@ -1012,21 +1029,12 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                 }
         };
         if (there) {
-            if constexpr (HOLD > 0) {
+            const char *from = first + ty * pitch;
+            for (int k = ty; k < n; k += TY * U, from += U * step) {
+                uint4_t raw[U];
 #pragma unroll
-                for (int k = 0; k < HOLD; k += U)
-                    if (k < n) {
-                        const uint4_t raw[U] = {keep[k], keep[k + 1], keep[k + 2], keep[k + 3]};
-                        gather(k, raw);
-                    }
-            } else {
-                const char *from = first + ty * pitch;
-                for (int k = ty; k < n; k += TY * U, from += U * step) {
-                    uint4_t raw[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
-                    gather(k, raw);
-                }
+                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
+                gather(k, raw);
             }
         }
         __syncthreads(); // the previous group's pairs have been read
@@ -1055,27 +1063,69 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                         arg_unpack<DT>(raw[u], v);
 #pragma unroll
                         for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : exp_of(v[e] - shift[e]) * inv[e];
-                        store_vec<V, true>(dst, DT, (o * axis + k + u * TY) * inner + col, v);
+                        store_vec<V, true>(dst, DT, at + (k + u * TY) * inner, v);
                     }
         };
         if (there) {
-            if constexpr (HOLD > 0) {
+            const char *from = first + ty * pitch;
+            for (int k = ty; k < n; k += TY * U, from += U * step) {
+                uint4_t raw[U];
 #pragma unroll
-                for (int k = 0; k < HOLD; k += U)
-                    if (k < n) {
-                        const uint4_t raw[U] = {keep[k], keep[k + 1], keep[k + 2], keep[k + 3]};
-                        emit(k, raw);
-                    }
-            } else {
-                const char *from = first + ty * pitch;
-                for (int k = ty; k < n; k += TY * U, from += U * step) {
-                    uint4_t raw[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
-                    emit(k, raw);
-                }
+                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
+                emit(k, raw);
             }
         }
+    }
+}
+
+// An axis of at most HOLD elements, read once: a thread per vector holds it in registers, nothing to merge.
+template <bool LOG, int DT, int HOLD>
+__global__ __launch_bounds__(64) void softmax_axis_short_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, AxisGroups groups) {
+    constexpr int V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V;
+    const int64_t vecs = (inner + V - 1) / V, pitch = inner * ES, last = round_up8(groups.count, groups.share);
+    AXHIP_ARGS_NOW(n);
+    for (int64_t b = blockIdx.x; b < last; b += gridDim.x) {
+        const int64_t g = axis_group(b, groups.share);
+        if (g >= groups.count) continue;
+        const AxisOrigin origin = axis_origin(groups, g, outer, vecs);
+        if (static_cast<int>(threadIdx.x) >= origin.left) continue;
+        const int64_t at = origin.o * n * inner + axis_column<V>(origin, threadIdx.x, vecs, inner, n * inner);
+        const char *first = static_cast<const char *>(src) + at * ES;
+        uint4_t raw[HOLD];
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) raw[k] = axis_load(first + min(k, n - 1) * pitch); // (no branch: all of them before the first wait)
+        float m[V], l[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            m[e] = -INFINITY;
+            l[e] = 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) { // (past the axis: its last element again, which changes no maximum)
+            float t[V];
+            arg_unpack<DT>(raw[k], t);
+#pragma unroll
+            for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
+        }
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k)
+            if (k < n) {
+                float t[V];
+                arg_unpack<DT>(raw[k], t);
+#pragma unroll
+                for (int e = 0; e < V; ++e) l[e] += exp_of(t[e] - m[e]);
+            }
+#pragma unroll
+        for (int e = 0; e < V; ++e) l[e] = LOG ? log_of(l[e]) : 1.0f / l[e];
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k)
+            if (k < n) {
+                float v[V];
+                arg_unpack<DT>(raw[k], v);
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - m[e] - l[e] : exp_of(v[e] - m[e]) * l[e];
+                store_vec<V, true>(dst, DT, at + k * inner, v);
+            }
     }
 }
 
@@ -1087,22 +1137,36 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
 // than a cache line: the blocks that share the lines run on the same XCD (block b lands on XCD b % 8), so the second one
 // finds them in that L2.
 template <bool LOG, int DT, int RPT, int THREADS>
-__global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int tx_log2) {
+__global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *src, void *dst, int64_t outer, int64_t inner, int n, int tx_log2, AxisGroups groups) {
     constexpr int V = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / V, NW = THREADS / WAVE;
     __shared__ float red[NW][WAVE][V + 1];
     const int TX = 1 << tx_log2, TY = THREADS >> tx_log2;
     const int tid = threadIdx.x, tx = tid & (TX - 1), ty = tid >> tx_log2, wave = tid / WAVE;
-    const int64_t ctiles = ((inner + V - 1) / V + TX - 1) >> tx_log2, tiles = outer * ctiles, pitch = inner * ES;
-    const int share = tx_log2 < 3 ? 3 - tx_log2 : 0; // log2 of the blocks per cache line of a row
-    const uint32_t slot = blockIdx.x / 8, xcd = blockIdx.x % 8;
-    const int64_t tile = (static_cast<int64_t>((slot >> share) * 8 + xcd) << share) + (slot & ((1 << share) - 1));
-    if (tile >= tiles) return; // (whole block)
-    const int64_t o = tile / ctiles, at = (((tile - o * ctiles) << tx_log2) + tx) * V, col = at < inner - V ? at : inner - V;
-    const bool there = at < inner;
-    const char *first = static_cast<const char *>(src) + o * n * pitch + col * ES;
+    const int64_t vecs = (inner + V - 1) / V, pitch = inner * ES, tile = axis_group(blockIdx.x, groups.share);
+    AXHIP_ARGS_NOW(n);
+    if (tile >= groups.count) return; // (whole block)
+    const AxisOrigin origin = axis_origin(groups, tile, outer, vecs);
+    const int64_t at = origin.o * n * inner + axis_column<V>(origin, tx, vecs, inner, n * inner);
+    const bool there = tx < origin.left;
+    const char *first = static_cast<const char *>(src) + at * ES;
     uint4_t raw[RPT];
 #pragma unroll
     for (int r = 0; r < RPT; ++r) raw[r] = axis_load(ty + r * TY < n ? first + ty * pitch + r * (TY * pitch) : first);
+    // fp32, or few rows: the values stay unpacked, and the exponentials of a softmax take their place
+    constexpr bool KEEP = RPT * V <= 64;
+    float kept[KEEP ? RPT : 1][V];
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) arg_unpack<DT>(raw[r], kept[r]);
+    }
+    auto value = [&](int r, float (&v)[V]) {
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[e] = kept[r][e];
+        } else {
+            arg_unpack<DT>(raw[r], v);
+        }
+    };
     // column statistic over the block: lanes of a wave that share tx, then the waves -- a thread per value merges them and
     // hands the result to all (every thread merging its V columns itself is 16 V LDS reads of straight-line code, twice)
     auto across = [&](float (&x)[V], bool is_max) { // (TX <= WAVE)
@@ -1135,7 +1199,7 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float t[V];
-            arg_unpack<DT>(raw[r], t);
+            value(r, t);
 #pragma unroll
             for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
         }
@@ -1147,9 +1211,13 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float t[V];
-            arg_unpack<DT>(raw[r], t);
+            value(r, t);
 #pragma unroll
-            for (int e = 0; e < V; ++e) l[e] += exp_of(t[e] - ref[e]);
+            for (int e = 0; e < V; ++e) {
+                const float p = exp_of(t[e] - ref[e]);
+                l[e] += p;
+                if (KEEP && !LOG) kept[r][e] = p;
+            }
         }
     across(l, false);
     float shift[V], inv[V]; // result = e^(x - shift) * inv, or x - shift - inv with the logarithm of the sum as inv
@@ -1163,10 +1231,10 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float v[V];
-            arg_unpack<DT>(raw[r], v);
+            value(r, v);
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : exp_of(v[e] - shift[e]) * inv[e];
-            store_vec<V, true>(dst, DT, (o * n + ty + r * TY) * inner + col, v);
+            for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : (KEEP ? v[e] : exp_of(v[e] - shift[e])) * inv[e];
+            store_vec<V, true>(dst, DT, at + (ty + r * TY) * inner, v);
         }
 }
 
@@ -1189,35 +1257,67 @@ __global__ __launch_bounds__(256) void softmax_strided_kernel(const void *src, i
     }
 }
 
+// Groups of 2^tx_log2 lanes over `cols` columns, rows of `vecs` vectors.  They keep to slices where that leaves few lanes
+// without a column (an eighth where a row takes several groups, three eighths where a group takes several rows: what it
+// reads is then one piece of memory, sum of bf16 [5242, 64, 100] 15.1 -> 12.2 us), and where there are few groups, whose
+// time is latency (sum of bf16 [3, 333, 333] 4.8 us numbered through, 4.3 slice by slice).
+// On one XCD run the neighbours that share a cache line, and 16 where rows are no whole number of lines, so that the lines
+// at the groups' edges are read and written in one L2 (softmax fp32 [5242, 64, 100] 80 -> 55 us, sum 27.7 -> 21.5), if there
+// are enough to go round.
+AxisGroups axis_groups(int tx_log2, int64_t outer, int64_t vecs, int64_t row_bytes) {
+    const int lanes = 1 << tx_log2, line = tx_log2 < 3 ? 3 - tx_log2 : 0;
+    const int64_t cols = outer * vecs;
+    AxisGroups g{(cols + lanes - 1) >> tx_log2, 0, lanes, 0};
+    const bool few = g.count < 1024;
+    if (vecs >= lanes) {
+        const int64_t per = (vecs + lanes - 1) >> tx_log2;
+        if (few || per * lanes * 8 <= vecs * 9) {
+            g.per_slice = per;
+            g.count = outer * per;
+        }
+    } else if (const int whole = lanes / static_cast<int>(vecs) * static_cast<int>(vecs); few || whole * 8 >= lanes * 5) {
+        g.width = whole;
+        g.count = (cols + whole - 1) / whole;
+    }
+    g.share = row_bytes % 128 != 0 && g.count >= 4096 ? std::max(line, 4) : line;
+    return g;
+}
+
 // one launch: RED is sum, max or min; the result is multiplied by `scale`
 int launch_reduce_axis(const void *src, int dtype, int64_t outer, int64_t axis, int64_t inner, int red, float scale, void *dst, int dst_dtype, hipStream_t s) {
     const int es = dtype == AXHIP_DTYPE_F32 ? 4 : 2;
     const bool bytes = dtype == AXHIP_DTYPE_U8 || dst_dtype == AXHIP_DTYPE_U8;
     if (red != AXHIP_RED_PROD && !bytes && inner >= 16 / es) { // (products, truth values, rows shorter than a vector: the element-wise kernel)
-        const int64_t vecs = (inner + 16 / es - 1) / (16 / es);
-        // a short axis with plenty of results: a thread per vector walks it alone (no merge through LDS)
-        const bool flat = axis <= 32 && outer * ((vecs + 255) / 256) >= 1024;
+        const int64_t vecs = (inner + 16 / es - 1) / (16 / es), cols = outer * vecs;
+        // A thread per vector walks a short axis alone (no merge through LDS): up to four elements always (bf16 [1.9 M, 2, 9]
+        // 43 us, [4096, 2, 4096] 14), up to eight with plenty of results, up to 32 where the rows are whole cache lines as well
+        // (bf16 [1927, 17, 1024] 13.3 us against 15.1); other rows are read in longer runs by thread rows that share a slice
+        // (bf16 [286790, 13, 9] 25.6 us, 35.6 by a thread each).
+        const bool flat = axis <= 4 || (axis <= 8 && cols >= 64 * 1024) || (axis <= 32 && cols >= 128 * 1024 && inner * es % 128 == 0);
         // 32-vector column groups from 512 of them on (sum over axis 1 of bf16 [256, 1024, 512] 44.5 -> 38.2 us, 75 -> 88 %
-        // of the HBM peak against 8-vector ones; AXHIP_REDUCE_AXIS_WIDE_FROM=<n>, read once, moves the threshold), never
-        // wider than the row, and no more thread rows than the axis gives four elements each
+        // of the HBM peak against 8-vector ones; AXHIP_REDUCE_AXIS_WIDE_FROM=<n>, read once, moves the threshold), and no
+        // more thread rows than the axis gives four elements each
         static const int wide_from = [] { const char *e = getenv("AXHIP_REDUCE_AXIS_WIDE_FROM"); return e ? atoi(e) : 512; }();
-        int tx_log2 = outer * ((vecs + 31) / 32) >= wide_from ? 5 : 3;
-        while (tx_log2 > 3 && ((vecs + (1 << tx_log2) - 1) >> tx_log2 << tx_log2) * 8 > vecs * 9) --tx_log2; // (an eighth of the lanes idle at most)
-        while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= vecs) --tx_log2;
-        while (tx_log2 < 6 && (256 >> tx_log2) * 4 > axis && (int64_t(1) << tx_log2) < vecs) ++tx_log2;
+        auto groups_of = [&](int log2) { return (cols + (int64_t(1) << log2) - 1) >> log2; };
+        int tx_log2 = groups_of(5) >= wide_from ? 5 : 3;
+        while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= cols) --tx_log2;
+        while (tx_log2 > 3 && (256 >> (tx_log2 - 1)) * 3 <= axis && (int64_t(1) << (tx_log2 - 1)) >= vecs) --tx_log2;
+        while (tx_log2 < 6 && (256 >> tx_log2) * 4 > axis && (int64_t(1) << tx_log2) < cols) ++tx_log2;
+        // (few groups for the CUs: narrower ones, as far as they hold a row and half of the threads have an element)
+        while (tx_log2 > 0 && groups_of(tx_log2) <= 512 && (256 >> (tx_log2 - 1)) <= 2 * axis && (int64_t(1) << (tx_log2 - 1)) >= vecs) --tx_log2;
         if (flat) tx_log2 = 8;
-        auto groups_of = [&](int log2) { return outer * ((vecs + (int64_t(1) << log2) - 1) >> log2); };
         // fewer work-groups than CUs: larger ones, as far as the axis has elements for them, and narrower ones, as far as
         // a thread still has more than eight
         const bool large = !flat && groups_of(tx_log2) <= 256 && axis >= (256 >> tx_log2) * 4;
         while (large && tx_log2 > 1 && groups_of(tx_log2) <= 128 && axis > (1024 >> tx_log2) * 8) --tx_log2;
-        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(round_up8(groups_of(tx_log2), tx_log2 < 3 ? 3 - tx_log2 : 0), 256 * 64));
+        const AxisGroups groups = axis_groups(tx_log2, outer, vecs, inner * es);
+        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(round_up8(groups.count, groups.share), 256 * 64));
         const int n = static_cast<int>(axis);
 #define AXHIP_RED_AXIS(RED, DT)                                                                                                            \
     do {                                                                                                                                   \
-        if (flat) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, true>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2);        \
-        else if (large) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 1024, false>), dim3(blocks), dim3(1024), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2); \
-        else hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, false>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2);             \
+        if (flat) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, true>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2, groups);        \
+        else if (large) hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 1024, false>), dim3(blocks), dim3(1024), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2, groups); \
+        else hipLaunchKernelGGL((reduce_axis_kernel<RED, DT, 256, false>), dim3(blocks), dim3(256), 0, s, src, dst, outer, inner, n, dst_dtype, scale, tx_log2, groups);             \
     } while (0)
 #define AXHIP_RED_VEC(RED)                                                                                                                 \
     do {                                                                                                                                   \
@@ -1904,7 +2004,34 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
     // row's last two vectors share out twice, and the second of them may find the first one's results there.
     const bool shared_columns = src == dst && inner % (16 / es) != 0;
     if (inner >= 16 / es && !shared_columns) {
-        const int64_t ivecs = (inner + 16 / es - 1) / (16 / es), bytes = outer * axis * inner * es;
+        const int64_t vecs = (inner + 16 / es - 1) / (16 / es), cols = outer * vecs, bytes = outer * axis * inner * es;
+        const int n = static_cast<int>(axis);
+        // A thread per vector holds a short axis: up to eight elements always, up to 24 (fp32: 20) where that fills the chip.
+        if (axis <= 8 || (axis <= (es == 4 ? 20 : 24) && cols >= 64 * 1024)) {
+            const AxisGroups groups = axis_groups(6, outer, vecs, inner * es);
+            const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(round_up8(groups.count, groups.share), 256 * 256));
+#define AXHIP_SMS_H(LOG, DT, H) hipLaunchKernelGGL((softmax_axis_short_kernel<LOG, DT, H>), dim3(blocks), dim3(64), 0, s, src, dst, outer, inner, n, groups)
+#define AXHIP_SMS_DT(LOG, DT)                                                                                                              \
+    do {                                                                                                                                   \
+        if (axis <= 4) AXHIP_SMS_H(LOG, DT, 4);                                                                                            \
+        else if (axis <= 8) AXHIP_SMS_H(LOG, DT, 8);                                                                                       \
+        else if (axis <= 16) AXHIP_SMS_H(LOG, DT, 16);                                                                                     \
+        else AXHIP_SMS_H(LOG, DT, 24);                                                                                                     \
+    } while (0)
+#define AXHIP_SMS(LOG)                                                                                                                     \
+    do {                                                                                                                                   \
+        if (dtype == AXHIP_DTYPE_F32) AXHIP_SMS_DT(LOG, AXHIP_DTYPE_F32);                                                                  \
+        else if (dtype == AXHIP_DTYPE_F16) AXHIP_SMS_DT(LOG, AXHIP_DTYPE_F16);                                                             \
+        else AXHIP_SMS_DT(LOG, AXHIP_DTYPE_BF16);                                                                                          \
+    } while (0)
+            if (is_log) AXHIP_SMS(true);
+            else AXHIP_SMS(false);
+#undef AXHIP_SMS
+#undef AXHIP_SMS_DT
+#undef AXHIP_SMS_H
+            AXHIP_CHECK_HIP(hipGetLastError());
+            return AXHIP_OK;
+        }
         // An axis that a block can hold is read once.  Up to 512 elements: four rows per thread (256 threads up to 256
         // elements, so that several blocks share a CU), as wide as that allows; bf16 [64, 256, 2048] 72 -> 40 us, fp32
         // [256, 128, 1024] 76 -> 58 us against the two-sweep kernel.  Longer axes of large arrays take 1024-thread blocks of
@@ -1915,20 +2042,21 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
         // sweeps are two trips to memory and little else, take four rows per thread whatever the axis: the code of sixteen
         // takes longer to arrive than the array.
         const bool small = bytes <= (int64_t(24) << 20);
-        const bool tile_pays = axis <= 512 || (axis <= 4096 && (small || (dtype == AXHIP_DTYPE_F32 ? axis <= 2048 || outer * ((ivecs + 7) / 8) < 512 : axis >= 1024)));
+        const bool tile_pays = axis <= 512 || (axis <= 4096 && (small || (dtype == AXHIP_DTYPE_F32 ? axis <= 2048 || (cols + 7) / 8 < 512 : axis >= 1024)));
         if (tile_pays && softmax_axis_tile_enabled()) {
             const bool narrow = axis <= 256;
             int tx_log2 = axis <= 1024 ? 4 : axis <= 2048 ? 3 : 2;
             if (small || axis <= 512)
                 for (tx_log2 = narrow ? 4 : 3; tx_log2 > 0 && ((narrow ? 1024 : 4096) >> tx_log2) < axis; --tx_log2) {}
-            while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= ivecs) --tx_log2;
-            const int TXv = 1 << tx_log2, TYv = (narrow ? 256 : 1024) >> tx_log2;
-            const int64_t tiles = outer * ((ivecs + TXv - 1) / TXv);
-            const int64_t nblocks = round_up8(tiles, tx_log2 < 3 ? 3 - tx_log2 : 0);
+            while (tx_log2 > 0 && (int64_t(1) << (tx_log2 - 1)) >= cols) --tx_log2;
+            // (fewer tiles than CUs: narrower ones, as far as they hold a row and no thread is left without an element)
+            while (tx_log2 > 0 && cols <= (int64_t(256) << tx_log2) && ((narrow ? 256 : 1024) >> (tx_log2 - 1)) <= axis && (int64_t(1) << (tx_log2 - 1)) >= vecs) --tx_log2;
+            const int TYv = (narrow ? 256 : 1024) >> tx_log2;
+            const AxisGroups groups = axis_groups(tx_log2, outer, vecs, inner * es);
+            const int64_t nblocks = round_up8(groups.count, groups.share);
             if (launch_fits(nblocks, narrow ? 256 : 1024)) { // (else the two-sweep kernel, whose work-groups take several tiles)
                 const bool few = (axis + TYv - 1) / TYv <= 4; // rows per thread
-                const int n = static_cast<int>(axis);
-#define AXHIP_SMT_R(LOG, DT, R, T) hipLaunchKernelGGL((softmax_axis_tile_kernel<LOG, DT, R, T>), dim3(static_cast<unsigned>(nblocks)), dim3(T), 0, s, src, dst, outer, inner, n, tx_log2)
+#define AXHIP_SMT_R(LOG, DT, R, T) hipLaunchKernelGGL((softmax_axis_tile_kernel<LOG, DT, R, T>), dim3(static_cast<unsigned>(nblocks)), dim3(T), 0, s, src, dst, outer, inner, n, tx_log2, groups)
 #define AXHIP_SMT_DT(LOG, DT)                                                                                                              \
     do {                                                                                                                                   \
         if (narrow) AXHIP_SMT_R(LOG, DT, 4, 256);                                                                                          \
@@ -1950,16 +2078,12 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
                 return AXHIP_OK;
             }
         }
-        // a short axis with plenty of results: a thread per vector walks it alone
-        const bool flat = axis <= 32 && outer * ((ivecs + 255) / 256) >= 1024;
-        const bool wide = outer * ((ivecs + 31) / 32) >= 1024;
-        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(outer * (flat ? (ivecs + 255) / 256 : wide ? (ivecs + 31) / 32 : (ivecs + 7) / 8), 256 * 64));
+        const bool wide = (cols + 31) / 32 >= 1024;
+        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(wide ? (cols + 31) / 32 : (cols + 7) / 8, 256 * 64));
 #define AXHIP_SM_TX(LOG, DT, TX) hipLaunchKernelGGL((softmax_strided_vec_kernel<LOG, DT, TX>), dim3(blocks), dim3(256), 0, s, src, outer, axis, inner, dst)
 #define AXHIP_SM_DT(LOG, DT)                                                                                                               \
     do {                                                                                                                                   \
-        if (flat && axis <= 16) hipLaunchKernelGGL((softmax_strided_vec_kernel<LOG, DT, 256, 16>), dim3(blocks), dim3(256), 0, s, src, outer, axis, inner, dst); \
-        else if (flat) AXHIP_SM_TX(LOG, DT, 256);                                                                                          \
-        else if (wide) AXHIP_SM_TX(LOG, DT, 32);                                                                                           \
+        if (wide) AXHIP_SM_TX(LOG, DT, 32);                                                                                           \
         else AXHIP_SM_TX(LOG, DT, 8);                                                                                                      \
     } while (0)
 #define AXHIP_SM(LOG)                                                                                                                      \

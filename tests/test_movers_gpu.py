@@ -585,3 +585,35 @@ def test_softmax_along_inner_axes_in_place(dt, outer, axis, inner):
     want = np.exp(x - x.max(1, keepdims=True))
     want /= want.sum(1, keepdims=True)
     assert np.all(np.abs(got - want) <= want * (half + (6 * 17 + axis) * 2.0**-23) + (2.0**-25 if dt == F16 else 1e-37))
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("axis,inner,few,many", [(2, 9, 7, 40001), (3, 35, 11, 30000), (4, 8, 300, 70001), (5, 129, 3, 9001), (8, 12, 5, 50000), (9, 17, 401, 25001), (16, 64, 9, 9001),
+                                                 (17, 300, 2, 2001), (20, 100, 50, 5500), (21, 9, 64, 34001), (24, 40, 33, 14001), (25, 100, 7, 5501), (32, 128, 3, 8301), (33, 9, 950, 20001),
+                                                 (48, 100, 77, 3001), (64, 17, 481, 6001), (100, 33, 5, 2500), (300, 12, 9, 1501)])
+def test_short_axes_and_narrow_rows(dt, axis, inner, few, many):
+    """Groups of columns that run from slice into slice -- rows of one vector to some dozens, whole slices to a group and not,
+    few slices and enough to fill the chip (neighbours dealt to one XCD, the short axis in registers, walked by one
+    thread).  Tolerances as for rows off the vector grid; what lies behind the results is left alone."""
+    rng = np.random.default_rng(axis * 1000 + inner)
+    half = {F32: 0.0, F16: 2.0**-11, BF16: 2.0**-8}[dt]
+    for outer in (1, few, many):
+        bits = axo.to_bits((rng.standard_normal((outer, axis, inner), np.float32) * 2), dt)
+        d = gh.to_dev(bits)
+        x = axo.to_f32(bits, dt).astype(np.float64)
+        mark = np.resize(bits, 32)
+        shift = np.exp(x - x.max(1, keepdims=True))
+        total = shift.sum(1, keepdims=True)
+        for what, want, tol in (("max", x.max(1), 0.0), ("sum", x.sum(1), axis * 2.0**-24 * np.abs(x).sum(1) + half * np.abs(x.sum(1)) * (1 + 2.0**-10)),
+                                ("softmax", shift / total, shift / total * (half + (6 * 17 + axis) * 2.0**-23) + (2.0**-25 if dt == F16 else 1e-37))):
+            out = gh.empty_dev((want.size + 32,), dt)
+            out[want.size:].copy_(gh.to_dev(mark))
+            gh.sync()
+            if what == "softmax":
+                capi.check(capi.lib().axhip_softmax_axis(d.data_ptr(), dt, outer, axis, inner, 0, out.data_ptr(), None))
+            else:
+                capi.check(capi.lib().axhip_reduce_axis(d.data_ptr(), dt, outer, axis, inner, capi.RED[what], out.data_ptr(), dt, None))
+            gh.sync()
+            got = gh.to_host(out, gh.np_store_dtype(dt))
+            assert np.all(np.abs(axo.to_f32(got[:want.size], dt).reshape(want.shape) - want) <= tol), (what, outer)
+            assert np.array_equal(got[want.size:], mark), (what, outer)
