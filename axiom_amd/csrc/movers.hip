@@ -1513,9 +1513,12 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
             // 17 us), except that fp32's 32 elements are too few (fp32 [5000, 33, 65] 30 us against 40).
             const bool lines = t.dst_stride_j * es % 128 == 0;
             const int64_t narrow = std::min(t.nJ, t.nL);
-            const bool together = es == 2 ? !lines || narrow <= 128 : !lines && narrow > 64;
-            // (output rows that one large tile holds whole keep it: bf16 [134, 104, 2624] 32.5 us against 37.6)
-            const int nv = together && !(es == 2 && t.nL > 64 && t.nL <= 128) ? 8 : 16;
+            // Output rows that one large tile holds whole keep it (bf16 [134, 104, 2624] 32.5 us against 37.6), and above 36 MiB,
+            // where the channels are busy for long, the diagonal order too (that array 32.7 us against 33.5, [2000, 128, 128]
+            // 28.8 against 31.3; but [300, 72, 500] 11.7 against 10.8).
+            const bool row_tiles = es == 2 && t.nL > 64 && t.nL <= 128;
+            const bool together = row_tiles ? a.total * es <= (int64_t(36) << 20) : es == 2 ? !lines || narrow <= 128 : !lines && narrow > 64;
+            const int nv = together && !row_tiles ? 8 : 16;
             const int64_t edge = nv * (16 / es);
             t.tiles_j = (t.nJ + edge - 1) / edge; t.tiles_l = (t.nL + edge - 1) / edge;
             blocks = blocks / (((t.nJ + 63) / 64) * ((t.nL + 63) / 64)) * t.tiles_j * t.tiles_l;

@@ -617,3 +617,14 @@ def test_short_axes_and_narrow_rows(dt, axis, inner, few, many):
             got = gh.to_host(out, gh.np_store_dtype(dt))
             assert np.all(np.abs(axo.to_f32(got[:want.size], dt).reshape(want.shape) - want) <= tol), (what, outer)
             assert np.array_equal(got[want.size:], mark), (what, outer)
+
+
+@pytest.mark.parametrize("others,rows,cols", [(3000, 100, 70), (2300, 128, 72), (40, 100, 70), (3, 65, 129)])
+def test_transposes_whose_output_rows_one_tile_holds(others, rows, cols):
+    """Output rows of 65 to 128 16-bit elements, in arrays above and below the size where the order of the tiles changes."""
+    x = torch.randint(-30000, 30000, (others, rows, cols), dtype=torch.int16, device="cuda")
+    y = torch.full((others * cols * rows + 64,), 77, dtype=torch.int16, device="cuda")
+    gh.sync()
+    capi.check(capi.lib().axhip_strided_copy(x.data_ptr(), BF16, y.data_ptr(), BF16, 3, i64([others, cols, rows]), i64([rows * cols, 1, cols]), None))
+    gh.sync()
+    assert torch.equal(y[:-64].view(others, cols, rows), x.transpose(1, 2)) and bool((y[-64:] == 77).all())
