@@ -1204,36 +1204,54 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
             for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
         }
     across(m, true);
+    // e^(x - m).  Where the exponentials are worked out twice (not KEEP) it is 2^(x log2(e) - ref), one fused multiply and add:
+    // ref is m log2(e) rounded, and all terms of a column share the factor that the rounding makes.  From 2^20 on that factor
+    // could be anything: there x - m is formed first as well (for the whole wavefront, which holds every column of the
+    // block).  bf16 [30, 1537, 640] 42.7 us, 45.2 with the difference for all.
+    const float LOG2E = 1.44269504088896340736f;
+    bool far = KEEP;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        if (m[e] == -INFINITY && !LOG) m[e] = 0.0f; // (nothing finite: every term is e^-inf = 0)
+        far = far || fabsf(m[e]) >= 1048576.0f;
+    }
+    far = KEEP || __builtin_amdgcn_ballot_w64(far) != 0;
     float ref[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) ref[e] = m[e] == -INFINITY ? 0.0f : m[e]; // (nothing finite: every term is e^-inf = 0)
+    for (int e = 0; e < V; ++e) ref[e] = far ? 0.0f : m[e] * LOG2E;
+    auto power = [&](float (&t)[V]) {
+        if (far) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) t[e] -= m[e];
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) t[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[e], LOG2E, -ref[e]));
+    };
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float t[V];
             value(r, t);
+            power(t);
 #pragma unroll
             for (int e = 0; e < V; ++e) {
-                const float p = exp_of(t[e] - ref[e]);
-                l[e] += p;
-                if (KEEP && !LOG) kept[r][e] = p;
+                l[e] += t[e];
+                if (KEEP && !LOG) kept[r][e] = t[e];
             }
         }
     across(l, false);
-    float shift[V], inv[V]; // result = e^(x - shift) * inv, or x - shift - inv with the logarithm of the sum as inv
+    float inv[V]; // result = e^(x - m) * inv, or x - m - inv with the logarithm of the sum as inv
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
-        shift[e] = LOG ? m[e] : ref[e];
-        inv[e] = LOG ? log_of(l[e]) : 1.0f / l[e];
-    }
+    for (int e = 0; e < V; ++e) inv[e] = LOG ? log_of(l[e]) - (far ? 0.0f : __builtin_fmaf(m[e], LOG2E, -ref[e]) * 0.69314718055994530942f) : 1.0f / l[e];
     if (!there) return;
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
         if (ty + r * TY < n) {
             float v[V];
             value(r, v);
+            if (!LOG && !KEEP) power(v);
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : (KEEP ? v[e] : exp_of(v[e] - shift[e])) * inv[e];
+            for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - m[e] - inv[e] : v[e] * inv[e];
             store_vec<V, true>(dst, DT, at + (ty + r * TY) * inner, v);
         }
 }

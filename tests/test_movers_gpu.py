@@ -538,7 +538,8 @@ def test_transposes_off_the_vector_grid_are_bit_exact(dt, rows, cols, others, sk
 
 @pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("outer,axis,inner", [(3, 40, 9), (2, 100, 64), (4, 300, 33), (1, 1030, 24), (1, 4097, 17), (2, 4100, 8), (1100, 5, 512), (1100, 24, 516), (1030, 16, 35), (40, 30, 3)])
-def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner):
+@pytest.mark.parametrize("far", [True, False], ids=["lowest", "thousands"])
+def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner, far):
     """Values around +-1000, a column of the type's lowest value alone (uniform: every result is 1 / axis) and one that it
     masks in part, in every kernel and on both kinds of rows.  x - max is one rounding, 2^-24 |x - max|, however large x is;
     the exponentials add 2^-22 per unit of an argument that matters (up to 17: below e^-17 a term is under the sum's own
@@ -546,8 +547,9 @@ def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner):
     rng = np.random.default_rng(axis * inner + dt)
     x = (rng.normal(size=(outer, axis, inner)) * 3 + np.where(rng.random((outer, 1, inner)) < 0.5, 1000.0, -1000.0)).astype(np.float32)
     lowest = {F32: np.finfo(np.float32).min, F16: -65504.0, BF16: axo.to_f32(np.array([0xFF7F], np.uint16), BF16)[0]}[dt]
-    x[:, :, 0] = lowest
-    x[:, 1::2, 1] = lowest
+    if far: # (past this magnitude the tile kernel takes the difference first, for a whole wavefront)
+        x[:, :, 0] = lowest
+        x[:, 1::2, 1] = lowest
     bits = axo.to_bits(x, dt)
     xf, half = axo.to_f32(bits, dt).astype(np.float64), {F32: 2.0**-24, F16: 2.0**-11, BF16: 2.0**-8}[dt]
     z = xf - xf.max(1, keepdims=True)
