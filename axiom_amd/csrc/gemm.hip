@@ -1,11 +1,11 @@
 // C = op(A) op(B) (+ bias) (+ residual), activation epilogue: the dispatch, and
 //
 //   gemm_mfma_nt_256_kernel    large bf16 / f16 x W^T: 256 x 256 tiles
-//   gemm_mfma_f32_ring_kernel  fp32 x W^T on the fp32 matrix instruction
+//   gemm_mfma_f32_ring_kernel  large fp32 products, b along k or [k, n], on the fp32 matrix instruction
 //   gemm_generic_kernel        any dtype / any transpose combination, 16x16 LDS tiles, fp32 FMA
 //
 // The other 16-bit kernels are in gemm_tile_*.hip (middle-sized products), gemm_small.hip (few rows or few output
-// tiles) and gemm_skinny.hip (at most eight rows).
+// tiles) and gemm_skinny.hip (at most eight rows), the smaller fp32 products in gemm_f32.hip.
 #include "common.hpp"
 #include "gemm_f32.hpp"
 #include "gemm_small.hpp"
@@ -371,10 +371,9 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 
 // ------------------------------------------------------------------ fp32, MFMA
 // C = A B^T in fp32 on v_mfma_f32_32x32x2_f32 (fp32 products, fp32 accumulation: no precision is given up against
-// the FMA kernel), A [M,K] and B [N,K] both K-contiguous.  Same skeleton as the 16-bit ring kernel: a k-tile is 32
-// floats, i.e. the same 128-byte LDS rows, XOR swizzle and direct-to-LDS loads; a lane's 16-byte fragment read holds
-// four k values that feed four successive MFMAs (which k a lane contributes to which MFMA is free as long as A and B
-// agree).  K only has to be a multiple of 4: the chunks of the last k-tile that lie past K are sent out of the
+// the FMA kernel), A [M,K] and B [N,K] both K-contiguous.  A ring of S k-tiles of 32 floats, i.e. the 128-byte LDS rows,
+// XOR swizzle and direct-to-LDS loads of the 256 x 256 kernel; a lane's 16-byte fragment read holds four k values that
+// feed four successive MFMAs (which k a lane contributes to which MFMA is free as long as A and B agree).  K only has to be a multiple of 4: the chunks of the last k-tile that lie past K are sent out of the
 // descriptor's range and arrive as zeros.  At 1/16 of the 16-bit MFMA rate the kernel is bound by the matrix pipe,
 // not by the ring.
 // NN: B is [K,N].  Its k-tile then is 32 rows of TNR floats, which the same loads bring in (N a multiple of 4), and a
@@ -542,9 +541,9 @@ static bool skinny_enabled() {
 }
 
 namespace {
-// whether (and into how many padded columns) a product is repacked before it runs on the k-contiguous kernels: fp32, and
-// 16-bit ones with A stored [k, m]; the workspace that axhip_gemm_workspace_bytes asks for does not depend on the type,
-// so that a program's figures stay what they were when every such product was repacked
+// Whether a product is of a form that may have to be repacked (and into how many padded columns): large, with an operand
+// stored the other way or a k off the vector grid.  axhip_gemm_workspace_bytes answers for the form; the kernels that read
+// such operands as they lie (16-bit ones with A along k, most fp32 ones) leave the memory alone.
 struct Repack { bool on, a, b; int64_t kp; };
 Repack repack_plan(const AxhipGemmParams &p) {
     const int64_t kvec = p.dtype == AXHIP_DTYPE_F32 ? 4 : 8;
@@ -831,11 +830,11 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
     const bool nt = !p.trans_a && p.trans_b && p.k % 8 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.stride_a % 8 == 0 &&
                     p.stride_b % 8 == 0 && al16(a) && al16(b) && p.ldc < (1 << 21);
-    // (measured against the tiled kernels, whose k loop costs about 5.5 us per 1024 elements of k whatever N is: one or
-    // two rows always win -- 1 x 4096 x 4096 23.2 -> 4.4 us --, up to four while W stays below 48 M elements, up to
-    // eight on long-k products of up to 24 M elements; beyond that the per-lane sums make the kernel VALU-bound)
-    // (fp32: the tiled fp32 kernels are an order of magnitude off on such shapes -- 1 x 4096 x 4096 138 -> 12 us --, so
-    // every product of up to eight rows goes here)
+    // One or two rows: 1 x 4096 x 4096 in bf16 4.2 us with W in the caches and 7.7 from HBM, 5.6 and 8.9 on the kernels of
+    // gemm_small.hip; 2 x 1280 x 5120 4.5 and 6.2, 5.5 and 9.1.  With more rows the sums per lane grow and the other kernels
+    // do not: the rest of the line dates from kernels that had a k loop of 5.5 us per 1024 elements (fp32: 138 us for
+    // 1 x 4096 x 4096) and lies too far out for those there are now -- bf16 4 x 4096 x 4096 8.5 us here and 5.8 there,
+    // 8 x 1280 x 5120 11.2 and 5.6; fp32 8 x 4096 x 4096 22.5 and 12.5, level at three or four rows.
     const int64_t w_elems = p.n * p.k;
     const bool skinny_pays = p.m <= 2 || (p.m <= 8 && p.dtype == AXHIP_DTYPE_F32) || (p.m <= 4 && w_elems <= (int64_t(48) << 20)) ||
                              (p.m <= 8 && p.k >= 2048 && w_elems <= (int64_t(24) << 20));

@@ -69,7 +69,7 @@ __device__ __forceinline__ void small_finish(const TileArgs &g, const float4_t (
         };
         if (g.bias) add4(bias);
         if (g.residual) add4(res);
-gemm_epilogue16_all(g.epilogue, y);
+        gemm_epilogue16_all(g.epilogue, y);
         const uint32_t w0 = BF16 ? pack_bf16x2(y[0], y[1]) : pack_f16x2(y[0], y[1]), w1 = BF16 ? pack_bf16x2(y[2], y[3]) : pack_f16x2(y[2], y[3]);
         if (valid - first == 4 && (reinterpret_cast<uintptr_t>(c) & 7u) == 0) {
             *reinterpret_cast<uint2_t *>(c) = uint2_t{w0, w1};

@@ -16,9 +16,9 @@ struct SdpaArgs {
     int nqb; // query blocks per (batch, head)
     int dtype;
     int64_t qs[3], ks[3], vs[3], os[3], ms[2];
-    // key split of sdpa_mfma_kernel (decoding: few query rows, few heads, a long key sequence): `ksplit` work-groups
+    // key split of sdpa_direct16_kernel and sdpa_mfma_kernel (decoding: few query rows, few heads, a long key sequence): `ksplit` work-groups
     // per (batch, head) take `kchunk` keys each and leave normalised fp32 partial outputs and the base-2 logarithm of
-    // their softmax denominators (reference maximum included) for sdpa_splitk_merge_kernel
+    // their softmax denominators (reference maximum included) for sdpa_merge_kernel
     int ksplit, kchunk;
     float *opart, *lse;
 };

@@ -132,7 +132,7 @@ def by_grid(dirs: list[str], needles: tuple[str, ...] = ("gemm", "Cijk")) -> Non
     import csv
 
     def short(n: str) -> str:
-        n = n.replace("(axhip::GemmArgs, int, int)", "").split("(")[0]
+        n = n.replace("(anonymous namespace)::", "").replace("(axhip::GemmArgs, int, int)", "").split("(")[0]
         return n if len(n) < 70 else "..." + n[-60:]
 
     for d in dirs:

@@ -423,11 +423,12 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
  * C[b] = op(A[b]) * op(B[b]) (+ bias[N]) (+ residual[b]) for b < batch;
  * row-major, lda/ldb/ldc and batch strides in elements (stride 0 shares an
  * operand across the batch).  fp32 accumulation; bf16/f16 on MFMA.
- * The matrix-core kernels read both operands along k (trans_a = 0,
- * trans_b = 1: x W^T) in 16-byte vectors.  On a large product an operand
- * stored the other way is transposed first, and a k that is not a multiple of
- * 8 (fp32: 4) zero-padded, into temporary memory that the library takes and
- * returns in stream order (hipMallocAsync / hipFreeAsync on `stream`). */
+ * The matrix-core kernels read A along k (trans_a = 0) and B either way, at
+ * any alignment.  A large product with A stored [k, m], and a large fp32 one
+ * off the vector grid (k, or n of a B stored [k, n], not a multiple of 4)
+ * where copying first is the faster way, is repacked: transposed, k
+ * zero-padded, into temporary memory that the library takes and returns in
+ * stream order (hipMallocAsync / hipFreeAsync on `stream`). */
 typedef struct {
     int32_t dtype;
     int32_t trans_a, trans_b;
@@ -441,8 +442,13 @@ typedef struct {
 } AxhipGemmParams;
 
 int axhip_gemm(const void *a, const void *b, void *c, const AxhipGemmParams *params_host, void *stream);
-/* The same with the repacked operands in memory handed in by the caller (0
- * bytes for every product that is not repacked). */
+/* The same with temporary memory handed in by the caller.  0 bytes below
+ * 2^30 floating-point operations and for x W^T in whole 16-byte vectors; for
+ * a large product with an operand stored the other way, or a k off that grid,
+ * the size of the operands repacked -- also where the kernel that the product
+ * gets reads them as they lie and leaves the memory alone.  Less is refused
+ * with AXHIP_ERR_WORKSPACE; NULL leaves the allocation, if one is needed, to
+ * the library. */
 size_t axhip_gemm_workspace_bytes(const AxhipGemmParams *params_host);
 int axhip_gemm_ws(const void *a, const void *b, void *c, const AxhipGemmParams *params_host,
                   void *workspace, size_t workspace_bytes, void *stream);

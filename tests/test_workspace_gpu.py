@@ -1,6 +1,8 @@
 """The *_ws entry points: the four calls that need temporary device memory take it from a caller's workspace and
 allocate nothing.  Each is compared bit for bit with its allocating form on the same inputs, is refused with
-AXHIP_ERR_WORKSPACE when the workspace is too small, and asks for no memory where the plain call takes none."""
+AXHIP_ERR_WORKSPACE when the workspace is too small, and asks for no memory where a call of its form never takes any
+(a large product with an operand stored the other way, or a k off the vector grid, asks for the size of its operands
+repacked, whether or not its kernel reads them as they lie)."""
 import ctypes as C
 
 import numpy as np
