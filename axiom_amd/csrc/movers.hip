@@ -978,21 +978,62 @@ __global__ __launch_bounds__(256) void reduce_strided_kernel(const void *src, in
 
 namespace axhip {
 // ----------------------------------------------- softmax along an inner axis
-__device__ __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f); } // (v_exp_f32, v_log_f32: base 2)
-__device__ __forceinline__ float log_of(float x) { return __builtin_amdgcn_logf(x) * 0.69314718055994530942f; }
+constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f; // (v_exp_f32 and v_log_f32 are base 2)
+
+// (fmaxf of a value as it was loaded makes sure first that it is no signalling NaN: an instruction for each element)
+__device__ __forceinline__ float max_of(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// e^(x - m) for V columns whose maxima m are known.  Below |m| = 2^20 it is 2^(x log2(e) - ref) in one fused multiply and
+// add: ref is m log2(e) rounded, and all terms of a column share the factor 2^rest that the rounding makes.  From there on
+// that factor could be anything, and with FAR the difference x - m is formed first (float16 holds nothing that far).  A
+// maximum below -2^20 that later elements may replace counts as -2^20: its terms are 0 and nothing overflows.
+constexpr float FAR_FROM_ZERO = 1048576.0f;
+template <int DT, int V> __device__ __forceinline__ bool far_from_zero(const float (&m)[V]) {
+    float top = 0.0f;
+#pragma unroll
+    for (int e = 0; e < V; ++e) top = fmaxf(top, fabsf(m[e]));
+    return DT != AXHIP_DTYPE_F16 && __builtin_expect(top >= FAR_FROM_ZERO, false);
+}
+__device__ __forceinline__ float exp_reference(float m) { // (never fused into what uses it)
+#pragma clang fp contract(off)
+    return fmaxf(m, -FAR_FROM_ZERO) * LOG2E;
+}
+template <int V, bool FAR> struct ExpFrom {
+    float m[V], ref[V];
+    __device__ __forceinline__ explicit ExpFrom(const float (&top)[V]) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            m[e] = top[e];
+            ref[e] = FAR ? 0.0f : exp_reference(top[e]);
+        }
+    }
+    __device__ __forceinline__ void power(float (&t)[V]) const {
+#pragma unroll
+        for (int e = 0; e < V; ++e) t[e] = __builtin_amdgcn_exp2f(FAR ? (t[e] - m[e]) * LOG2E : __builtin_fmaf(t[e], LOG2E, -ref[e]));
+    }
+    // the logarithm of the sum of e^(x - m), from the sum of the powers
+    __device__ __forceinline__ float log_sum(float sum, int e) const {
+        return __builtin_amdgcn_logf(sum) * LN2 - (FAR ? 0.0f : __builtin_fmaf(m[e], LOG2E, -ref[e]) * LN2);
+    }
+};
 
 // softmax / log-softmax along the middle extent of a contiguous (outer, axis, inner) view, inner >= V, in the layout of
 // reduce_axis_kernel (any alignment, the last vector of a row moved left to end with it).  One sweep gathers a running
-// maximum and the sum of e^(x - maximum) per inner position (rescaled once per four elements), the thread rows merge
-// their pairs through LDS, a second sweep over the same elements writes the result: two reads of the input (the second
-// mostly from the caches) and one write.  x - maximum is formed before the factor log2(e): it is exact to one rounding of
-// the difference whatever the magnitude of x, where x log2(e) is off by 6e-5 for x around 1000, and it stays finite for
-// every finite x (a column that holds nothing but the type's lowest value is uniform).
+// maximum and the sum of e^(x - maximum) per inner position (rescaled once per four elements), the pairs are merged in the
+// registers of each wavefront and then through LDS (all 32 of a column through LDS, in every thread: bf16 [770, 640, 64]
+// 59 us, so 39, and fp32 [2, 5000, 64] 39.5 and 35.4), a second sweep over the same elements writes the result: two
+// reads of the input (the second mostly from the caches) and one write.  A group with a maximum far from zero -- the type's
+// lowest value, say, of which a column is uniform -- takes a third one for its sums.
 template <bool LOG, int DT, int TX>
 __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *src, int64_t outer, int64_t axis, int64_t inner, void *dst) {
     constexpr int TY = 256 / TX, U = 4, V = DT == AXHIP_DTYPE_F32 ? 4 : 8;
-    __shared__ float sm[TY][TX][V + 1], sl[TY][TX][V + 1];
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    constexpr int NW = 256 / WAVE;
+    __shared__ float sm[NW][TX][V + 1], sl[NW][TX][V + 1];
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX, wave = threadIdx.x / WAVE;
     constexpr int ES = 16 / V;
     const int64_t vecs = (inner + V - 1) / V, pitch = inner * ES;
     const AxisGroups groups{(outer * vecs + TX - 1) / TX, 0, TX, 0};
@@ -1003,10 +1044,11 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
         const bool there = tx < origin.left;
         const char *first = static_cast<const char *>(src) + at * ES;
         const int64_t step = TY * pitch;
-        float m[V], l[V];
+        float m[V], ref[V], l[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             m[e] = -INFINITY;
+            ref[e] = exp_reference(m[e]);
             l[e] = 0.0f;
         }
         auto gather = [&](int k, const uint4_t (&raw)[U]) { // running maximum and rescaled sum over U axis elements
@@ -1019,62 +1061,101 @@ __global__ __launch_bounds__(256) void softmax_strided_vec_kernel(const void *sr
                 }
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
-                    const float mx = fmaxf(fmaxf(fmaxf(t[0][e], t[1][e]), fmaxf(t[2][e], t[3][e])), m[e]);
-                    const float ref = mx == -INFINITY ? 0.0f : mx; // (nothing finite yet: every term below is e^-inf = 0)
+                    const float mx = max_of(max_of(t[0][e], t[1][e], t[2][e]), t[3][e], m[e]);
+                    const float now = exp_reference(mx);
                     float add = 0.0f;
 #pragma unroll
-                    for (int u = 0; u < U; ++u) add += exp_of(t[u][e] - ref);
-                    l[e] = l[e] * exp_of(m[e] - ref) + add;
+                    for (int u = 0; u < U; ++u) add += __builtin_amdgcn_exp2f(__builtin_fmaf(t[u][e], LOG2E, -now));
+                    l[e] = l[e] * __builtin_amdgcn_exp2f(ref[e] - now) + add;
                     m[e] = mx;
+                    ref[e] = now;
                 }
         };
         if (there) {
-            const char *from = first + ty * pitch;
-            for (int k = ty; k < n; k += TY * U, from += U * step) {
+            const char *row = first + ty * pitch;
+            for (int k = ty; k < n; k += TY * U, row += U * step) {
                 uint4_t raw[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
+                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? row + u * step : first);
                 gather(k, raw);
             }
         }
-        __syncthreads(); // the previous group's pairs have been read
+        // the pairs of a wavefront in registers, then those of the wavefronts through LDS
+        across_lanes(m, TX, [](float p, float q) { return fmaxf(p, q); });
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            sm[ty][tx][e] = m[e];
-            sl[ty][tx][e] = l[e];
+        for (int e = 0; e < V; ++e) l[e] *= __builtin_amdgcn_exp2f(ref[e] - exp_reference(m[e]));
+        across_lanes(l, TX, [](float p, float q) { return p + q; });
+        __syncthreads(); // the previous group's pairs have been read
+        if (threadIdx.x % WAVE < TX) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                sm[wave][tx][e] = m[e];
+                sl[wave][tx][e] = l[e];
+            }
         }
         __syncthreads();
-        float shift[V], inv[V]; // result = e^(x - shift) * inv, or x - shift - inv with the logarithm of the sum as inv
+        float inv[V]; // result = e^(x - m) * inv, or x - m - inv with the logarithm of the sum as inv
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-            float M = sm[0][tx][e];
-            for (int y = 1; y < TY; ++y) M = fmaxf(M, sm[y][tx][e]);
-            const float ref = M == -INFINITY ? 0.0f : M;
-            float L = 0.0f;
-            for (int y = 0; y < TY; ++y) L += sl[y][tx][e] * exp_of(sm[y][tx][e] - ref);
-            shift[e] = M;
-            inv[e] = LOG ? log_of(L) : 1.0f / L;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) m[e] = fmaxf(m[e], sm[w][tx][e]);
+            ref[e] = exp_reference(m[e]);
+            inv[e] = 0.0f;
         }
-        auto emit = [&](int k, const uint4_t (&raw)[U]) {
+#pragma unroll 2
+        for (int w = 0; w < NW; ++w)
+#pragma unroll
+            for (int e = 0; e < V; ++e) inv[e] += sl[w][tx][e] * __builtin_amdgcn_exp2f(exp_reference(sm[w][tx][e]) - ref[e]);
+        auto emit = [&](const auto &from) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) inv[e] = LOG ? from.log_sum(inv[e], e) : 1.0f / inv[e];
+            if (!there) return;
+            const char *row = first + ty * pitch;
+            for (int k = ty; k < n; k += TY * U, row += U * step) {
+                uint4_t raw[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? row + u * step : first);
 #pragma unroll
                 for (int u = 0; u < U; ++u)
                     if (k + u * TY < n) {
                         float v[V];
                         arg_unpack<DT>(raw[u], v);
+                        if (!LOG) from.power(v);
 #pragma unroll
-                        for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - shift[e] - inv[e] : exp_of(v[e] - shift[e]) * inv[e];
+                        for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - m[e] - inv[e] : v[e] * inv[e];
                         store_vec<V, true>(dst, DT, at + (k + u * TY) * inner, v);
                     }
-        };
-        if (there) {
-            const char *from = first + ty * pitch;
-            for (int k = ty; k < n; k += TY * U, from += U * step) {
-                uint4_t raw[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) raw[u] = axis_load(k + u * TY < n ? from + u * step : first);
-                emit(k, raw);
             }
+        };
+        if (__builtin_amdgcn_ballot_w64(there && far_from_zero<DT>(m)) == 0) { // (every wavefront holds every column of the group)
+            emit(ExpFrom<V, false>(m));
+            continue;
         }
+        // the sums above mean nothing: a third sweep, now that the maxima are known
+        const ExpFrom<V, true> from(m);
+#pragma unroll
+        for (int e = 0; e < V; ++e) l[e] = inv[e] = 0.0f;
+        if (there)
+#pragma unroll 1
+            for (int k = ty; k < n; k += TY) {
+                float t[V];
+                arg_unpack<DT>(axis_load(first + k * pitch), t);
+                from.power(t);
+#pragma unroll
+                for (int e = 0; e < V; ++e) l[e] += t[e];
+            }
+        across_lanes(l, TX, [](float p, float q) { return p + q; });
+        __syncthreads(); // the first sums have been read
+        if (threadIdx.x % WAVE < TX) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) sl[wave][tx][e] = l[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+#pragma unroll
+            for (int w = 0; w < NW; ++w) inv[e] += sl[w][tx][e];
+        emit(from);
     }
 }
 
@@ -1107,23 +1188,46 @@ __global__ __launch_bounds__(64) void softmax_axis_short_kernel(const void *src,
 #pragma unroll
             for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
         }
+        if (DT == AXHIP_DTYPE_F32 && far_from_zero<DT>(m)) {
 #pragma unroll
-        for (int k = 0; k < HOLD; ++k)
-            if (k < n) {
+            for (int k = 0; k < HOLD; ++k) {
                 float t[V];
                 arg_unpack<DT>(raw[k], t);
 #pragma unroll
-                for (int e = 0; e < V; ++e) l[e] += exp_of(t[e] - m[e]);
+                for (int e = 0; e < V; ++e) raw[k][e] = __builtin_bit_cast(uint32_t, t[e] - m[e]);
             }
 #pragma unroll
-        for (int e = 0; e < V; ++e) l[e] = LOG ? log_of(l[e]) : 1.0f / l[e];
+            for (int e = 0; e < V; ++e) m[e] = 0.0f;
+        }
+        const ExpFrom<V, DT == AXHIP_DTYPE_BF16> from(m);
+        float odd[V]; // (in two halves, by pairs: fewer roundings on the way of each term)
+#pragma unroll
+        for (int e = 0; e < V; ++e) odd[e] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < HOLD; k += 2)
+            if (k < n) {
+                float t[V], u[V];
+                arg_unpack<DT>(raw[k], t);
+                from.power(t);
+                if (k + 1 < n) {
+                    arg_unpack<DT>(raw[k + 1], u);
+                    from.power(u);
+#pragma unroll
+                    for (int e = 0; e < V; ++e) t[e] += u[e];
+                }
+#pragma unroll
+                for (int e = 0; e < V; ++e) (k % 4 == 0 ? l : odd)[e] += t[e];
+            }
+#pragma unroll
+        for (int e = 0; e < V; ++e) l[e] = LOG ? from.log_sum(l[e] + odd[e], e) : 1.0f / (l[e] + odd[e]);
 #pragma unroll
         for (int k = 0; k < HOLD; ++k)
             if (k < n) {
                 float v[V];
                 arg_unpack<DT>(raw[k], v);
+                if (!LOG) from.power(v);
 #pragma unroll
-                for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - m[e] - l[e] : exp_of(v[e] - m[e]) * l[e];
+                for (int e = 0; e < V; ++e) v[e] = LOG ? v[e] - m[e] - l[e] : v[e] * l[e];
                 store_vec<V, true>(dst, DT, at + k * inner, v);
             }
     }
@@ -1204,28 +1308,29 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
             for (int e = 0; e < V; ++e) m[e] = fmaxf(m[e], t[e]);
         }
     across(m, true);
-    // e^(x - m).  Where the exponentials are worked out twice (not KEEP) it is 2^(x log2(e) - ref), one fused multiply and add:
-    // ref is m log2(e) rounded, and all terms of a column share the factor that the rounding makes.  From 2^20 on that factor
-    // could be anything: there x - m is formed first as well (for the whole wavefront, which holds every column of the
-    // block).  bf16 [30, 1537, 640] 42.7 us, 45.2 with the difference for all.
-    const float LOG2E = 1.44269504088896340736f;
-    bool far = KEEP;
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
+    for (int e = 0; e < V; ++e)
         if (m[e] == -INFINITY && !LOG) m[e] = 0.0f; // (nothing finite: every term is e^-inf = 0)
-        far = far || fabsf(m[e]) >= 1048576.0f;
-    }
-    far = KEEP || __builtin_amdgcn_ballot_w64(far) != 0;
-    float ref[V];
+    // (every wavefront holds every column of the block)
+    const bool far = DT != AXHIP_DTYPE_F16 && __builtin_amdgcn_ballot_w64(far_from_zero<DT>(m)) != 0;
+    if (KEEP && __builtin_expect(far, false)) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) ref[e] = far ? 0.0f : m[e] * LOG2E;
-    auto power = [&](float (&t)[V]) {
-        if (far) {
+        for (int r = 0; r < RPT; ++r)
+#pragma unroll
+            for (int e = 0; e < V; ++e) kept[KEEP ? r : 0][e] -= m[e];
+#pragma unroll
+        for (int e = 0; e < V; ++e) m[e] = 0.0f;
+    }
+    float top[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) top[e] = !KEEP && far ? 0.0f : m[e];
+    const ExpFrom<V, false> from(top);
+    auto power = [&](float (&t)[V]) { // (bf16 [30, 1537, 640] in the caches 34.9 us, 37.1 with a subtraction of m or of 0 from all)
+        if (!KEEP && far) {
 #pragma unroll
             for (int e = 0; e < V; ++e) t[e] -= m[e];
         }
-#pragma unroll
-        for (int e = 0; e < V; ++e) t[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[e], LOG2E, -ref[e]));
+        from.power(t);
     };
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
@@ -1236,13 +1341,13 @@ __global__ __launch_bounds__(THREADS) void softmax_axis_tile_kernel(const void *
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 l[e] += t[e];
-                if (KEEP && !LOG) kept[r][e] = t[e];
+                if (KEEP && !LOG) kept[KEEP ? r : 0][e] = t[e];
             }
         }
     across(l, false);
     float inv[V]; // result = e^(x - m) * inv, or x - m - inv with the logarithm of the sum as inv
 #pragma unroll
-    for (int e = 0; e < V; ++e) inv[e] = LOG ? log_of(l[e]) - (far ? 0.0f : __builtin_fmaf(m[e], LOG2E, -ref[e]) * 0.69314718055994530942f) : 1.0f / l[e];
+    for (int e = 0; e < V; ++e) inv[e] = LOG ? from.log_sum(l[e], e) : 1.0f / l[e];
     if (!there) return;
 #pragma unroll
     for (int r = 0; r < RPT; ++r)
@@ -2054,11 +2159,11 @@ int axhip_softmax_axis(const void *src, int32_t dtype, int64_t outer, int64_t ax
             return AXHIP_OK;
         }
         // An axis that a block can hold is read once.  Up to 512 elements: four rows per thread (256 threads up to 256
-        // elements, so that several blocks share a CU), as wide as that allows; bf16 [64, 256, 2048] 72 -> 40 us, fp32
-        // [256, 128, 1024] 76 -> 58 us against the two-sweep kernel.  Longer axes of large arrays take 1024-thread blocks of
+        // elements, so that several blocks share a CU), as wide as that allows; bf16 [64, 256, 2048] 40 -> 37 us, fp32
+        // [256, 128, 1024] 79 -> 57 us against the two-sweep kernel.  Longer axes of large arrays take 1024-thread blocks of
         // sixteen rows per thread, where they pay (one block per CU, whose load, arithmetic and store phases do not overlap):
-        // fp32 axes of up to 2048 elements (126 against 179 us on [16, 2048, 2048]), 16-bit axes of 1024 to 4096 (274 against
-        // 348 us on [64, 2048, 2048]), TX = 16, 8 or 4 vectors for axes of up to 1024, 2048 or 4096; fp32 axes of more than 2048
+        // fp32 axes of up to 2048 elements (118 against 186 us on [16, 2048, 2048]), 16-bit axes of 1024 to 4096 (252 against
+        // 352 us on [64, 2048, 2048]), TX = 16, 8 or 4 vectors for axes of up to 1024, 2048 or 4096; fp32 axes of more than 2048
         // only where the two-sweep kernel would leave the chip short of work-groups.  Small arrays, whose two
         // sweeps are two trips to memory and little else, take four rows per thread whatever the axis: the code of sixteen
         // takes longer to arrive than the array.

@@ -572,6 +572,44 @@ def test_softmax_along_inner_axes_of_large_values(dt, outer, axis, inner, far):
 
 
 @pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,axis,inner", [(1100, 24, 20), (3, 300, 33), (1, 4097, 17), (2, 4100, 136)])
+@pytest.mark.parametrize("hidden", ["lowest", "large", "inf"])
+def test_softmax_along_inner_axes_of_masked_columns(dt, outer, axis, inner, hidden):
+    """Ordinary columns whose first half is hidden, or all but one row in 32, or all but the last: a maximum that starts far
+    below the column's own leaves no trace, and the hidden elements are 0 exactly (a column of nothing but -inf is NaN, and a
+    NaN makes its own column so).  The bound is the one above with arguments up to 17; a few units of magnitude leave x - max
+    its one rounding."""
+    rng = np.random.default_rng(axis * inner + dt)
+    x = (rng.normal(size=(outer, axis, inner)) * 3).astype(np.float32)
+    lowest = {F32: np.finfo(np.float32).min, F16: -65504.0, BF16: axo.to_f32(np.array([0xFF7F], np.uint16), BF16)[0]}[dt]
+    mask = np.zeros((axis, inner), bool)
+    mask[: axis // 2, 0::4] = True
+    mask[np.arange(axis) % 32 != 5, 1::4] = True
+    mask[:-1, 2::4] = True
+    x[:, mask] = {"lowest": lowest, "large": -60000.0 if dt == F16 else -1e30, "inf": -np.inf}[hidden]
+    if hidden == "inf":
+        x[:, :, 3] = -np.inf
+        x[:, axis // 3, 7] = np.nan
+    bits = axo.to_bits(x, dt)
+    xf, half = axo.to_f32(bits, dt).astype(np.float64), {F32: 2.0**-24, F16: 2.0**-11, BF16: 2.0**-8}[dt]
+    with np.errstate(invalid="ignore"):
+        z = np.exp(xf - xf.max(1, keepdims=True))
+    want = z / z.sum(1, keepdims=True)
+    undefined = np.isnan(want)
+    out = gh.empty_dev((outer, axis, inner), dt)
+    d = gh.to_dev(bits)
+    gh.sync()
+    capi.check(capi.lib().axhip_softmax_axis(d.data_ptr(), dt, outer, axis, inner, 0, out.data_ptr(), None))
+    gh.sync()
+    got = axo.to_f32(gh.to_host(out, gh.np_store_dtype(dt)), dt).reshape(outer, axis, inner)
+    assert np.array_equal(np.isnan(got), undefined)
+    got[undefined] = want[undefined] = 0.0
+    assert np.all(got[:, mask] == 0.0)
+    arith = (17 * 4 + axis + 8) * 2.0**-24
+    assert np.all(np.abs(got - want) <= want * (half * (1 + 2.0**-10) + 2 * arith) + (2.0**-25 if dt == F16 else 1e-37))
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("outer,axis,inner", [(3, 50, 129), (2, 300, 9), (1100, 5, 515), (1100, 24, 520), (40, 7, 64), (1, 4097, 17), (2, 4100, 24)])
 def test_softmax_along_inner_axes_in_place(dt, outer, axis, inner):
     """dst == src, with rows that are whole vectors and rows whose last vector is moved left over its neighbour's columns
