@@ -113,6 +113,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
+typedef int int2_t __attribute__((ext_vector_type(2)));
 
 // bf16 <-> f32 with the same rounding as Axiom's bfloat16_t: round to nearest
 // even, NaN canonicalised to 0x7FC0.

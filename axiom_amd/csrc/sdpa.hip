@@ -351,6 +351,65 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_mfma_kernel(const S
     }
 }
 
+// An explicit mask as the pipelined kernel reads it: bits, set where masked out or past the last key.  Word
+// ((plane * tiles + tile) * Sq + row) * 2 + g holds the 32 keys that the lanes of half-wave g own in a 64-key tile, in the
+// order of their score accumulators: bit 16 kt + i for key 32 kt + 8 (i / 4) + 4 g + i % 4.  Next to them, for each block of
+// 32 rows, the first tile with a key that one of its rows sees and the one past the last (0x7FFFFFFF, 0: no such tile).
+// Bound by one read of the mask; what it saves: 60 heads of 1282 x 128 under a mask of whole key tails 450 -> 80 us (the
+// bytes, read where they are used, cost two operations per score and head even when the rows are 4-byte aligned: 40 heads
+// of 1920 173 -> 81).  A work-group per block of rows: every byte of the mask is read once, whatever the number of heads that share it, and
+// rows may start anywhere (gfx950 loads 16 bytes from any address).
+__global__ __launch_bounds__(256) void sdpa_pack_mask_kernel(const uint8_t *mask, int64_t sb, int64_t sh, int planes_h, int Sq, int Skv, uint32_t *bits, int2_t *range) {
+    struct __attribute__((packed, aligned(1))) bytes16_t { uint4_t v; };
+    __shared__ int lo_s, hi_s;
+    const int nb32 = (Sq + 31) / 32, tiles = (Skv + BN - 1) / BN;
+    const int plane = blockIdx.x / nb32, blk = blockIdx.x % nb32;
+    const int row = blk * 32 + threadIdx.x % 32;
+    const uint8_t *M = mask + (plane / planes_h) * sb + (plane % planes_h) * sh + static_cast<int64_t>(row) * Skv;
+    if (threadIdx.x == 0) {
+        lo_s = 0x7FFFFFFF;
+        hi_s = 0;
+    }
+    __syncthreads();
+    int lo = 0x7FFFFFFF, hi = 0;
+    if (row < Sq) {
+        for (int t = threadIdx.x / 32; t < tiles; t += 8) {
+            uint2_t out = {0, 0};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) { // keys 16 c .. 16 c + 15 of the tile
+                const int key = t * BN + 16 * c;
+                uint4_t v;
+                if (key + 16 <= Skv) {
+                    v = reinterpret_cast<const bytes16_t *>(M + key)->v;
+                } else {
+                    v = uint4_t{~0u, ~0u, ~0u, ~0u};
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (key + i < Skv && M[key + i] == 0) v[i / 4] &= ~(0xFFu << (8 * (i % 4)));
+                }
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t set = (((v[w] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v[w]) & 0x80808080u; // bit 7 of every nonzero byte
+                    const uint32_t nibble = ((set >> 7) * 0x10204080u) >> 28;
+                    const int word = 4 * c + w; // keys 4 word .. 4 word + 3
+                    out[word % 2] |= nibble << (16 * (word / 8) + 4 * ((word % 8) / 2));
+                }
+            }
+            reinterpret_cast<uint2_t *>(bits)[(plane * static_cast<int64_t>(tiles) + t) * Sq + row] = out;
+            if ((out.x & out.y) != ~0u) {
+                lo = min(lo, t);
+                hi = t + 1;
+            }
+        }
+        if (hi > 0) {
+            atomicMin(&lo_s, lo);
+            atomicMax(&hi_s, hi);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) range[blockIdx.x] = int2_t{lo_s, hi_s};
+}
+
 // --------------------------------- pipelined MFMA kernel, head_dim 128 and 64
 // Same tiling as sdpa_mfma_kernel, restructured for throughput:
 //  * K and V tiles go HBM -> LDS directly (buffer_load ... lds), no staging
@@ -385,23 +444,29 @@ __device__ __forceinline__ int4_t make_rsrc(const void *base, int bytes) {
 
 // NW waves per work-group (4: two work-groups share a CU; 8: one work-group per CU, each
 // K/V tile fetched once for 256 query rows instead of 128).
-// Head sizes between the compiled ones (a.D = 40 .. 56 on D = 64, 72 .. 120 on D = 128, multiples of 8) run as the next
-// compiled size with zeros in the missing dims: the Q fragments beyond a.D stay zero, the lanes that would fetch a K/V
-// chunk beyond a.D are sent outside the tile's descriptor (the load writes zeros to LDS), the output keeps a.D columns.
-// SPLIT = 2 (problems too small to give every SIMD two waves otherwise): the work-group's waves form two halves that
-// take the same 32 * NW / 2 query rows and one half of the keys each, through K/V tile buffers of their own; the second
-// half hands its accumulators, reference maximum and row sums to the first through LDS at the end.  No causal mask, no
-// explicit mask, at least two key tiles.
+// Head sizes between the compiled ones (a.D = 40 .. 56 on D = 64, 72 .. 120 on D = 128, multiples of 8) run in the rows of
+// the next compiled size with zeros in the missing dims: the Q fragments beyond a.D stay zero, the lanes that would fetch
+// a K/V chunk beyond a.D are sent outside the tile's descriptor (the load writes zeros to LDS), the output keeps a.D
+// columns.  PAD: how many dims of the row are computed -- up to 80 dims take 5 + 6 MFMAs per 32 keys instead of the 8 + 8
+// of 128 (128 heads of 4096 x 80, causal: 460 -> 401 us).
+// SPLIT = 2 (problems too small to give every SIMD two waves otherwise): the work-group's waves form two groups, which
+// take the same 32 * NW / 2 query rows and one part of the key tiles each, through K/V tile buffers of their own; the
+// second hands its accumulators, reference maximum and row sums to the first through LDS at the end.  A part may be empty.
+// (Four parts of 32 rows: 6 heads of 1344 x 64 11.6 us instead of 12.2, 10 of 356 17.7 instead of 7.9.)
 // (Four K and four V tile buffers with counted waits, so that a tile is requested three steps before its use, made the
 // 4-wave head_dim-64 kernel 5 % slower on small problems: its step is not waiting for tiles.)
 // (PAD: such a head size; the exact sizes keep a kernel without its tests.)
-template <bool BF16, bool HAS_MASK, int NW, int D, int SPLIT = 1, bool PAD = false>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_kernel(const SdpaArgs a) {
+// MASK: how the explicit mask is read.  MASK_BYTES: from the caller's bytes.  MASK_BITS: from the bits that
+// sdpa_pack_mask_kernel made of it -- one word per lane and tile, tiles beyond the block's first and last visible key left out.
+enum SdpaMask { MASK_NONE = 0, MASK_BYTES = 1, MASK_BITS = 2 };
+template <bool BF16, int MASK, int NW, int D, int SPLIT = 1, int PAD = 0>
+__global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void sdpa_mfma_pipelined_kernel(const SdpaArgs a) {
     static_assert(D == 128 || D == 64, "head sizes with a direct-to-LDS pipeline");
-    static_assert(SPLIT == 1 || (SPLIT == 2 && !HAS_MASK && NW == 4 && D == 64), "key split: the 64 KiB of static LDS hold two sets of head_dim-64 tiles");
+    static_assert(NW % SPLIT == 0 && SPLIT * D <= 256, "key split: the parts' tile buffers have to fit the LDS");
     constexpr int NWH = NW / SPLIT;       // waves that share a key range
-    constexpr int KT = D / 16;            // k-steps of the score product
-    constexpr int DT = D / 32;            // 32-row tiles of O^T
+    constexpr int DE = PAD ? PAD : D;     // dims that are computed
+    constexpr int KT = (DE + 15) / 16;    // k-steps of the score product
+    constexpr int DT = (DE + 31) / 32;    // 32-row tiles of O^T
     constexpr int BMW = 32 * NWH;         // query rows per work-group
     constexpr int ROWB = 2 * D;           // bytes per LDS row
     constexpr int CHUNKS = ROWB / 16;     // 16-byte chunks per row
@@ -412,43 +477,41 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
 
     const int tid = threadIdx.x;
     const int lane = tid % WAVE;
-    const int part = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE / NWH); // which half of the keys
-    const int wave = SPLIT == 1 ? tid / WAVE : __builtin_amdgcn_readfirstlane(tid / WAVE % NWH); // position among the waves of its half
+    const int part = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE / NWH); // which part of the keys
+    const int wave = SPLIT == 1 ? tid / WAVE : __builtin_amdgcn_readfirstlane(tid / WAVE % NWH); // position among the waves of its part
     unsigned char *const lds = lds_all + part * 4 * TILEB;
     const int ql = lane % 32, g = lane / 32;
 
-    // Work-group -> (batch*head, query block(s)).  Under a causal mask query block i needs
-    // i+1 key blocks, so a work-group takes the pair (i, nqb-1-i): every work-group then
-    // carries the same load and the launch has no ragged tail.  Work-groups are dealt to
-    // the 8 XCDs round-robin by id; one (batch, head) stays on one XCD so that its K/V
-    // live in that XCD's L2.
+    // Work-group -> (batch*head, query block).  Under a causal mask query block i needs i+1 key blocks: the longest
+    // blocks of every (batch, head) come first.  Work-groups are dealt to the 8 XCDs round-robin by id; one
+    // (batch, head) stays on one XCD so that its K/V live in that XCD's L2.
     const int L = blockIdx.x;
     const int BH = a.B * a.H;
     const int nqb = (a.Sq + BMW - 1) / BMW;
-    const int per_bh = a.causal ? (nqb + 1) / 2 : nqb; // work-groups per (batch, head)
-    int bh, slot;
-    if (BH % 8 == 0) {
+    int bh, qb;
+    if (a.causal) {
+        bh = L % BH;
+        qb = nqb - 1 - L / BH;
+    } else if (BH % 8 == 0) {
         const int xcd = L % 8, j = L / 8;
-        bh = (j / per_bh) * 8 + xcd;
-        slot = j % per_bh;
+        bh = (j / nqb) * 8 + xcd;
+        qb = j % nqb;
     } else {
-        bh = L / per_bh;
-        slot = L % per_bh;
+        bh = L / nqb;
+        qb = L % nqb;
     }
     const int b = bh / a.H, h = bh % a.H;
-    const int npass = (a.causal && slot != nqb - 1 - slot) ? 2 : 1;
 
     const uint16_t *Q = static_cast<const uint16_t *>(a.q) + b * a.qs[0] + h * a.qs[1];
     const uint16_t *K = static_cast<const uint16_t *>(a.k) + b * a.ks[0] + h * a.ks[1];
     const uint16_t *V = static_cast<const uint16_t *>(a.v) + b * a.vs[0] + h * a.vs[1];
     uint16_t *O = static_cast<uint16_t *>(a.o) + b * a.os[0] + h * a.os[1];
-    const uint8_t *M = HAS_MASK ? a.mask + b * a.ms[0] + h * a.ms[1] : nullptr;
-    // Explicit masks are read as the eight 4-byte words that cover this lane's keys of a tile (the lane's 32 keys are
-    // 8 runs of 4 consecutive ones), a step before the tile's score MFMAs are issued, and applied by starting the
-    // masked elements' accumulators at -inf: the mask costs two VALU operations per score and no pass of its own.
-    // Needs 4-byte aligned rows (else, and for the ragged last tile, single bytes are read after the MFMAs).
-    const bool mask_words = HAS_MASK && a.Skv % 4 == 0 && (reinterpret_cast<uintptr_t>(M) & 3u) == 0;
+    const uint8_t *M = MASK == MASK_BYTES ? a.mask + b * a.ms[0] + h * a.ms[1] : nullptr;
+    // MASK_BYTES: the mask is read as the eight 4-byte words that cover this lane's keys of a tile (the lane's 32 keys are
+    // 8 runs of 4 consecutive ones; rows may start anywhere), a step before the tile's score MFMAs are issued, and
+    // applied by starting the masked elements' accumulators at -inf: two VALU operations per score and no pass of its own.
     uint32_t mk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int plane = b * a.mask_plane[0] + h * a.mask_plane[1]; // MASK_BITS: which of the packed masks
 
     const int dv = PAD ? a.D : D; // the head size in memory (<= D, a multiple of 8)
     const int krow_bytes = static_cast<int>(a.ks[2]) * 2, vrow_bytes = static_cast<int>(a.vs[2]) * 2;
@@ -456,24 +519,30 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
     const int4_t vrsrc = make_rsrc(V, (a.Skv - 1) * vrow_bytes + dv * 2);
 
     // ---- HBM -> LDS mapping.  A wave-wide load moves RPL rows; load n of wave w covers
-    // tile rows RPL*NW*n + RPL*w + lane / CHUNKS; the lane fetches the chunk that belongs at
+    // tile rows RPL*NWH*n + RPL*w + lane / CHUNKS; the lane fetches the chunk that belongs at
     // position lane % CHUNKS of the swizzled row (the swizzles only see row & 15).
     const int ld_r = RPL * wave + lane / CHUNKS;
     // (a chunk beyond the head size in memory: an offset that stays outside the descriptor whatever tile offset is
     // added to it -- a (batch, head) slice spans less than 2^31 bytes)
-    const int k_chunk = (lane % CHUNKS) ^ swizzle_k<D>(ld_r), v_chunk = (lane % CHUNKS) ^ swizzle_v<D>(ld_r);
-    const int k_voff = k_chunk * 8 < dv ? ld_r * krow_bytes + k_chunk * 16 : static_cast<int>(0x80000000u);
-    const int v_voff = v_chunk * 8 < dv ? ld_r * vrow_bytes + v_chunk * 16 : static_cast<int>(0x80000000u);
+    // (loads that move 8 rows: the odd ones have the swizzle of the rows 8 further down)
+    constexpr int NVOFF = RPL * NWH < 16 ? 2 : 1;
+    int k_voff[NVOFF], v_voff[NVOFF];
+#pragma unroll
+    for (int o = 0; o < NVOFF; ++o) {
+        const int k_chunk = (lane % CHUNKS) ^ swizzle_k<D>(ld_r + 8 * o), v_chunk = (lane % CHUNKS) ^ swizzle_v<D>(ld_r + 8 * o);
+        k_voff[o] = k_chunk * 8 < dv ? ld_r * krow_bytes + k_chunk * 16 : static_cast<int>(0x80000000u);
+        v_voff[o] = v_chunk * 8 < dv ? ld_r * vrow_bytes + v_chunk * 16 : static_cast<int>(0x80000000u);
+    }
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)); // LDS addresses fit 32 bits
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + RPL * wave * ROWB);
     // load n (0 .. NLOAD-1) of this wave's share of a K / V tile
-    // (tile: counted from the first tile of this half's key range, tile0 -- set per pass below)
+    // (tile: counted from the first tile of this part's key range, tile0 -- set below)
     int tile0 = 0;
     auto load_k1 = [&](int tile, int buf, int n) {
-        load_to_lds_16(krsrc, lds_wave + buf * TILEB + n * RPL * NWH * ROWB, k_voff + ((tile0 + tile) * BN + RPL * NWH * n) * krow_bytes);
+        load_to_lds_16(krsrc, lds_wave + buf * TILEB + n * RPL * NWH * ROWB, k_voff[n % NVOFF] + ((tile0 + tile) * BN + RPL * NWH * n) * krow_bytes);
     };
     auto load_v1 = [&](int tile, int buf, int n) {
-        load_to_lds_16(vrsrc, lds_wave + (2 + buf) * TILEB + n * RPL * NWH * ROWB, v_voff + ((tile0 + tile) * BN + RPL * NWH * n) * vrow_bytes);
+        load_to_lds_16(vrsrc, lds_wave + (2 + buf) * TILEB + n * RPL * NWH * ROWB, v_voff[n % NVOFF] + ((tile0 + tile) * BN + RPL * NWH * n) * vrow_bytes);
     };
     auto load_k = [&](int tile, int buf) {
 #pragma unroll
@@ -500,9 +569,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             }
     }
 
-    for (int pass = 0; pass < npass; ++pass) {
-        // heavier block of the pair first
-        const int qb = a.causal ? (pass == 0 ? nqb - 1 - slot : slot) : slot;
+    {
         const int q0 = qb * BMW;
         const int qw0 = q0 + wave * 32; // first query row of this wave
         const int q = qw0 + ql;
@@ -533,11 +600,24 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
 
         int kv_end = a.Skv;
         if (a.causal) kv_end = min(a.Skv, q0 + BMW);
-        const int ntiles_all = (kv_end + BN - 1) / BN; // >= 1
-        // key split: the first half takes the larger share; `nsteps` is what the work-group's barriers are counted by
-        const int nsteps = SPLIT == 1 ? ntiles_all : (ntiles_all + 1) / 2;
-        const int ntiles = SPLIT == 1 ? ntiles_all : part == 0 ? nsteps : ntiles_all - nsteps; // >= 1 (the launcher sees to two tiles)
-        tile0 = SPLIT == 1 ? 0 : part * nsteps;
+        int first = 0, beyond = (kv_end + BN - 1) / BN; // key tiles of this query block
+        if constexpr (MASK == MASK_BITS) { // those with a key that some row of the block sees (if none: one tile, all of it masked)
+            const int nb32 = (a.Sq + 31) / 32;
+            int lo = 0x7FFFFFFF, hi = 0;
+            for (int w = 0; w < NWH; ++w)
+                if (q0 / 32 + w < nb32) {
+                    const int2_t r = a.mask_range[plane * static_cast<int64_t>(nb32) + q0 / 32 + w];
+                    lo = min(lo, r.x);
+                    hi = max(hi, r.y);
+                }
+            beyond = __builtin_amdgcn_readfirstlane(min(beyond, hi));
+            first = max(0, min(__builtin_amdgcn_readfirstlane(lo), beyond - 1));
+        }
+        const int ntiles_all = max(beyond - first, 1);
+        // key split: `nsteps` is what the work-group's barriers are counted by; the last part may be short or empty
+        const int nsteps = (ntiles_all + SPLIT - 1) / SPLIT;
+        const int ntiles = SPLIT == 1 ? ntiles_all : max(0, min(nsteps, ntiles_all - part * nsteps));
+        tile0 = first + (SPLIT == 1 ? 0 : min(part * nsteps, ntiles_all - 1));
 
         // v_maximum3_f32: NaN-propagating maximum, which (unlike maxnum) needs no input canonicalisation
         auto max3 = [](float x, float y, float z) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z); };
@@ -558,23 +638,33 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             return max_across_halves(max3(m0, s[0][15], __builtin_elementwise_maximum(m2, s[1][15])));
         };
 
-        // initial value of the score accumulators of tile `tile`: `base`, or -inf where the mask words (already in
-        // mk) say so
-        auto init_scores = [&](int tile, float base, float16_t (&s)[2]) {
-            const bool use_words = HAS_MASK && mask_words && (tile0 + tile) * BN + BN <= a.Skv;
+        // initial value of the score accumulators of a tile: `base`, or -inf where the mask (already in mk) says so
+        auto init_scores = [&](float base, float16_t (&s)[2]) {
+            if constexpr (MASK == MASK_BITS) {
+                if (__builtin_amdgcn_ballot_w64(mk[0] != 0) != 0) { // (most tiles of a padding mask have no masked key)
+    #pragma unroll
+                    for (int kt = 0; kt < 2; ++kt)
+    #pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            const uint32_t dead = static_cast<uint32_t>(static_cast<int32_t>(mk[0] << (31 - (kt * 16 + i))) >> 31);
+                            s[kt][i] = __uint_as_float((dead & 0xFF800000u) | (~dead & __float_as_uint(base)));
+                        }
+                    return;
+                }
+            }
     #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
     #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     bool dead = false;
-                    if constexpr (HAS_MASK) dead = use_words && ((mk[kt * 4 + i / 4] >> (8 * (i % 4))) & 0xFFu) != 0;
+                    if constexpr (MASK == MASK_BYTES) dead = ((mk[kt * 4 + i / 4] >> (8 * (i % 4))) & 0xFFu) != 0;
                     s[kt][i] = dead ? NEG_INF_F : base;
                 }
         };
 
         // S^T = K Q^T for one tile (two 32-key sub-tiles); prologue only
         auto scores = [&](const unsigned char *Kb, float16_t (&s)[2]) {
-            init_scores(0, 0.0f, s);
+            init_scores(0.0f, s);
     #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
     #pragma unroll
@@ -585,19 +675,36 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             }
         };
 
-        // the mask words of this lane's keys of one tile: bytes 32 kt + 8 i4 + 4 g .. + 3 of the tile's 64, kt < 2, i4 < 4
+        // the mask of this lane's keys of one tile: bits, or bytes 32 kt + 8 i4 + 4 g .. + 3 of the tile's 64, kt < 2, i4 < 4;
+        // keys past the last count as masked (rows past the last are never stored: nothing masked)
         auto load_mask_words = [&](int tile) {
-            if constexpr (HAS_MASK) {
+            if constexpr (MASK == MASK_BITS) {
+                if (q_ok) mk[0] = a.mask_bits[((plane * static_cast<int64_t>(a.mask_tiles) + tile0 + tile) * a.Sq + q) * 2 + g];
+            }
+            if constexpr (MASK == MASK_BYTES) {
                 const int kvb = (tile0 + tile) * BN;
-                if (mask_words && q_ok && kvb + BN <= a.Skv) {
-                    const uint32_t *row = reinterpret_cast<const uint32_t *>(M + static_cast<int64_t>(q) * a.Skv + kvb + 4 * g);
+                if (q_ok) {
+                    const uint8_t *row = M + static_cast<int64_t>(q) * a.Skv + kvb + 4 * g;
+                    const int left = a.Skv - kvb - 4 * g; // bytes of the row from there on
+                    if (kvb + BN <= a.Skv) {
     #pragma unroll
-                    for (int w8 = 0; w8 < 8; ++w8) mk[w8] = row[(w8 / 4) * 8 + (w8 % 4) * 2];
+                        for (int w8 = 0; w8 < 8; ++w8) mk[w8] = reinterpret_cast<const uint32_unaligned_t *>(row + (w8 / 4) * 32 + (w8 % 4) * 8)->v;
+                    } else {
+    #pragma unroll
+                        for (int w8 = 0; w8 < 8; ++w8) {
+                            const int at = (w8 / 4) * 32 + (w8 % 4) * 8;
+                            mk[w8] = ~0u;
+                            if (at + 4 <= left) mk[w8] = reinterpret_cast<const uint32_unaligned_t *>(row + at)->v;
+                            else
+                                for (int i = 0; i < 3; ++i)
+                                    if (at + i < left && row[at + i] == 0) mk[w8] &= ~(0xFFu << (8 * i));
+                        }
+                    }
                 }
             }
         };
 
-        // Key masking of tile j (diagonal, key tail, explicit mask), then the row maximum.
+        // Key masking of tile j (diagonal, key tail), then the row maximum.
         auto mask_and_max = [&](int kv0, float16_t (&s)[2]) {
             const int kv_limit = a.causal ? min(a.Skv - 1, q) : a.Skv - 1;
     #pragma unroll
@@ -605,11 +712,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
     #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int kv = kv0 + kt * 32 + (i / 4) * 8 + g * 4 + (i % 4);
-                    bool dead = kv > kv_limit;
-                    if constexpr (HAS_MASK) {
-                        if (!(mask_words && kv0 + BN <= a.Skv) && q_ok && kv < a.Skv) dead = dead || M[static_cast<int64_t>(q) * a.Skv + kv] != 0;
-                    }
-                    if (dead) s[kt][i] = NEG_INF_F;
+                    if (kv > kv_limit) s[kt][i] = NEG_INF_F;
                 }
             return row_max(s);
         };
@@ -642,8 +745,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
         //   slots  0..NS-1      score MFMAs of the NEXT tile (K fragments from Kn)
         //   slots NS..NS+NP-1   O^T += V^T P^T of the CURRENT tile (V fragments from Vb)
         // LDS fragment reads run PF slots ahead of their MFMA.  The VALU work of the current
-        // tile's softmax (exp2, pack, row sum: 16 pairs) is dealt out over the score slots (D = 128: one pair in
-        // 12 of them and in the first four PV slots; D = 64: two pairs in each), always ahead of the P fragment
+        // tile's softmax (exp2, pack, row sum: 16 pairs) is dealt out over the score slots (128 dims: one pair in
+        // 12 of them and in the first four PV slots; fewer: one or two pairs in each), always ahead of the P fragment
         // that the PV MFMAs need; the row maximum of the next tile is spread over PV slots.  A scheduling
         // barrier closes every slot so the compiler keeps this order.
         auto fused = [&](int j, const unsigned char *Kn, const unsigned char *Vb, const float16_t (&cur)[2], float16_t (&nxt)[2], float &mx_next) {
@@ -677,9 +780,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             for (int m = 0; m < NS + NP; ++m) {
                 if (m + PF < NS + NP) read_frag(m + PF);
                 if (m < NS) {
-                    if constexpr (HAS_MASK) {
+                    if constexpr (MASK != MASK_NONE) {
                         if (m == 0) { // both sub-tiles at once: the mask words are then free for the tile after
-                            init_scores(j + 1, -m_use, nxt);
+                            init_scores(-m_use, nxt);
                             if (j + 2 < ntiles) load_mask_words(j + 2);
                         }
                     } else if (m % KT == 0) {
@@ -687,18 +790,19 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
                         for (int i = 0; i < 16; ++i) nxt[m / KT][i] = -m_use; // logits come out relative to the reference
                     }
                     nxt[m / KT] = mfma_32x32x16<BF16>(fr[m % RING], qf[m % KT], nxt[m / KT]);
-                    if constexpr (D == 128) {
+                    if constexpr (KT == 8) {
                         if (m % 4 != 3) exp_pair((m / 4) * 3 + m % 4);
-                    } else {
-                        exp_pair(2 * m);
-                        exp_pair(2 * m + 1);
+                    } else { // 16 pairs over NS < 16 slots, two in the first ones
+                        constexpr int TWO = 16 - NS;
+                        exp_pair(m < TWO ? 2 * m : m + TWO);
+                        if (m < TWO) exp_pair(2 * m + 1);
                     }
                 } else {
                     const int idx = m - NS, ks = idx / DT, dt = idx % DT;
                     const uint4_t pf = {w[4 * ks], w[4 * ks + 1], w[4 * ks + 2], w[4 * ks + 3]};
                     oacc[dt] = mfma_32x32x16<BF16>(fr[m % RING], pf, oacc[dt]);
-                    constexpr int MAX0 = D == 128 ? 4 : 0; // first PV slot that works on the next tile's maximum
-                    if (D == 128 && idx < 4) exp_pair(12 + idx);
+                    constexpr int MAX0 = KT == 8 ? 4 : 0; // first PV slot that works on the next tile's maximum
+                    if (KT == 8 && idx < 4) exp_pair(12 + idx);
                     if (idx >= MAX0 && idx < MAX0 + 8) { // two partial maxima per slot over the next tile's 32 scores
                         const int c = idx - MAX0, kt = c / 4, i0 = (c % 4) * 4;
                         if (c % 4 < 2) {
@@ -707,14 +811,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
                             pm[kt * 2 + c % 4 - 2] = max3(max3(pm[kt * 2 + c % 4 - 2], nxt[kt][i0], nxt[kt][i0 + 1]), nxt[kt][i0 + 2], nxt[kt][i0 + 3]);
                         }
                     }
-                    if (idx == (D == 128 ? MAX0 + 8 : MAX0 + 7)) mx_next = max_across_halves(max3(max3(pm[0], pm[1], pm[2]), pm[3], NEG_INF_F));
+                    if (idx == (NP > MAX0 + 8 ? MAX0 + 8 : MAX0 + 7)) mx_next = max_across_halves(max3(max3(pm[0], pm[1], pm[2]), pm[3], NEG_INF_F));
                 }
                 // the tile prefetch is spread over the slots instead of bursting at the step start:
-                // K(j+2) in slots 1, 3, .., V(j+1) in slots 2, 4, ..
+                // K(j+2) in slots 1, 3, .., V(j+1) in slots 2, 4, .. (the last of a full set in slot 0)
                 if (m % 2 == 1 && m / 2 < NLOAD) {
                     if (want_k) load_k1(j + 2, j & 1, m / 2);
                 } else if (m % 2 == 0 && m >= 2 && m / 2 - 1 < NLOAD) {
                     if (want_v) load_v1(j + 1, (j + 1) & 1, m / 2 - 1);
+                } else if (m == 0 && 2 * NLOAD == NS + NP) { // as many loads as half of the slots
+                    if (want_v) load_v1(j + 1, (j + 1) & 1, NLOAD - 1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -740,7 +846,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             const unsigned char *Vb = lds + (2 + (j & 1)) * TILEB;
             const unsigned char *Kn = lds + ((j + 1) & 1) * TILEB;
             if (active) {
-                const bool need_mask = (a.causal && kv0 + BN - 1 > qw0) || (kv0 + BN > a.Skv) || (HAS_MASK && !mask_words);
+                const bool need_mask = (a.causal && kv0 + BN - 1 > qw0) || (MASK == MASK_NONE && kv0 + BN > a.Skv);
                 float mloc = mx_cur;
                 if (need_mask) mloc = mask_and_max(kv0, cur);
                 update_max(mloc, cur);
@@ -760,30 +866,37 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
             if (j + 1 < nsteps) step(j + 1, sB, mxB, sA, mxA);
         }
 
-        if constexpr (SPLIT == 2) {
-            // The second half's state goes to the first through LDS (the tile buffers are free: every step ends in a
-            // barrier), value-major so that the 64 lanes of a wave touch consecutive words.  Both halves hold sums of
+        if constexpr (SPLIT > 1) {
+            // The other parts' states go to the first through LDS (the tile buffers are free: every step ends in a
+            // barrier), value-major so that the 64 lanes of a wave touch consecutive words.  All hold sums of
             // 2^(logit - reference) with a reference of their own: brought to the larger one and added.
-            float *xch = reinterpret_cast<float *>(lds_all) + wave * (DT * 16 + 2) * WAVE + lane;
-            if (part == 1) {
+            constexpr int STATE = (DT * 16 + 2) * WAVE; // floats of one wave
+            float *const xch = reinterpret_cast<float *>(lds_all) + wave * STATE + lane;
+            if (part > 0) {
+                float *const mine = xch + (part - 1) * NWH * STATE;
     #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
     #pragma unroll
-                    for (int i = 0; i < 16; ++i) xch[(dt * 16 + i) * WAVE] = oacc[dt][i];
-                xch[DT * 16 * WAVE] = m_run;
-                xch[(DT * 16 + 1) * WAVE] = l_run;
+                    for (int i = 0; i < 16; ++i) mine[(dt * 16 + i) * WAVE] = oacc[dt][i];
+                mine[DT * 16 * WAVE] = m_run;
+                mine[(DT * 16 + 1) * WAVE] = l_run;
             }
             __syncthreads();
-            if (part == 1) return; // (one pass: no causal mask)
-            const float m_other = xch[DT * 16 * WAVE], l_other = xch[(DT * 16 + 1) * WAVE];
-            const float m_new = __builtin_elementwise_maximum(m_run, m_other);
-            const float a_mine = m_run == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-            const float a_other = m_other == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_other - m_new);
-            l_run = l_run * a_mine + l_other * a_other;
+            if (part > 0) return;
     #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+            for (int other = 0; other < SPLIT - 1; ++other) {
+                const float *const from = xch + other * NWH * STATE;
+                const float m_other = from[DT * 16 * WAVE], l_other = from[(DT * 16 + 1) * WAVE];
+                const float m_new = __builtin_elementwise_maximum(m_run, m_other);
+                const float a_mine = m_run == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                const float a_other = m_other == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_other - m_new);
+                m_run = m_new;
+                l_run = l_run * a_mine + l_other * a_other;
     #pragma unroll
-                for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a_mine + xch[(dt * 16 + i) * WAVE] * a_other;
+                for (int dt = 0; dt < DT; ++dt)
+    #pragma unroll
+                    for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a_mine + from[(dt * 16 + i) * WAVE] * a_other;
+            }
         }
 
         const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
@@ -818,9 +931,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sdpa_mfma_pipelined_
 //    matrix pipe: next to MFMAs every one of them costs about 18 cycles.
 //  * the score accumulators of a tile exist once (the softmax of tile j ends before the MFMAs of tile j+1 start in
 //    the same wave), which leaves registers for everything else without spills.
-//  * a work-group is persistent: it walks the units blockIdx.x, blockIdx.x + gridDim.x, ... and requests the first K
-//    and V tiles of the next segment (the second query block of a causal pair, or the next unit) during the last two
-//    steps of the one at hand, so a segment does not start with an empty pipeline.
+//  * a work-group is persistent: it walks several segments (a (batch, head) and a query block) and requests the first K
+//    and V tiles of the next one during the last two steps of the one at hand, so a segment does not start with an empty
+//    pipeline.  Under a causal mask the segments are dealt in pairs (i, n-1-i) of equal sums where these fill their last
+//    round, else longest first, every other round in reverse, which leaves the sums within about one block of each other
+//    (96 heads of 1433, 288 pairs: 95 -> 70 us; 128 heads of 4096, 1024 pairs: 493 us in pairs, 510 otherwise -- fewer
+//    work-groups share a (batch, head) at a time).
 //  * the output is written as 16 bytes per lane after one exchange between the half-waves.
 // No explicit mask and exact head sizes only (the pipelined kernel keeps those cases).
 template <bool BF16, int D>
@@ -840,30 +956,35 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
 
     const int BH = a.B * a.H;
     const int nqb = (a.Sq + BMW - 1) / BMW;
-    const int per_bh = a.causal ? (nqb + 1) / 2 : nqb;
-    const int n_wg = per_bh * BH; // units of work: a (batch, head) and a query block (a pair of them under a causal mask)
     const int krow_bytes = static_cast<int>(a.ks[2]) * 2, vrow_bytes = static_cast<int>(a.vs[2]) * 2;
-    // A work-group walks the units blockIdx.x, blockIdx.x + gridDim.x, ... (units are dealt to the 8 XCDs round-robin by
-    // id, and gridDim.x is a multiple of 8: one (batch, head) stays on one XCD); a unit is one or two segments (passes).
+    // Segment r of a work-group.  Causal, a.pairs = 0: unit r * gridDim.x + blockIdx.x, longest blocks first, counted from the
+    // other end in odd rounds -- in eights, since work-groups are dealt to the 8 XCDs round-robin by id: one
+    // (batch, head) stays on one XCD.  Causal, a.pairs = 1: blocks i and nqb-1-i (nqb is even) in turn, neighbouring
+    // work-groups on one (batch, head).
     struct Segment { int bh, qb, ntiles; };
-    auto segment_of = [&](int L, int pass) {
-        int bh, slot;
-        if (BH % 8 == 0) {
+    auto segment_of = [&](int r) __attribute__((always_inline)) { // ntiles = 0: no such segment
+        const int G = gridDim.x, w = blockIdx.x;
+        const bool pairs = a.causal && a.pairs;
+        const int per_bh = pairs ? nqb / 2 : nqb;
+        int L, bh, qb;
+        if (pairs) L = r / 2 * G + w;
+        else L = r * G + (a.causal && r % 2 == 1 && G % 8 == 0 ? G - 8 - w / 8 * 8 + w % 8 : w);
+        if (L >= per_bh * BH) return Segment{0, 0, 0};
+        if (a.causal && !pairs) {
+            bh = L % BH;
+            qb = nqb - 1 - L / BH; // query block i needs i + 1 key blocks
+        } else if (BH % 8 == 0) {
             const int xcd = L % 8, j = L / 8;
             bh = (j / per_bh) * 8 + xcd;
-            slot = j % per_bh;
+            qb = j % per_bh;
         } else {
             bh = L / per_bh;
-            slot = L % per_bh;
+            qb = L % per_bh;
         }
-        const int qb = a.causal ? (pass == 0 ? nqb - 1 - slot : slot) : slot;
+        if (pairs && r % 2 == 0) qb = nqb - 1 - qb; // the longer one of the pair first
         int kv_end = a.Skv;
         if (a.causal) kv_end = min(a.Skv, qb * BMW + BMW);
         return Segment{bh, qb, (kv_end + BN - 1) / BN};
-    };
-    auto passes_of = [&](int L) {
-        const int slot = BH % 8 == 0 ? (L / 8) % per_bh : L % per_bh;
-        return (a.causal && slot != nqb - 1 - slot) ? 2 : 1;
     };
     auto k_rsrc_of = [&](int bh) { return make_rsrc(static_cast<const uint16_t *>(a.k) + (bh / a.H) * a.ks[0] + (bh % a.H) * a.ks[1], (a.Skv - 1) * krow_bytes + D * 2); };
     auto v_rsrc_of = [&](int bh) { return make_rsrc(static_cast<const uint16_t *>(a.v) + (bh / a.H) * a.vs[0] + (bh % a.H) * a.vs[1], (a.Skv - 1) * vrow_bytes + D * 2); };
@@ -906,17 +1027,17 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
     auto wait_tiles = [&] { __builtin_amdgcn_s_waitcnt(0x0F70); asm volatile("" :: "v"(touch)); }; // vmcnt(0) (and the touch register stays reserved until here)
 
     bool prefetched = false; // the first tiles of the segment at hand were requested during the previous one
-    for (int L = blockIdx.x; L < n_wg; L += gridDim.x) {
-    const int npass = passes_of(L);
-    for (int pass = 0; pass < npass; ++pass) {
-        const Segment seg = segment_of(L, pass);
+    for (int r = 0;; ++r) {
+        const Segment seg = segment_of(r);
+        if (seg.ntiles == 0) break;
         const int b = seg.bh / a.H, h = seg.bh % a.H;
         const uint16_t *Q = static_cast<const uint16_t *>(a.q) + b * a.qs[0] + h * a.qs[1];
         uint16_t *O = static_cast<uint16_t *>(a.o) + b * a.os[0] + h * a.os[1];
         const int4_t krsrc = k_rsrc_of(seg.bh), vrsrc = v_rsrc_of(seg.bh);
         // the segment after this one: its first K and V tiles are requested in this segment's last two steps
-        const bool has_next = pass + 1 < npass || L + static_cast<int>(gridDim.x) < n_wg;
-        const Segment nxt = has_next ? (pass + 1 < npass ? segment_of(L, pass + 1) : segment_of(L + gridDim.x, 0)) : seg;
+        const Segment following = segment_of(r + 1);
+        const bool has_next = following.ntiles > 0;
+        const Segment nxt = has_next ? following : seg;
         const int4_t krsrc_n = k_rsrc_of(nxt.bh), vrsrc_n = v_rsrc_of(nxt.bh);
         const int qb = seg.qb;
         const int q0 = qb * BMW;
@@ -952,7 +1073,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
             const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
             return __builtin_elementwise_maximum(__uint_as_float(r[0]), __uint_as_float(r[1]));
         };
-        auto row_max = [&](const float16_t (&s)[2]) {
+        auto row_max = [&](const float16_t (&s)[2]) __attribute__((always_inline)) {
             float m0 = max3(s[0][0], s[0][1], s[0][2]), m1 = max3(s[0][8], s[0][9], s[0][10]);
             float m2 = max3(s[1][0], s[1][1], s[1][2]), m3 = max3(s[1][8], s[1][9], s[1][10]);
             m0 = max3(m0, s[0][3], s[0][4]); m1 = max3(m1, s[0][11], s[0][12]);
@@ -962,7 +1083,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
             m0 = max3(m0, s[0][7], m1); m2 = max3(m2, s[1][7], m3);
             return max_across_halves(max3(m0, s[0][15], __builtin_elementwise_maximum(m2, s[1][15])));
         };
-        auto mask_and_max = [&](int kv0, float16_t (&s)[2]) {
+        auto mask_and_max = [&](int kv0, float16_t (&s)[2]) __attribute__((always_inline)) {
             const int kv_limit = a.causal ? min(a.Skv - 1, q) : a.Skv - 1;
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
@@ -973,7 +1094,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
                 }
             return row_max(s);
         };
-        auto update_max = [&](float mloc, float16_t (&cur)[2]) {
+        auto update_max = [&](float mloc, float16_t (&cur)[2]) __attribute__((always_inline)) {
             const float ref = m_run == NEG_INF_F ? 0.0f : m_run;
             const float m_new = __builtin_elementwise_maximum(m_run, mloc + ref);
             if (__builtin_amdgcn_ballot_w64(m_new - m_run > RESCALE_THRESHOLD) != 0) {
@@ -1002,7 +1123,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
         uint32_t w[16];
 
         // softmax of the tile in s (scores relative to the reference): masks, row maximum, rescale, P = 2^s packed to w
-        auto softmax_phase = [&](int j) {
+        auto softmax_phase = [&](int j) __attribute__((always_inline)) {
             const int kv0 = j * BN;
             const bool need_mask = (a.causal && kv0 + BN - 1 > qw0) || (kv0 + BN > a.Skv);
             const float mloc = need_mask ? mask_and_max(kv0, s) : row_max(s);
@@ -1025,7 +1146,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
         };
         // the NM MFMAs of a step: O^T += V^T P^T of tile j (P in w, V fragments from Vb) and S^T = K Q^T of tile j+1
         // (K fragments from Kn) alternate, so consecutive MFMAs never share an accumulator
-        auto mfma_phase = [&](const unsigned char *Kn, const unsigned char *Vb) {
+        auto mfma_phase = [&](const unsigned char *Kn, const unsigned char *Vb) __attribute__((always_inline)) {
             constexpr int RING = PF + 1;
             uint4_t fr[RING];
             // slot m: even -> score MFMA (m / 2): sub-tile kt = (m/2) & 1, k-step t = (m/2) >> 1; odd -> PV MFMA (m / 2): ks = idx / DT, dt = idx % DT
@@ -1076,7 +1197,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
         }
         __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): K buffer 0 is read
 
-        auto request = [&](int j, auto par) { // K(j+2) into the buffer of K(j), V(j+1) into the buffer of V(j-1)
+        auto request = [&](int j, auto par) __attribute__((always_inline)) { // K(j+2) into the buffer of K(j), V(j+1) into the buffer of V(j-1)
             constexpr int PAR = decltype(par)::value;
             if (j + 2 < ntiles) load_k(krsrc, j + 2, PAR);
             else if (pf_next && j + 2 - ntiles < nxt.ntiles) load_k(krsrc_n, j + 2 - ntiles, PAR);
@@ -1086,7 +1207,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
         auto active_at = [&](int j) { return !(a.causal && j * BN > qw0 + 31); };
         // One interval per tile, one barrier each: group 0 runs MFMAs(j+1) then softmax(j+1), group 1 softmax(j) then
         // MFMAs(j+1) -- the two waves of a SIMD are always in opposite phases.  PAR = j & 1 picks the tile buffers.
-        auto interval0 = [&](int j, auto par) {
+        auto interval0 = [&](int j, auto par) __attribute__((always_inline)) {
             constexpr int PAR = decltype(par)::value;
             wait_tiles();
             bar();
@@ -1094,7 +1215,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
             if (active_at(j)) mfma_phase(lds + (1 - PAR) * TILEB, lds + (2 + PAR) * TILEB);
             if (j + 1 < ntiles && active_at(j + 1)) softmax_phase(j + 1);
         };
-        auto interval1 = [&](int j, auto par) {
+        auto interval1 = [&](int j, auto par) __attribute__((always_inline)) {
             constexpr int PAR = decltype(par)::value;
             wait_tiles();
             bar();
@@ -1141,7 +1262,6 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
                     if (q_ok) *reinterpret_cast<uint4_t *>(orow + d) = wv;
                 }
         }
-    }
     }
 }
 
@@ -1605,9 +1725,15 @@ bool sdpa_decode_split = [] {
     return !(e && e[0] == '0');
 }();
 
-// AXHIP_SDPA_KEY_SPLIT=0 keeps small head_dim-64 problems on the unsplit kernel (for A/B timing)
-bool sdpa_key_split = [] {
+// AXHIP_SDPA_KEY_SPLIT=0 keeps small problems on the unsplit pipelined kernel, 2 splits the keys of every problem (for A/B timing)
+int sdpa_key_split = [] {
     const char *e = getenv("AXHIP_SDPA_KEY_SPLIT");
+    return e ? atoi(e) : -1;
+}();
+
+// AXHIP_SDPA_MASK_BITS=0: explicit masks are read as bytes by every kernel (for A/B timing)
+bool sdpa_mask_bits = [] {
+    const char *e = getenv("AXHIP_SDPA_MASK_BITS");
     return !(e && e[0] == '0');
 }();
 
@@ -1728,6 +1854,42 @@ DirectPlan direct_plan(const AxhipSdpaParams &p, bool has_mask) {
     return d;
 }
 
+// An explicit mask that is packed to bits first (sdpa_pack_mask_kernel)
+struct MaskPlan { bool on; int planes_b, planes_h, tiles, nb32; size_t bits_bytes, bytes; };
+MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
+    MaskPlan m{};
+    const bool half = p.dtype == AXHIP_DTYPE_BF16 || p.dtype == AXHIP_DTYPE_F16;
+    // (below 16 M scores the second launch, 4.7 us, costs more than reading bytes does: 128 heads of 384 x 202 21 us as bytes,
+    // 24 as bits; 64 heads of 832 x 832 37 and 25)
+    if (!half || !has_mask || !sdpa_mask_bits || p.head_dim <= 32 || p.head_dim > 128 || p.seq_q < 64 || p.seq_kv <= 0 ||
+        static_cast<int64_t>(p.batch) * p.heads * p.seq_q * p.seq_kv < (int64_t(16) << 20))
+        return m;
+    m.planes_b = p.mask_strides[0] == 0 ? 1 : p.batch;
+    m.planes_h = p.mask_strides[1] == 0 ? 1 : p.heads;
+    m.tiles = (p.seq_kv + BN - 1) / BN;
+    m.nb32 = (p.seq_q + 31) / 32;
+    const int64_t planes = static_cast<int64_t>(m.planes_b) * m.planes_h;
+    if (!launch_fits(planes * m.nb32, 256)) return m;
+    m.on = true;
+    m.bits_bytes = CallScratch::rounded(static_cast<size_t>(planes) * m.tiles * p.seq_q * 8);
+    m.bytes = m.bits_bytes + static_cast<size_t>(planes) * m.nb32 * sizeof(int2_t);
+    return m;
+}
+
+template <bool BF16, int MASK, int D, int PAD> void launch_pipelined_as(const SdpaArgs &a, int nw, bool split, unsigned grid, hipStream_t s) {
+    if (nw == 8) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 1, PAD>), dim3(grid), dim3(512), 0, s, a);
+    else if (!split) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 4, D, 1, PAD>), dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 4, D, 2, PAD>), dim3(grid), dim3(256), 0, s, a);
+}
+
+template <bool BF16, int MASK> void launch_pipelined(const SdpaArgs &a, int nw, bool split, unsigned grid, hipStream_t s) {
+    if (a.D == 64) launch_pipelined_as<BF16, MASK, 64, 0>(a, nw, split, grid, s);
+    else if (a.D == 128) launch_pipelined_as<BF16, MASK, 128, 0>(a, nw, split, grid, s);
+    else if (a.D < 64) launch_pipelined_as<BF16, MASK, 64, 64>(a, nw, split, grid, s);
+    else if (a.D <= 80) launch_pipelined_as<BF16, MASK, 128, 80>(a, nw, split, grid, s);
+    else launch_pipelined_as<BF16, MASK, 128, 128>(a, nw, split, grid, s);
+}
+
 template <bool BF16, int D> int launch_mfma(const SdpaArgs &a, hipStream_t s) {
     const unsigned grid = static_cast<unsigned>(a.nqb) * static_cast<unsigned>(a.B * a.H);
     constexpr size_t lds = D > 128 ? sdpa_mfma_lds_bytes<D>() : 0;
@@ -1774,8 +1936,8 @@ extern "C" {
 int axhip_sdpa_d128_occupancy(int waves) {
     int n = -1;
     hipError_t e = waves == 8
-        ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, sdpa_mfma_pipelined_kernel<true, false, 8, 128>, 512, 0)
-        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, sdpa_mfma_pipelined_kernel<true, false, 4, 128>, 256, 0);
+        ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, sdpa_mfma_pipelined_kernel<true, MASK_NONE, 8, 128>, 512, 0)
+        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, sdpa_mfma_pipelined_kernel<true, MASK_NONE, 4, 128>, 256, 0);
     return e == hipSuccess ? n : -static_cast<int>(e);
 }
 
@@ -1801,6 +1963,7 @@ size_t axhip_sdpa_workspace_bytes(const AxhipSdpaParams *params, int has_mask) {
     if (!params || validate(*params) != AXHIP_OK) return 0;
     if (pick_kernel(*params, nullptr, nullptr, nullptr, nullptr) != SdpaKind::MFMA) return 0;
     const DirectPlan direct = direct_plan(*params, has_mask != 0);
+    if (has_mask) return CallScratch::rounded(mask_plan(*params, true).bytes); // (with a mask the keys of a decoding step are not split)
     return CallScratch::rounded(direct.on ? direct.split.bytes : decode_split_plan(*params, has_mask != 0).bytes);
 }
 
@@ -1903,61 +2066,61 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         case 32: rc = bf ? launch_mfma<true, 32>(a, s) : launch_mfma<false, 32>(a, s); break;
         case 256: rc = bf ? launch_mfma<true, 256>(a, s) : launch_mfma<false, 256>(a, s); break;
         default: {
-            // 8-wave work-groups (256 query rows, each K/V tile fetched once for all of them) when that still gives
-            // every CU a work-group; 4-wave work-groups (128 rows, two per CU) for shorter or narrower problems
-            const int nqb8 = (p.seq_q + 255) / 256;
-            const int64_t g8 = static_cast<int64_t>(a.causal ? (nqb8 + 1) / 2 : nqb8) * a.B * a.H;
-            const bool wide = p.seq_q > 128 && sdpa_d128_waves != 4 && (g8 >= 256 || sdpa_d128_waves == 8);
-            // Problems with 4-wave work-groups for at most half of the CUs split the keys between the two halves of a
-            // work-group of 64 query rows instead: twice the work-groups, half the steps each (12 heads of 1024 rows:
-            // 14.8 -> 10.6 us).  With a work-group for nearly every CU (Whisper's 20 heads of 1500 frames: 240) the
-            // split changes nothing -- a SIMD issues the same instructions as one wave or as two.
-            const int64_t g4 = static_cast<int64_t>((p.seq_q + 127) / 128) * a.B * a.H;
-            if (p.head_dim > 32 && p.head_dim <= 64 && !mask && !a.causal && p.seq_kv > BN && g4 <= 128 && sdpa_key_split) {
-                last_schedule = "key_split";
-                const unsigned gs = static_cast<unsigned>((p.seq_q + 63) / 64) * static_cast<unsigned>(a.B * a.H);
-                if (p.head_dim == 64) {
-                    if (bf) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<true, false, 4, 64, 2>), dim3(gs), dim3(256), 0, s, a);
-                    else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<false, false, 4, 64, 2>), dim3(gs), dim3(256), 0, s, a);
-                } else {
-                    if (bf) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<true, false, 4, 64, 2, true>), dim3(gs), dim3(256), 0, s, a);
-                    else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<false, false, 4, 64, 2, true>), dim3(gs), dim3(256), 0, s, a);
-                }
-                break;
-            }
-            const int bmw = wide ? 256 : 128;
-            const int nqbw = (p.seq_q + bmw - 1) / bmw;
-            const unsigned g = static_cast<unsigned>(a.causal ? (nqbw + 1) / 2 : nqbw) * static_cast<unsigned>(a.B * a.H);
-#define AXHIP_LAUNCH_DX(BF, MK, DD)                                                                                       \
-    do {                                                                                                                  \
-        if (p.head_dim == DD) {                                                                                           \
-            if (wide) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF, MK, 8, DD>), dim3(g), dim3(512), 0, s, a);            \
-            else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF, MK, 4, DD>), dim3(g), dim3(256), 0, s, a);                 \
-        } else {                                                                                                          \
-            if (wide) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF, MK, 8, DD, 1, true>), dim3(g), dim3(512), 0, s, a);   \
-            else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF, MK, 4, DD, 1, true>), dim3(g), dim3(256), 0, s, a);        \
-        }                                                                                                                 \
-    } while (0)
-#define AXHIP_LAUNCH_D(DD)                                                                                                \
-    do {                                                                                                                  \
-        if (bf && mask) AXHIP_LAUNCH_DX(true, true, DD);                                                                  \
-        else if (bf) AXHIP_LAUNCH_DX(true, false, DD);                                                                    \
-        else if (mask) AXHIP_LAUNCH_DX(false, true, DD);                                                                  \
-        else AXHIP_LAUNCH_DX(false, false, DD);                                                                           \
-    } while (0)
-            last_schedule = wide ? "pipelined8" : "pipelined4";
-            if (p.head_dim == 128 && !mask && wide && sdpa_pingpong) {
+            // The work-group, by how many there are of which size for 256 CUs (timings of 90 problems of 8 .. 4096 blocks of
+            // 128 rows, none slower than with any other choice by more than 5 %):
+            //  * key_split, 64 rows whose keys the two halves of the work-group share, where even those blocks are one round
+            //    (16 heads of 1000 x 64: 14.7 -> 10.7 us; 24 of 260 7.7 -> 9.2); a causal problem has half the keys, so two
+            //    rounds still profit (20 heads of 1500: 19.6 -> 14.4).  Beyond 64 dims the two sets of tiles take a CU's LDS
+            //    to themselves: one round, and enough keys (8 heads of 500 x 128: 13.5 -> 12.3; of 128 7.7 -> 8.1).
+            //  * pingpong (128 dims, no mask), persistent with 256 rows, where every CU gets a block.
+            //  * pipelined4, 128 rows and two work-groups per CU, else -- causal blocks in work-groups of their own, longest
+            //    first: in pairs (i, n-1-i) of equal length half of the CUs had nothing to do (8 heads of 832 x 128: 28.0 -> 19.3).
+            //  * pipelined8, 256 rows, where that is one round of work-groups and 128 rows would be a round and a part
+            //    (42 heads of 1024 x 128: 40.0 -> 29.3), or where 128 rows would leave a second block nearly empty.
+            const int64_t slices64 = static_cast<int64_t>(p.batch) * p.heads;
+            const int64_t g64 = slices64 * ((p.seq_q + 63) / 64), g128 = slices64 * ((p.seq_q + 127) / 128), g256 = slices64 * ((p.seq_q + 255) / 256);
+            const int keys = a.causal ? std::min(p.seq_q, p.seq_kv) : p.seq_kv;
+            const bool small = p.head_dim <= 64 ? g64 <= (a.causal ? 512 : 256) : g64 <= 256 && (mask || keys >= 384);
+            const bool split = p.seq_kv > BN && sdpa_key_split != 0 && (small || sdpa_key_split == 2);
+            const bool pingpong = p.head_dim == 128 && !mask && !split && p.seq_q > 128 && (a.causal ? g256 >= 256 : g128 > 256) && sdpa_pingpong && sdpa_d128_waves != 4;
+            const bool wide = !split && !pingpong && p.seq_q > 128 && sdpa_d128_waves != 4 &&
+                              (sdpa_d128_waves == 8 || (!a.causal && ((g128 > 256 && g256 <= 256) || (p.seq_q <= 192 && g256 >= 256))));
+            const unsigned g = static_cast<unsigned>(split ? g64 : wide || pingpong ? g256 : g128);
+            last_schedule = split ? "key_split" : wide ? "pipelined8" : "pipelined4";
+            if (pingpong) {
                 last_schedule = "pingpong";
                 // persistent work-groups, one per CU (a multiple of 8: a (batch, head) keeps its XCD)
                 // (head_dim 64 stays on the pipelined kernel: with twice the softmax work per MFMA the two phases are
                 // too uneven -- measured 846 against 867 TFLOP/s on bf16 B4 H32 S4096 causal)
-                const unsigned gp = std::min<unsigned>(g, 256);
+                // (pairs where their last round of work-groups is full to 4 %)
+                const int64_t nqb256 = (p.seq_q + 255) / 256, pairs = slices64 * (nqb256 / 2);
+                a.pairs = a.causal && nqb256 % 2 == 0 && (pairs + 255) / 256 * 256 * 100 <= pairs * 104;
+                const unsigned gp = std::min<unsigned>(a.pairs ? static_cast<unsigned>(pairs) : g, 256);
                 if (bf) hipLaunchKernelGGL((sdpa_mfma_pingpong_kernel<true, 128>), dim3(gp), dim3(512), 0, s, a);
                 else hipLaunchKernelGGL((sdpa_mfma_pingpong_kernel<false, 128>), dim3(gp), dim3(512), 0, s, a);
-            } else if (p.head_dim <= 64) AXHIP_LAUNCH_D(64);
-            else AXHIP_LAUNCH_D(128);
-#undef AXHIP_LAUNCH_D
-#undef AXHIP_LAUNCH_DX
+            } else {
+                const int nw = wide ? 8 : 4;
+                const MaskPlan mp = mask_plan(p, mask != nullptr);
+                if (mask && mp.on && workspace && workspace_bytes >= CallScratch::rounded(mp.bytes)) {
+                    uint32_t *bits = static_cast<uint32_t *>(workspace);
+                    int2_t *range = reinterpret_cast<int2_t *>(static_cast<char *>(workspace) + mp.bits_bytes);
+                    a.mask_bits = bits;
+                    a.mask_range = range;
+                    a.mask_tiles = mp.tiles;
+                    a.mask_plane[0] = mp.planes_b > 1 ? mp.planes_h : 0;
+                    a.mask_plane[1] = mp.planes_h > 1 ? 1 : 0;
+                    hipLaunchKernelGGL(sdpa_pack_mask_kernel, dim3(static_cast<unsigned>(mp.planes_b * mp.planes_h * mp.nb32)), dim3(256), 0, s, mask, a.ms[0], a.ms[1],
+                                       mp.planes_h, p.seq_q, p.seq_kv, bits, range);
+                    if (bf) launch_pipelined<true, MASK_BITS>(a, nw, split, g, s);
+                    else launch_pipelined<false, MASK_BITS>(a, nw, split, g, s);
+                } else if (mask) {
+                    if (bf) launch_pipelined<true, MASK_BYTES>(a, nw, split, g, s);
+                    else launch_pipelined<false, MASK_BYTES>(a, nw, split, g, s);
+                } else {
+                    if (bf) launch_pipelined<true, MASK_NONE>(a, nw, split, g, s);
+                    else launch_pipelined<false, MASK_NONE>(a, nw, split, g, s);
+                }
+            }
         }
             break;
         }

@@ -21,6 +21,11 @@ struct SdpaArgs {
     // their softmax denominators (reference maximum included) for sdpa_merge_kernel
     int ksplit, kchunk;
     float *opart, *lse;
+    int pairs; // sdpa_mfma_pingpong_kernel, causal: query blocks i and n - 1 - i go to one work-group
+    // an explicit mask as sdpa_pack_mask_kernel left it: the plane of (b, h) is b * mask_plane[0] + h * mask_plane[1]
+    const uint32_t *mask_bits;
+    const int2_t *mask_range;
+    int mask_tiles, mask_plane[2];
 };
 
 constexpr float NEG_INF_F = -__builtin_huge_valf();

@@ -116,7 +116,9 @@ int axhip_sdpa_fwd(const void *q, const void *k, const void *v, void *o,
  * behind the caller's back).  axhip_sdpa_workspace_bytes answers 0 for every
  * problem that needs none; has_mask: whether a mask will be passed.  Steps of
  * fewer than 8 M key elements (slices x keys x dims) only run faster with it:
- * without one, or with less, they run undivided and allocate nothing. */
+ * without one, or with less, they run undivided and allocate nothing.  So do
+ * 16-bit problems of 16 M scores and more under a mask, which take it for the
+ * mask as bits. */
 size_t axhip_sdpa_workspace_bytes(const AxhipSdpaParams *params_host, int has_mask);
 int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o,
                       const uint8_t *mask, const AxhipSdpaParams *params_host,
@@ -128,7 +130,7 @@ const char *axhip_sdpa_kernel_name(const AxhipSdpaParams *params_host);
 /* diagnostic: the schedule the calling thread's last axhip_sdpa_fwd launched ("pingpong", "pipelined8",
  * "pipelined4", "key_split", "decode_split", "direct", "register_staged", "mfma_f32", "generic", "empty"); several
  * schedules share one kernel name.  AXHIP_SDPA_PINGPONG=0 in the environment (read when the library loads)
- * sends "pingpong" problems to "pipelined8". */
+ * sends "pingpong" problems to "pipelined4" or "pipelined8". */
 const char *axhip_sdpa_last_schedule(void);
 
 /* ------------------------------------------------------------ fused chains

@@ -486,3 +486,98 @@ def test_f32_short_sequences(case):
     assert capi.lib().axhip_sdpa_last_schedule() == b"direct"
     want = naive_attention64(q, k, v, 1 / math.sqrt(D), causal, mask)
     assert np.allclose(got, want, rtol=1e-4, atol=1e-4), np.max(np.abs(got - want))
+
+
+def sdpa_ws(q, k, v, dt, causal, mask=None, mask_strides=(0, 0), mask_offset=0, give=True):
+    """The call with a caller's workspace (`give`) or none; the mask may start `mask_offset` bytes into its buffer."""
+    import ctypes as C
+    import torch
+    from axiom_amd import capi
+
+    lib = capi.lib()
+    B, H, Sq, D = q.shape
+    Skv = k.shape[2]
+    dq, dk, dv = gh.to_dev(q), gh.to_dev(k), gh.to_dev(v)
+    o = gh.empty_dev((B, H, Sq, D), dt)
+    o.fill_(0x7FC1)
+    p = capi.SdpaParams()
+    p.dtype, p.batch, p.heads, p.seq_q, p.seq_kv, p.head_dim, p.scale, p.is_causal = dt, B, H, Sq, Skv, D, -1.0, int(causal)
+    p.q_strides[:], p.o_strides[:] = gh.contiguous_strides(H, Sq, D), gh.contiguous_strides(H, Sq, D)
+    p.k_strides[:], p.v_strides[:] = gh.contiguous_strides(H, Skv, D), gh.contiguous_strides(H, Skv, D)
+    dm = None
+    if mask is not None:
+        p.mask_strides[:] = mask_strides
+        dm = torch.empty(mask.size + mask_offset, dtype=torch.uint8, device="cuda")
+        dm[mask_offset:].copy_(torch.from_numpy(np.ascontiguousarray(mask).reshape(-1)))
+    need = lib.axhip_sdpa_workspace_bytes(C.byref(p), int(mask is not None))
+    ws = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device="cuda") if need and give else None
+    gh.sync()
+    torch.cuda.synchronize()
+    capi.check(lib.axhip_sdpa_fwd_ws(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), o.data_ptr(), dm.data_ptr() + mask_offset if dm is not None else None,
+                                     C.byref(p), ws.data_ptr() if ws is not None else None, need if ws is not None else 0, None))
+    gh.sync()
+    if ws is not None:
+        assert bool((ws[need:] == 0x5A).all().item())
+    return axo.to_f32(gh.to_host(o, np.uint16), dt), need, lib.axhip_sdpa_last_schedule()
+
+
+@pytest.mark.parametrize("dt,D,S,Skv,causal,kind,offset", [
+    (BF16, 64, 257, 259, False, "tails", 1), (F16, 128, 300, 257, False, "heads", 3), (BF16, 80, 130, 513, True, "tails", 0),
+    (BF16, 40, 256, 320, True, "random", 2), (F16, 64, 64, 1025, False, "none seen", 0), (BF16, 128, 129, 640, False, "first keys", 1)])
+def test_masks_packed_to_bits(dt, D, S, Skv, causal, kind, offset):
+    """From 16 M scores on an explicit mask is packed to bits first, if the caller brings the memory: rows that start
+    anywhere, ragged last tiles, masks per batch, per (batch, head) and shared, leading and trailing tiles that no row
+    sees, rows (and whole slices) that see nothing.  Against float64 on some slices, and against the bytes read in
+    place, which is what a call without a workspace gets."""
+    B, H = 4, 66
+    r = np.random.default_rng(S * Skv)
+    planes_b, planes_h = (B, 1) if kind in ("tails", "none seen") else (B, H) if kind == "heads" else (1, 1)
+    mask = np.zeros((planes_b, planes_h, S, Skv), np.uint8)
+    if kind == "tails":
+        for b in range(B):
+            mask[b, :, :, [Skv, Skv // 2, 65, 1][b]:] = 1
+    elif kind == "heads":
+        mask[:] = r.random(mask.shape) < 0.5
+        mask[:, ::3, :, :70] = 7
+        mask[:, 1::3, 5:9] = 255
+    elif kind == "random":
+        mask[:] = r.random(mask.shape) < 0.3
+    elif kind == "none seen":
+        mask[1] = 1
+        mask[2, :, :, :1024] = 1
+    else:
+        mask[:, :, :, :200] = 1
+        mask[:, :, 64:, :500] = 1
+    q, k, v = inputs(B, H, S, Skv, D, dt, seed=S + D)
+    strides = (0 if planes_b == 1 else planes_h * S * Skv, 0 if planes_h == 1 else S * Skv)
+    got, need, _ = sdpa_ws(q, k, v, dt, causal, mask, strides, offset)
+    assert need > 0
+    plain, _, _ = sdpa_ws(q, k, v, dt, causal, mask, strides, offset, give=False)
+    assert np.isfinite(got).all()
+    # both round P and the output to 16 bits, in tiles that may start elsewhere: two roundings apart
+    assert np.max(np.abs(got - plain)) < 4e-2
+    for b, h in ((0, 0), (1, 1), (2, 17), (3, H - 1)):
+        qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
+        want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, mask[min(b, planes_b - 1), min(h, planes_h - 1)])
+        assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h)
+
+
+@pytest.mark.parametrize("dt,B,H,Sq,Skv,D,causal,schedule", [
+    (BF16, 1, 3, 64, 65, 64, True, b"key_split"), (BF16, 2, 5, 200, 200, 64, True, b"key_split"), (F16, 1, 4, 130, 70, 40, True, b"key_split"),
+    (BF16, 1, 3, 1000, 400, 128, True, b"key_split"), (F16, 2, 4, 400, 449, 128, False, b"key_split"), (BF16, 1, 2, 70, 700, 80, False, b"key_split"),
+    (F16, 1, 7, 385, 385, 72, True, b"key_split"), (BF16, 8, 16, 300, 130, 64, True, b"pipelined4"), (BF16, 8, 17, 257, 300, 80, True, b"pipelined4"),
+    (F16, 7, 6, 900, 65, 72, False, b"pipelined8"), (BF16, 40, 8, 140, 64, 128, True, b"pingpong"), (F16, 3, 40, 600, 600, 128, True, b"pingpong"),
+    (BF16, 7, 41, 513, 200, 128, True, b"pingpong")])
+def test_work_groups_by_the_number_of_blocks(dt, B, H, Sq, Skv, D, causal, schedule):
+    """Causal problems split their keys too (a part may be empty), run one query block per work-group, and walk the
+    persistent kernel's segments in pairs or longest first (an odd block count, a (batch, head) count that 8 does not
+    divide); head sizes up to 80 leave out the dims they lack."""
+    q, k, v = inputs(B, H, Sq, Skv, D, dt, seed=9 + Sq)
+    got, _, ran = sdpa_ws(q, k, v, dt, causal)
+    assert ran == schedule
+    assert np.isfinite(got).all()
+    for sl in sorted({0, B * H - 1, *range(1, B * H, max(1, B * H // 6))}):
+        b, h = divmod(sl, H)
+        qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
+        want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, None)
+        assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, sl
