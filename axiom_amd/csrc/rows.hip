@@ -379,8 +379,7 @@ int axhip_fused_rows(const AxhipRowsProgram *program, void *stream) {
     AXHIP_REQUIRE(P.rows < (int64_t(1) << 31), AXHIP_ERR_UNSUPPORTED, "axhip_fused_rows: more than 2^31 rows");
     rc = ensure_init();
     if (rc) return rc;
-    RowsPlan pl = plan_rows(P);
-    if (pl.kind == RowsPlan::EMPTY) return AXHIP_OK;
+    if (P.rows == 0 || P.cols == 0) return AXHIP_OK;
     hipStream_t s = resolve_stream(stream);
     // a kernel compiled for this program's shape (built in, or compiled now if this is its first launch) ...
     int launch_rc = AXHIP_OK;
@@ -390,6 +389,7 @@ int axhip_fused_rows(const AxhipRowsProgram *program, void *stream) {
         AXHIP_CHECK_HIP(hipGetLastError());
         return AXHIP_OK;
     }
+    const RowsPlan pl = plan_rows(P);
     // ... or the interpreter, a work-group of (at least) 256 threads for 256 / group rows, or of 1024 for a streamed row
     if (pl.kind == RowsPlan::RESIDENT || pl.kind == RowsPlan::STREAMED) {
         const int64_t threads = pl.kind == RowsPlan::STREAMED ? 1024 : std::max(256, pl.group), rows = pl.kind == RowsPlan::STREAMED ? 1 : threads / pl.group;
