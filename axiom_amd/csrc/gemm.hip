@@ -16,6 +16,7 @@
 #include <cstdlib>
 #include <mutex>
 #include <set>
+#include <utility>
 #include <type_traits>
 
 namespace axhip {
@@ -98,28 +99,22 @@ __device__ __forceinline__ void gemm_load_to_lds(const int4_t &rsrc, uint32_t ld
 
 __device__ __forceinline__ int4_t gemm_rsrc(const void *base, int bytes) {
     const uint64_t pa = reinterpret_cast<uint64_t>(base);
-    return int4_t{static_cast<int>(static_cast<uint32_t>(pa)), static_cast<int>(static_cast<uint32_t>(pa >> 32) & 0xFFFFu), bytes, 0x00020000};
+    // (the same in every lane: kept in scalar registers)
+    return int4_t{__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(pa))),
+                  __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(pa >> 32) & 0xFFFFu)), __builtin_amdgcn_readfirstlane(bytes), 0x00020000};
 }
 
 // The epilogue for 16x16 accumulator tiles computed as B-fragment x A-fragment^T: lane (l16, g4) holds, of tile
-// (i, j), row 16 i + l16 and the four consecutive columns 16 j + 4 g4 .. + 3 -- one 8-byte store where C allows it
-// (even ldc, 4-byte aligned origin), 2-byte stores otherwise.  C and the residual go through buffer descriptors that
-// cover exactly the block's valid rows (a row past the end is dropped by the bounds check); columns are masked.
-// Requires 128 * ldc * 2 < 2^31.
+// (i, j), row 16 i + l16 and the four consecutive columns 16 j + 4 g4 .. + 3.
 typedef float float4_t __attribute__((ext_vector_type(4)));
 template <bool BF16, int RESIDUAL_T, int OP> // RESIDUAL_T: 0 no, 1 yes, 2 decided at run time
 __device__ __forceinline__ void gemm_store_tiles16_as(const GemmArgs &g, const float4_t (&acc)[8][4], int64_t m_base, int64_t n_base, int64_t coff, int l16, int g4, unsigned char *stage) {
     const bool RESIDUAL = RESIDUAL_T == 1 || (RESIDUAL_T == 2 && g.residual != nullptr);
-    const int ldc2 = static_cast<int>(g.ldc) * 2;
     const int cols_valid = static_cast<int>(min<int64_t>(64, g.N - n_base));
     const int rows_valid = static_cast<int>(min<int64_t>(128, g.M - m_base));
-    const int extent = (rows_valid - 1) * ldc2 + cols_valid * 2;
     const int64_t origin = coff + m_base * g.ldc + n_base;
     uint16_t *cbase = static_cast<uint16_t *>(g.c) + origin;
     const uint16_t *rbase = static_cast<const uint16_t *>(RESIDUAL ? g.residual : g.c) + origin;
-    const __amdgpu_buffer_rsrc_t crsrc = __builtin_amdgcn_make_buffer_rsrc(cbase, 0, extent, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(rbase), 0, extent, 0x00020000);
-    const bool wide = (g.ldc & 1) == 0 && (reinterpret_cast<uintptr_t>(cbase) & 3u) == 0 && (reinterpret_cast<uintptr_t>(rbase) & 3u) == 0;
     float bias[4][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -128,29 +123,26 @@ __device__ __forceinline__ void gemm_store_tiles16_as(const GemmArgs &g, const f
             const int col = 16 * j + 4 * g4 + e;
             bias[j][e] = g.bias && col < cols_valid ? load16<BF16>(g.bias, n_base + col) : 0.0f;
         }
-    // A block with all 64 columns inside and 16-byte aligned rows goes through the wave's 16 KiB of LDS (free once the
-    // k loop has ended): the finished 16-bit values are written in accumulator layout and read back row by row, so that
-    // every global store carries 16 bytes per lane and a store instruction fills eight whole 128-byte lines.  While C is
+    // The block goes through the wave's 16 KiB of LDS (free once the k loop has ended): the finished 16-bit values are
+    // written in accumulator layout and read back row by row, so that every global store carries 16 bytes per lane and a
+    // store instruction fills eight whole 128-byte lines -- of rows that may start anywhere.  While C is
     // written no MFMA runs anywhere on the chip (all work-groups end their k loops together), so the write phase is
     // pure HBM time: 8-byte stores, 32 bytes of a row per instruction, take 9.3 us for the 32 MiB of 4096^2 values.
-    const bool staged = stage != nullptr && cols_valid == 64 && (g.ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(cbase) & 15u) == 0;
-    // rows outside, columns inside: the four stores that complete a row's 128-byte line follow one another (with the
-    // column tiles outside, 16 rows apart in between, the same kernel takes 7 % longer on 4096^3)
+    const int lane = 16 * g4 + l16;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+        const int row = 16 * i + l16;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int col = 16 * j + 4 * g4;
-            if (col >= cols_valid) continue;
-            const bool whole = wide && col + 4 <= cols_valid;
-            const int voff = (16 * i + l16) * ldc2 + col * 2;
             float x[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] = acc[i][j][e] + bias[j][e];
-            if (RESIDUAL) {
-                if (whole) {
-                    const uint2_t r = __builtin_bit_cast(uint2_t, __builtin_amdgcn_raw_buffer_load_b64(rrsrc, voff, 0, 0));
-                    const uint32_t rw[2] = {r.x, r.y};
+            if (RESIDUAL && row < rows_valid) {
+                const uint16_t *r = rbase + static_cast<int64_t>(row) * g.ldc + col;
+                if (col + 4 <= cols_valid) {
+                    const uint2_t t = reinterpret_cast<const uint2_unaligned_t *>(r)->v;
+                    const uint32_t rw[2] = {t.x, t.y};
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const uint16_t h = static_cast<uint16_t>(rw[e / 2] >> (16 * (e % 2)));
@@ -159,10 +151,7 @@ __device__ __forceinline__ void gemm_store_tiles16_as(const GemmArgs &g, const f
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (col + e < cols_valid) {
-                            const uint16_t h = __builtin_amdgcn_raw_buffer_load_b16(rrsrc, voff + 2 * e, 0, 0);
-                            x[e] += BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
-                        }
+                        if (col + e < cols_valid) x[e] += BF16 ? bf16_bits_to_f32(r[e]) : f16_bits_to_f32(r[e]);
                 }
             }
             uint32_t w[2];
@@ -171,26 +160,25 @@ __device__ __forceinline__ void gemm_store_tiles16_as(const GemmArgs &g, const f
                 const float y0 = gemm_epilogue16(OP, x[e]), y1 = gemm_epilogue16(OP, x[e + 1]);
                 w[e / 2] = BF16 ? pack_bf16x2(y0, y1) : pack_f16x2(y0, y1);
             }
-            if (staged) {
-                const int r = 16 * i + l16; // 128-byte rows; the 16-byte chunk index is XOR-ed with the row so that neither pass meets bank conflicts
-                *reinterpret_cast<uint2_t *>(stage + r * 128 + (((2 * j + (g4 >> 1)) ^ (r & 7)) * 16) + (g4 & 1) * 8) = uint2_t{w[0], w[1]};
-            } else if (whole) {
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b64(rrsrc, 0, 0, 0)), uint2_t{w[0], w[1]}), crsrc, voff, 0, 0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < cols_valid)
-                        __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(w[e / 2] >> (16 * (e % 2))), crsrc, voff + 2 * e, 0, 0);
-            }
+            // 128-byte rows; the 16-byte chunk index is XOR-ed with the row so that neither pass meets bank conflicts
+            *reinterpret_cast<uint2_t *>(stage + row * 128 + (((2 * j + (g4 >> 1)) ^ (row & 7)) * 16) + (g4 & 1) * 8) = uint2_t{w[0], w[1]};
         }
     }
-    if (staged) {
-        const int lane = 16 * g4 + l16;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (other lanes' values: the hardware keeps the order, the compiler is told to)
+    __builtin_amdgcn_wave_barrier();
+    const int q = lane & 7, left = cols_valid - 8 * q; // columns of this lane's chunk and behind
 #pragma unroll
-        for (int n = 0; n < 16; ++n) {
-            const int r = 8 * n + (lane >> 3), q = lane & 7;
-            const uint4_t v = *reinterpret_cast<const uint4_t *>(stage + r * 128 + ((q ^ (r & 7)) * 16));
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b128(rrsrc, 0, 0, 0)), v), crsrc, r * ldc2 + q * 16, 0, 0);
+    for (int n = 0; n < 16; ++n) {
+        const int r = 8 * n + (lane >> 3);
+        const uint4_t v = *reinterpret_cast<const uint4_t *>(stage + r * 128 + ((q ^ (r & 7)) * 16));
+        if (r >= rows_valid) continue;
+        uint16_t *c = cbase + static_cast<int64_t>(r) * g.ldc + 8 * q;
+        if (left >= 8) {
+            reinterpret_cast<uint4_unaligned_t *>(c)->v = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (e < left) c[e] = static_cast<uint16_t>(v[e / 2] >> (16 * (e % 2)));
         }
     }
 }
@@ -255,7 +243,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
     }
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(big_lds));
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + 8 * wave * BIG_ROWB);
-    auto load_one = [&](const int4_t &ar, const int4_t &br, int kt, int buf, int n) { // n: 0..3 of A, 4..7 of B
+    auto load_one = [&](const int4_t &ar, const int4_t &br, int kt, int buf, int n) __attribute__((always_inline)) { // n: 0..3 of A, 4..7 of B
         const int soff = kt * BIG_ROWB;
         if (n < 4) gemm_load_to_lds(ar, lds_wave + buf * 2 * BIG_TILEB + n * 64 * BIG_ROWB, a_voff[n % 4], soff);
         else gemm_load_to_lds(br, lds_wave + buf * 2 * BIG_TILEB + BIG_TILEB + (n - 4) * 64 * BIG_ROWB, b_voff[n % 4], soff);
@@ -274,14 +262,14 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
         for (int j = 0; j < 4; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     uint4_t fa[8], fb[2][4];
-    auto read_a = [&](int buf, int s, int i) {
+    auto read_a = [&](int buf, int s, int i) __attribute__((always_inline)) {
         fa[i] = *reinterpret_cast<const uint4_t *>(big_lds + buf * 2 * BIG_TILEB + (wm + 16 * i) * BIG_ROWB + f_off[s]);
     };
-    auto read_b = [&](int slot, int buf, int s, int j) {
+    auto read_b = [&](int slot, int buf, int s, int j) __attribute__((always_inline)) {
         fb[slot][j] = *reinterpret_cast<const uint4_t *>(big_lds + buf * 2 * BIG_TILEB + BIG_TILEB + (wn + 16 * j) * BIG_ROWB + f_off[s]);
     };
     // D = (B fragment) x (A fragment)^T: the lane holds four consecutive columns of one row of C
-    auto mfma = [&](int slot, int i, int j) {
+    auto mfma = [&](int slot, int i, int j) __attribute__((always_inline)) {
         if constexpr (BF16)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fb[slot][j]), __builtin_bit_cast(bf16x8_t, fa[i]), acc[i][j], 0, 0, 0);
         else
@@ -602,8 +590,7 @@ bool half_aligned(const AxhipGemmParams &p, const void *a, const void *b) {
 // rounds its work-groups take on the 256 CUs (whole rounds of the tile kernels, of which a CU holds one; the small ones
 // share a CU, and a part of a round costs about half of what is missing from a whole one) and u how full the first is.
 // The coefficients are fitted to 300 products of m 16 .. 3000, n 128 .. 5120, k 128 .. 4096, bf16, operands from the
-// caches: mean error 3 - 9 %, and the kernel picked is on average 1 % slower than the fastest of all.  Rows off the
-// 16-byte grid cost the small kernels 1.9 times per element of k (odd k of 842 .. 2045).
+// caches: mean error 3 - 9 %, and the kernel picked is on average 1 % slower than the fastest of all.
 struct HalfKernel {
     enum Kind { BIG256, TILE, SMALL } kind;
     int shape, waves;
@@ -616,7 +603,7 @@ constexpr HalfKernel HALF_KERNELS[] = {
     {HalfKernel::TILE, TILE_192x128, 8, 5.7f, 0.0063f, 0.0024f, 4.9f, true, true, false},
     {HalfKernel::TILE, TILE_128x128, 8, 4.9f, 0.0048f, 0.0014f, 4.1f, true, true, false},
     {HalfKernel::TILE, TILE_64x128, 8, 4.9f, 0.0032f, 0.0009f, 3.7f, true, true, false},
-    {HalfKernel::TILE, TILE_128x128, 8, 9.5f, 0.0095f, 0.0f, 5.0f, true, true, true}, // (through registers)
+    {HalfKernel::TILE, TILE_128x128, 8, 6.5f, 0.0080f, 0.0f, 5.9f, true, true, true}, // (through registers)
     {HalfKernel::SMALL, SMALL_64x64, 8, 4.35f, 0.00245f, 0.00148f, 3.6f, true, true, false},
     {HalfKernel::SMALL, SMALL_64x64, 4, 4.15f, 0.00324f, 0.00047f, 1.65f, true, true, false},
     {HalfKernel::SMALL, SMALL_32x64, 8, 3.50f, 0.00170f, 0.00085f, 2.3f, true, true, false},
@@ -631,27 +618,44 @@ constexpr HalfKernel HALF_KERNELS[] = {
     {HalfKernel::SMALL, SMALL_16x16, 4, 2.94f, 0.00069f, 0.00004f, 0.02f, true, false, false},
 };
 
+// Unaligned rows: what an operand whose rows start on odd elements, on other even ones, or on other multiples of four
+// adds to the small kernels' time per element of k, and a quarter of it to the tile kernel's (18 products of k 75 .. 3582,
+// which the kernels picked run in 0.91 of the time that one factor for all alignments led to).
+float half_misalignment(int64_t ld) { return ld % 2 != 0 ? 0.55f : ld % 4 != 0 ? 0.45f : ld % 8 != 0 ? 0.1f : 0.0f; }
+
+struct HalfChoice { const HalfKernel *best; float cost; };
+// One candidate.  (The candidates are a parameter of the template so that their tiles are constants here: divisions by what a
+// table holds took 0.5 us of the 3.5 that a small product costs its caller.)
+template <size_t I> void consider_half_kernel(const AxhipGemmParams &p, bool aligned, float misaligned, HalfChoice &c) {
+    constexpr const HalfKernel &h = HALF_KERNELS[I];
+    if (p.trans_b ? !h.nt : !h.nn) return;
+    if (h.kind != HalfKernel::SMALL && h.ragged == aligned) return;
+    if (h.kind == HalfKernel::BIG256 && (p.k % TK != 0 || p.m < BIG || p.n < BIG || p.ldc >= (1 << 21))) return;
+    constexpr uint32_t tm = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.kind == HalfKernel::TILE ? h.shape : 0].tm : SMALL_GEOMETRY[h.kind == HalfKernel::SMALL ? h.shape : 0].tm;
+    constexpr uint32_t tn = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.kind == HalfKernel::TILE ? h.shape : 0].tn : SMALL_GEOMETRY[h.kind == HalfKernel::SMALL ? h.shape : 0].tn;
+    const uint32_t rows = (static_cast<uint32_t>(p.m) + tm - 1) / tm, cols = (static_cast<uint32_t>(p.n) + tn - 1) / tn;
+    if (!launch_fits(static_cast<int64_t>(rows) * cols + 7, 64 * h.waves)) return;
+    const float k = static_cast<float>((p.k + 63) / 64 * 64);
+    const float full = static_cast<float>(p.batch) * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
+    float r = 1.0f;
+    if (full > 1.0f) {
+        float whole = full < 1e9f ? static_cast<float>(static_cast<int>(full)) : full;
+        if (whole < full) whole += 1.0f;
+        r = h.kind == HalfKernel::SMALL ? 0.5f * (whole + full) : whole;
+    }
+    const float slower = aligned ? 1.0f : h.kind == HalfKernel::SMALL ? 1.0f + misaligned : 1.0f + 0.25f * misaligned;
+    const float cost = h.start + k * (h.per_k + h.per_k_full * std::min(full, 1.0f)) * slower * r + h.per_round * (r - 1.0f);
+    if (!c.best || cost < c.cost) c = {&h, cost};
+}
+template <size_t... I> const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned, std::index_sequence<I...>) {
+    HalfChoice c{nullptr, 0.0f};
+    const float misaligned = aligned ? 0.0f : half_misalignment(p.lda) + half_misalignment(p.ldb);
+    (consider_half_kernel<I>(p, aligned, misaligned, c), ...);
+    return c.best;
+}
 // (NULL: no kernel whose work-groups, as many as the product has tiles, can be launched at once)
 const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
-    const HalfKernel *best = nullptr;
-    float best_cost = 0.0f;
-    const uint32_t m = static_cast<uint32_t>(p.m), n = static_cast<uint32_t>(p.n);
-    const float k = static_cast<float>((p.k + 63) / 64 * 64), batch = static_cast<float>(p.batch);
-    for (const HalfKernel &h : HALF_KERNELS) {
-        if (p.trans_b ? !h.nt : !h.nn) continue;
-        if (h.kind != HalfKernel::SMALL && h.ragged == aligned) continue;
-        if (h.kind == HalfKernel::BIG256 && (p.k % TK != 0 || p.m < BIG || p.n < BIG || p.ldc >= (1 << 21))) continue;
-        const uint32_t tm = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tm : SMALL_GEOMETRY[h.shape].tm;
-        const uint32_t tn = h.kind == HalfKernel::BIG256 ? BIG : h.kind == HalfKernel::TILE ? TILE_GEOMETRY[h.shape].tn : SMALL_GEOMETRY[h.shape].tn;
-        const uint32_t rows = (m + tm - 1) / tm, cols = (n + tn - 1) / tn;
-        if (!launch_fits(static_cast<int64_t>(rows) * cols + 7, 64 * h.waves)) continue;
-        const float full = batch * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
-        const float whole = std::ceil(full), r = full <= 1.0f ? 1.0f : h.kind == HalfKernel::SMALL ? 0.5f * (whole + full) : whole;
-        const float per_k = (h.per_k + h.per_k_full * std::min(full, 1.0f)) * (h.kind == HalfKernel::SMALL && !aligned ? 1.9f : 1.0f);
-        const float cost = h.start + k * per_k * r + h.per_round * (r - 1.0f);
-        if (!best || cost < best_cost) { best_cost = cost; best = &h; }
-    }
-    return best;
+    return choose_half_kernel(p, aligned, std::make_index_sequence<sizeof(HALF_KERNELS) / sizeof(HALF_KERNELS[0])>{});
 }
 
 // ---- fp32 products: which kernel

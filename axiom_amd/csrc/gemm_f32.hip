@@ -176,6 +176,21 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
         // columns col .. col + 3.  (NN: a lane whose columns were moved left to end with the rows owns those at and
         // behind the place it was moved from)
         const int col = n0 + (NN ? 4 * NJ * xg + 4 * f : 16 * f + 4 * xg);
+        if (col + 4 + (NN ? NJ : 0) <= g.N) { // all four, and none of them moved
+            const int64_t to = static_cast<int64_t>(m) * g.ldc + col;
+            auto add4 = [&](const float *p) {
+                const Floats<4> t = *reinterpret_cast<const Floats<4> *>(p);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += t.v[e];
+            };
+            if (bias) add4(bias + col);
+            if (res) add4(res + to);
+            Floats<4> y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y.v[e] = gemm_epilogue(g.epilogue, v[e]);
+            *reinterpret_cast<Floats<4> *>(C + to) = y;
+            continue;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             int at = col + e;

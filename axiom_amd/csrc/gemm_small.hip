@@ -58,8 +58,8 @@ __device__ __forceinline__ void small_finish(const TileArgs &g, const float4_t (
         float y[4] = {v[0], v[1], v[2], v[3]};
         auto widen = [](uint32_t h) { return BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h); };
         auto add4 = [&](const uint16_t *p) {
-            if (valid - first == 4 && (reinterpret_cast<uintptr_t>(p) & 7u) == 0) {
-                const uint2_t q = *reinterpret_cast<const uint2_t *>(p);
+            if (valid - first == 4) {
+                const uint2_t q = reinterpret_cast<const uint2_unaligned_t *>(p)->v;
                 y[0] += widen(q.x & 0xFFFFu); y[1] += widen(q.x >> 16); y[2] += widen(q.y & 0xFFFFu); y[3] += widen(q.y >> 16);
             } else {
 #pragma unroll
@@ -71,8 +71,8 @@ __device__ __forceinline__ void small_finish(const TileArgs &g, const float4_t (
         if (g.residual) add4(res);
         gemm_epilogue16_all(g.epilogue, y);
         const uint32_t w0 = BF16 ? pack_bf16x2(y[0], y[1]) : pack_f16x2(y[0], y[1]), w1 = BF16 ? pack_bf16x2(y[2], y[3]) : pack_f16x2(y[2], y[3]);
-        if (valid - first == 4 && (reinterpret_cast<uintptr_t>(c) & 7u) == 0) {
-            *reinterpret_cast<uint2_t *>(c) = uint2_t{w0, w1};
+        if (valid - first == 4) { // (any alignment)
+            reinterpret_cast<uint2_unaligned_t *>(c)->v = uint2_t{w0, w1};
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(const TileArgs g) {
         else off[n] = static_cast<uint32_t>(min(row, rows_b - 1)) * g.ldb * 2;
     }
     uint4_t regs[NL];
-    auto load = [&](int piece) { // (past the last piece: the row's end, or the last row, again)
+    auto load = [&](int piece) { // (past the end of k: the row's end, or the last row, again)
 #pragma unroll
         for (int n = 0; n < NL; ++n) {
             const uint32_t at = NN && n >= NA ? static_cast<uint32_t>(min(64 * piece + 8 * (n - NA) + ld_r, g.K - 1)) * g.ldb * 2
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(const TileArgs g) {
         }
 #pragma unroll
         for (int n = 0; n < NL; ++n) *reinterpret_cast<uint4_t *>(st + n * 1024 + lane * 16) = regs[n];
-        load(p + W);
+        if (p + W < pieces) load(p + W);
         wave_lds_fence();
         uint4_t fa[2][MI], fb[2][NJ];
         small_read_fragments<NN, MI, NJ>(fa, fb, st, l16, g4);

@@ -318,3 +318,24 @@ def test_f32_products_of_plain_matrices_on_the_ring(M, N, K, batch):
     got = c.double()
     x64, w64 = da.double(), gh.to_dev(W).double()
     assert bool(((got - x64 @ w64).abs() <= (K + 2) * 2.0**-24 * (x64.abs() @ w64.abs())).all())
+
+
+@pytest.mark.parametrize("dt", [BF16, F16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("K", [9, 65, 127, 193, 257, 321, 385, 449, 513, 577, 641, 705])
+def test_half_products_through_registers_of_every_number_of_k_tiles(dt, nn, K):
+    """Unaligned rows on the tile kernel that loads through registers, from one k-tile to what its pipeline holds twice
+    over, and the unaligned stores of C (rows of an odd number of columns, ragged last tiles).  The bound of
+    test_half_products_at_the_edges_of_tiles."""
+    import torch
+
+    M, N = 1930, 2001
+    g = axo.PCG64(K)
+    x, W = axo.to_bits(g.normal((M, K)), dt), axo.to_bits(g.normal((K, N) if nn else (N, K)) / np.sqrt(K), dt)
+    bias, res = axo.to_bits(g.normal((N,)) * 0.1, dt), axo.to_bits(g.normal((M, N)), dt)
+    got = axo.to_f32(gh.gemm(x, W, dt, trans_b=not nn, bias=bias, residual=res), dt).reshape(M, N)
+    on = lambda t: torch.from_numpy(np.ascontiguousarray(axo.to_f32(t, dt))).cuda().double()
+    x64, w64, extra = on(x), on(W) if nn else on(W).t().contiguous(), on(bias) + on(res)
+    want, magnitude = x64 @ w64 + extra, x64.abs() @ w64.abs() + on(bias).abs() + on(res).abs()
+    tol = (2.0**-8 if dt == BF16 else 2.0**-11) * want.abs() + (K + 2) * 2.0**-24 * magnitude + (0.0 if dt == BF16 else 2.0**-25)
+    assert bool(((torch.from_numpy(got).cuda().double() - want).abs() <= tol).all())
