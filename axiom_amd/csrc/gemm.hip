@@ -358,23 +358,33 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 }
 
 // ------------------------------------------------------------------ fp32, MFMA
-// C = A B^T in fp32 on v_mfma_f32_32x32x2_f32 (fp32 products, fp32 accumulation: no precision is given up against
-// the FMA kernel), A [M,K] and B [N,K] both K-contiguous.  A ring of S k-tiles of 32 floats, i.e. the 128-byte LDS rows,
-// XOR swizzle and direct-to-LDS loads of the 256 x 256 kernel; a lane's 16-byte fragment read holds four k values that
-// feed four successive MFMAs (which k a lane contributes to which MFMA is free as long as A and B agree).  K only has to be a multiple of 4: the chunks of the last k-tile that lie past K are sent out of the
-// descriptor's range and arrive as zeros.  At 1/16 of the 16-bit MFMA rate the kernel is bound by the matrix pipe,
-// not by the ring.
-// NN: B is [K,N].  Its k-tile then is 32 rows of TNR floats, which the same loads bring in (N a multiple of 4), and a
-// lane's four k values of its column are four 4-byte reads -- as many LDS cycles as the one of 16 bytes, and no pass that
-// transposes B first.
+// C = A B^T (B [N,K]) or A B (NN: B [K,N]) in fp32 on v_mfma_f32_32x32x2_f32: fp32 products, fp32 accumulation, so no
+// precision is given up against the FMA kernel.  Work-group tile TM x TNR, four wavefronts with a quarter of it each; a
+// ring of S k-tiles of 32 floats, i.e. the 128-byte LDS rows, XOR swizzle and direct-to-LDS loads of the 256 x 256 kernel.
+// A lane's 16-byte fragment read holds four k values that feed four successive MFMAs (which k a lane contributes to which
+// MFMA is free as long as A and B agree).  NN: a k-tile of B is 32 rows of TNR floats, and a lane's four k values of its
+// column are four 4-byte reads -- as many LDS cycles as the one of 16 bytes, and no pass that transposes B first.
+// At 1/16 of the 16-bit rate the matrix pipe is the bound, so nothing but the barrier may stand between two MFMAs of a
+// wavefront, of which a SIMD has one: four more wavefronts, one per SIMD, issue the loads (a direct-to-LDS load holds the
+// issue of its wavefront for longer than an MFMA takes, wherever it stands: 64 x 1536 x 4096 on 64 x 64 tiles 84 us, with
+// loaders 76), the fragments of the next eight k are read under the MFMAs of these, the barrier of a k-tile comes before its
+// last steps (by then every wavefront has read the whole tile), and behind it the reads turn to the next tile.  What is
+// left, one k-tile of 64 x 64: 1024 cycles of MFMAs in 1380.  Two wavefronts a SIMD with half of each k-tile, or two sums
+// in turn, were no faster.  1024^3: 26.3 -> 24.5 us, 2048^3 155 -> 138.
+// Rows may start anywhere: the loads need 4-byte alignment.  The chunk that K ends in is fetched as the four floats that
+// end with the row and shifted into place in LDS by the lane that loaded it; chunks behind it, and k-tiles past the last,
+// are sent out of the descriptor's range and arrive as zeros.  NN rows that are no whole chunks: the last column tile is
+// moved left to end with them (N >= TNR); the columns it shares with its neighbour are the neighbour's to store.
 template <int TM, int TNR, int S, bool NN>
-__global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
+__global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
     constexpr int MI = TM / 64, NJ = TNR / 64;
-    constexpr int NLA = TM / 32, NLB = TNR / 32;
+    constexpr int NLA = TM / 32, NLB = TNR / 32, NL = NLA + NLB; // loads of 1 KiB per wavefront and k-tile
     constexpr int KF = 32;                            // floats per k-tile
     constexpr int STAGEB = (TM + TNR) * BIG_ROWB;
     extern __shared__ __attribute__((aligned(1024))) unsigned char big_lds[];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const bool loader = __builtin_amdgcn_readfirstlane(tid / WAVE) >= 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE) % 4;
     const int l32 = lane % 32, g2 = lane / 32;
 
     const int per_xcd = gridDim.x / 8;
@@ -385,111 +395,158 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const int gsz = min(GR, tiles_m - first_m);
     const int rem = t - group * GR * tiles_n;
     const int tm = first_m + rem % gsz, tn = rem / gsz;
-    const int64_t m0 = static_cast<int64_t>(tm) * TM, n0 = static_cast<int64_t>(tn) * TNR;
+    const int64_t m0 = static_cast<int64_t>(tm) * TM, n_low = static_cast<int64_t>(tn) * TNR;
+    const int64_t n0 = NN && g.N % 4 != 0 ? min<int64_t>(n_low, g.N - TNR) : n_low;
     const int64_t bz = blockIdx.y;
     const float *A = static_cast<const float *>(g.a) + bz * g.sa + m0 * g.a_rs;
     const float *B = static_cast<const float *>(g.b) + bz * g.sb + n0 * (NN ? 1 : g.b_cs);
     const int arow_bytes = static_cast<int>(g.a_rs) * 4, brow_bytes = static_cast<int>(NN ? g.b_rs : g.b_cs) * 4;
     const int rows_a = static_cast<int>(min<int64_t>(TM, g.M - m0)), rows_b = static_cast<int>(min<int64_t>(TNR, g.N - n0));
-    const int K = static_cast<int>(g.K);
+    const int K = static_cast<int>(g.K), nk = (K + KF - 1) / KF;
     const int4_t arsrc = gemm_rsrc(A, (rows_a - 1) * arow_bytes + K * 4);
     const int4_t brsrc = gemm_rsrc(B, NN ? (K - 1) * brow_bytes + rows_b * 4 : (rows_b - 1) * brow_bytes + K * 4);
 
     const int ld_r = 8 * wave + (lane >> 3);
-    const int ld_c = (lane & 7) ^ ((ld_r >> 1) & 7); // source chunk of this lane: floats 4 ld_c .. 4 ld_c + 3 of the k-tile
+    const int ld_k = 4 * ((lane & 7) ^ ((ld_r >> 1) & 7)); // this lane's chunk of a row along k: floats ld_k .. ld_k + 3 of the k-tile
     constexpr int OUT_OF_RANGE = 0x7FFFFFF0;
-    int a_voff[NLA], b_voff[NLB];
+    int a_row[NLA], b_row[NLB]; // where the rows of this lane's chunks start (NN, b: where the chunks of k-tile 0 do)
 #pragma unroll
-    for (int n = 0; n < NLA; ++n) a_voff[n] = (32 * n + ld_r) * arow_bytes + ld_c * 16;
+    for (int n = 0; n < NLA; ++n) a_row[n] = (32 * n + ld_r) * arow_bytes;
 #pragma unroll
     for (int n = 0; n < NLB; ++n) {
         const int at = (4 * n + wave) * 1024 + lane * 16; // of the tile
-        if (NN) b_voff[n] = at % (TNR * 4) < rows_b * 4 ? at / (TNR * 4) * brow_bytes + at % (TNR * 4) : OUT_OF_RANGE;
-        else b_voff[n] = (32 * n + ld_r) * brow_bytes + ld_c * 16;
+        if (NN) b_row[n] = at % (TNR * 4) < rows_b * 4 ? at / (TNR * 4) * brow_bytes + at % (TNR * 4) : OUT_OF_RANGE;
+        else b_row[n] = (32 * n + ld_r) * brow_bytes;
     }
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(big_lds));
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + 8 * wave * BIG_ROWB);
-    auto load_tile = [&](int kt, int stage) {
-        const int soff = kt * BIG_ROWB;
-        const bool k_ok = kt * KF + ld_c * 4 < K; // false only for the trailing chunks of a ragged last k-tile
-#pragma unroll
-        for (int n = 0; n < NLA; ++n) gemm_load_to_lds(arsrc, lds_wave + stage * STAGEB + n * 32 * BIG_ROWB, k_ok ? a_voff[n] : OUT_OF_RANGE, soff);
-#pragma unroll
-        for (int n = 0; n < NLB; ++n) {
-            const bool ok = NN ? kt * KF + ((4 * n + wave) * 1024 + lane * 16) / (TNR * 4) < K : k_ok;
-            gemm_load_to_lds(brsrc, lds_wave + stage * STAGEB + TM * BIG_ROWB + n * 32 * BIG_ROWB, ok ? b_voff[n] : OUT_OF_RANGE, NN ? kt * KF * brow_bytes : soff);
+    auto load = [&](int kt, int stage_off, int n) __attribute__((always_inline)) { // n: of A, then of B
+        const int k0 = kt * KF;
+        const int along = k0 + ld_k < K ? min(k0 + ld_k, K - 4) * 4 : OUT_OF_RANGE; // of a row along k
+        if (n < NLA) {
+            gemm_load_to_lds(arsrc, lds_wave + stage_off + n * 32 * BIG_ROWB, along == OUT_OF_RANGE ? OUT_OF_RANGE : a_row[n < NLA ? n : 0] + along, 0);
+        } else {
+            const int nb = n < NLA ? 0 : n - NLA;
+            const uint32_t to = lds_wave + stage_off + TM * BIG_ROWB + nb * 32 * BIG_ROWB;
+            if (NN) gemm_load_to_lds(brsrc, to, k0 + ((4 * nb + wave) * 1024 + lane * 16) / (TNR * 4) < K ? b_row[nb] : OUT_OF_RANGE, kt < nk ? k0 * brow_bytes : 0);
+            else gemm_load_to_lds(brsrc, to, along == OUT_OF_RANGE ? OUT_OF_RANGE : b_row[nb] + along, 0);
         }
     };
+    // the last k-tile, where K is no multiple of 4: this lane's chunks that K ends in, already in LDS, are put in place
+    auto mend = [&](int stage_off) __attribute__((always_inline)) {
+        const int drop = (nk - 1) * KF + ld_k + 4 - K; // floats in front of the chunk
+        if (drop <= 0 || drop >= 4) return;
+#pragma unroll
+        for (int n = 0; n < (NN ? NLA : NL); ++n) {
+            float4_t *c = reinterpret_cast<float4_t *>(big_lds + stage_off + n * 32 * BIG_ROWB + wave * 1024 + lane * 16);
+            *c = __builtin_bit_cast(float4_t, __builtin_bit_cast(unsigned __int128, *c) >> (32 * drop));
+        }
+    };
+
+#define AXHIP_FENCE() __builtin_amdgcn_sched_barrier(0)
+#define AXHIP_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | 0x0F70 | (((n) >> 4) << 14))
+    static_assert(S >= 3 && NL * (S - 1) < 64, "vmcnt is a 6-bit counter");
+    if (loader) {
+#pragma unroll
+        for (int st = 0; st < S - 1; ++st)
+#pragma unroll
+            for (int n = 0; n < NL; ++n) load(st, st * STAGEB, n);
+        AXHIP_VMCNT(NL * (S - 2)); // tile 0 has landed
+        __syncthreads();
+        int next = STAGEB, to = (S - 1) * STAGEB; // stages of tile kt + 1, and of kt + S - 1 (that of kt - 1: everyone has read it)
+        for (int kt = 0; kt < nk; ++kt) {
+#pragma unroll
+            for (int n = 0; n < NL; ++n) load(kt + S - 1, to, n);
+            AXHIP_VMCNT(NL * (S - 2)); // tile kt + 1 has landed
+            if (K % 4 != 0 && kt + 2 == nk) mend(next);
+            __syncthreads();
+            next = next + STAGEB == S * STAGEB ? 0 : next + STAGEB;
+            to = to + STAGEB == S * STAGEB ? 0 : to + STAGEB;
+        }
+        AXHIP_VMCNT(0); // no load is still on its way into LDS
+        return;
+    }
 
     const int wm = (wave / 2) * (TM / 2), wn = (wave % 2) * (TNR / 2);
     int f_off[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) f_off[ks] = l32 * BIG_ROWB + (((2 * ks + g2) ^ ((l32 >> 1) & 7)) * 16);
 
-    float16_t acc[MI][NJ];
+    // The sums of a k-tile are added to those of all before: chains of 32 fp32 additions, however large K (2048^3, one
+    // chain: 8.1e-7 off the exact result, now 1.8e-7; no more than the kernels without shared tiles at any K).
+    float16_t acc[MI][NJ], sum[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+            for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.0f;
 
-    float4_t fa[2][MI], fb[2][NJ];
-    auto read_frags = [&](int slot, int stage, int ks) {
-        const unsigned char *As = big_lds + stage * STAGEB + wm * BIG_ROWB;
-        const unsigned char *Bs = big_lds + stage * STAGEB + (NN ? TM : TM + wn) * BIG_ROWB;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            if constexpr (NN) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) fb[slot][j][c] = reinterpret_cast<const float *>(Bs)[(8 * ks + 4 * g2 + c) * TNR + wn + 32 * j + l32];
-            } else {
-                fb[slot][j] = *reinterpret_cast<const float4_t *>(Bs + 32 * j * BIG_ROWB + f_off[ks]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < MI; ++i) fa[slot][i] = *reinterpret_cast<const float4_t *>(As + 32 * i * BIG_ROWB + f_off[ks]);
+    // fragments of LOOK steps of eight k are on their way while one is multiplied: with one block a wavefront has four MFMAs
+    // for these, less than a read takes next to three other wavefronts'
+    constexpr int LOOK = MI * NJ == 1 ? 2 : 1, SLOTS_F = 2 * LOOK;
+    float4_t fa[SLOTS_F][MI], fb[SLOTS_F][NJ];
+    auto read_a = [&](int slot, int stage_off, int step, int i) __attribute__((always_inline)) {
+        fa[slot][i] = *reinterpret_cast<const float4_t *>(big_lds + stage_off + (wm + 32 * i) * BIG_ROWB + f_off[step]);
     };
-    auto multiply = [&](int slot) {
+    auto read_b = [&](int slot, int stage_off, int step, int j) __attribute__((always_inline)) {
+        const unsigned char *Bs = big_lds + stage_off + (NN ? TM : TM + wn) * BIG_ROWB;
+        if constexpr (NN) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) fb[slot][j][c] = reinterpret_cast<const float *>(Bs)[(8 * step + 4 * g2 + c) * TNR + wn + 32 * j + l32];
+        } else {
+            fb[slot][j] = *reinterpret_cast<const float4_t *>(Bs + 32 * j * BIG_ROWB + f_off[step]);
+        }
+    };
+    // eight k: 4 MI NJ MFMAs; behind MFMA x what `between(x)` does
+    auto multiply = [&](int slot, bool first, auto between) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], first && c == 0 ? float16_t{} : acc[i][j], 0, 0, 0);
+                    AXHIP_FENCE();
+                    between((c * MI + i) * NJ + j);
+                    AXHIP_FENCE();
+                }
     };
 
-    const int nk = (K + KF - 1) / KF;
-    constexpr int INFLIGHT = (NLA + NLB) * (S - 2);
-    static_assert(INFLIGHT < 64, "vmcnt is a 6-bit counter");
-    constexpr int WAIT_OLDEST = (INFLIGHT & 0xF) | 0x0F70 | ((INFLIGHT >> 4) << 14);
+    __syncthreads();
 #pragma unroll
-    for (int st = 0; st < S - 1; ++st)
-        if (st < nk) load_tile(st, st);
-
-    auto step = [&](auto stage_tag, int kt) {
-        constexpr int ST = decltype(stage_tag)::value;
-        if (kt + S - 2 < nk) __builtin_amdgcn_s_waitcnt(WAIT_OLDEST);
-        else __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        if (kt + S - 1 < nk) load_tile(kt + S - 1, (ST + S - 1) % S);
-        read_frags(0, ST, 0);
+    for (int ks = 0; ks < LOOK; ++ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) read_a(ks, 0, ks, i);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) read_b(ks, 0, ks, j);
+    }
+    int cur = 0; // offset of k-tile kt's stage
+    for (int kt = 0; kt < nk; ++kt) {
+        const int next = cur + STAGEB == S * STAGEB ? 0 : cur + STAGEB;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            if (ks + 1 < 4) read_frags((ks + 1) & 1, ST, ks + 1);
-            multiply(ks & 1);
-        }
-    };
-    auto steps = [&](auto self, auto stage_tag, int kt0) -> void {
-        constexpr int ST = decltype(stage_tag)::value;
-        if constexpr (ST < S) {
-            if (kt0 + ST < nk) {
-                step(stage_tag, kt0 + ST);
-                self(self, std::integral_constant<int, ST + 1>{}, kt0);
+            constexpr int LAST = 4 - LOOK; // from here on the reads are the next tile's
+            const int from = ks >= LAST ? next : cur;
+            if (ks == LAST) {
+                __syncthreads(); // tile kt + 1 has landed, and tile kt is no longer read
+                AXHIP_FENCE();
             }
+            multiply(ks % SLOTS_F, ks == 0, [&](int x) __attribute__((always_inline)) {
+                if (x < MI) read_a((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
+                if (x < NJ) read_b((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
+            });
         }
-    };
-    for (int kt0 = 0; kt0 < nk; kt0 += S) steps(steps, std::integral_constant<int, 0>{}, kt0);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) sum[i][j][e] += acc[i][j][e];
+        cur = next;
+    }
+#undef AXHIP_VMCNT
+#undef AXHIP_FENCE
 
     // epilogue: accumulator element e of tile (i, j) is C[m + 32 i + 8 (e / 4) + 4 g2 + e % 4][n + 32 j + l32]
     float *Cb = static_cast<float *>(g.c) + bz * g.sc;
@@ -497,7 +554,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int64_t col = n0 + wn + 32 * j + l32;
-        if (col >= g.N) continue;
+        if (col >= g.N || col < n_low) continue;
         const float bias = g.bias ? static_cast<const float *>(g.bias)[col] : 0.0f;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -505,7 +562,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
             for (int e = 0; e < 16; ++e) {
                 const int64_t row = m0 + wm + 32 * i + 8 * (e / 4) + 4 * g2 + e % 4;
                 if (row >= g.M) continue;
-                float x = acc[i][j][e] + bias;
+                float x = sum[i][j][e] + bias;
                 if (Rb) x += Rb[row * g.ldc + col];
                 Cb[row * g.ldc + col] = gemm_epilogue(g.epilogue, x);
             }
@@ -659,24 +716,27 @@ const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
 }
 
 // ---- fp32 products: which kernel
-// The tile of the ring kernel, by rounds of work-groups x tile area (it is bound by the matrix pipe), and that product.
-constexpr int F32_RING_TILES[4][2] = {{128, 128}, {64, 128}, {128, 192}, {64, 64}};
-struct F32Ring { int tile; float area; }; // area: rounds x tile, in tiles of 128 x 128
+// The ring kernel's tiles with the time each takes, in us: start + k per_k r + per_round (r - 1), r being the rounds its
+// work-groups take on the 256 CUs, fitted to 60 products of m 11 .. 4117, n 64 .. 51865, k 64 .. 8192.  Tiles of 64 x 64 fill
+// the chip soonest and share a CU; larger ones read less from LDS and L2 for each MFMA.
+struct F32RingTile { int tm, tn; float start, per_k, per_round; };
+constexpr F32RingTile F32_RING_TILES[3] = {{128, 128, 13.0f, 0.067f, 4.5f}, {64, 128, 8.5f, 0.0325f, 4.0f}, {64, 64, 6.2f, 0.0170f, 1.3f}};
+struct F32Ring { int tile; float cost; };
 F32Ring f32_ring_tile(const AxhipGemmParams &p) {
     F32Ring best{0, 0.0f};
-    float best_cost = 0.0f;
-    for (int c = 0; c < 4; ++c) {
-        const int tm = F32_RING_TILES[c][0], tn = F32_RING_TILES[c][1];
-        const int64_t tiles = ((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) * p.batch;
-        const float rounds = static_cast<float>((tiles + 255) / 256), area = static_cast<float>(tm * tn) / 16384.0f, cost = rounds * (0.05f + area);
-        if (c == 0 || cost < best_cost) { best_cost = cost; best = {c, rounds * area}; }
+    const float k = static_cast<float>((p.k + 31) / 32 * 32);
+    for (int c = 0; c < 3; ++c) {
+        const F32RingTile &t = F32_RING_TILES[c];
+        const int64_t tiles = ((p.m + t.tm - 1) / t.tm) * ((p.n + t.tn - 1) / t.tn) * p.batch;
+        const float r = static_cast<float>((tiles + 255) / 256), cost = t.start + k * t.per_k * r + t.per_round * (r - 1.0f);
+        if (c == 0 || cost < best.cost) best = {c, cost};
     }
     return best;
 }
-// A along k, whole 16-byte vectors, offsets of 32 bits
+// A along k, offsets of 32 bits, rows of b as [k, n] of whole chunks or at least a tile (128 columns at most)
 bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
-    return !p.trans_a && (p.trans_b || (p.n % 4 == 0 && p.n < (1 << 24) && (p.k + 64) * p.ldb < (int64_t(1) << 29))) && p.k >= 32 && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && p.stride_a % 4 == 0 && p.stride_b % 4 == 0 &&
-           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0 && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
+    return !p.trans_a && (p.trans_b || ((p.n % 4 == 0 || p.n >= 128) && p.n < (1 << 24) && (p.k + 64) * p.ldb < (int64_t(1) << 29))) && p.k >= 32 &&
+           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 3u) == 0 && p.lda < (1 << 21) && p.ldb < (1 << 21) && p.k < (1 << 24) &&
            p.m * p.n * p.batch >= 64 * 64 * 16 && f32_mfma_enabled();
 }
 // The time of the kernels of gemm_f32.hip in us, as for the 16-bit ones above: start + k (per_k + (per_k_full +
@@ -701,11 +761,7 @@ int choose_f32_kernel(const AxhipGemmParams &p, bool ring, double repacked) {
     const float k = static_cast<float>(p.k), u = p.k % 4 != 0 || (!p.trans_b && p.n % 4 != 0) ? 1.0f : 0.0f;
     int best = -1;
     float best_cost = 0.0f;
-    if (ring) {
-        // (less than fitted: where the two are close, the ring is no slower than before)
-        const float padded = static_cast<float>((p.k + 31) / 32 * 32);
-        best_cost = 0.85f * (3.7f + (0.0718f * padded + 9.4f) * f32_ring_tile(p).area + (repacked > 0.0 ? 4.7f + 2.1e-7f * static_cast<float>(repacked) : 0.0f));
-    }
+    if (ring) best_cost = f32_ring_tile(p).cost + (repacked > 0.0 ? 4.7f + 2.1e-7f * static_cast<float>(repacked) : 0.0f);
     for (int i = 0; i < F32_SHAPES; ++i) {
         const F32Kernel &h = F32_KERNELS[i];
         const int64_t rows = (p.m + F32_GEOMETRY[i].tm - 1) / F32_GEOMETRY[i].tm, cols = (p.n + F32_GEOMETRY[i].tn - 1) / F32_GEOMETRY[i].tn;
@@ -883,18 +939,20 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
             }
             const int tiles_m = static_cast<int>((p.m + tm_rows - 1) / tm_rows), tiles_n = static_cast<int>((p.n + tn_cols - 1) / tn_cols);
             const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-            AXHIP_REQUIRE(launch_fits(int64_t(8) * per_xcd, 256), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(256), lds_bytes, s, g, tiles_m, tiles_n);
+            AXHIP_REQUIRE(launch_fits(int64_t(8) * per_xcd, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
             return AXHIP_OK;
         };
         int rc2;
         switch (f32_ring_tile(p).tile) {
-#define AXHIP_RING(TM, TN) \
-    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, 3, false>, TM, TN, 3 * (TM + TN) * BIG_ROWB) : launch(gemm_mfma_f32_ring_kernel<TM, TN, 3, true>, TM, TN, 3 * (TM + TN) * BIG_ROWB)
-        case 0: AXHIP_RING(128, 128); break;
-        case 1: AXHIP_RING(64, 128); break;
-        case 3: AXHIP_RING(64, 64); break;
-        default: AXHIP_RING(128, 192); break;
+#define AXHIP_RING(TM, TN, S) \
+    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, S, false>, TM, TN, S * (TM + TN) * BIG_ROWB) : launch(gemm_mfma_f32_ring_kernel<TM, TN, S, true>, TM, TN, S * (TM + TN) * BIG_ROWB)
+        case 0: AXHIP_RING(128, 128, 3); break;
+        case 1: AXHIP_RING(64, 128, 3); break;
+        default: // (one work-group per CU: a fourth stage hides the rest of a load's latency, 80 -> 76 us for k of 4096; more: three of them share a CU's LDS)
+            if ((p.m + 63) / 64 * ((p.n + 63) / 64) * p.batch <= 256) AXHIP_RING(64, 64, 4);
+            else AXHIP_RING(64, 64, 3);
+            break;
 #undef AXHIP_RING
         }
         if (rc2) return rc2;

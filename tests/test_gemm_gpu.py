@@ -339,3 +339,42 @@ def test_half_products_through_registers_of_every_number_of_k_tiles(dt, nn, K):
     want, magnitude = x64 @ w64 + extra, x64.abs() @ w64.abs() + on(bias).abs() + on(res).abs()
     tol = (2.0**-8 if dt == BF16 else 2.0**-11) * want.abs() + (K + 2) * 2.0**-24 * magnitude + (0.0 if dt == BF16 else 2.0**-25)
     assert bool(((torch.from_numpy(got).cuda().double() - want).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", [
+    (1025, 1027, 33, 1), (1000, 1001, 95, 2), (513, 2049, 127, 1), (1919, 1921, 129, 1), (1920, 1920, 730, 1),  # 64 x 64 and 64 x 128, K of every remainder of 4
+    (2300, 130, 161, 8), (700, 2813, 385, 1), (4000, 3999, 1001, 1)])
+def test_f32_products_of_rows_that_start_anywhere_on_the_ring(nn, M, N, K, batch):
+    """The ring kernel without 16-byte alignment: k that ends inside a chunk (what lies behind it in memory are other rows,
+    here with infinities and NaNs next to the operands), column tiles moved left to end with the rows, bias and residual.
+    The bound of the tests above; its sums are chains of 32 and then one per k-tile, so the error is also held to that of
+    chains that long: (32 + K / 32 + 4) half ulps of the sum of magnitudes."""
+    import ctypes as C
+
+    import torch
+
+    from axiom_amd import capi
+
+    g = axo.PCG64(M + 3 * N + K)
+    x, W = g.normal((batch, M, K)).astype(np.float32), (g.normal((batch, K, N) if nn else (batch, N, K)) / np.sqrt(K)).astype(np.float32)
+    def off_grid(t):  # one float into a buffer of NaNs
+        buf = torch.full((t.size + 600,), float("nan"), device="cuda")
+        buf[1:1 + t.size] = gh.to_dev(t).flatten()
+        return buf, buf[1:1 + t.size].view(t.shape)
+    (_, da), (_, db) = off_grid(x), off_grid(W)
+    bias, res = gh.to_dev((g.normal((N,)) * 0.1).astype(np.float32)), gh.to_dev(g.normal((batch, M, N)).astype(np.float32))
+    c = gh.empty_dev((batch, M, N), F32)
+    p = capi.GemmParams()
+    p.dtype, p.m, p.n, p.k, p.batch, p.lda, p.ldb, p.ldc, p.trans_b = F32, M, N, K, batch, K, N if nn else K, N, int(not nn)
+    p.stride_a, p.stride_b, p.stride_c = M * K, K * N, M * N
+    p.bias, p.residual = bias.data_ptr(), res.data_ptr()
+    torch.cuda.synchronize()
+    gh.sync()
+    capi.check(capi.lib().axhip_gemm(da.data_ptr(), db.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    for b in range(batch):
+        x64, w64 = da[b].double(), db[b].double() if nn else db[b].double().t().contiguous()
+        want, magnitude = x64 @ w64 + bias.double() + res[b].double(), x64.abs() @ w64.abs() + bias.double().abs() + res[b].double().abs()
+        err = (c[b].double() - want).abs()
+        assert bool((err <= min(K + 2, 36 + K / 32) * 2.0**-24 * magnitude).all())
