@@ -29,6 +29,7 @@ struct GemmArgs {
     int64_t M, N, K;
     int64_t a_rs, a_cs, b_rs, b_cs, ldc; // element strides of op(A)[m][k], op(B)[k][n]
     int64_t sa, sb, sc;                   // batch strides
+    int batch;                            // products of this launch
 };
 
 // ------------------------------------------------------------------- generic
@@ -211,18 +212,17 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
     const int l16 = lane % 16, g4 = lane / 16;
 
-    // work-group -> C tile: XCD x (work-groups x, x+8, ...) owns a contiguous range of the
-    // tile order; within it tiles run down groups of 4 tile rows
-    const int per_xcd = gridDim.x / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles_m * tiles_n) return;
+    // the tiles of a product run down groups of 4 tile rows
+    int product;
+    const int t = tile_of_work_group(tiles_m * tiles_n, g.batch, product);
+    if (t < 0) return;
     constexpr int GR = 4;
     const int group = t / (GR * tiles_n), first_m = group * GR;
     const int gsz = min(GR, tiles_m - first_m);
     const int rem = t - group * GR * tiles_n;
     const int tm = first_m + rem % gsz, tn = rem / gsz;
     const int64_t m0 = static_cast<int64_t>(tm) * BIG, n0 = static_cast<int64_t>(tn) * BIG;
-    const int64_t bz = blockIdx.y;
+    const int64_t bz = product;
     const uint16_t *A = static_cast<const uint16_t *>(g.a) + bz * g.sa + m0 * g.a_rs;
     const uint16_t *B = static_cast<const uint16_t *>(g.b) + bz * g.sb + n0 * g.b_cs;
     const int arow_bytes = static_cast<int>(g.a_rs) * 2, brow_bytes = static_cast<int>(g.b_cs) * 2;
@@ -387,9 +387,9 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE) % 4;
     const int l32 = lane % 32, g2 = lane / 32;
 
-    const int per_xcd = gridDim.x / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles_m * tiles_n) return;
+    int product;
+    const int t = tile_of_work_group(tiles_m * tiles_n, g.batch, product);
+    if (t < 0) return;
     constexpr int GR = 4;
     const int group = t / (GR * tiles_n), first_m = group * GR;
     const int gsz = min(GR, tiles_m - first_m);
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const int tm = first_m + rem % gsz, tn = rem / gsz;
     const int64_t m0 = static_cast<int64_t>(tm) * TM, n_low = static_cast<int64_t>(tn) * TNR;
     const int64_t n0 = NN && g.N % 4 != 0 ? min<int64_t>(n_low, g.N - TNR) : n_low;
-    const int64_t bz = blockIdx.y;
+    const int64_t bz = product;
     const float *A = static_cast<const float *>(g.a) + bz * g.sa + m0 * g.a_rs;
     const float *B = static_cast<const float *>(g.b) + bz * g.sb + n0 * (NN ? 1 : g.b_cs);
     const int arow_bytes = static_cast<int>(g.a_rs) * 4, brow_bytes = static_cast<int>(NN ? g.b_rs : g.b_cs) * 4;
@@ -774,9 +774,8 @@ int choose_f32_kernel(const AxhipGemmParams &p, bool ring, double repacked) {
     return best;
 }
 
-int launch_big(const GemmArgs &g, bool bf, int batch, hipStream_t s) {
+int launch_big(const GemmArgs &g, bool bf, hipStream_t s) {
     const int tiles_m = static_cast<int>((g.M + BIG - 1) / BIG), tiles_n = static_cast<int>((g.N + BIG - 1) / BIG);
-    const dim3 grid(static_cast<unsigned>(8 * ((tiles_m * tiles_n + 7) / 8)), static_cast<unsigned>(batch));
     constexpr size_t lds_bytes = 4 * BIG_TILEB;
     static const bool configured = [] {
         bool ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_nt_256_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
@@ -784,8 +783,10 @@ int launch_big(const GemmArgs &g, bool bf, int batch, hipStream_t s) {
         return ok;
     }();
     AXHIP_REQUIRE(configured, AXHIP_ERR_UNSUPPORTED, "axhip_gemm: cannot reserve %zu bytes of LDS", lds_bytes);
-    if (bf) hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<true>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
-    else hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<false>), grid, dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
+    launch_products(g, static_cast<int64_t>(tiles_m) * tiles_n, 512, 2, [&](const GemmArgs &part, unsigned grid) {
+        if (bf) hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<true>), dim3(grid), dim3(512), lds_bytes, s, part, tiles_m, tiles_n);
+        else hipLaunchKernelGGL((gemm_mfma_nt_256_kernel<false>), dim3(grid), dim3(512), lds_bytes, s, part, tiles_m, tiles_n);
+    });
     return AXHIP_OK;
 }
 
@@ -796,14 +797,14 @@ TileArgs tile_args(const AxhipGemmParams &p, const void *a, const void *b, void 
     t.M = static_cast<int>(p.m); t.N = static_cast<int>(p.n); t.K = static_cast<int>(p.k);
     t.lda = static_cast<int>(p.lda); t.ldb = static_cast<int>(p.ldb); t.ldc = static_cast<int>(p.ldc);
     t.epilogue = p.epilogue_op;
+    t.batch = static_cast<int>(p.batch);
     return t;
 }
 
 int launch_half(const AxhipGemmParams &p, const void *a, const void *b, void *c, const HalfKernel &k, bool aligned, bool bf, hipStream_t s) {
     const TileArgs t = tile_args(p, a, b, c);
-    const int batch = static_cast<int>(p.batch);
-    if (k.kind == HalfKernel::SMALL) return launch_small(t, bf, !p.trans_b, k.shape, k.waves, batch, s);
-    return p.trans_b ? launch_tile_nt(t, bf, k.shape, aligned, batch, s) : launch_tile_nn(t, bf, k.shape, aligned, batch, s);
+    if (k.kind == HalfKernel::SMALL) return launch_small(t, bf, !p.trans_b, k.shape, k.waves, s);
+    return p.trans_b ? launch_tile_nt(t, bf, k.shape, aligned, s) : launch_tile_nn(t, bf, k.shape, aligned, s);
 }
 
 int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *params, CallScratch *scratch_in, void *workspace, size_t workspace_bytes, void *stream) {
@@ -884,7 +885,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     g.M = p.m; g.N = p.n; g.K = p.k;
     g.a_rs = p.trans_a ? 1 : p.lda; g.a_cs = p.trans_a ? p.lda : 1;
     g.b_rs = p.trans_b ? 1 : p.ldb; g.b_cs = p.trans_b ? p.ldb : 1;
-    g.ldc = p.ldc; g.sa = p.stride_a; g.sb = p.stride_b; g.sc = p.stride_c;
+    g.ldc = p.ldc; g.sa = p.stride_a; g.sb = p.stride_b; g.sc = p.stride_c; g.batch = static_cast<int>(p.batch);
 
     const bool half = p.dtype != AXHIP_DTYPE_F32;
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
@@ -920,10 +921,10 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         launch_skinny(k, static_cast<int>(p.m), rows_per_wave, blocks, s);
     } else if (const HalfKernel *k = half_kernel()) {
         const bool aligned = half_aligned(p, a, b), bf = p.dtype == AXHIP_DTYPE_BF16;
-        rc = k->kind == HalfKernel::BIG256 ? launch_big(g, bf, static_cast<int>(p.batch), s) : launch_half(p, a, b, c, *k, aligned, bf, s);
+        rc = k->kind == HalfKernel::BIG256 ? launch_big(g, bf, s) : launch_half(p, a, b, c, *k, aligned, bf, s);
         if (rc) return rc;
     } else if (f32_shape >= 0) {
-        rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, static_cast<int>(p.batch), s);
+        rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, s);
         if (rc) return rc;
     } else if (f32 && takes_f32_ring(p, a, b)) {
         // fp32 x W^T on the fp32 MFMA
@@ -938,9 +939,9 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
                 }
             }
             const int tiles_m = static_cast<int>((p.m + tm_rows - 1) / tm_rows), tiles_n = static_cast<int>((p.n + tn_cols - 1) / tn_cols);
-            const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-            AXHIP_REQUIRE(launch_fits(int64_t(8) * per_xcd, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * per_xcd), static_cast<unsigned>(p.batch)), dim3(512), lds_bytes, s, g, tiles_m, tiles_n);
+            const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
+            AXHIP_REQUIRE(launch_fits(tiles + 7, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+            launch_products(g, tiles, 512, 4, [&](const GemmArgs &part, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds_bytes, s, part, tiles_m, tiles_n); });
             return AXHIP_OK;
         };
         int rc2;

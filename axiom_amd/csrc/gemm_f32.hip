@@ -26,11 +26,12 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
     constexpr int W = F32_WAVES, TM = 16 * MI, TN = 16 * NJ, KP = 32 * P, U = 2 * P;
     constexpr int NA = 2 * MI, NS = NA + (NN ? 0 : 2 * NJ); // staged loads of 8 rows x 128 bytes per 32 k
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, l16 = lane % 16, g4 = lane / 16;
-    const int tiles_m = (g.M + TM - 1) / TM, tiles = tiles_m * ((g.N + TN - 1) / TN), per_xcd = (tiles + 7) / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles) return;
+    const int tiles_m = (g.M + TM - 1) / TM;
+    int product;
+    const int t = tile_of_work_group(tiles_m * ((g.N + TN - 1) / TN), g.batch, product);
+    if (t < 0) return;
     const int m0 = (t % tiles_m) * TM, n0 = (t / tiles_m) * TN;
-    const int64_t bz = blockIdx.y;
+    const int64_t bz = product;
     const float *A = static_cast<const float *>(g.a) + bz * g.sa, *B = static_cast<const float *>(g.b) + bz * g.sb;
 
     // rows and columns past the end repeat the last ones: they are not stored
@@ -208,29 +209,29 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
     }
 }
 
-template <bool NN, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, int batch, hipStream_t s) {
+template <bool NN, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, hipStream_t s) {
     constexpr int stages = F32_WAVES * P * 2 * (MI + (NN ? 0 : NJ)) * 1024, sum = F32_WAVES * MI * NJ * 1024, lds = stages > sum ? stages : sum;
     const auto kernel = gemm_f32_direct_kernel<NN, MI, NJ, P>;
     static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     AXHIP_CHECK_HIP(configured);
     const int64_t tiles = static_cast<int64_t>((g.M + 16 * MI - 1) / (16 * MI)) * ((g.N + 16 * NJ - 1) / (16 * NJ));
     AXHIP_REQUIRE(launch_fits(tiles + 7, 64 * F32_WAVES), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * ((tiles + 7) / 8)), static_cast<unsigned>(batch)), dim3(64 * F32_WAVES), lds, s, g);
+    launch_products(g, tiles, 64 * F32_WAVES, 4, [&](const TileArgs &part, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * F32_WAVES), lds, s, part); });
     return AXHIP_OK;
 }
-template <bool NN> int launch_shape(const TileArgs &g, int shape, int batch, hipStream_t s) {
+template <bool NN> int launch_shape(const TileArgs &g, int shape, hipStream_t s) {
     switch (shape) {
-    case F32_16x16: return launch_kernel<NN, 1, 1, 2>(g, batch, s);
-    case F32_16x32: return launch_kernel<NN, 1, 2, 2>(g, batch, s);
-    case F32_16x64: return launch_kernel<NN, 1, 4, 1>(g, batch, s);
-    case F32_32x32: return launch_kernel<NN, 2, 2, 1>(g, batch, s);
-    case F32_32x64: return launch_kernel<NN, 2, 4, 1>(g, batch, s);
-    default: return launch_kernel<NN, 4, 4, 1>(g, batch, s);
+    case F32_16x16: return launch_kernel<NN, 1, 1, 2>(g, s);
+    case F32_16x32: return launch_kernel<NN, 1, 2, 2>(g, s);
+    case F32_16x64: return launch_kernel<NN, 1, 4, 1>(g, s);
+    case F32_32x32: return launch_kernel<NN, 2, 2, 1>(g, s);
+    case F32_32x64: return launch_kernel<NN, 2, 4, 1>(g, s);
+    default: return launch_kernel<NN, 4, 4, 1>(g, s);
     }
 }
 } // namespace
 
-int launch_f32_direct(const TileArgs &g, bool nn, int shape, int batch, hipStream_t s) {
-    return nn ? launch_shape<true>(g, shape, batch, s) : launch_shape<false>(g, shape, batch, s);
+int launch_f32_direct(const TileArgs &g, bool nn, int shape, hipStream_t s) {
+    return nn ? launch_shape<true>(g, shape, s) : launch_shape<false>(g, shape, s);
 }
 } // namespace axhip

@@ -10,6 +10,6 @@ struct F32Geometry { int tm, tn, tk; };
 constexpr F32Geometry F32_GEOMETRY[F32_SHAPES] = {{16, 16, 64}, {16, 32, 64}, {16, 64, 32}, {32, 32, 32}, {32, 64, 32}, {64, 64, 32}};
 
 // a [M, K]; b [N, K], or [K, N] (nn).  K >= 1, N >= 4; no alignment beyond the elements'.
-int launch_f32_direct(const TileArgs &g, bool nn, int shape, int batch, hipStream_t s);
+int launch_f32_direct(const TileArgs &g, bool nn, int shape, hipStream_t s);
 
 } // namespace axhip

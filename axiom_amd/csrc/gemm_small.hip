@@ -105,13 +105,13 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(const TileArgs g) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
     const int l16 = lane % 16, g4 = lane / 16;
     const int tiles_m = (g.M + 16 * MI - 1) / (16 * MI);
-    const int tiles = tiles_m * ((g.N + 16 * NJ - 1) / (16 * NJ)), per_xcd = (tiles + 7) / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles) return;
+    int product;
+    const int t = tile_of_work_group(tiles_m * ((g.N + 16 * NJ - 1) / (16 * NJ)), g.batch, product);
+    if (t < 0) return;
     const int m0 = (t % tiles_m) * 16 * MI, n_low = (t / tiles_m) * 16 * NJ;
     // (NN: the last column tile is moved left to end with the rows; the columns it shares are its neighbour's to store)
     const int n0 = NN ? max(0, min(n_low, g.N - 16 * NJ)) : n_low;
-    const int64_t bz = blockIdx.y;
+    const int64_t bz = product;
     const char *A = reinterpret_cast<const char *>(static_cast<const uint16_t *>(g.a) + bz * g.sa + static_cast<int64_t>(m0) * g.lda);
     const char *B = reinterpret_cast<const char *>(static_cast<const uint16_t *>(g.b) + bz * g.sb + (NN ? static_cast<int64_t>(n0) : static_cast<int64_t>(n0) * g.ldb));
     const int rows_a = min(16 * MI, g.M - m0), rows_b = min(16 * NJ, g.N - n0);
@@ -175,36 +175,36 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(const TileArgs g) {
     small_finish<BF16, MI, NJ, W>(g, acc, m0, n0, n_low, bz * g.sc, small_lds);
 }
 
-template <bool BF16, bool NN, int MI, int NJ, int W> int launch_kernel(const TileArgs &g, int batch, hipStream_t s) {
+template <bool BF16, bool NN, int MI, int NJ, int W> int launch_kernel(const TileArgs &g, hipStream_t s) {
     constexpr int stages = W * (MI + NJ) * 2048, sums = W * MI * NJ * 1024, lds = stages > sums ? stages : sums;
     const auto kernel = gemm_small_kernel<BF16, NN, MI, NJ, W>;
     static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     AXHIP_CHECK_HIP(configured);
     const int64_t tiles = static_cast<int64_t>((g.M + 16 * MI - 1) / (16 * MI)) * ((g.N + 16 * NJ - 1) / (16 * NJ));
     AXHIP_REQUIRE(launch_fits(tiles + 7, 64 * W), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * ((tiles + 7) / 8)), static_cast<unsigned>(batch)), dim3(64 * W), lds, s, g);
+    launch_products(g, tiles, 64 * W, 2, [&](const TileArgs &part, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), lds, s, part); });
     return AXHIP_OK;
 }
-template <bool BF16, bool NN, int MI, int NJ> int launch_waves(const TileArgs &g, int waves, int batch, hipStream_t s) {
-    return waves == 8 ? launch_kernel<BF16, NN, MI, NJ, 8>(g, batch, s) : launch_kernel<BF16, NN, MI, NJ, 4>(g, batch, s);
+template <bool BF16, bool NN, int MI, int NJ> int launch_waves(const TileArgs &g, int waves, hipStream_t s) {
+    return waves == 8 ? launch_kernel<BF16, NN, MI, NJ, 8>(g, s) : launch_kernel<BF16, NN, MI, NJ, 4>(g, s);
 }
-template <bool BF16> int launch_shape(const TileArgs &g, bool nn, int shape, int waves, int batch, hipStream_t s) {
+template <bool BF16> int launch_shape(const TileArgs &g, bool nn, int shape, int waves, hipStream_t s) {
     if (nn) switch (shape) {
-        case SMALL_16x64: return launch_waves<BF16, true, 1, 4>(g, waves, batch, s);
-        case SMALL_32x64: return launch_waves<BF16, true, 2, 4>(g, waves, batch, s);
-        default: return launch_waves<BF16, true, 4, 4>(g, waves, batch, s);
+        case SMALL_16x64: return launch_waves<BF16, true, 1, 4>(g, waves, s);
+        case SMALL_32x64: return launch_waves<BF16, true, 2, 4>(g, waves, s);
+        default: return launch_waves<BF16, true, 4, 4>(g, waves, s);
         }
     switch (shape) {
-    case SMALL_16x16: return launch_waves<BF16, false, 1, 1>(g, waves, batch, s);
-    case SMALL_32x16: return launch_waves<BF16, false, 2, 1>(g, waves, batch, s);
-    case SMALL_32x32: return launch_waves<BF16, false, 2, 2>(g, waves, batch, s);
-    case SMALL_32x64: return launch_waves<BF16, false, 2, 4>(g, waves, batch, s);
-    default: return launch_waves<BF16, false, 4, 4>(g, waves, batch, s);
+    case SMALL_16x16: return launch_waves<BF16, false, 1, 1>(g, waves, s);
+    case SMALL_32x16: return launch_waves<BF16, false, 2, 1>(g, waves, s);
+    case SMALL_32x32: return launch_waves<BF16, false, 2, 2>(g, waves, s);
+    case SMALL_32x64: return launch_waves<BF16, false, 2, 4>(g, waves, s);
+    default: return launch_waves<BF16, false, 4, 4>(g, waves, s);
     }
 }
 } // namespace
 
-int launch_small(const TileArgs &g, bool bf16, bool nn, int shape, int waves, int batch, hipStream_t s) {
-    return bf16 ? launch_shape<true>(g, nn, shape, waves, batch, s) : launch_shape<false>(g, nn, shape, waves, batch, s);
+int launch_small(const TileArgs &g, bool bf16, bool nn, int shape, int waves, hipStream_t s) {
+    return bf16 ? launch_shape<true>(g, nn, shape, waves, s) : launch_shape<false>(g, nn, shape, waves, s);
 }
 } // namespace axhip

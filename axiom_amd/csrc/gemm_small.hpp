@@ -10,6 +10,6 @@ struct SmallGeometry { int tm, tn; };
 constexpr SmallGeometry SMALL_GEOMETRY[SMALL_SHAPES] = {{16, 16}, {32, 16}, {32, 32}, {16, 64}, {32, 64}, {64, 64}};
 
 // `waves`: 4 or 8 wavefronts share k.  K >= 8 and, NN, N >= 8; no alignment beyond the elements'.
-int launch_small(const TileArgs &g, bool bf16, bool nn, int shape, int waves, int batch, hipStream_t s);
+int launch_small(const TileArgs &g, bool bf16, bool nn, int shape, int waves, hipStream_t s);
 
 } // namespace axhip

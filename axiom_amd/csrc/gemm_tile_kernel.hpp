@@ -110,12 +110,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 1) void gemm_tile_kernel(const T
     const int l16 = lane % 16, g4 = lane / 16;
     const int wk = wave / (WM * WN), wt = wave % (WM * WN), wm = (wt / WN) * 16 * MI, wn = (wt % WN) * 64;
 
-    // work-group -> tile: XCD x (work-groups x, x + 8, ...) owns a contiguous range of the tile order, which runs down
-    // groups of GR tile rows, so that an XCD's L2 sees a compact block of C and each panel of A and B few times
+    // the tiles of a product run down groups of GR tile rows, so that an XCD's L2 sees a compact block of C and each panel of
+    // A and B few times
     const int tiles_m = (g.M + TM - 1) / TM, tiles_n = (g.N + TN - 1) / TN;
-    const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-    const int t = (static_cast<int>(blockIdx.x) % 8) * per_xcd + static_cast<int>(blockIdx.x) / 8;
-    if (t >= tiles_m * tiles_n) return;
+    int product;
+    const int t = tile_of_work_group(tiles_m * tiles_n, g.batch, product);
+    if (t < 0) return;
     constexpr int GR = TM >= 128 ? 4 : 8;
     const int group = t / (GR * tiles_n), first_m = group * GR;
     const int gsz = min(GR, tiles_m - first_m);
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 1) void gemm_tile_kernel(const T
     // (through registers, NN: the last column tile is moved left to end with the rows, so that no chunk of B reaches past
     // one; the columns it shares with its neighbour are the neighbour's to store)
     const int n0 = NN && !DMA ? max(0, min(n_low, g.N - TN)) : n_low;
-    const int64_t bz = blockIdx.y;
+    const int64_t bz = product;
     const uint16_t *A = static_cast<const uint16_t *>(g.a) + bz * g.sa + static_cast<int64_t>(m0) * g.lda;
     const uint16_t *B = static_cast<const uint16_t *>(g.b) + bz * g.sb + (NN ? static_cast<int64_t>(n0) : static_cast<int64_t>(n0) * g.ldb);
     const int rows_a = min(TM, g.M - m0), cols_b = min(TN, g.N - n0);
@@ -423,7 +423,7 @@ template <int MI, int WM, int WN, int WK, int TK, int S> constexpr size_t tile_l
 }
 
 template <bool BF16, bool NN, bool DMA, int MI, int WM, int WN, int WK, int TK, int S>
-int launch_tile_kernel(const TileArgs &g, int batch, hipStream_t s) {
+int launch_tile_kernel(const TileArgs &g, hipStream_t s) {
     constexpr size_t lds = tile_lds_bytes<MI, WM, WN, WK, TK, S>();
     static_assert(lds <= 160 * 1024, "LDS of a CU");
     const auto kernel = gemm_tile_kernel<BF16, NN, DMA, MI, WM, WN, WK, TK, S>;
@@ -432,7 +432,7 @@ int launch_tile_kernel(const TileArgs &g, int batch, hipStream_t s) {
     constexpr int TM = 16 * MI * WM, TN = 64 * WN;
     const int64_t tiles = static_cast<int64_t>((g.M + TM - 1) / TM) * ((g.N + TN - 1) / TN);
     AXHIP_REQUIRE(launch_fits(tiles + 7, 64 * WM * WN * WK), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(8 * ((tiles + 7) / 8)), static_cast<unsigned>(batch)), dim3(64 * WM * WN * WK), lds, s, g);
+    launch_products(g, tiles, 64 * WM * WN * WK, 2, [&](const TileArgs &part, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WM * WN * WK), lds, s, part); });
     return AXHIP_OK;
 }
 

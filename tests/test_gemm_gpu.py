@@ -378,3 +378,42 @@ def test_f32_products_of_rows_that_start_anywhere_on_the_ring(nn, M, N, K, batch
         want, magnitude = x64 @ w64 + bias.double() + res[b].double(), x64.abs() @ w64.abs() + bias.double().abs() + res[b].double().abs()
         err = (c[b].double() - want).abs()
         assert bool((err <= min(K + 2, 36 + K / 32) * 2.0**-24 * magnitude).all())
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch,shared", [
+    (16, 16, 64, 3, False), (40, 72, 96, 5, True), (50, 200, 128, 7, False),    # one tile a product, fewer products than XCDs
+    (192, 1536, 264, 9, False), (130, 390, 200, 11, True), (640, 320, 512, 8, False), # 3 .. 15 tiles: products change inside an XCD's range
+    (513, 700, 130, 3, False), (257, 2050, 2112, 2, True), (16, 64, 32, 1000, False)])
+def test_batches_are_dealt_over_all_xcds(dtype, nn, M, N, K, batch, shared):
+    """Every tile of every product is computed once, with its own residual; `shared`: one b for the whole batch (stride 0).
+    The bound of the tests above: K + 2 roundings of fp32 on the sum of magnitudes, half an ulp of the stored type."""
+    import ctypes as C
+
+    import torch
+
+    from axiom_amd import capi
+
+    g = axo.PCG64(M + 3 * N + K + batch)
+    nb = 1 if shared else batch
+    half_ulp = {F32: 0.0, F16: 2.0**-11, BF16: 2.0**-8}[dtype]
+    td = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dtype]
+    da = gh.to_dev(g.normal((batch, M, K)).astype(np.float32)).to(td)
+    db = gh.to_dev((g.normal((nb, K, N) if nn else (nb, N, K)) / np.sqrt(K)).astype(np.float32)).to(td)
+    bias, res = gh.to_dev((g.normal((N,)) * 0.1).astype(np.float32)).to(td), gh.to_dev(g.normal((batch, M, N)).astype(np.float32)).to(td)
+    c = torch.full((batch, M, N), float("nan"), device="cuda", dtype=td)
+    p = capi.GemmParams()
+    p.dtype, p.m, p.n, p.k, p.batch, p.lda, p.ldb, p.ldc, p.trans_b = dtype, M, N, K, batch, K, N if nn else K, N, int(not nn)
+    p.stride_a, p.stride_b, p.stride_c = M * K, 0 if shared else K * N, M * N
+    p.bias, p.residual = bias.data_ptr(), res.data_ptr()
+    torch.cuda.synchronize()
+    gh.sync()
+    capi.check(capi.lib().axhip_gemm(da.data_ptr(), db.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    for b in range(batch):
+        x, w = da[b].double(), db[0 if shared else b].double()
+        w = w if nn else w.t().contiguous()
+        want = x @ w + bias.double() + res[b].double()
+        magnitude = x.abs() @ w.abs() + bias.double().abs() + res[b].double().abs()
+        assert bool(((c[b].double() - want).abs() <= (K + 2) * 2.0**-24 * magnitude + half_ulp * want.abs() + 2.0**-24).all())
