@@ -370,12 +370,14 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // loaders 76), the fragments of the next eight k are read under the MFMAs of these, the barrier of a k-tile comes before its
 // last steps (by then every wavefront has read the whole tile), and behind it the reads turn to the next tile.  What is
 // left, one k-tile of 64 x 64: 1024 cycles of MFMAs in 1380.  Two wavefronts a SIMD with half of each k-tile, or two sums
-// in turn, were no faster.  1024^3: 26.3 -> 24.5 us, 2048^3 155 -> 138.
+// in turn, were no faster.  The values of a finished block then take bias, residual and activation together: with a branch on the activation for each,
+// 60 KB of code that every CU read anew, 4096 x 4096 x 512 + GELU took 228 us instead of 176 and 1024^3 24.5 instead of 22.
+// 1024^3: 26.3 -> 22 us, 2048^3 155 -> 134.
 // Rows may start anywhere: the loads need 4-byte alignment.  The chunk that K ends in is fetched as the four floats that
 // end with the row and shifted into place in LDS by the lane that loaded it; chunks behind it, and k-tiles past the last,
 // are sent out of the descriptor's range and arrive as zeros.  NN rows that are no whole chunks: the last column tile is
 // moved left to end with them (N >= TNR); the columns it shares with its neighbour are the neighbour's to store.
-template <int TM, int TNR, int S, bool NN>
+template <int TM, int TNR, int S, bool NN, bool TURNS>
 __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
     constexpr int MI = TM / 64, NJ = TNR / 64;
     constexpr int NLA = TM / 32, NLB = TNR / 32, NL = NLA + NLB; // loads of 1 KiB per wavefront and k-tile
@@ -473,14 +475,14 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     for (int ks = 0; ks < 4; ++ks) f_off[ks] = l32 * BIG_ROWB + (((2 * ks + g2) ^ ((l32 >> 1) & 7)) * 16);
 
     // The sums of a k-tile are added to those of all before: chains of 32 fp32 additions, however large K (2048^3, one
-    // chain: 8.1e-7 off the exact result, now 1.8e-7; no more than the kernels without shared tiles at any K).
-    float16_t acc[MI][NJ], sum[MI][NJ];
+    // chain: 8.1e-7 off the exact result, now 1.8e-7; no more than the kernels without shared tiles at any K).  TURNS:
+    // two accumulators in turn, one is added up under the next k-tile's MFMAs.
+    constexpr int TURN = TURNS ? 1 : 0;
+    float16_t acc[1 + TURN][MI][NJ], sum[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.0f;
+        for (int j = 0; j < NJ; ++j) sum[i][j] = acc[TURN][i][j] = float16_t{};
 
     // fragments of LOOK steps of eight k are on their way while one is multiplied: with one block a wavefront has four MFMAs
     // for these, less than a read takes next to three other wavefronts'
@@ -498,17 +500,17 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
             fb[slot][j] = *reinterpret_cast<const float4_t *>(Bs + 32 * j * BIG_ROWB + f_off[step]);
         }
     };
-    // eight k: 4 MI NJ MFMAs; behind MFMA x what `between(x)` does
-    auto multiply = [&](int slot, bool first, auto between) __attribute__((always_inline)) {
+    // eight k: 4 MI NJ MFMAs; behind MFMA (c, i, j) what `between` does
+    auto multiply = [&](int slot, int p, bool first, auto between) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], first && c == 0 ? float16_t{} : acc[i][j], 0, 0, 0);
+                    acc[p][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], first && c == 0 ? float16_t{} : acc[p][i][j], 0, 0, 0);
                     AXHIP_FENCE();
-                    between((c * MI + i) * NJ + j);
+                    between(c, i, j);
                     AXHIP_FENCE();
                 }
     };
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
         for (int j = 0; j < NJ; ++j) read_b(ks, 0, ks, j);
     }
     int cur = 0; // offset of k-tile kt's stage
-    for (int kt = 0; kt < nk; ++kt) {
+    auto tile = [&](int p) __attribute__((always_inline)) {
         const int next = cur + STAGEB == S * STAGEB ? 0 : cur + STAGEB;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -532,23 +534,44 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
                 __syncthreads(); // tile kt + 1 has landed, and tile kt is no longer read
                 AXHIP_FENCE();
             }
-            multiply(ks % SLOTS_F, ks == 0, [&](int x) __attribute__((always_inline)) {
+            multiply(ks % SLOTS_F, p, ks == 0, [&](int c, int i, int j) __attribute__((always_inline)) {
+                const int x = (c * MI + i) * NJ + j;
                 if (x < MI) read_a((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
                 if (x < NJ) read_b((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
+                if (TURNS && (ks == 1 || ks == 2)) {
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) sum[i][j][8 * (ks - 1) + 2 * c + e] += acc[p ^ TURN][i][j][8 * (ks - 1) + 2 * c + e];
+                }
             });
         }
+        cur = next;
+    };
+    auto add_up = [&](int p) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) sum[i][j][e] += acc[i][j][e];
-        cur = next;
+                for (int e = 0; e < 16; ++e) sum[i][j][e] += acc[p][i][j][e];
+    };
+    if constexpr (TURNS) {
+        for (int kt = 0; kt < nk; kt += 2) {
+            tile(0);
+            if (kt + 1 < nk) tile(TURN);
+        }
+        if (nk % 2 == 0) add_up(TURN);
+        else add_up(0);
+    } else {
+        for (int kt = 0; kt < nk; ++kt) {
+            tile(0);
+            add_up(0);
+        }
     }
 #undef AXHIP_VMCNT
 #undef AXHIP_FENCE
 
-    // epilogue: accumulator element e of tile (i, j) is C[m + 32 i + 8 (e / 4) + 4 g2 + e % 4][n + 32 j + l32]
+    // epilogue: accumulator element e of tile (i, j) is C[m + 32 i + 8 (e / 4) + 4 g2 + e % 4][n + 32 j + l32].  The 16
+    // values of a tile take each step together: one branch on the epilogue, one set of loads on their way.
     float *Cb = static_cast<float *>(g.c) + bz * g.sc;
     const float *Rb = g.residual ? static_cast<const float *>(g.residual) + bz * g.sc : nullptr;
 #pragma unroll
@@ -557,15 +580,21 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
         if (col >= g.N || col < n_low) continue;
         const float bias = g.bias ? static_cast<const float *>(g.bias)[col] : 0.0f;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i) {
+            const int64_t row0 = m0 + wm + 32 * i + 4 * g2, at0 = row0 * g.ldc + col;
+            const int rows = static_cast<int>(min<int64_t>(32, g.M - row0)); // (row 8 (e / 4) + e % 4 of these)
+            float x[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int64_t row = m0 + wm + 32 * i + 8 * (e / 4) + 4 * g2 + e % 4;
-                if (row >= g.M) continue;
-                float x = sum[i][j][e] + bias;
-                if (Rb) x += Rb[row * g.ldc + col];
-                Cb[row * g.ldc + col] = gemm_epilogue(g.epilogue, x);
+            for (int e = 0; e < 16; ++e) x[e] = sum[i][j][e] + bias;
+            if (Rb) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) x[e] += 8 * (e / 4) + e % 4 < rows ? Rb[at0 + (8 * (e / 4) + e % 4) * g.ldc] : 0.0f;
             }
+            gemm_epilogue_all(g.epilogue, x);
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (8 * (e / 4) + e % 4 < rows) Cb[at0 + (8 * (e / 4) + e % 4) * g.ldc] = x[e];
+        }
     }
 }
 
@@ -720,7 +749,7 @@ const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
 // work-groups take on the 256 CUs, fitted to 60 products of m 11 .. 4117, n 64 .. 51865, k 64 .. 8192.  Tiles of 64 x 64 fill
 // the chip soonest and share a CU; larger ones read less from LDS and L2 for each MFMA.
 struct F32RingTile { int tm, tn; float start, per_k, per_round; };
-constexpr F32RingTile F32_RING_TILES[3] = {{128, 128, 13.0f, 0.067f, 4.5f}, {64, 128, 8.5f, 0.0325f, 4.0f}, {64, 64, 6.2f, 0.0170f, 1.3f}};
+constexpr F32RingTile F32_RING_TILES[3] = {{128, 128, 11.0f, 0.067f, 3.5f}, {64, 128, 6.8f, 0.0325f, 3.0f}, {64, 64, 4.5f, 0.0170f, 1.3f}};
 struct F32Ring { int tile; float cost; };
 F32Ring f32_ring_tile(const AxhipGemmParams &p) {
     F32Ring best{0, 0.0f};
@@ -946,13 +975,17 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         };
         int rc2;
         switch (f32_ring_tile(p).tile) {
-#define AXHIP_RING(TM, TN, S) \
-    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, S, false>, TM, TN, S * (TM + TN) * BIG_ROWB) : launch(gemm_mfma_f32_ring_kernel<TM, TN, S, true>, TM, TN, S * (TM + TN) * BIG_ROWB)
-        case 0: AXHIP_RING(128, 128, 3); break;
-        case 1: AXHIP_RING(64, 128, 3); break;
+#define AXHIP_RING(TM, TN, S, TURNS) \
+    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, S, false, TURNS>, TM, TN, S * (TM + TN) * BIG_ROWB) \
+                    : launch(gemm_mfma_f32_ring_kernel<TM, TN, S, true, TURNS>, TM, TN, S * (TM + TN) * BIG_ROWB)
+        // (two accumulators in turn on the one work-group of a CU, where nothing else fills the pipe meanwhile; elsewhere their
+        // registers cost a second work-group its place: 2048^3 145 us instead of 134 on 64 x 128 tiles, and 128 x 128 tiles
+        // 182 instead of 176 for 4096 x 4096 x 512)
+        case 0: AXHIP_RING(128, 128, 3, false); break;
+        case 1: AXHIP_RING(64, 128, 3, false); break;
         default: // (one work-group per CU: a fourth stage hides the rest of a load's latency, 80 -> 76 us for k of 4096; more: three of them share a CU's LDS)
-            if ((p.m + 63) / 64 * ((p.n + 63) / 64) * p.batch <= 256) AXHIP_RING(64, 64, 4);
-            else AXHIP_RING(64, 64, 3);
+            if ((p.m + 63) / 64 * ((p.n + 63) / 64) * p.batch <= 256) AXHIP_RING(64, 64, 4, true);
+            else AXHIP_RING(64, 64, 3, false);
             break;
 #undef AXHIP_RING
         }

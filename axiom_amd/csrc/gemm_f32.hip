@@ -188,7 +188,8 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
             if (res) add4(res + to);
             Floats<4> y;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y.v[e] = gemm_epilogue(g.epilogue, v[e]);
+            for (int e = 0; e < 4; ++e) y.v[e] = v[e];
+            gemm_epilogue_all(g.epilogue, y.v);
             *reinterpret_cast<Floats<4> *>(C + to) = y;
             continue;
         }

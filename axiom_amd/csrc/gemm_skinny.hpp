@@ -27,10 +27,10 @@ __device__ __forceinline__ float gemm_epilogue16(int op, float x) {
 }
 
 // ... of N values: one branch for all of them
-template <int N> __device__ __forceinline__ void gemm_epilogue16_all(int op, float (&x)[N]) {
+template <bool HALF, int N> __device__ __forceinline__ void gemm_epilogue_all_as(int op, float (&x)[N]) {
 #define AXHIP_EPILOGUE_CASE(OP)                                                   \
     case OP:                                                                      \
-        _Pragma("unroll") for (int e = 0; e < N; ++e) x[e] = gemm_epilogue16(OP, x[e]); \
+        _Pragma("unroll") for (int e = 0; e < N; ++e) x[e] = HALF ? gemm_epilogue16(OP, x[e]) : gemm_epilogue(OP, x[e]); \
         break;
     switch (op) {
         AXHIP_EPILOGUE_CASE(AXHIP_OP_RELU)
@@ -42,14 +42,15 @@ template <int N> __device__ __forceinline__ void gemm_epilogue16_all(int op, flo
     }
 #undef AXHIP_EPILOGUE_CASE
 }
+template <int N> __device__ __forceinline__ void gemm_epilogue16_all(int op, float (&x)[N]) { gemm_epilogue_all_as<true>(op, x); }
+template <int N> __device__ __forceinline__ void gemm_epilogue_all(int op, float (&x)[N]) { gemm_epilogue_all_as<false>(op, x); }
 
 // x W^T with at most 8 rows of x (a decoding step: one token, or a handful, against a weight matrix), both operands
 // along k.  The product is bound by reading W once, and a tiling by output tiles would give the chip N / 128
 // work-groups.  Here a wavefront owns R rows of W (R = 1, 2 or 4: enough wavefronts for every SIMD) and walks k with
 // its 64 lanes side by side -- every load covers 1 KiB of one row -- keeping M x R fp32 sums per lane
 // (16-bit: v_dot2_f32 on the packed pairs, products exact, fp32 accumulation; fp32: FMAs), which the lanes add up at
-// the end; lane 0
-// applies bias, residual and activation.
+// the end.
 struct SkinnyArgs {
     const void *x, *w;
     void *c;

@@ -204,6 +204,19 @@ def test_skinny_products_of_a_decoding_step_match_fp64(dt, M, N, K, extras):
         assert np.max(np.abs(got - want)) < 2e-2 + 2.0**-8 * np.max(np.abs(want))
 
 
+def test_the_fp32_ring_adds_up_odd_and_even_numbers_of_k_tiles():
+    """Whole numbers, exact in every order of the sum: 64 x 64 tiles with one work-group per CU (two accumulators in turn) and
+    with several, two to five k-tiles and a ragged last one, rows off the tile, with and without each epilogue step."""
+    for M, N in ((1000, 980), (1500, 1284)):
+        for K in (64, 96, 100, 128, 131, 160):
+            r = np.random.default_rng(M + K)
+            a, b = (r.integers(-4, 5, s).astype(np.float32) for s in ((M, K), (K, N)))
+            bias, res = (r.integers(-9, 10, s).astype(np.float32) for s in ((N,), (M, N)))
+            assert np.array_equal(gh.gemm(a, b, F32)[0], a @ b), (M, N, K)
+            got = gh.gemm(a, np.ascontiguousarray(b.T), F32, trans_b=True, bias=bias, residual=res, epilogue="relu")[0]
+            assert np.array_equal(got, np.maximum(a @ b + bias + res, 0.0)), (M, N, K)
+
+
 @pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])
 def test_seeded_random_shapes_match_fp64(dt):
     """Forty seeded random products per dtype, shaped to land on every kernel and tile shape (matrix-core ring tiles,
