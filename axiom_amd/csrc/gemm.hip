@@ -920,14 +920,15 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
     const bool nt = !p.trans_a && p.trans_b && p.k % 8 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.stride_a % 8 == 0 &&
                     p.stride_b % 8 == 0 && al16(a) && al16(b) && p.ldc < (1 << 21);
-    // One or two rows: 1 x 4096 x 4096 in bf16 4.2 us with W in the caches and 7.7 from HBM, 5.6 and 8.9 on the kernels of
-    // gemm_small.hip; 2 x 1280 x 5120 4.5 and 6.2, 5.5 and 9.1.  With more rows the sums per lane grow and the other kernels
-    // do not: the rest of the line dates from kernels that had a k loop of 5.5 us per 1024 elements (fp32: 138 us for
-    // 1 x 4096 x 4096) and lies too far out for those there are now -- bf16 4 x 4096 x 4096 8.5 us here and 5.8 there,
-    // 8 x 1280 x 5120 11.2 and 5.6; fp32 8 x 4096 x 4096 22.5 and 12.5, level at three or four rows.
+    // Its wavefronts, one per row of W, each read all of x: with the outputs, m n, grow the reads from L1, and the other
+    // kernels share them (W from HBM, us here and there: bf16 4 x 2048 x 4096 7.8 and 8.6, 6 x 2048 x 4096 9.2 and 8.4, 8 x 768 x
+    // 3072 5.5 and 5.6, 3 x 4096 x 4096 10.8 and 9.8; fp32 4 x 2048 x 2048 7.5 and 8.0, 6 x 2048 x 2048 8.8 and 8.0, 8 x 768 x
+    // 3072 7.2 and 8.0).  With one or two rows W alone counts (1 x 51865 x 4096 70 and 84, fp32 138 and 164), unless rows of W
+    // so short that a wavefront has hardly anything to wait for meet so many of them (bf16 1 x 51865 x 512 16.6 and 12.3,
+    // 2 x 51865 x 1280 29.9 and 26.0, 1 x 51865 x 1280 25.0 and 26.2).  Few bytes in all: fp32 4 x 3072 x 768 4.3 and 5.0.
     const int64_t w_elems = p.n * p.k;
-    const bool skinny_pays = p.m <= 2 || (p.m <= 8 && p.dtype == AXHIP_DTYPE_F32) || (p.m <= 4 && w_elems <= (int64_t(48) << 20)) ||
-                             (p.m <= 8 && p.k >= 2048 && w_elems <= (int64_t(24) << 20));
+    const bool f32_rows = p.dtype == AXHIP_DTYPE_F32;
+    const bool skinny_pays = p.m <= 8 && (p.m * p.n <= 8192 || (p.m <= 2 && (f32_rows || p.m * p.n <= 64 * p.k)) || (f32_rows && p.m * w_elems <= 10000000));
     const bool f32_nt = p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && al16(a) && al16(b);
     // (the kernel carries leading dimensions as 32-bit element counts)
     const bool ld32 = p.lda < (int64_t(1) << 31) && p.ldb < (int64_t(1) << 31) && p.ldc < (int64_t(1) << 31);

@@ -4,8 +4,7 @@
 // work-groups.  Here a wavefront owns R rows of W (R = 1, 2 or 4: enough wavefronts for every SIMD) and walks k with
 // its 64 lanes side by side -- every load covers 1 KiB of one row -- keeping M x R fp32 sums per lane
 // (16-bit: v_dot2_f32 on the packed pairs, products exact, fp32 accumulation; fp32: FMAs), which the lanes add up at
-// the end; lane 0
-// applies bias, residual and activation.
+// the end.
 #include "gemm_skinny.hpp"
 
 namespace axhip {
@@ -28,12 +27,56 @@ template <int DT> __device__ __forceinline__ float dot16b(const uint4_t &a, cons
     return acc;
 }
 
+// The sums of P values (a power of two) over the wavefront, value i in the lanes [64 / P i, 64 / P (i + 1)): at each step
+// that still has several values a lane hands half of them over and adds up the other half -- P - 1 exchanges and adds, and
+// one a step from there on.  Every sum is formed as the butterfly over lanes 32, 16, .. 1 apart forms it.
+template <int CTRL> __device__ __forceinline__ float skinny_dpp(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xF, 0xF, false));
+}
+template <int P> __device__ __forceinline__ float skinny_sums(float (&v)[P], int lane) {
+    auto halve = [&](int p, auto swap) __attribute__((always_inline)) { // (swap(x, y): x's low and y's low lanes, x's high and y's high)
+#pragma unroll
+        for (int i = 0; i < (p > 1 ? p / 2 : 1); ++i) {
+            const auto t = swap(__float_as_uint(v[i]), __float_as_uint(v[p > 1 ? i + p / 2 : i]));
+            v[i] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+        }
+    };
+    auto step = [&](int p, int d, auto from) __attribute__((always_inline)) { // (from(x): x of the lane d away)
+        if (p <= 1) {
+            v[0] += from(v[0]);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < p / 2; ++i) {
+            const float mine = lane & d ? v[i + p / 2] : v[i], other = lane & d ? v[i] : v[i + p / 2];
+            v[i] = mine + from(other);
+        }
+    };
+    halve(P, [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); });
+    halve(P / 2, [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); });
+    step(P / 4, 8, [](float x) { return skinny_dpp<0x128>(x); }); // (row_ror:8)
+    if constexpr (P <= 4) v[0] += skinny_dpp<0x124>(v[0]);        // (row_ror:4: lanes 8 apart hold the same)
+    else step(P / 8, 4, [](float x) { return __shfl_xor(x, 4, WAVE); });
+    step(P / 16, 2, [](float x) { return skinny_dpp<0x4E>(x); }); // (quad_perm)
+    step(P / 32, 1, [](float x) { return skinny_dpp<0xB1>(x); });
+    return v[0];
+}
+
 template <int DT, int M, int R>
 __global__ __launch_bounds__(256) void gemm_skinny_kernel(const SkinnyArgs a) {
     constexpr int E = DT == AXHIP_DTYPE_F32 ? 4 : 8, ES = 16 / E; // elements per 16-byte vector, bytes per element
     const int lane = threadIdx.x % 64;
     const int n0 = (blockIdx.x * 4 + threadIdx.x / 64) * R;
     if (n0 >= a.N) return; // (whole wavefronts)
+    // After the sums, lane 64 / P i finishes value i = m R + r: one epilogue for all of them, and what it adds is requested
+    // before W is (value after value in lane 0, each with its own loads and branches, 4 x 1280 x 1280 in bf16 took 5.7 us instead of
+    // 4.0, 8 x 1280 x 5120 14.5 instead of 11.0, fp32 8 x 4096 x 4096 31.4 instead of 27.7).
+    constexpr int P = M * R <= 1 ? 1 : M * R <= 2 ? 2 : M * R <= 4 ? 4 : M * R <= 8 ? 8 : M * R <= 16 ? 16 : 32;
+    const int value = lane / (64 / P), n = n0 + value % R;
+    const bool writes = lane % (64 / P) == 0 && value < M * R && n < a.N;
+    const int64_t at = static_cast<int64_t>(value / R) * a.ldc + n;
+    const float bias = writes && a.bias ? load_any(a.bias, DT, n) : 0.0f;
+    const float residual = writes && a.residual ? load_any(a.residual, DT, at) : 0.0f;
     float acc[M][R];
 #pragma unroll
     for (int m = 0; m < M; ++m)
@@ -62,20 +105,11 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(const SkinnyArgs a) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) acc[m][r] = dot16b<DT>(wf[u][r], xf[u][m], acc[m][r]);
     }
+    float v[P];
 #pragma unroll
-    for (int m = 0; m < M; ++m)
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            float v = acc[m][r];
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, WAVE);
-            const int n = n0 + r;
-            if (lane == 0 && n < a.N) {
-                if (a.bias) v += load_any(a.bias, a.dtype, n);
-                if (a.residual) v += load_any(a.residual, a.dtype, static_cast<int64_t>(m) * a.ldc + n);
-                store_any(a.c, a.dtype, static_cast<int64_t>(m) * a.ldc + n, gemm_epilogue(a.epilogue, v));
-            }
-        }
+    for (int i = 0; i < P; ++i) v[i] = i < M * R ? acc[i / R][i % R] : 0.0f;
+    const float sum = skinny_sums<P>(v, lane);
+    if (writes) store_any(a.c, DT, at, gemm_epilogue(a.epilogue, sum + bias + residual));
 }
 
 void launch_skinny(const SkinnyArgs &k, int m, int rows_per_wave, unsigned blocks, hipStream_t s) {

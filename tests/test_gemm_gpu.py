@@ -204,6 +204,23 @@ def test_skinny_products_of_a_decoding_step_match_fp64(dt, M, N, K, extras):
         assert np.max(np.abs(got - want)) < 2e-2 + 2.0**-8 * np.max(np.abs(want))
 
 
+@pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(m, 37, 264) for m in range(1, 9)] + [(2, 3001, 24576), (3, 2051, 32768)])
+def test_skinny_sums_reach_their_row_and_column(dt, M, N, K):
+    """One to eight rows of x on one row of W per wavefront, and two and three on two (W of 64 M elements and more), W's last
+    one alone: whole numbers whose products add up without rounding, with bias, residual and RELU."""
+    g = axo.PCG64(M * 31 + N)
+    x, W = np.zeros((M, K), np.float32), np.zeros((N, K), np.float32)
+    hit = (np.arange(N) * 8191) % K  # row n of W picks column hit[n] of x, and its last one
+    W[np.arange(N), hit] += 2.0
+    W[:, K - 1] += 1.0
+    x[:] = (np.arange(M)[:, None] * 37 + np.arange(K)[None, :] * 11) % 23 - 11.0
+    bias, res = (np.round(4 * g.normal(s)).astype(np.float32) for s in ((N,), (M, N)))
+    got = axo.to_f32(gh.gemm(*(axo.to_bits(t, dt) for t in (x, W)), dt, trans_b=True, bias=axo.to_bits(bias, dt), residual=axo.to_bits(res, dt), epilogue="relu")[0], dt)
+    want = np.maximum(2.0 * x[:, hit] + x[:, K - 1 :] + bias + res, 0.0)
+    assert np.array_equal(got, want)
+
+
 def test_the_fp32_ring_adds_up_odd_and_even_numbers_of_k_tiles():
     """Whole numbers, exact in every order of the sum: 64 x 64 tiles with one work-group per CU (two accumulators in turn) and
     with several, two to five k-tiles and a ragged last one, rows off the tile, with and without each epilogue step."""
