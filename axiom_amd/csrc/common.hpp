@@ -348,26 +348,31 @@ __device__ __forceinline__ void store_vec(void *p, int dt, int64_t i, const floa
     }
 }
 
-// wavefront (64 lanes) all-reduce through cross-lane shuffles
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+// Combinations of lanes 32 or 16 apart: combine(own, other's) in both, without a trip through LDS (a shuffle is one, and six
+// of them in a row are most of a short kernel's tail).
+template <class F> __device__ __forceinline__ float across32(float v, F combine) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return combine(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float wave_prod(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v *= __shfl_xor(v, o, WAVE);
-    return v;
+template <class F> __device__ __forceinline__ float across16(float v, F combine) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return combine(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-    return v;
+template <int CTRL, class F> __device__ __forceinline__ float across_dpp(float v, F combine) {
+    return combine(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xF, 0xF, false)));
 }
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, WAVE));
-    return v;
+// All-reduce over the wavefront (64 lanes, all of them active), lanes 32, 16, .. 1 apart: by then lanes a row's rotation
+// apart hold what those that far apart in the butterfly do.
+template <class F> __device__ __forceinline__ float wave_all(float v, F combine) {
+    v = across16(across32(v, combine), combine);
+    v = across_dpp<0x124>(across_dpp<0x128>(v, combine), combine); // row_ror:8, row_ror:4
+    return across_dpp<0x121>(across_dpp<0x122>(v, combine), combine);
 }
+__device__ __forceinline__ float lanes_add(float a, float b) { return a + b; }
+__device__ __forceinline__ float lanes_max(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ float wave_sum(float v) { return wave_all(v, lanes_add); }
+__device__ __forceinline__ float wave_prod(float v) { return wave_all(v, [](float a, float b) { return a * b; }); }
+__device__ __forceinline__ float wave_max(float v) { return wave_all(v, lanes_max); }
+__device__ __forceinline__ float wave_min(float v) { return wave_all(v, [](float a, float b) { return fminf(a, b); }); }
 
 } // namespace axhip

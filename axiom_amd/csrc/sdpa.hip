@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_mfma_kernel(const S
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, s[kt][i]);
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
+            mloc = across32(mloc, lanes_max);
             const float m_new = fmaxf(m_run, mloc * a.scale_log2e);
             // rescale only when some row's maximum outgrew its reference by the threshold
             // (-inf - -inf = NaN compares false: a row with no visible key yet keeps -inf)
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_mfma_kernel(const S
     }
 
     // ---- epilogue: O = O^T / l, written as 4 consecutive dims (8 bytes) per store
-    const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
+    const float l_tot = across32(l_run, lanes_add);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     if constexpr (SPLITK) {
         if (q_ok) {
@@ -899,7 +899,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
             }
         }
 
-        const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
+        const float l_tot = across32(l_run, lanes_add);
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         if (q_ok) {
             uint16_t *orow = O + static_cast<int64_t>(q) * a.os[2];
@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(512, 1) void sdpa_mfma_pingpong_kernel(const SdpaAr
         prefetched = pf_next;
 
         l_run += l_run1;
-        const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
+        const float l_tot = across32(l_run, lanes_add);
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         // A lane holds 4 consecutive dims per (dt, i4); the half-waves trade every second group so that each lane
         // stores 8 consecutive dims (16 bytes): lanes 0-31 the even groups, lanes 32-63 the odd ones
@@ -1470,7 +1470,7 @@ __global__ __launch_bounds__(256) void sdpa_mfma_f32_kernel(const SdpaArgs a) {
         for (int u = 0; u < NSUB; ++u)
 #pragma unroll
             for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, s[u][i]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
+        mloc = across32(mloc, lanes_max);
         const float m_new = fmaxf(m_run, mloc * a.scale_log2e);
         if (__builtin_amdgcn_ballot_w64(m_new - m_run > RESCALE_THRESHOLD) != 0) {
             const float alpha = m_new == NEG_INF_F ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
@@ -1532,7 +1532,7 @@ __global__ __launch_bounds__(256) void sdpa_mfma_f32_kernel(const SdpaArgs a) {
         }
     }
 
-    const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
+    const float l_tot = across32(l_run, lanes_add);
     if constexpr (SPLIT == 1) {
         // ---- epilogue: O = O^T / l, four consecutive dims per store
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
