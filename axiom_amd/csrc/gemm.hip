@@ -928,7 +928,8 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     // 2 x 51865 x 1280 29.9 and 26.0, 1 x 51865 x 1280 25.0 and 26.2).  Few bytes in all: fp32 4 x 3072 x 768 4.3 and 5.0.
     const int64_t w_elems = p.n * p.k;
     const bool f32_rows = p.dtype == AXHIP_DTYPE_F32;
-    const bool skinny_pays = p.m <= 8 && (p.m * p.n <= 8192 || (p.m <= 2 && (f32_rows || p.m * p.n <= 64 * p.k)) || (f32_rows && p.m * w_elems <= 10000000));
+    const bool alone = f32_rows ? f32_shape < 0 && !takes_f32_ring(p, a, b) : !takes_half_kernels(p); // (else the FMA kernel)
+    const bool skinny_pays = p.m <= 8 && (p.m * p.n <= 8192 || (p.m <= 2 && (f32_rows || p.m * p.n <= 64 * p.k)) || (f32_rows && p.m * w_elems <= 10000000) || alone);
     const bool f32_nt = p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && al16(a) && al16(b);
     // (the kernel carries leading dimensions as 32-bit element counts)
     const bool ld32 = p.lda < (int64_t(1) << 31) && p.ldb < (int64_t(1) << 31) && p.ldc < (int64_t(1) << 31);

@@ -1,5 +1,6 @@
 """GPU parity of axhip_gemm (the nn::Linear / ops::matmul path) against float64
 and against the CPU oracle's matmul."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -219,6 +220,27 @@ def test_skinny_sums_reach_their_row_and_column(dt, M, N, K):
     got = axo.to_f32(gh.gemm(*(axo.to_bits(t, dt) for t in (x, W)), dt, trans_b=True, bias=axo.to_bits(bias, dt), residual=axo.to_bits(res, dt), epilogue="relu")[0], dt)
     want = np.maximum(2.0 * x[:, hit] + x[:, K - 1 :] + bias + res, 0.0)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])
+def test_few_rows_too_far_apart_for_the_tiled_kernels(dt):
+    """Four rows of x 2^21 elements apart, past the 32-bit offsets of the 16-bit tile kernels, and more outputs than the kernel
+    for a few rows otherwise takes."""
+    from axiom_amd import capi
+
+    M, N, K, lda = 4, 2304, 512, 1 << 21
+    r = np.random.default_rng(3)
+    x, W = r.integers(-3, 4, (M, K)).astype(np.float32), r.integers(-2, 3, (N, K)).astype(np.float32)
+    far = np.zeros((M, lda), np.float32)
+    far[:, :K] = x
+    a, b, c = gh.to_dev(axo.to_bits(far, dt)), gh.to_dev(axo.to_bits(W, dt)), gh.empty_dev((M, N), dt)
+    p = capi.GemmParams()
+    p.dtype, p.trans_a, p.trans_b, p.m, p.n, p.k, p.batch = dt, 0, 1, M, N, K, 1
+    p.lda, p.ldb, p.ldc, p.stride_a, p.stride_b, p.stride_c = lda, K, N, M * lda, N * K, M * N
+    gh.sync()
+    capi.check(capi.lib().axhip_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    assert np.array_equal(axo.to_f32(gh.to_host(c, gh.np_store_dtype(dt)), dt), x @ W.T if dt == F32 else axo.to_f32(axo.to_bits(x @ W.T, dt), dt))
 
 
 def test_the_fp32_ring_adds_up_odd_and_even_numbers_of_k_tiles():
