@@ -717,6 +717,32 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
             return row_max(s);
         };
 
+        // Explicit mask: a masked score starts at -inf, and its key may hold anything -- but -inf plus a product with an
+        // infinity or a NaN is NaN, which the maximum of the row passes on.  Where it did, the mask of the tile is put on the
+        // finished scores; a row whose maximum still is NaN sees one.  (A compare and a branch per tile where K is finite.)
+        auto mask_again = [&](int tile, float16_t (&s)[2]) {
+            uint32_t dead = 0; // bit 16 kt + i: key 32 kt + 8 (i / 4) + 4 g + i % 4 of the tile
+            if constexpr (MASK == MASK_BITS) {
+                if (q_ok) dead = a.mask_bits[((plane * static_cast<int64_t>(a.mask_tiles) + tile) * a.Sq + q) * 2 + g];
+            }
+            if constexpr (MASK == MASK_BYTES) {
+                if (q_ok) {
+                    const uint8_t *row = M + static_cast<int64_t>(q) * a.Skv;
+    #pragma unroll 1
+                    for (int n = 0; n < 32; ++n) {
+                        const int key = tile * BN + 32 * (n / 16) + 8 * (n % 16 / 4) + 4 * g + n % 4;
+                        dead |= (key >= a.Skv || row[key] != 0 ? 1u : 0u) << n;
+                    }
+                }
+            }
+    #pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+    #pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if ((dead >> (kt * 16 + i)) & 1u) s[kt][i] = NEG_INF_F;
+            return row_max(s);
+        };
+
         // Running maximum and the (rare) rescale of the accumulators.  The score accumulators of a
         // tile start at MINUS the reference maximum that was current when its MFMAs were issued, so
         // `cur` already holds logit - reference and the exponentials need no subtraction; mloc is
@@ -849,6 +875,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
                 const bool need_mask = (a.causal && kv0 + BN - 1 > qw0) || (MASK == MASK_NONE && kv0 + BN > a.Skv);
                 float mloc = mx_cur;
                 if (need_mask) mloc = mask_and_max(kv0, cur);
+                if constexpr (MASK != MASK_NONE) {
+                    if (__builtin_expect(__builtin_amdgcn_ballot_w64(q_ok && __builtin_isnan(mloc)) != 0, 0)) mloc = mask_again(tile0 + j, cur);
+                }
                 update_max(mloc, cur);
                 // The next tile's scores are issued unconditionally so that they share a basic
                 // block with this tile's softmax; after the last tile (or the last one this wave

@@ -85,7 +85,10 @@ int axhip_stream_sync(void *stream);
  * (0 = broadcast).  is_causal masks kv_pos > q_pos (top-left aligned,
  * src/backends/cpu/flash_attention_cpu.cpp:78-89).  scale <= 0 means
  * 1/sqrt(D) (src/tensor/operations.cpp:4013-4015).  A row whose keys are all
- * masked yields zeros.  fp32 accumulation; output in `dtype`.
+ * masked yields zeros.  K may hold anything, infinities and NaN too, where a
+ * key is masked; V there meets a weight of zero and has to be finite (a block
+ * of keys that no row of a tile sees may not be read at all).  fp32
+ * accumulation; output in `dtype`.
  * bf16/f16 with D a multiple of 8 up to 256, and fp32 with D a multiple of
  * 4 up to 128, run on MFMA (16-byte aligned base
  * pointers, strides that are multiples of 8 elements; fp32: 4); everything

@@ -518,7 +518,7 @@ def sdpa_ws(q, k, v, dt, causal, mask=None, mask_strides=(0, 0), mask_offset=0, 
     gh.sync()
     if ws is not None:
         assert bool((ws[need:] == 0x5A).all().item())
-    return axo.to_f32(gh.to_host(o, np.uint16), dt), need, lib.axhip_sdpa_last_schedule()
+    return axo.to_f32(gh.to_host(o, gh.np_store_dtype(dt)), dt), need, lib.axhip_sdpa_last_schedule()
 
 
 @pytest.mark.parametrize("dt,D,S,Skv,causal,kind,offset", [
@@ -581,3 +581,37 @@ def test_work_groups_by_the_number_of_blocks(dt, B, H, Sq, Skv, D, causal, sched
         qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
         want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, None)
         assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, sl
+
+
+@pytest.mark.parametrize("dt,D,B,H,S,Skv,causal,planes,give,schedule", [
+    (BF16, 64, 1, 3, 70, 131, False, (1, 1), False, b"key_split"), (F16, 128, 2, 4, 200, 449, True, (2, 1), False, b"key_split"),
+    (BF16, 64, 8, 33, 100, 192, False, (8, 33), False, b"pipelined4"), (F16, 80, 8, 17, 257, 131, True, (1, 1), False, b"pipelined4"),
+    (BF16, 128, 7, 6, 900, 199, False, (7, 1), False, b"pipelined8"), (F16, 40, 7, 6, 900, 512, False, (1, 1), True, b"pipelined8"),
+    (BF16, 64, 4, 66, 257, 259, False, (4, 1), True, b"pipelined4"), (BF16, 128, 4, 66, 130, 513, True, (1, 1), True, b"pipelined4"),
+    (F16, 64, 1, 8, 2048, 2048, False, (1, 1), True, b"key_split"), (BF16, 80, 1, 8, 2048, 1281, True, (1, 1), True, b"key_split"),
+    (BF16, 32, 2, 3, 130, 131, False, (2, 1), False, b"register_staged"), (F16, 256, 1, 3, 130, 131, False, (1, 1), False, b"register_staged"),
+    (F32, 64, 1, 3, 130, 131, False, (1, 1), False, b"direct"), (F32, 128, 4, 16, 130, 131, True, (4, 1), False, b"mfma_f32")])
+def test_masked_keys_may_hold_anything(dt, D, B, H, S, Skv, causal, planes, give, schedule):
+    """K is NaN or infinite at keys that a mask leaves out: whole tiles and ragged ends of them for every row, single keys
+    for every second one.  The rows that do not see such a key are what they are without it; the others are NaN."""
+    mask = np.zeros((*planes, S, Skv), np.uint8)
+    end = Skv - 67
+    mask[..., end:] = 1
+    mask[..., ::2, 5] = 1
+    mask[..., ::2, end // 2] = 255
+    mask[-1, -1, :, 9:12] = 1
+    q, k, v = inputs(B, H, S, Skv, D, dt, seed=S + D)
+    kf = axo.to_f32(k, dt).copy()
+    kf[:, :, end:] = np.array([np.nan, np.inf, -np.inf], np.float32)[np.arange(Skv - end) % 3, None]
+    kf[:, :, [5, end // 2]] = np.array([np.inf, np.nan], np.float32)[:, None]
+    got, _, ran = sdpa_ws(q, axo.to_bits(kf, dt), v, dt, causal, mask, (0 if planes[0] == 1 else planes[1] * S * Skv, 0 if planes[1] == 1 else S * Skv), 1, give)
+    assert ran == schedule
+    kf[:, :, [5, end // 2]] = 0.0 # (masked for the rows that are compared)
+    kf[:, :, end:] = 0.0
+    for b, h in {(0, 0), (B - 1, H - 1), (B // 2, H // 2)}:
+        qs, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, v))
+        want = naive_attention64(qs, kf[b:b + 1, h:h + 1], vs, 1 / math.sqrt(D), causal, mask[min(b, planes[0] - 1), min(h, planes[1] - 1)])[0, 0]
+        out = got[b, h]
+        err = np.abs(out[::2] - want[::2])
+        assert np.max(err) < (1e-4 + 1e-4 * np.max(np.abs(want)) if dt == F32 else 2e-2), (b, h)
+        assert np.isnan(out[end // 2 | 1::2]).all() # (causal: from the row on that reaches the key)
