@@ -114,3 +114,24 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(capi, "LIB_PATH", tmp_path / "libaxhip.so")
     with pytest.raises(FileNotFoundError):
         capi.lib()
+
+
+@pytest.mark.parametrize("batch,heads,seq_q,seq_kv,causal,planes,packed", [
+    (4, 16, 704, 704, 0, "batch", True), (4, 16, 512, 512, 0, "batch", False), (4, 12, 1024, 1024, 1, "batch", True), (4, 11, 1024, 1024, 1, "batch", False),
+    (4, 16, 1024, 1024, 0, "own", False), (4, 16, 1023, 1023, 0, "own", False), (4, 32, 2048, 2048, 0, "own", True), (4, 32, 2047, 2047, 0, "own", False),
+    (16, 2, 2048, 2048, 0, "batch", True), (16, 2, 1501, 1501, 0, "batch", False), (4, 8, 1501, 1501, 0, "batch", True),
+    (1, 16, 64, 65536, 0, "own", True), (1, 16, 64, 65535, 0, "own", False), (1, 16, 63, 65536, 0, "one", False), (1, 8, 4096, 4096, 0, "one", True)])
+def test_memory_for_a_packed_mask_is_asked_for_where_packing_pays(batch, heads, seq_q, seq_kv, causal, planes, packed):
+    """What packing a mask costs is by its bytes, what it saves by the scores: by how many slices share the mask, and whether
+    its rows are aligned."""
+    lib = capi.lib()
+    p = capi.SdpaParams()
+    p.dtype, p.batch, p.heads, p.seq_q, p.seq_kv, p.head_dim, p.is_causal = capi.DTYPE_BF16, batch, heads, seq_q, seq_kv, 64, causal
+    p.q_strides[:] = p.o_strides[:] = (heads * seq_q * 64, seq_q * 64, 64)
+    p.k_strides[:] = p.v_strides[:] = (heads * seq_kv * 64, seq_kv * 64, 64)
+    plane = seq_q * seq_kv
+    p.mask_strides[:] = {"own": (heads * plane, plane), "batch": (plane, 0), "one": (0, 0)}[planes]
+    masks = {"own": batch * heads, "batch": batch, "one": 1}[planes]
+    need = lib.axhip_sdpa_workspace_bytes(C.byref(p), 1)
+    assert (need > 0) == packed
+    assert not packed or masks * plane // 8 <= need <= masks * seq_q * ((seq_kv + 63) // 64) * 8 + masks * (seq_q // 32 + 1) * 8 + 512
