@@ -617,3 +617,30 @@ def test_masked_keys_may_hold_anything(dt, D, B, H, S, Skv, causal, planes, give
         err = np.abs(out[::2] - want[::2])
         assert np.max(err) < (1e-4 + 1e-4 * np.max(np.abs(want)) if dt == F32 else 2e-2), (b, h)
         assert np.isnan(out[end // 2 | 1::2]).all() # (causal: from the row on that reaches the key)
+
+
+@pytest.mark.parametrize("dt,D,B,H,S,Skv,causal,planes,offset", [
+    (BF16, 64, 1, 8, 2048, 2048, False, (1, 1), 0), (F16, 64, 2, 4, 2000, 2049, False, (1, 1), 1), (BF16, 128, 1, 8, 2048, 2048, False, (1, 1), 3),
+    (F16, 80, 1, 8, 2048, 1539, False, (1, 1), 0), (BF16, 40, 1, 8, 1985, 2112, False, (1, 1), 2), (BF16, 64, 3, 4, 2111, 2012, True, (1, 1), 0),
+    (F16, 128, 1, 8, 2048, 3088, True, (1, 1), 1), (BF16, 72, 2, 4, 2000, 3200, True, (2, 1), 0)])
+def test_packed_masks_with_the_keys_split(dt, D, B, H, S, Skv, causal, planes, offset):
+    """Few slices under a packed mask: the two halves of a work-group share the key tiles between the first and the last one
+    that some row of its block sees -- none, one, two, .. five of them here, so that a half's share is short or empty."""
+    r = np.random.default_rng(S + Skv + D)
+    tiles = (Skv + 63) // 64
+    mask = np.ones((*planes, S, Skv), np.uint8)
+    for blk in range((S + 63) // 64):
+        first = 0 if causal else (7 * blk) % (tiles - 5)
+        first, seen = max(0, min(first, blk - 2)) if causal else first, blk % 6
+        rows = slice(64 * blk, 64 * blk + 64)
+        mask[..., rows, 64 * first : 64 * (first + seen)] = r.random(mask[..., rows, 64 * first : 64 * (first + seen)].shape) < 0.4
+    mask[..., S // 2 : S // 2 + 70, :] = 0 # (and all of them)
+    mask[..., -9:, : Skv - 1] = 1          # (the last rows: the last key alone)
+    mask[..., -9:, Skv - 1] = 0
+    q, k, v = inputs(B, H, S, Skv, D, dt, seed=S + D)
+    got, need, ran = sdpa_ws(q, k, v, dt, causal, mask, (0 if planes[0] == 1 else planes[1] * S * Skv, 0 if planes[1] == 1 else S * Skv), offset)
+    assert need > 0 and ran == b"key_split"
+    for b, h in {(0, 0), (B - 1, H - 1)}:
+        qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
+        want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, mask[min(b, planes[0] - 1), min(h, planes[1] - 1)])
+        assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h)
