@@ -23,6 +23,7 @@ int rows_setup_device(); // per-device set-up of the fused-row kernels (rows.hip
         if (_e != hipSuccess) {                                                        \
             ::axhip::set_last_error("%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e), \
                                     __FILE__, __LINE__);                               \
+            (void)hipGetLastError(); /* reported here: the next launch's check is not to find it */ \
             return static_cast<int>(_e);                                               \
         }                                                                              \
     } while (0)

@@ -120,3 +120,15 @@ def test_long_axis_reductions_with_a_caller_workspace(dt):
     # many results over a short axis: one pass, no temporary memory
     assert lib.axhip_reduce_axis_workspace_bytes(dx.data_ptr(), dt, 4096, 4, 1024) == 0
     assert lib.axhip_argreduce_workspace_bytes(dx.data_ptr(), dt, 4096, 4, 1024) == 0
+
+
+def test_a_refused_allocation_is_not_the_next_call_s_error():
+    lib = capi.lib()
+    p = C.c_void_p()
+    assert lib.axhip_malloc(C.byref(p), 1 << 50) != 0 and not p.value  # more than any card holds
+    x = gh.to_dev(axo.PCG64(4).normal((5, 70)))
+    y = torch.empty_like(x)
+    gh.sync()
+    capi.check(lib.axhip_softmax_axis(x.data_ptr(), capi.DTYPE_F32, 5, 70, 1, 0, y.data_ptr(), None))
+    gh.sync()
+    assert torch.allclose(y, torch.softmax(x, 1), atol=1e-6)
