@@ -468,8 +468,13 @@ Tensor detail::sdpa(const Tensor &query, const Tensor &key, const Tensor &value,
     // (a decoding step's partial results live in a block of this layer's cache: the block goes back when this
     // function returns and is handed out again in stream order)
     const size_t ws_bytes = axhip_sdpa_workspace_bytes(&p, mask_ptr != nullptr);
-    const std::unique_ptr<Storage> ws = ws_bytes ? make_storage(ws_bytes, Device::GPU) : nullptr;
-    AXHIP_CALL(axhip_sdpa_fwd_ws(ptr(q), ptr(k), ptr(v), out.storage()->raw(), mask_ptr, &p, ws ? ws->raw() : nullptr, ws_bytes, nullptr));
+    std::unique_ptr<Storage> ws;
+    try {
+        if (ws_bytes) ws = make_storage(ws_bytes, Device::GPU);
+    } catch (const DeviceError &) {
+        if (!mask_ptr) throw; // (a masked problem only runs faster with it: on a card with no room left it reads the mask in place)
+    }
+    AXHIP_CALL(axhip_sdpa_fwd_ws(ptr(q), ptr(k), ptr(v), out.storage()->raw(), mask_ptr, &p, ws ? ws->raw() : nullptr, ws ? ws_bytes : 0, nullptr));
     return out; // asynchronous; .cpu() / item() synchronise
 }
 

@@ -6,8 +6,10 @@
 #include <map>
 
 #include <atomic>
+#include <dlfcn.h>
 #include <thread>
 
+#include "axhip.h"
 #include "oracle_util.hpp"
 #include "test_framework.hpp"
 
@@ -17,6 +19,17 @@ using axtest::max_abs_diff;
 static std::vector<float> host_floats(const Tensor &t) {
     Tensor c = t.cpu().astype(DType::Float32).ascontiguousarray();
     return std::vector<float>(c.typed_data<float>(), c.typed_data<float>() + c.size());
+}
+
+// The library's allocation function as this program's host layer calls it: refuses blocks of `refused_bytes`, as a full card does.
+static std::atomic<size_t> refused_bytes{0}, refusals{0};
+extern "C" int axhip_malloc(void **p, size_t bytes) {
+    static const auto real = reinterpret_cast<int (*)(void **, size_t)>(dlsym(RTLD_NEXT, "axhip_malloc"));
+    if (bytes != 0 && bytes == refused_bytes) {
+        ++refusals;
+        return 2;
+    }
+    return real(p, bytes);
 }
 
 // ------------------------------------------------------------ device semantics
@@ -609,6 +622,27 @@ GPU_TEST(FlashAttentionGPU, BoolMasks) { // tests/test_flash_attention.cpp (mask
     ASSERT_TENSORS_CLOSE(ops::scaled_dot_product_attention(q.gpu(), k.gpu(), v.gpu(), m2.gpu(), -1, false).cpu(), axtest::oracle_sdpa(q, k, v, m2, -1, false), 1e-4, 1e-4);
     ASSERT_TENSORS_CLOSE(ops::scaled_dot_product_attention(q.gpu(), k.gpu(), v.gpu(), m4, -1, false).cpu(), axtest::oracle_sdpa(q, k, v, m4, -1, false), 1e-4, 1e-4); // host mask is moved over
     EXPECT_THROW(ops::scaled_dot_product_attention(q.gpu(), k.gpu(), v.gpu(), Tensor::zeros({8, 8}, DType::Bool), -1, false), ShapeError);
+}
+GPU_TEST(FlashAttentionGPU, MaskedProblemsRunWithoutTheirWorkspaceWhereItDoesNotFit) {
+    auto [q, k, v] = make_inputs(1, 16, 1280, 1280, 64, DType::BFloat16); // (26 M scores: the mask is packed where there is room)
+    Tensor m({1280, 1280}, DType::Bool);
+    for (size_t i = 0; i < 1280; ++i)
+        for (size_t j = 0; j < 1280; ++j) m.set_item<int>({i, j}, j > 900 || (i + j) % 3 == 0);
+    AxhipSdpaParams p{};
+    p.dtype = AXHIP_DTYPE_BF16;
+    p.batch = 1, p.heads = 16, p.seq_q = p.seq_kv = 1280, p.head_dim = 64;
+    for (int64_t *s : {p.q_strides, p.k_strides, p.v_strides, p.o_strides}) s[0] = 16 * 1280 * 64, s[1] = 1280 * 64, s[2] = 64;
+    const size_t bytes = axhip_sdpa_workspace_bytes(&p, 1);
+    EXPECT_TRUE(bytes > 0);
+    auto qg = q.gpu(), kg = k.gpu(), vg = v.gpu(), mg = m.gpu();
+    auto packed = ops::scaled_dot_product_attention(qg, kg, vg, mg, -1, false).cpu();
+    backends::hip::empty_cache();
+    refused_bytes = bytes;
+    refusals = 0;
+    auto in_place = ops::scaled_dot_product_attention(qg, kg, vg, mg, -1, false).cpu();
+    refused_bytes = 0;
+    EXPECT_TRUE(refusals > 0);
+    EXPECT_LE(max_abs_diff(packed, in_place), 2e-2); // (two orders of the same sums, rounded to bf16)
 }
 GPU_TEST(FlashAttentionGPU, HalfTypesRunOnMfma) { // tests/test_flash_attention.cpp:233-249 (vs f32 computation of the same inputs)
     for (DType dt : {DType::Float16, DType::BFloat16})
