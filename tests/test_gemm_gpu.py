@@ -206,10 +206,10 @@ def test_skinny_products_of_a_decoding_step_match_fp64(dt, M, N, K, extras):
 
 
 @pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])
-@pytest.mark.parametrize("M,N,K", [(m, 37, 264) for m in range(1, 9)] + [(2, 3001, 24576), (3, 2051, 32768)])
+@pytest.mark.parametrize("M,N,K", [(m, 37, 264) for m in range(1, 9)] + [(2, 3001, 24576), (3, 2051, 32768), (5, 1025, 65536), (8, 1023, 65792)])
 def test_skinny_sums_reach_their_row_and_column(dt, M, N, K):
-    """One to eight rows of x on one row of W per wavefront, and two and three on two (W of 64 M elements and more), W's last
-    one alone: whole numbers whose products add up without rounding, with bias, residual and RELU."""
+    """One to eight rows of x on one row of W per wavefront, and two, three, five and eight on two (W of 64 M elements and more),
+    W's last one alone or not: whole numbers whose products add up without rounding, with bias, residual and RELU."""
     g = axo.PCG64(M * 31 + N)
     x, W = np.zeros((M, K), np.float32), np.zeros((N, K), np.float32)
     hit = (np.arange(N) * 8191) % K  # row n of W picks column hit[n] of x, and its last one
@@ -220,6 +220,19 @@ def test_skinny_sums_reach_their_row_and_column(dt, M, N, K):
     got = axo.to_f32(gh.gemm(*(axo.to_bits(t, dt) for t in (x, W)), dt, trans_b=True, bias=axo.to_bits(bias, dt), residual=axo.to_bits(res, dt), epilogue="relu")[0], dt)
     want = np.maximum(2.0 * x[:, hit] + x[:, K - 1 :] + bias + res, 0.0)
     assert np.array_equal(got, want)
+
+
+def test_skinny_sums_of_four_rows_of_w():
+    """Four rows of W per wavefront, up to 32 sums over its lanes: a setting that is read once, so it has a process of its own."""
+    import os
+    import subprocess
+    import sys
+
+    if os.environ.get("AXHIP_GEMM_SKINNY_ROWS"):
+        pytest.skip("already inside a forced run")
+    r = subprocess.run([sys.executable, "-m", "pytest", "-x", "-q", "-p", "no:cacheprovider", __file__, "-k", "test_skinny_sums_reach and 37-264"],
+                       env=dict(os.environ, AXHIP_GEMM_SKINNY_ROWS="4"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert r.returncode == 0 and "24 passed" in r.stdout, r.stdout[-3000:]
 
 
 @pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])

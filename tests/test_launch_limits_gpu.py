@@ -65,6 +65,34 @@ def test_products_of_many_row_tiles(dt, m, n, k):
     assert torch.equal(c[at], want)
 
 
+@pytest.mark.parametrize("dt,k,trans_b", [(BF16, 16, 1), (BF16, 16, 0), (F32, 32, 1), (F32, 32, 0)], ids=["bf16-nt", "bf16-nn", "f32-nt", "f32-nn"])
+def test_more_products_than_a_launch_may_have_tiles_for(dt, k, trans_b):
+    """65535 products of one row and 16385 columns, 129 tiles each at the widest: whichever kernel runs needs several launches,
+    which have to go on with the next product's a, b, c and residual.  b of product z is that of z - 1 a row (or column)
+    further on; sums of k exact terms, all compared."""
+    batch, n = 65535, 16385
+    kind = torch.float32 if dt == F32 else torch.bfloat16
+    a = torch.empty(batch, k, dtype=kind, device="cuda").random_(-2, 3)
+    b = torch.empty((n + batch, k) if trans_b else (k, n + batch), dtype=kind, device="cuda").random_(-1, 2)
+    bias, res = (torch.empty(s, dtype=kind, device="cuda").random_(-5, 6) for s in ((n,), (batch, n)))
+    c = torch.full((batch, n), 99.0, dtype=kind, device="cuda")
+    p = capi.GemmParams()
+    p.dtype, p.trans_b, p.m, p.n, p.k, p.batch = dt, trans_b, 1, n, k, batch
+    p.lda, p.ldb, p.ldc, p.stride_a, p.stride_b, p.stride_c = k, k if trans_b else n + batch, n, k, k if trans_b else 1, n
+    p.bias, p.residual = bias.data_ptr(), res.data_ptr()
+    gh.sync()
+    torch.cuda.synchronize()
+    capi.check(capi.lib().axhip_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    for z in range(0, batch, 1024):
+        count = min(1024, batch - z)
+        width = n + count - 1
+        window = b[z : z + width].t() if trans_b else b[:, z : z + width]
+        all_pairs = a[z : z + count].float() @ window.float()  # (product, column of the window)
+        want = all_pairs.as_strided((count, n), (width + 1, 1)) + bias.float() + res[z : z + count].float()
+        assert torch.equal(c[z : z + count].float(), want), z
+
+
 @pytest.mark.parametrize("outer,a,b", [(1 << 21, 65, 65), ((1 << 24) + 300, 16, 17)])
 def test_transposed_copy_of_many_small_slices(outer, a, b):
     """fp32 slices of several tiles (63 GiB in and out) and of one, of which there are more than a launch may have."""
