@@ -969,10 +969,24 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
                     configured.insert(reinterpret_cast<const void *>(kernel));
                 }
             }
-            const int tiles_m = static_cast<int>((p.m + tm_rows - 1) / tm_rows), tiles_n = static_cast<int>((p.n + tn_cols - 1) / tn_cols);
-            const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
-            AXHIP_REQUIRE(launch_fits(tiles + 7, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-            launch_products(g, tiles, 512, 4, [&](const GemmArgs &part, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds_bytes, s, part, tiles_m, tiles_n); });
+            // (more tiles than a launch may have: a strip of the longer side at a time; rows where b is [k, n], of which n < 2^24)
+            const int64_t tiles_m = (p.m + tm_rows - 1) / tm_rows, tiles_n = (p.n + tn_cols - 1) / tn_cols;
+            const bool by_rows = !p.trans_b || tiles_m >= tiles_n;
+            const int64_t across = by_rows ? tiles_n : tiles_m, size = by_rows ? p.m : p.n;
+            AXHIP_REQUIRE(launch_fits(across + 7, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+            const int64_t strip = products_per_launch(across, 512) * (by_rows ? tm_rows : tn_cols);
+            for (int64_t at = 0; at < size; at += strip) {
+                GemmArgs part = g;
+                (by_rows ? part.M : part.N) = std::min(strip, size - at);
+                const int64_t in_c = 4 * at * (by_rows ? g.ldc : 1);
+                if (by_rows) part.a = static_cast<const char *>(g.a) + 4 * at * g.a_rs;
+                else part.b = static_cast<const char *>(g.b) + 4 * at * g.b_cs;
+                part.c = static_cast<char *>(g.c) + in_c;
+                if (g.residual) part.residual = static_cast<const char *>(g.residual) + in_c;
+                if (g.bias && !by_rows) part.bias = static_cast<const char *>(g.bias) + 4 * at;
+                const int rows = static_cast<int>((part.M + tm_rows - 1) / tm_rows), cols = static_cast<int>((part.N + tn_cols - 1) / tn_cols);
+                launch_products(part, static_cast<int64_t>(rows) * cols, 512, 4, [&](const GemmArgs &some, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds_bytes, s, some, rows, cols); });
+            }
             return AXHIP_OK;
         };
         int rc2;

@@ -65,6 +65,32 @@ def test_products_of_many_row_tiles(dt, m, n, k):
     assert torch.equal(c[at], want)
 
 
+@pytest.mark.parametrize("m,n,trans_b", [(2, (1 << 29) + 41, 1), ((1 << 29) + 41, 3, 1), ((1 << 29) + 41, 4, 0), ((1 << 30) + 17, 1, 1)])
+def test_fp32_products_of_more_tiles_than_a_launch_may_have(m, n, trans_b):
+    """Long and narrow products of k exact terms, rows of the long operand overlapping: the strips have to go on in a or b, c,
+    the bias and the residual (which is c)."""
+    k, step = 32, 4
+    a, lda = (torch.empty(m * step + k, device="cuda").random_(-3, 4), step) if m > n else (torch.empty(m, k, device="cuda").random_(-3, 4), k)
+    b = (torch.empty(n * step + k, device="cuda").random_(0, 2) if n > m else torch.empty((n, k) if trans_b else (k, n), device="cuda").random_(0, 2))
+    bias = torch.empty(n, device="cuda").random_(-5, 6)
+    c = torch.empty(m, n, device="cuda").random_(-9, 10)
+    p = capi.GemmParams()
+    p.dtype, p.trans_b, p.m, p.n, p.k, p.lda, p.ldb, p.ldc, p.batch = F32, trans_b, m, n, k, lda, (step if n > m else k) if trans_b else n, n, 1
+    p.bias, p.residual = bias.data_ptr(), c.data_ptr()
+    at = torch.cat([places(max(m, n)), torch.arange((1 << 29) - 1024, 1 << 29, device="cuda")])  # (where the next strip starts, among them)
+    kk = torch.arange(k, device="cuda")
+    before = c[at] if m > n else c[:, at]
+    if m > n:
+        want = a[at[:, None] * step + kk] @ (b.t() if trans_b else b) + bias + before
+    else:
+        want = a @ b[at[:, None] * step + kk].t() + bias[at] + before
+    gh.sync()
+    torch.cuda.synchronize()
+    capi.check(capi.lib().axhip_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    assert torch.equal(c[at] if m > n else c[:, at], want)
+
+
 @pytest.mark.parametrize("dt,k,trans_b", [(BF16, 16, 1), (BF16, 16, 0), (F32, 32, 1), (F32, 32, 0)], ids=["bf16-nt", "bf16-nn", "f32-nt", "f32-nn"])
 def test_more_products_than_a_launch_may_have_tiles_for(dt, k, trans_b):
     """65535 products of one row and 16385 columns, 129 tiles each at the widest: whichever kernel runs needs several launches,
