@@ -920,16 +920,18 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
     const bool nt = !p.trans_a && p.trans_b && p.k % 8 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.stride_a % 8 == 0 &&
                     p.stride_b % 8 == 0 && al16(a) && al16(b) && p.ldc < (1 << 21);
-    // Its wavefronts, one per row of W, each read all of x: with the outputs, m n, grow the reads from L1, and the other
-    // kernels share them (W from HBM, us here and there: bf16 4 x 2048 x 4096 7.8 and 8.6, 6 x 2048 x 4096 9.2 and 8.4, 8 x 768 x
-    // 3072 5.5 and 5.6, 3 x 4096 x 4096 10.8 and 9.8; fp32 4 x 2048 x 2048 7.5 and 8.0, 6 x 2048 x 2048 8.8 and 8.0, 8 x 768 x
-    // 3072 7.2 and 8.0).  With one or two rows W alone counts (1 x 51865 x 4096 70 and 84, fp32 138 and 164), unless rows of W
-    // so short that a wavefront has hardly anything to wait for meet so many of them (bf16 1 x 51865 x 512 16.6 and 12.3,
-    // 2 x 51865 x 1280 29.9 and 26.0, 1 x 51865 x 1280 25.0 and 26.2).  Few bytes in all: fp32 4 x 3072 x 768 4.3 and 5.0.
+    // fp32: always.  A lane adds up every 64th product; the kernels with shared tiles add up an eighth of k, or k-tile after
+    // k-tile, and come out 1.5 to 2.9 times as far from the exact sums, although most products are faster there (W from HBM,
+    // here and there: 8 x 4096 x 4096 26.3 us, error 1.6e-7, and 14.9, 4.1e-7; 8 x 1280 x 1280 6.1, 1.1e-7 and 5.3, 2.4e-7;
+    // 6 x 2048 x 2048 8.3, 1.2e-7 and 7.0, 2.9e-7; 4 x 20096 x 560 15.8, 0.9e-7 and 18.3, 1.7e-7).
+    // 16 bits: its wavefronts, one per row of W, each read all of x.  With the outputs, m n, grow the reads from L1, and the other
+    // kernels share them (W from HBM, us here and there: 4 x 2048 x 4096 7.8 and 8.6, 6 x 2048 x 4096 9.2 and 8.4, 8 x 768 x
+    // 3072 5.5 and 5.6, 3 x 4096 x 4096 10.8 and 9.8).  With one or two rows W alone counts (1 x 51865 x 4096 70 and 84), unless
+    // rows of W so short that a wavefront has hardly anything to wait for meet so many of them (1 x 51865 x 512 16.6 and 12.3,
+    // 2 x 51865 x 1280 29.9 and 26.0, 1 x 51865 x 1280 25.0 and 26.2).
     const int64_t w_elems = p.n * p.k;
-    const bool f32_rows = p.dtype == AXHIP_DTYPE_F32;
-    const bool alone = f32_rows ? f32_shape < 0 && !takes_f32_ring(p, a, b) : !takes_half_kernels(p); // (else the FMA kernel)
-    const bool skinny_pays = p.m <= 8 && (p.m * p.n <= 8192 || (p.m <= 2 && (f32_rows || p.m * p.n <= 64 * p.k)) || (f32_rows && p.m * w_elems <= 10000000) || alone);
+    const bool alone = !takes_half_kernels(p); // (else the FMA kernel)
+    const bool skinny_pays = p.m <= 8 && (f32 || p.m * p.n <= 8192 || (p.m <= 2 && p.m * p.n <= 64 * p.k) || alone);
     const bool f32_nt = p.dtype == AXHIP_DTYPE_F32 && !p.trans_a && p.trans_b && p.k % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0 && al16(a) && al16(b);
     // (the kernel carries leading dimensions as 32-bit element counts)
     const bool ld32 = p.lda < (int64_t(1) << 31) && p.ldb < (int64_t(1) << 31) && p.ldc < (int64_t(1) << 31);

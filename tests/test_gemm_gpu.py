@@ -235,6 +235,18 @@ def test_skinny_sums_of_four_rows_of_w():
     assert r.returncode == 0 and "24 passed" in r.stdout, r.stdout[-3000:]
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 3072, 4096), (5, 4376, 5720), (8, 4728, 1056), (8, 1160, 5120), (4, 20096, 560)])
+def test_fp32_products_of_a_few_rows_keep_short_sums(M, N, K):
+    """A lane's chain is the K / 64 products it owns, then six steps over the lanes.  An addition is off by 0.41 u of its
+    result in the mean square; a chain of n terms adds up n / 2 of the final sum's variance, a step over the lanes all of it:
+    u sqrt(K / 128 + 7) times 0.41, and 0.55 with room for the sample.  (Chains of K / 8: twice to four times as much.)"""
+    r = np.random.default_rng(M * N)
+    x, W = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((N, K)).astype(np.float32)
+    want = x.astype(np.float64) @ W.T.astype(np.float64)
+    got = gh.gemm(x, W, F32, trans_b=True)[0]
+    assert np.linalg.norm(got - want) <= 0.55 * 2.0**-24 * np.sqrt(K / 128 + 7) * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("dt", [F32, BF16, F16], ids=["f32", "bf16", "f16"])
 def test_few_rows_too_far_apart_for_the_tiled_kernels(dt):
     """Four rows of x 2^21 elements apart, past the 32-bit offsets of the 16-bit tile kernels, and more outputs than the kernel
