@@ -462,7 +462,7 @@ enum SdpaMask { MASK_NONE = 0, MASK_BYTES = 1, MASK_BITS = 2 };
 template <bool BF16, int MASK, int NW, int D, int SPLIT = 1, int PAD = 0>
 __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void sdpa_mfma_pipelined_kernel(const SdpaArgs a) {
     static_assert(D == 128 || D == 64, "head sizes with a direct-to-LDS pipeline");
-    static_assert(NW % SPLIT == 0 && SPLIT * D <= 256, "key split: the parts' tile buffers have to fit the LDS");
+    static_assert(SPLIT == 1 || (SPLIT == 2 && NW == 4), "key split: two parts, whose tile buffers fit the LDS");
     constexpr int NWH = NW / SPLIT;       // waves that share a key range
     constexpr int DE = PAD ? PAD : D;     // dims that are computed
     constexpr int KT = (DE + 15) / 16;    // k-steps of the score product
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
             first = max(0, min(__builtin_amdgcn_readfirstlane(lo), beyond - 1));
         }
         const int ntiles_all = max(beyond - first, 1);
-        // key split: `nsteps` is what the work-group's barriers are counted by; the last part may be short or empty
+        // key split: `nsteps` is what the work-group's barriers are counted by; the second part may be short or empty
         const int nsteps = (ntiles_all + SPLIT - 1) / SPLIT;
         const int ntiles = SPLIT == 1 ? ntiles_all : max(0, min(nsteps, ntiles_all - part * nsteps));
         tile0 = first + (SPLIT == 1 ? 0 : min(part * nsteps, ntiles_all - 1));
@@ -840,13 +840,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
                     if (idx == (NP > MAX0 + 8 ? MAX0 + 8 : MAX0 + 7)) mx_next = max_across_halves(max3(max3(pm[0], pm[1], pm[2]), pm[3], NEG_INF_F));
                 }
                 // the tile prefetch is spread over the slots instead of bursting at the step start:
-                // K(j+2) in slots 1, 3, .., V(j+1) in slots 2, 4, .. (the last of a full set in slot 0)
+                // K(j+2) in slots 1, 3, .., V(j+1) in slots 2, 4, ..
                 if (m % 2 == 1 && m / 2 < NLOAD) {
                     if (want_k) load_k1(j + 2, j & 1, m / 2);
                 } else if (m % 2 == 0 && m >= 2 && m / 2 - 1 < NLOAD) {
                     if (want_v) load_v1(j + 1, (j + 1) & 1, m / 2 - 1);
-                } else if (m == 0 && 2 * NLOAD == NS + NP) { // as many loads as half of the slots
-                    if (want_v) load_v1(j + 1, (j + 1) & 1, NLOAD - 1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -895,37 +893,30 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void s
             if (j + 1 < nsteps) step(j + 1, sB, mxB, sA, mxA);
         }
 
-        if constexpr (SPLIT > 1) {
-            // The other parts' states go to the first through LDS (the tile buffers are free: every step ends in a
-            // barrier), value-major so that the 64 lanes of a wave touch consecutive words.  All hold sums of
+        if constexpr (SPLIT == 2) {
+            // The second part's state goes to the first through LDS (the tile buffers are free: every step ends in a
+            // barrier), value-major so that the 64 lanes of a wave touch consecutive words.  Both hold sums of
             // 2^(logit - reference) with a reference of their own: brought to the larger one and added.
-            constexpr int STATE = (DT * 16 + 2) * WAVE; // floats of one wave
-            float *const xch = reinterpret_cast<float *>(lds_all) + wave * STATE + lane;
-            if (part > 0) {
-                float *const mine = xch + (part - 1) * NWH * STATE;
+            float *const xch = reinterpret_cast<float *>(lds_all) + wave * (DT * 16 + 2) * WAVE + lane;
+            if (part == 1) {
     #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
     #pragma unroll
-                    for (int i = 0; i < 16; ++i) mine[(dt * 16 + i) * WAVE] = oacc[dt][i];
-                mine[DT * 16 * WAVE] = m_run;
-                mine[(DT * 16 + 1) * WAVE] = l_run;
+                    for (int i = 0; i < 16; ++i) xch[(dt * 16 + i) * WAVE] = oacc[dt][i];
+                xch[DT * 16 * WAVE] = m_run;
+                xch[(DT * 16 + 1) * WAVE] = l_run;
             }
             __syncthreads();
-            if (part > 0) return;
+            if (part == 1) return;
+            const float m_other = xch[DT * 16 * WAVE], l_other = xch[(DT * 16 + 1) * WAVE];
+            const float m_new = __builtin_elementwise_maximum(m_run, m_other);
+            const float a_mine = m_run == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+            const float a_other = m_other == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_other - m_new);
+            l_run = l_run * a_mine + l_other * a_other;
     #pragma unroll
-            for (int other = 0; other < SPLIT - 1; ++other) {
-                const float *const from = xch + other * NWH * STATE;
-                const float m_other = from[DT * 16 * WAVE], l_other = from[(DT * 16 + 1) * WAVE];
-                const float m_new = __builtin_elementwise_maximum(m_run, m_other);
-                const float a_mine = m_run == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-                const float a_other = m_other == NEG_INF_F ? 0.0f : __builtin_amdgcn_exp2f(m_other - m_new);
-                m_run = m_new;
-                l_run = l_run * a_mine + l_other * a_other;
+            for (int dt = 0; dt < DT; ++dt)
     #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-    #pragma unroll
-                    for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a_mine + from[(dt * 16 + i) * WAVE] * a_other;
-            }
+                for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a_mine + xch[(dt * 16 + i) * WAVE] * a_other;
         }
 
         const float l_tot = across32(l_run, lanes_add);
