@@ -1883,18 +1883,21 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
     m.planes_b = p.mask_strides[0] == 0 ? 1 : p.batch;
     m.planes_h = p.mask_strides[1] == 0 ? 1 : p.heads;
     // Packing is a launch, 4.7 us, and one more read of the mask, which rows off the 16-byte grid slow down; it saves time per
-    // score, and tiles that nobody sees (510 calls; us from bytes and from bits, keys masked at random / whole tails of them):
-    //  * 24 M scores, half as many counted under a causal mask: 64 heads of 512 x 64, 4 masks 16.1 and 20.1 / 15.6 and 18.2;
-    //    of 704 32.6 and 28.5 / 32.6 and 26.3; causal 48 of 1024 32.6 and 29.8 / 32.6 and 27.2, 36 of 832 18.3 and 20.6 / 18.3 and 19.3.
-    //  * a mask that two slices share, six where rows are unaligned: 32 heads of 2048 x 64, 16 masks 79.7 and 67.1; of
-    //    1501 x 1501 54.0 and 56.3, 4 masks 54.1 and 50.1.  One mask each: 64 heads of 1024 x 64 44.4 and 48.9, of 1023 41.5 and 67.7.
-    //  * else aligned rows that are few (16 heads of 64 x 65536, one mask each, 964 and 826; 65535 893 and 954), since the keys
-    //    are walked by few work-groups then, or very many (128 of 2048 x 64 321 and 324 / 321 and 277).
-    const int64_t rows = static_cast<int64_t>(m.planes_b) * m.planes_h * p.seq_q, scores = static_cast<int64_t>(p.batch) * p.heads * p.seq_q * p.seq_kv;
-    const int64_t computed = p.is_causal ? scores / 2 : scores;
-    const bool aligned = p.seq_kv % 16 == 0;
-    if (computed < (int64_t(24) << 20)) return m;
-    if ((aligned ? 2 : 6) * rows * p.seq_kv > scores && !(aligned && (rows <= 4096 || computed >= (int64_t(256) << 20)))) return m;
+    // score, and tiles that nobody sees (550 calls; us from bytes and from bits, keys masked at random / whole tails of them).  The scores
+    // of a causal problem are those that are computed, key j for query i >= j; the whole mask is packed all the same.
+    //  * 24 M scores: 64 heads of 512 x 64, 4 masks 16.1 and 20.1 / 15.6 and 18.2; of 704 32.6 and 28.5 / 32.6 and 26.3; causal 48 of
+    //    1024 32.6 and 29.8 / 32.6 and 27.2, 36 of 832 18.3 and 20.6 / 18.3 and 19.3, 16 of 64 queries and 65536 keys 6.7 and 82.
+    //  * a mask that two slices share, six where rows are unaligned: 32 heads of 2048 x 64, 16 masks 79.7 and 67.1 (causal 61.9 and
+    //    55.8 / 62.1 and 50.1); of 1501 x 1501 54.0 and 56.3, 4 masks 54.1 and 50.1.  One mask each: 64 heads of 1024 x 64 44.4
+    //    and 48.9, of 1023 41.5 and 67.7; causal 128 of 2048 x 64 189 and 245 / 188 and 230, 32 of 4096 x 128 221 and 296 / 219 and 283.
+    //  * else, not causal, aligned rows that are few (16 heads of 64 x 65536, one mask each, 964 and 826; 65535 893 and 954), since the
+    //    keys are walked by few work-groups then, or very many (128 of 2048 x 64 321 and 324 / 321 and 284, x 128 406 and 421 / 400 and 364).
+    const int64_t slices = static_cast<int64_t>(p.batch) * p.heads, sq = p.seq_q, skv = p.seq_kv, both = std::min(sq, skv);
+    const int64_t mask_bytes = static_cast<int64_t>(m.planes_b) * m.planes_h * sq * skv;
+    const int64_t scores = slices * (p.is_causal ? both * (both + 1) / 2 + (sq - both) * skv : sq * skv);
+    const bool aligned = skv % 16 == 0, shared = mask_bytes * (aligned ? 1 : 3) <= (p.is_causal ? scores : scores / 2);
+    if (scores < (int64_t(24) << 20)) return m;
+    if (!shared && !(aligned && !p.is_causal && (mask_bytes <= 4096 * skv || scores >= (int64_t(256) << 20)))) return m;
     m.tiles = (p.seq_kv + BN - 1) / BN;
     m.nb32 = (p.seq_q + 31) / 32;
     const int64_t planes = static_cast<int64_t>(m.planes_b) * m.planes_h;

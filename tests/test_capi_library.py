@@ -120,10 +120,12 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     (4, 16, 704, 704, 0, "batch", True), (4, 16, 512, 512, 0, "batch", False), (4, 12, 1024, 1024, 1, "batch", True), (4, 11, 1024, 1024, 1, "batch", False),
     (4, 16, 1024, 1024, 0, "own", False), (4, 16, 1023, 1023, 0, "own", False), (4, 32, 2048, 2048, 0, "own", True), (4, 32, 2047, 2047, 0, "own", False),
     (16, 2, 2048, 2048, 0, "batch", True), (16, 2, 1501, 1501, 0, "batch", False), (4, 8, 1501, 1501, 0, "batch", True),
-    (1, 16, 64, 65536, 0, "own", True), (1, 16, 64, 65535, 0, "own", False), (1, 16, 63, 65536, 0, "one", False), (1, 8, 4096, 4096, 0, "one", True)])
+    (1, 16, 64, 65536, 0, "own", True), (1, 16, 64, 65535, 0, "own", False), (1, 16, 63, 65536, 0, "one", False), (1, 8, 4096, 4096, 0, "one", True),
+    (4, 32, 2048, 2048, 1, "own", False), (1, 32, 4096, 4096, 1, "own", False), (16, 2, 2048, 2048, 1, "batch", True), (1, 16, 64, 65536, 1, "own", False),
+    (2, 8, 512, 8192, 1, "batch", False), (2, 8, 8192, 512, 1, "batch", True), (32, 3, 1501, 1501, 1, "batch", False), (16, 6, 1501, 1501, 1, "batch", True)])
 def test_memory_for_a_packed_mask_is_asked_for_where_packing_pays(batch, heads, seq_q, seq_kv, causal, planes, packed):
-    """What packing a mask costs is by its bytes, what it saves by the scores: by how many slices share the mask, and whether
-    its rows are aligned."""
+    """What packing a mask costs is by its bytes, what it saves by the scores that are computed: by how many slices share the
+    mask, whether its rows are aligned, and how much of it a causal mask leaves."""
     lib = capi.lib()
     p = capi.SdpaParams()
     p.dtype, p.batch, p.heads, p.seq_q, p.seq_kv, p.head_dim, p.is_causal = capi.DTYPE_BF16, batch, heads, seq_q, seq_kv, 64, causal

@@ -523,10 +523,10 @@ def sdpa_ws(q, k, v, dt, causal, mask=None, mask_strides=(0, 0), mask_offset=0, 
 
 @pytest.mark.parametrize("dt,D,B,H,S,Skv,causal,kind,offset,schedule", [
     (BF16, 64, 4, 96, 257, 259, False, "tails", 1, b"pipelined4"), (F16, 128, 4, 8, 128, 6160, False, "heads", 3, b"key_split"),
-    (BF16, 80, 4, 96, 258, 513, True, "tails", 0, b"pipelined4"), (BF16, 40, 4, 160, 256, 320, True, "random", 2, b"pipelined4"),
+    (BF16, 80, 4, 96, 386, 513, True, "tails", 0, b"pipelined4"), (BF16, 40, 4, 160, 288, 320, True, "random", 2, b"pipelined4"),
     (F16, 64, 4, 96, 64, 1025, False, "none seen", 0, b"pipelined4"), (BF16, 128, 4, 80, 129, 640, False, "first keys", 1, b"pipelined8")])
 def test_masks_packed_to_bits(dt, D, B, H, S, Skv, causal, kind, offset, schedule):
-    """From 24 M scores on (48 M under a causal mask) an explicit mask that slices share, or that has few rows, is packed to
+    """From 24 M scores on (of which a causal mask leaves about half) an explicit mask that slices share, or that has few rows, is packed to
     bits first, if the caller brings the memory: rows that start
     anywhere, ragged last tiles, masks per batch, per (batch, head) and shared, leading and trailing tiles that no row
     sees, rows (and whole slices) that see nothing.  Against float64 on some slices, and against the bytes read in
@@ -589,8 +589,8 @@ def test_work_groups_by_the_number_of_blocks(dt, B, H, Sq, Skv, D, causal, sched
     (BF16, 64, 1, 3, 70, 131, False, (1, 1), False, b"key_split"), (F16, 128, 2, 4, 200, 449, True, (2, 1), False, b"key_split"),
     (BF16, 64, 8, 33, 100, 192, False, (8, 33), False, b"pipelined4"), (F16, 80, 8, 17, 257, 131, True, (1, 1), False, b"pipelined4"),
     (BF16, 128, 7, 6, 900, 199, False, (7, 1), False, b"pipelined8"), (F16, 40, 7, 6, 900, 672, False, (1, 1), True, b"pipelined8"),
-    (BF16, 64, 4, 96, 257, 259, False, (4, 1), True, b"pipelined4"), (BF16, 128, 4, 96, 257, 513, True, (1, 1), True, b"pipelined4"),
-    (F16, 64, 1, 8, 2048, 2048, False, (1, 1), True, b"key_split"), (BF16, 80, 1, 8, 2048, 3088, True, (1, 1), True, b"key_split"),
+    (BF16, 64, 4, 96, 257, 259, False, (4, 1), True, b"pipelined4"), (BF16, 128, 4, 96, 385, 513, True, (1, 1), True, b"pipelined4"),
+    (F16, 64, 1, 8, 2048, 2048, False, (1, 1), True, b"key_split"), (BF16, 80, 1, 5, 3200, 3088, True, (1, 1), True, b"key_split"),
     (BF16, 32, 2, 3, 130, 131, False, (2, 1), False, b"register_staged"), (F16, 256, 1, 3, 130, 131, False, (1, 1), False, b"register_staged"),
     (F32, 64, 1, 3, 130, 131, False, (1, 1), False, b"direct"), (F32, 128, 4, 16, 130, 131, True, (4, 1), False, b"mfma_f32")])
 def test_masked_keys_may_hold_anything(dt, D, B, H, S, Skv, causal, planes, give, schedule):
@@ -622,7 +622,7 @@ def test_masked_keys_may_hold_anything(dt, D, B, H, S, Skv, causal, planes, give
 @pytest.mark.parametrize("dt,D,B,H,S,Skv,causal,planes,offset", [
     (BF16, 64, 1, 8, 2048, 2048, False, (1, 1), 0), (F16, 64, 2, 4, 2000, 2049, False, (1, 1), 1), (BF16, 128, 1, 8, 2048, 2048, False, (1, 1), 3),
     (F16, 80, 1, 8, 2048, 1539, False, (1, 1), 0), (BF16, 40, 1, 8, 1985, 2112, False, (1, 1), 2), (BF16, 64, 3, 4, 2111, 2012, True, (1, 1), 0),
-    (F16, 128, 1, 8, 2048, 3088, True, (1, 1), 1), (BF16, 72, 2, 4, 2000, 3200, True, (2, 1), 0)])
+    (F16, 128, 1, 5, 3200, 3088, True, (1, 1), 1), (BF16, 72, 2, 2, 4000, 3200, True, (2, 1), 0)])
 def test_packed_masks_with_the_keys_split(dt, D, B, H, S, Skv, causal, planes, offset):
     """Few slices under a packed mask: the two halves of a work-group share the key tiles between the first and the last one
     that some row of its block sees -- none, one, two, .. five of them here, so that a half's share is short or empty."""
