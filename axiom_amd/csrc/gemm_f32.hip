@@ -177,35 +177,42 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
         // columns col .. col + 3.  (NN: a lane whose columns were moved left to end with the rows owns those at and
         // behind the place it was moved from)
         const int col = n0 + (NN ? 4 * NJ * xg + 4 * f : 16 * f + 4 * xg);
-        if (col + 4 + (NN ? NJ : 0) <= g.N) { // all four, and none of them moved
-            const int64_t to = static_cast<int64_t>(m) * g.ldc + col;
-            auto add4 = [&](const float *p) {
-                const Floats<4> t = *reinterpret_cast<const Floats<4> *>(p);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += t.v[e];
-            };
-            if (bias) add4(bias + col);
-            if (res) add4(res + to);
-            Floats<4> y;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) y.v[e] = v[e];
-            gemm_epilogue_all(g.epilogue, y.v);
-            *reinterpret_cast<Floats<4> *>(C + to) = y;
-            continue;
-        }
+        const bool whole = col + 4 <= g.N; // all four, and none of them moved (col and n0 are multiples of four, and NJ divides four)
+        int at[4];                         // (-1: not this lane's)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            int at = col + e;
+            at[e] = col + e;
             if constexpr (NN) {
-                const int first = at / NJ * NJ; // (n0 is a multiple of NJ)
-                at = min(first, g.N - NJ) + (at - first);
-                if (at < first) continue;
+                const int first = at[e] / NJ * NJ;
+                at[e] = min(first, g.N - NJ) + (at[e] - first);
+                if (at[e] < first) at[e] = -1;
             }
-            if (at >= g.N) continue;
-            float y = v[e] + (bias ? bias[at] : 0.0f);
-            const int64_t to = static_cast<int64_t>(m) * g.ldc + at;
-            if (res) y += res[to];
-            C[to] = gemm_epilogue(g.epilogue, y);
+            if (at[e] >= g.N) at[e] = -1;
+        }
+        // one epilogue for both kinds of lanes: with one each, which a wavefront at the end of the rows goes through both of,
+        // a b 2496 x 128 x 64 took 5.1 us instead of 4.5
+        float y[4] = {v[0], v[1], v[2], v[3]};
+        auto add4 = [&](const float *row) {
+            if (whole) {
+                const Floats<4> t = *reinterpret_cast<const Floats<4> *>(row + col);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] += t.v[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (at[e] >= 0) y[e] += row[at[e]];
+            }
+        };
+        const int64_t row0 = static_cast<int64_t>(m) * g.ldc;
+        if (bias) add4(bias);
+        if (res) add4(res + row0);
+        gemm_epilogue_all(g.epilogue, y);
+        if (whole) {
+            *reinterpret_cast<Floats<4> *>(C + row0 + col) = Floats<4>{{y[0], y[1], y[2], y[3]}};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (at[e] >= 0) C[row0 + at[e]] = y[e];
         }
     }
 }
