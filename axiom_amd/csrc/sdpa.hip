@@ -1901,7 +1901,6 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
     m.tiles = (p.seq_kv + BN - 1) / BN;
     m.nb32 = (p.seq_q + 31) / 32;
     const int64_t planes = static_cast<int64_t>(m.planes_b) * m.planes_h;
-    if (!launch_fits(planes * m.nb32, 256)) return m; // (its blocks have a quarter of the attention kernel's rows)
     if (!launch_fits(planes * m.nb32, 256)) return m;
     m.on = true;
     m.bits_bytes = CallScratch::rounded(static_cast<size_t>(planes) * m.tiles * p.seq_q * 8);

@@ -137,16 +137,3 @@ def test_memory_for_a_packed_mask_is_asked_for_where_packing_pays(batch, heads, 
     need = lib.axhip_sdpa_workspace_bytes(C.byref(p), 1)
     assert (need > 0) == packed
     assert not packed or masks * plane // 8 <= need <= masks * seq_q * ((seq_kv + 63) // 64) * 8 + masks * (seq_q // 32 + 1) * 8 + 512
-
-
-@pytest.mark.parametrize("slices,packed", [(1 << 15, True), ((1 << 16) - 1, True), (1 << 16, False), ((1 << 18) - 1, False)])
-def test_a_mask_is_packed_only_where_one_launch_packs_it(slices, packed):
-    """256 blocks of 32 rows a slice, of 256 threads each: 2^32 threads and more are no launch, while the attention kernel's 64 blocks
-    of 128 rows still are one.  (8192 rows of 16 keys, a mask each: 2^32 scores and more.)"""
-    lib = capi.lib()
-    p = capi.SdpaParams()
-    p.dtype, p.batch, p.heads, p.seq_q, p.seq_kv, p.head_dim = capi.DTYPE_BF16, slices, 1, 8192, 16, 64
-    p.q_strides[:] = p.o_strides[:] = (8192 * 64, 8192 * 64, 64)
-    p.k_strides[:] = p.v_strides[:] = (16 * 64, 16 * 64, 64)
-    p.mask_strides[:] = (8192 * 16, 8192 * 16)
-    assert (lib.axhip_sdpa_workspace_bytes(C.byref(p), 1) > 0) == packed
