@@ -369,8 +369,8 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // issue of its wavefront for longer than an MFMA takes, wherever it stands: 64 x 1536 x 4096 on 64 x 64 tiles 84 us, with
 // loaders 76), the fragments of the next eight k are read under the MFMAs of these, the barrier of a k-tile comes before its
 // last steps (by then every wavefront has read the whole tile), and behind it the reads turn to the next tile.  What is
-// left, one k-tile of 64 x 64: 1024 cycles of MFMAs in 1380.  Two wavefronts a SIMD with half of each k-tile, or two sums
-// in turn, were no faster.  The values of a finished block then take bias, residual and activation together: with a branch on the activation for each,
+// left, one k-tile of 64 x 64, one work-group a CU: 1024 cycles of MFMAs in 1310, and 10.9 k cycles of a launch outside of the k
+// loop (counted for 1024 x 1024 over 1024, 2048 and 4096).  Two wavefronts a SIMD with half of each k-tile were no faster.  The values of a finished block then take bias, residual and activation together: with a branch on the activation for each,
 // 60 KB of code that every CU read anew, 4096 x 4096 x 512 + GELU took 228 us instead of 176 and 1024^3 24.5 instead of 22.
 // 1024^3: 26.3 -> 22 us, 2048^3 155 -> 134.
 // Rows may start anywhere: the loads need 4-byte alignment.  The chunk that K ends in is fetched as the four floats that
@@ -474,8 +474,8 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) f_off[ks] = l32 * BIG_ROWB + (((2 * ks + g2) ^ ((l32 >> 1) & 7)) * 16);
 
-    // The sums of a k-tile are added to those of all before: chains of 32 fp32 additions, however large K (2048^3, one
-    // chain: 8.1e-7 off the exact result, now 1.8e-7; no more than the kernels without shared tiles at any K).  TURNS:
+    // The sums of a k-tile are added to those of all before: chains of 32 fp32 additions, then one of K / 32, in place of one
+    // of K (2048^3, one chain: 8.1e-7 off the exact result, now 1.8e-7).  TURNS:
     // two accumulators in turn, one is added up under the next k-tile's MFMAs.
     constexpr int TURN = TURNS ? 1 : 0;
     float16_t acc[1 + TURN][MI][NJ], sum[MI][NJ];
@@ -773,7 +773,7 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 // products of m 9 .. 8192, n 64 .. 4096, k 64 .. 4096 (mean error 5 - 8 %); on average the one picked is
 // 2 % slower than the fastest, and 2.3 times as fast as the ring and FMA kernels, which had these products to themselves:
 // 99 x 1024 x 5120 104 -> 18 us, 186 x 640 x 958 35 -> 8, 48 x 384 x 2048 77 -> 6.3.  Large products with both operands
-// along k stay on the ring: 2048^3 157 us against 188.
+// along k stay on the ring: 2048^3 134 us against 188.
 struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
     {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f},
@@ -848,7 +848,8 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     if (p.m == 0 || p.n == 0 || p.batch == 0) return AXHIP_OK;
     AXHIP_REQUIRE(a && b && c, AXHIP_ERR_INVALID_ARG, "axhip_gemm: NULL matrix");
     if (p.batch >= 65536) {
-        // the batch index is a grid dimension (at most 65 535): a larger batch runs as consecutive launches
+        // larger batches run as consecutive calls: the batch is a grid dimension of the FMA kernel (at most 65 535), and a
+        // workspace has to hold the repacked operands of one call only
         const int64_t es = p.dtype == AXHIP_DTYPE_F32 ? 4 : 2;
         for (int64_t b0 = 0; b0 < p.batch; b0 += 65535) {
             AxhipGemmParams part = p;
@@ -864,9 +865,9 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     if (rc) return rc;
     hipStream_t s = resolve_stream(stream);
 
-    // The matrix kernels read A along k, the fp32 ring kernel in 16-byte vectors.  An operand stored the other way (A as
-    // [k, m]; B as [k, n] where its rows are no whole vectors), or a reduction length that is not a whole
-    // number of vectors, leaves only the FMA kernel below, a hundred times slower on a large product.  Such a product
+    // The matrix kernels read A along k, rows that start anywhere, and B either way (takes_half_kernels and takes_f32_ring say
+    // where they do not).  An operand they do not take, A as [k, m] above all, leaves only the FMA kernel below, a hundred
+    // times slower on a large product.  Such a product
     // is repacked first, into stream-ordered temporary memory (freed in stream order behind the product): the operand
     // that lies the other way is transposed; an unaligned k is zero-padded to the next multiple of 64 in both operands.
     const Repack rp = repack_plan(p);
@@ -960,7 +961,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, s);
         if (rc) return rc;
     } else if (f32 && takes_f32_ring(p, a, b)) {
-        // fp32 x W^T on the fp32 MFMA
+        // the fp32 MFMA, b along k or [k, n]
         auto launch = [&](auto kernel, int tm_rows, int tn_cols, size_t lds_bytes) -> int {
             static std::mutex mu;
             static std::set<const void *> configured;

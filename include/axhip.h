@@ -120,8 +120,9 @@ int axhip_sdpa_fwd(const void *q, const void *k, const void *v, void *o,
  * problem that needs none; has_mask: whether a mask will be passed.  Steps of
  * fewer than 8 M key elements (slices x keys x dims) only run faster with it:
  * without one, or with less, they run undivided and allocate nothing.  So do
- * 16-bit problems of 24 M scores and more under a mask that (batch, head)
- * slices share, which take it for the mask as bits. */
+ * 16-bit problems of 24 M scores and more under a mask whose packing to bits
+ * pays (one that (batch, head) slices share; one per slice of few or very many
+ * rows), which take it for the mask as bits. */
 size_t axhip_sdpa_workspace_bytes(const AxhipSdpaParams *params_host, int has_mask);
 int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o,
                       const uint8_t *mask, const AxhipSdpaParams *params_host,
