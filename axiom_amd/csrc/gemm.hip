@@ -1,13 +1,14 @@
 // C = op(A) op(B) (+ bias) (+ residual), activation epilogue: the dispatch, and
 //
 //   gemm_mfma_nt_256_kernel    large bf16 / f16 x W^T: 256 x 256 tiles
-//   gemm_mfma_f32_ring_kernel  large fp32 products, b along k or [k, n], on the fp32 matrix instruction
+//   gemm_mfma_f32_ring_kernel  large fp32 products, b along k or [k, n], by products of bf16 parts or on the fp32 matrix instruction
 //   gemm_generic_kernel        any dtype / any transpose combination, 16x16 LDS tiles, fp32 FMA
 //
 // The other 16-bit kernels are in gemm_tile_*.hip (middle-sized products), gemm_small.hip (few rows or few output
 // tiles) and gemm_skinny.hip (at most eight rows), the smaller fp32 products in gemm_f32.hip.
 #include "common.hpp"
 #include "gemm_f32.hpp"
+#include "gemm_f32_split.hpp"
 #include "gemm_small.hpp"
 #include "gemm_skinny.hpp"
 
@@ -368,25 +369,249 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // wavefront, of which a SIMD has one: four more wavefronts, one per SIMD, issue the loads (a direct-to-LDS load holds the
 // issue of its wavefront for longer than an MFMA takes, wherever it stands: 64 x 1536 x 4096 on 64 x 64 tiles 84 us, with
 // loaders 76), the fragments of the next eight k are read under the MFMAs of these, the barrier of a k-tile comes before its
-// last steps (by then every wavefront has read the whole tile), and behind it the reads turn to the next tile.  What is
-// left, one k-tile of 64 x 64, one work-group a CU: 1024 cycles of MFMAs in 1310, and 10.9 k cycles of a launch outside of the k
-// loop (counted for 1024 x 1024 over 1024, 2048 and 4096).  Two wavefronts a SIMD with half of each k-tile were no faster.  The values of a finished block then take bias, residual and activation together: with a branch on the activation for each,
-// 60 KB of code that every CU read anew, 4096 x 4096 x 512 + GELU took 228 us instead of 176 and 1024^3 24.5 instead of 22.
-// 1024^3: 26.3 -> 22 us, 2048^3 155 -> 134.
+// last steps (by then every wavefront has read the whole tile), and behind it the reads turn to the next tile.  One k-tile of
+// 64 x 64, one work-group a CU: 1024 cycles of MFMAs in 1310.  The values of a finished block then take bias, residual and
+// activation together: with a branch on the activation for each, 60 KB of code that every CU read anew, 4096 x 4096 x 512 + GELU
+// took 228 us instead of 176.
+// Products of parts (SplitRing) take its place wherever there is k enough; this form stays for short k, of whose tiles of
+// 64 x 64 three work-groups share a CU (8 x (2939 x 704 x 66) 44 us against 54), and for tiles whose parts have no finite sums.
 // Rows may start anywhere: the loads need 4-byte alignment.  The chunk that K ends in is fetched as the four floats that
 // end with the row and shifted into place in LDS by the lane that loaded it; chunks behind it, and k-tiles past the last,
 // are sent out of the descriptor's range and arrive as zeros.  NN rows that are no whole chunks: the last column tile is
 // moved left to end with them (N >= TNR); the columns it shares with its neighbour are the neighbour's to store.
-template <int TM, int TNR, int S, bool NN, bool TURNS>
-__global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
+
+// The same tiles by products of bf16 parts (gemm_f32_split.hpp).  Splitting an element takes seven VALU operations, of which about
+// five fit beside a 32-cycle MFMA of another wavefront, so each is split once for the whole work-group: the loading wavefronts keep
+// DEPTH k-tiles on their way in registers, split one and write its parts to LDS, in the order in which fragments are read: a block of
+// 32 rows, 8 k at a time, is 512 bytes, 16 a row (the row XOR-ed so that what 32 lanes write at a time meets all banks).
+// The multiplying ones, one per SIMD, hold all fragments of 32 k and refill them under the MFMAs of blocks that need them no
+// more.  Barrier kt: k-tile kt is in LDS and k-tile kt - 1 has been read.
+// What bounds it: with few work-groups the splitting (a k-tile of 128 x 128 x 32 on 64 CUs 2470 cycles, 2040 without MFMAs,
+// of which the MFMAs are 1536), with all CUs at work the power limit (3400 of the same cycles).  64 x 64 has two loading wavefronts per
+// SIMD for that reason (1024^3 22.5 us with one, 19.4 with two), and 64 k at a time for half the barriers.  v_mfma_f32_16x16x32, which leaves
+// less room beside it, took 3 % less on full chips and 10 % more on others.
+// 1024^3 22.2 -> 19.3 us, 2048^3 135 -> 97, 4096 x 2000 x 1000 138 -> 105.
+template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: floats per k-tile; LW: loading wavefronts
+    static constexpr int MI = TM / 64, NJ = TNR / 64, DEPTH = KF == 32 || LW == 8 ? 3 : 2;
+    static constexpr int CHUNKS = KF / 4, ROWS = WAVE / CHUNKS * LW;      // 16-byte chunks of a row along k, rows that the loading wavefronts fetch at a time
+    static constexpr int NLA = TM / ROWS, NLB = TNR / ROWS;               // loads of a lane per k-tile
+    static constexpr int PLANE_A = TM * KF * 2, PLANE_B = TNR * KF * 2, STAGEB = 3 * (PLANE_A + PLANE_B);
+
+    // where the 8 k of chunk pair kc of row r of an operand's plane lie
+    static __device__ __forceinline__ int at(int r, int kc) { return (r / 32) * (KF * 64) + kc * 512 + (((r % 32) ^ (((r / 16) & 3) | ((kc & 3) << 2)) ^ (kc / 4 * 2)) * 16); }
+
+    static __device__ __forceinline__ void load(const GemmArgs &g, const float *A, const float *B, int rows_a, int rows_b, unsigned char *lds, int wave, int lane) {
+        const int arow = static_cast<int>(g.a_rs) * 4, brow = static_cast<int>(NN ? g.b_rs : g.b_cs) * 4;
+        const int K = static_cast<int>(g.K), nk = (K + KF - 1) / KF;
+        const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, (rows_a - 1) * arow + K * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), 0, NN ? (K - 1) * brow + rows_b * 4 : (rows_b - 1) * brow + K * 4, 0x00020000);
+        constexpr uint32_t OUT_OF_RANGE = 0x7FFFFFF0u;
+        // rows along k: load n is row ROWS n + r0, floats k0 .. + 3 of the k-tile
+        const int r0 = WAVE / CHUNKS * wave + lane / CHUNKS, k0 = 4 * (lane % CHUNKS);
+        // b as [k, n]: load n is row bk + n, columns bn .. + 3 (of every 32 lanes 16 lie side by side and 16 on the next rows: what
+        // they write then meets all banks)
+        constexpr int WIDE = TNR / 64; // runs of 16 lanes to a row
+        const int run = wave * 4 + lane / 16, bk = (run / (2 * WIDE) * 2 + run % 2) * NLB, bn = (run / 2 % WIDE * 16 + lane % 16) * 4;
+        uint4_t regs[DEPTH][NLA + NLB];
+        auto fetch = [&](int set, int kt, int n) __attribute__((always_inline)) { // n: of a, then of b
+            const int k = kt * KF + k0;
+            const uint32_t along = k < K ? static_cast<uint32_t>(min(k, K - 4)) * 4u : OUT_OF_RANGE;
+            if (n < NLA) {
+                regs[set][n] = __builtin_amdgcn_raw_buffer_load_b128(ar, static_cast<uint32_t>((ROWS * n + r0) * arow) + along, 0, 0);
+            } else if constexpr (NN) {
+                const int row = kt * KF + bk + n - NLA;
+                regs[set][n] = __builtin_amdgcn_raw_buffer_load_b128(br, row < K && bn < rows_b ? static_cast<uint32_t>(row * brow + bn * 4) : OUT_OF_RANGE, 0, 0);
+            } else {
+                regs[set][n] = __builtin_amdgcn_raw_buffer_load_b128(br, static_cast<uint32_t>((ROWS * (n - NLA) + r0) * brow) + along, 0, 0);
+            }
+        };
+        // k-tile kt -> LDS; `behind(n)` once the registers of load n are free: the loads of a later k-tile stand between the splits of
+        // this one (side by side they wait for each other, 16 cycles of the CU's address path each)
+        auto write = [&](int set, int kt, auto behind) __attribute__((always_inline)) {
+            if (K % 4 != 0 && kt == nk - 1) {
+                const int drop = kt * KF + k0 + 4 - K; // floats in front of the chunk that K ends in
+                if (drop > 0 && drop < 4) {
+#pragma unroll
+                    for (int n = 0; n < NLA + (NN ? 0 : NLB); ++n) regs[set][n] = __builtin_bit_cast(uint4_t, __builtin_bit_cast(unsigned __int128, regs[set][n]) >> (32 * drop));
+                }
+            }
+            unsigned char *stage = lds + (kt & 1) * STAGEB;
+            if constexpr (NN) {
+                float4_t v[NLB];
+#pragma unroll
+                for (int n = 0; n < NLB; ++n) v[n] = __builtin_bit_cast(float4_t, regs[set][NLA + n]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t w[NLB / 2][3];
+#pragma unroll
+                    for (int n = 0; n < NLB / 2; ++n) split_pair(v[2 * n][j], v[2 * n + 1][j], w[n]);
+                    unsigned char *to = stage + 3 * PLANE_A + at(bn + j, bk / 8) + (bk % 8) * 2;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        if constexpr (NLB == 8) *reinterpret_cast<uint4_t *>(to + q * PLANE_B) = uint4_t{w[0][q], w[1][q], w[NLB / 2 - 2][q], w[NLB / 2 - 1][q]};
+                        else if constexpr (NLB == 4) *reinterpret_cast<uint2_t *>(to + q * PLANE_B) = uint2_t{w[0][q], w[NLB / 2 - 1][q]};
+                        else *reinterpret_cast<uint32_t *>(to + q * PLANE_B) = w[0][q];
+                    }
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < NLA + (NN ? 0 : NLB); ++n) {
+                const bool a = n < NLA;
+                const float4_t v = __builtin_bit_cast(float4_t, regs[set][n]);
+                uint32_t lo[3], hi[3];
+                split_pair(v[0], v[1], lo);
+                split_pair(v[2], v[3], hi);
+                unsigned char *to = stage + (a ? 0 : 3 * PLANE_A) + at(ROWS * (a ? n : n - NLA) + r0, k0 / 8) + (k0 / 4 & 1) * 8;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2_t *>(to + q * (a ? PLANE_A : PLANE_B)) = uint2_t{lo[q], hi[q]};
+                __builtin_amdgcn_sched_barrier(0);
+                behind(n);
+                if constexpr (NN) {
+#pragma unroll
+                    for (int x = n * NLB / NLA; x < (n + 1) * NLB / NLA; ++x) behind(NLA + x);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+#pragma unroll
+            for (int n = 0; n < NLA + NLB; ++n) fetch(d, d, n);
+        int kt = 0;
+        for (; kt + DEPTH <= nk; kt += DEPTH) { // (no branch inside: the compiler would wait for every load in flight where the paths meet)
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                write(d, kt + d, [&](int n) __attribute__((always_inline)) { fetch(d, kt + d + DEPTH, n); });
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < DEPTH - 1; ++d) {
+            if (kt + d < nk) {
+                write(d, kt + d, [](int) {});
+                __syncthreads();
+            }
+        }
+        __syncthreads(); // barrier nk
+    }
+
+    static __device__ __forceinline__ float16_t mfma(const uint4_t &a, const uint4_t &b, const float16_t &sum) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), sum, 0, 0, 0);
+    }
+
+    // -> sum[i][j]: as the fp32 MFMAs leave them, times SPLIT_SCALE^2
+    static __device__ __forceinline__ void multiply(int K, const unsigned char *lds, int wm, int wn, int lane, float16_t (&sum)[MI][NJ]) {
+        const int nk = (K + KF - 1) / KF, l32 = lane % 32, g2 = lane / 32;
+        // KF = 32, four blocks: the fragments of one are dead long before the next k-tile needs them.  KF = 64: the halves of a k-tile in turn
+        constexpr int SLOTS = KF / 32, BLOCKS = MI * NJ;
+        static_assert(SLOTS == 1 ? MI == 2 && NJ == 2 : MI == 1, "blocks");
+        uint4_t fa[SLOTS][MI][2][3], fb[SLOTS][NJ][2][3];
+        int a_off[SLOTS][MI][2], b_off[SLOTS][NJ][2];
+#pragma unroll
+        for (int h = 0; h < SLOTS; ++h)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) a_off[h][i][ks] = at(wm + 32 * i + l32, 4 * h + 2 * ks + g2);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) b_off[h][j][ks] = 3 * PLANE_A + at(wn + 32 * j + l32, 4 * h + 2 * ks + g2);
+            }
+        auto read_a = [&](int h, const unsigned char *stage, int i, int n) __attribute__((always_inline)) { // n: 3 ks + part
+            fa[h][i][n / 3][n % 3] = *reinterpret_cast<const uint4_t *>(stage + a_off[h][i][n / 3] + n % 3 * PLANE_A);
+        };
+        auto read_b = [&](int h, const unsigned char *stage, int j, int n) __attribute__((always_inline)) {
+            fb[h][j][n / 3][n % 3] = *reinterpret_cast<const uint4_t *>(stage + b_off[h][j][n / 3] + n % 3 * PLANE_B);
+        };
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) sum[i][j] = float16_t{};
+        float16_t t[2] = {float16_t{}, float16_t{}};
+        // block (i, j) of 32 k: twelve MFMAs, behind MFMA x what `between` does; the block before is added to its sum meanwhile
+        auto block = [&](int h, int i, int j, float16_t &before, auto between) __attribute__((always_inline)) {
+            const int turn = BLOCKS > 1 ? (i * NJ + j) & 1 : h;
+#pragma unroll
+            for (int x = 0; x < 12; ++x) {
+                const int n = x / 2, ks = x % 2;
+                t[turn] = mfma(fa[h][i][ks][SPLIT_A[n]], fb[h][j][ks][SPLIT_B[n]], x == 0 ? float16_t{} : t[turn]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (x >= 3 && x < 11) {
+#pragma unroll
+                    for (int e = 2 * (x - 3); e < 2 * (x - 3) + 2; ++e) before[e] += t[turn ^ 1][e];
+                }
+                between(x);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        __syncthreads(); // barrier 0
+        if constexpr (SLOTS == 1) {
+#pragma unroll
+            for (int n = 0; n < 6; ++n) {
+                read_a(0, lds, 0, n);
+                read_b(0, lds, 0, n);
+            }
+            for (int kt = 0; kt < nk; ++kt) {
+                const unsigned char *cur = lds + (kt & 1) * STAGEB, *next = lds + ((kt & 1) ^ 1) * STAGEB;
+                block(0, 0, 0, sum[1][1], [&](int x) __attribute__((always_inline)) {
+                    if (x < 6) read_b(0, cur, 1, x);
+                    else read_a(0, cur, 1, x - 6);
+                });
+                block(0, 0, 1, sum[0][0], [](int) {});
+                __syncthreads(); // barrier kt + 1 (behind the last k-tile: what is read below is not used)
+                block(0, 1, 0, sum[0][1], [&](int x) __attribute__((always_inline)) {
+                    if (x < 6) read_a(0, next, 0, x);
+                });
+                block(0, 1, 1, sum[1][0], [&](int x) __attribute__((always_inline)) {
+                    if (x < 6) read_b(0, next, 0, x);
+                });
+            }
+            sum[1][1] += t[1];
+        } else {
+            float16_t odd[NJ]; // the second halves' sums: two chains of K / 64 additions
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) odd[j] = float16_t{};
+            auto half = [&](int h, const unsigned char *stage) __attribute__((always_inline)) { // multiplies half h and reads the other one from `stage`
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    block(h, 0, j, j == 0 ? (h == 0 ? odd[NJ - 1] : sum[0][NJ - 1]) : (h == 0 ? sum[0][j - 1] : odd[j - 1]), [&](int x) __attribute__((always_inline)) {
+                        if (j == 0 && x < 6) read_a(h ^ 1, stage, 0, x);
+                        if (j == 0 && x < 6 * NJ) read_b(h ^ 1, stage, x / 6, x % 6);
+                    });
+            };
+#pragma unroll
+            for (int n = 0; n < 6; ++n) {
+                read_a(0, lds, 0, n);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) read_b(0, lds, j, n);
+            }
+            for (int kt = 0; kt < nk; ++kt) {
+                half(0, lds + (kt & 1) * STAGEB);
+                __syncthreads(); // barrier kt + 1
+                half(1, lds + ((kt & 1) ^ 1) * STAGEB);
+            }
+            odd[NJ - 1] += t[1];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) sum[0][j] += odd[j];
+        }
+    }
+};
+
+constexpr int RING_STAGES = 3;
+template <int TM, int TNR> constexpr int ring_lds_bytes() { return RING_STAGES * (TM + TNR) * BIG_ROWB; }
+template <int TM, int TNR, int KF, int LW> constexpr int split_lds_bytes() { // the ring or both stages of parts, and a flag of each wavefront
+    const int ring = ring_lds_bytes<TM, TNR>(), split = 2 * SplitRing<TM, TNR, KF, LW, false>::STAGEB;
+    return (ring > split ? ring : split) + 64;
+}
+
+template <int TM, int TNR, int KF, int LW, bool NN> // KF: 0 fp32 products, else products of parts
+__global__ __launch_bounds__(64 * (4 + LW), 1) void gemm_mfma_f32_ring_kernel(const GemmArgs g, const int tiles_m, const int tiles_n) {
     constexpr int MI = TM / 64, NJ = TNR / 64;
     constexpr int NLA = TM / 32, NLB = TNR / 32, NL = NLA + NLB; // loads of 1 KiB per wavefront and k-tile
-    constexpr int KF = 32;                            // floats per k-tile
-    constexpr int STAGEB = (TM + TNR) * BIG_ROWB;
+    constexpr int RK = 32, S = RING_STAGES, STAGEB = (TM + TNR) * BIG_ROWB; // (fp32 products: floats per k-tile, stages)
     extern __shared__ __attribute__((aligned(1024))) unsigned char big_lds[];
     const int tid = threadIdx.x, lane = tid % WAVE;
-    const bool loader = __builtin_amdgcn_readfirstlane(tid / WAVE) >= 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE) % 4;
+    const int wavefront = __builtin_amdgcn_readfirstlane(tid / WAVE), wave = wavefront % 4;
+    const bool loader = wavefront >= 4;
     const int l32 = lane % 32, g2 = lane / 32;
 
     int product;
@@ -404,10 +629,34 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const float *B = static_cast<const float *>(g.b) + bz * g.sb + n0 * (NN ? 1 : g.b_cs);
     const int arow_bytes = static_cast<int>(g.a_rs) * 4, brow_bytes = static_cast<int>(NN ? g.b_rs : g.b_cs) * 4;
     const int rows_a = static_cast<int>(min<int64_t>(TM, g.M - m0)), rows_b = static_cast<int>(min<int64_t>(TNR, g.N - n0));
-    const int K = static_cast<int>(g.K), nk = (K + KF - 1) / KF;
+    const int K = static_cast<int>(g.K), nk = (K + RK - 1) / RK;
     const int4_t arsrc = gemm_rsrc(A, (rows_a - 1) * arow_bytes + K * 4);
     const int4_t brsrc = gemm_rsrc(B, NN ? (K - 1) * brow_bytes + rows_b * 4 : (rows_b - 1) * brow_bytes + K * 4);
 
+    const int wm = (wave / 2) * (TM / 2), wn = (wave % 2) * (TNR / 2);
+
+    float16_t sum[MI][NJ];
+    bool fp32_products = true;
+    if constexpr (KF != 0) {
+        using Split = SplitRing<TM, TNR, KF, LW, NN>;
+        bool failed = false;
+        if (loader) {
+            Split::load(g, A, B, rows_a, rows_b, big_lds, wavefront - 4, lane);
+        } else {
+            Split::multiply(K, big_lds, wm, wn, lane, sum);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        failed = failed || split_failed(sum[i][j][e]);
+                        sum[i][j][e] *= SPLIT_UNSCALE;
+                    }
+        }
+        fp32_products = work_group_any<4 + LW>(failed, reinterpret_cast<uint32_t *>(big_lds + split_lds_bytes<TM, TNR, KF, LW>() - 64));
+    }
+    if (fp32_products) {
     const int ld_r = 8 * wave + (lane >> 3);
     const int ld_k = 4 * ((lane & 7) ^ ((ld_r >> 1) & 7)); // this lane's chunk of a row along k: floats ld_k .. ld_k + 3 of the k-tile
     constexpr int OUT_OF_RANGE = 0x7FFFFFF0;
@@ -423,7 +672,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(big_lds));
     const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(lds_base + 8 * wave * BIG_ROWB);
     auto load = [&](int kt, int stage_off, int n) __attribute__((always_inline)) { // n: of A, then of B
-        const int k0 = kt * KF;
+        const int k0 = kt * RK;
         const int along = k0 + ld_k < K ? min(k0 + ld_k, K - 4) * 4 : OUT_OF_RANGE; // of a row along k
         if (n < NLA) {
             gemm_load_to_lds(arsrc, lds_wave + stage_off + n * 32 * BIG_ROWB, along == OUT_OF_RANGE ? OUT_OF_RANGE : a_row[n < NLA ? n : 0] + along, 0);
@@ -436,7 +685,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
     };
     // the last k-tile, where K is no multiple of 4: this lane's chunks that K ends in, already in LDS, are put in place
     auto mend = [&](int stage_off) __attribute__((always_inline)) {
-        const int drop = (nk - 1) * KF + ld_k + 4 - K; // floats in front of the chunk
+        const int drop = (nk - 1) * RK + ld_k + 4 - K; // floats in front of the chunk
         if (drop <= 0 || drop >= 4) return;
 #pragma unroll
         for (int n = 0; n < (NN ? NLA : NL); ++n) {
@@ -448,7 +697,9 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
 #define AXHIP_FENCE() __builtin_amdgcn_sched_barrier(0)
 #define AXHIP_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | 0x0F70 | (((n) >> 4) << 14))
     static_assert(S >= 3 && NL * (S - 1) < 64, "vmcnt is a 6-bit counter");
-    if (loader) {
+    if (LW > 4 && wavefront >= 8) { // (four load)
+        for (int kt = 0; kt <= nk; ++kt) __syncthreads();
+    } else if (loader) {
 #pragma unroll
         for (int st = 0; st < S - 1; ++st)
 #pragma unroll
@@ -466,23 +717,19 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
             to = to + STAGEB == S * STAGEB ? 0 : to + STAGEB;
         }
         AXHIP_VMCNT(0); // no load is still on its way into LDS
-        return;
-    }
+    } else {
 
-    const int wm = (wave / 2) * (TM / 2), wn = (wave % 2) * (TNR / 2);
     int f_off[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) f_off[ks] = l32 * BIG_ROWB + (((2 * ks + g2) ^ ((l32 >> 1) & 7)) * 16);
 
     // The sums of a k-tile are added to those of all before: chains of 32 fp32 additions, then one of K / 32, in place of one
-    // of K (2048^3, one chain: 8.1e-7 off the exact result, now 1.8e-7).  TURNS:
-    // two accumulators in turn, one is added up under the next k-tile's MFMAs.
-    constexpr int TURN = TURNS ? 1 : 0;
-    float16_t acc[1 + TURN][MI][NJ], sum[MI][NJ];
+    // of K (2048^3, one chain: 8.1e-7 off the exact result, these 1.8e-7).
+    float16_t acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) sum[i][j] = acc[TURN][i][j] = float16_t{};
+        for (int j = 0; j < NJ; ++j) sum[i][j] = float16_t{};
 
     // fragments of LOOK steps of eight k are on their way while one is multiplied: with one block a wavefront has four MFMAs
     // for these, less than a read takes next to three other wavefronts'
@@ -501,14 +748,14 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
         }
     };
     // eight k: 4 MI NJ MFMAs; behind MFMA (c, i, j) what `between` does
-    auto multiply = [&](int slot, int p, bool first, auto between) __attribute__((always_inline)) {
+    auto multiply = [&](int slot, bool first, auto between) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    acc[p][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], first && c == 0 ? float16_t{} : acc[p][i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[slot][i][c], fb[slot][j][c], first && c == 0 ? float16_t{} : acc[i][j], 0, 0, 0);
                     AXHIP_FENCE();
                     between(c, i, j);
                     AXHIP_FENCE();
@@ -524,7 +771,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
         for (int j = 0; j < NJ; ++j) read_b(ks, 0, ks, j);
     }
     int cur = 0; // offset of k-tile kt's stage
-    auto tile = [&](int p) __attribute__((always_inline)) {
+    for (int kt = 0; kt < nk; ++kt) {
         const int next = cur + STAGEB == S * STAGEB ? 0 : cur + STAGEB;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -534,41 +781,23 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_f32_ring_kernel(const GemmAr
                 __syncthreads(); // tile kt + 1 has landed, and tile kt is no longer read
                 AXHIP_FENCE();
             }
-            multiply(ks % SLOTS_F, p, ks == 0, [&](int c, int i, int j) __attribute__((always_inline)) {
+            multiply(ks % SLOTS_F, ks == 0, [&](int c, int i, int j) __attribute__((always_inline)) {
                 const int x = (c * MI + i) * NJ + j;
                 if (x < MI) read_a((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
                 if (x < NJ) read_b((ks + LOOK) % SLOTS_F, from, (ks + LOOK) % 4, x);
-                if (TURNS && (ks == 1 || ks == 2)) {
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) sum[i][j][8 * (ks - 1) + 2 * c + e] += acc[p ^ TURN][i][j][8 * (ks - 1) + 2 * c + e];
-                }
             });
         }
         cur = next;
-    };
-    auto add_up = [&](int p) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) sum[i][j][e] += acc[p][i][j][e];
-    };
-    if constexpr (TURNS) {
-        for (int kt = 0; kt < nk; kt += 2) {
-            tile(0);
-            if (kt + 1 < nk) tile(TURN);
-        }
-        if (nk % 2 == 0) add_up(TURN);
-        else add_up(0);
-    } else {
-        for (int kt = 0; kt < nk; ++kt) {
-            tile(0);
-            add_up(0);
-        }
+            for (int j = 0; j < NJ; ++j) sum[i][j] += acc[i][j];
+    }
     }
 #undef AXHIP_VMCNT
 #undef AXHIP_FENCE
+    }
+    if (loader) return;
 
     // epilogue: accumulator element e of tile (i, j) is C[m + 32 i + 8 (e / 4) + 4 g2 + e % 4][n + 32 j + l32].  The 16
     // values of a tile take each step together: one branch on the epilogue, one set of loads on their way.
@@ -745,23 +974,33 @@ const HalfKernel *choose_half_kernel(const AxhipGemmParams &p, bool aligned) {
 }
 
 // ---- fp32 products: which kernel
-// The ring kernel's tiles with the time each takes, in us: start + k per_k r + per_round (r - 1), r being the rounds its
-// work-groups take on the 256 CUs, fitted to 60 products of m 11 .. 4117, n 64 .. 51865, k 64 .. 8192.  Tiles of 64 x 64 fill
-// the chip soonest and share a CU; larger ones read less from LDS and L2 for each MFMA.
-struct F32RingTile { int tm, tn; float start, per_k, per_round; };
-constexpr F32RingTile F32_RING_TILES[3] = {{128, 128, 11.0f, 0.067f, 3.5f}, {64, 128, 6.8f, 0.0325f, 3.0f}, {64, 64, 4.5f, 0.0170f, 1.3f}};
+// The ring kernel's tiles, by fp32 products and by products of parts, with the time each takes, in us: start + k (per_k +
+// (per_k_full + per_k_odd odd) u) r + per_round (r - 1), r being the rounds its work-groups take on the 256 CUs, u how full the
+// first is (all CUs at work lower the clock) and odd 1 for rows off the 16-byte grid.
+enum RingTile { RING_64x64, RING_64x128, RING_128x128_PARTS, RING_64x128_PARTS, RING_64x64_PARTS, RING_TILES };
+struct F32RingTile { int tm, tn, tk; float start, per_k, per_k_full, per_round, per_k_odd; };
+constexpr F32RingTile F32_RING_TILES[RING_TILES] = {{64, 64, 32, 4.25f, 0.0166f, 0.0f, 0.78f, 0.0f},
+                                                    {64, 128, 32, 5.20f, 0.0320f, 0.0f, 1.66f, 0.0015f},
+                                                    {128, 128, 32, 8.20f, 0.0297f, 0.0063f, 7.52f, 0.0020f},
+                                                    {64, 128, 64, 6.67f, 0.0204f, 0.0027f, 5.45f, 0.0021f},
+                                                    {64, 64, 64, 4.59f, 0.0120f, 0.0017f, 3.31f, 0.0016f}};
 struct F32Ring { int tile; float cost; };
-F32Ring f32_ring_tile(const AxhipGemmParams &p) {
+// (one candidate; the candidates are a parameter of the template, as those of the 16-bit kernels are)
+template <size_t I> void consider_f32_ring_tile(const AxhipGemmParams &p, float odd, F32Ring &best) {
+    constexpr F32RingTile t = F32_RING_TILES[I];
+    const float k = static_cast<float>((p.k + t.tk - 1) / t.tk * t.tk);
+    const uint64_t tiles = ((static_cast<uint64_t>(p.m) + t.tm - 1) / t.tm) * ((static_cast<uint64_t>(p.n) + t.tn - 1) / t.tn) * static_cast<uint64_t>(p.batch);
+    const float r = static_cast<float>(static_cast<int64_t>((tiles + 255) / 256)), u = tiles < 256 ? static_cast<float>(static_cast<int>(tiles)) * (1.0f / 256.0f) : 1.0f;
+    const float cost = t.start + k * (t.per_k + (t.per_k_full + t.per_k_odd * odd) * u) * r + t.per_round * (r - 1.0f);
+    if (I == 0 || cost < best.cost) best = {static_cast<int>(I), cost};
+}
+template <size_t... I> F32Ring f32_ring_tile(const AxhipGemmParams &p, std::index_sequence<I...>) {
     F32Ring best{0, 0.0f};
-    const float k = static_cast<float>((p.k + 31) / 32 * 32);
-    for (int c = 0; c < 3; ++c) {
-        const F32RingTile &t = F32_RING_TILES[c];
-        const int64_t tiles = ((p.m + t.tm - 1) / t.tm) * ((p.n + t.tn - 1) / t.tn) * p.batch;
-        const float r = static_cast<float>((tiles + 255) / 256), cost = t.start + k * t.per_k * r + t.per_round * (r - 1.0f);
-        if (c == 0 || cost < best.cost) best = {c, cost};
-    }
+    const float odd = p.k % 4 != 0 || (!p.trans_b && p.n % 4 != 0) ? 1.0f : 0.0f;
+    (consider_f32_ring_tile<I>(p, odd, best), ...);
     return best;
 }
+F32Ring f32_ring_tile(const AxhipGemmParams &p) { return f32_ring_tile(p, std::make_index_sequence<RING_TILES>{}); }
 // A along k, offsets of 32 bits, rows of b as [k, n] of whole chunks or at least a tile (128 columns at most)
 bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
     return !p.trans_a && (p.trans_b || ((p.n % 4 == 0 || p.n >= 128) && p.n < (1 << 24) && (p.k + 64) * p.ldb < (int64_t(1) << 29))) && p.k >= 32 &&
@@ -777,7 +1016,21 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
     {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f},
-    {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f}, {4.59f, 0.00939f, 0.00112f, 3.91f, 0.00138f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}};
+    {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f}, {5.30f, 0.00701f, 0.00159f, 3.70f, 0.00106f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}};
+
+template <size_t I> void consider_f32_kernel(const AxhipGemmParams &p, float k, float u, bool ring, int &best, float &best_cost) {
+    constexpr F32Kernel h = F32_KERNELS[I];
+    constexpr uint32_t tm = F32_GEOMETRY[I].tm, tn = F32_GEOMETRY[I].tn;
+    const uint32_t rows = (static_cast<uint32_t>(p.m) + tm - 1) / tm, cols = (static_cast<uint32_t>(p.n) + tn - 1) / tn; // (m, n < 2^30)
+    if (!launch_fits(static_cast<int64_t>(rows) * cols + 7, 512)) return; // (eight wavefronts a tile)
+    const float full = static_cast<float>(p.batch) * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
+    const float r = full <= 1.0f ? 1.0f : 0.5f * (std::ceil(full) + full);
+    const float cost = h.start + k * (h.per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
+    if ((best < 0 && !ring) || cost < best_cost) { best_cost = cost; best = static_cast<int>(I); }
+}
+template <size_t... I> void consider_f32_kernels(const AxhipGemmParams &p, float k, float u, bool ring, int &best, float &best_cost, std::index_sequence<I...>) {
+    (consider_f32_kernel<I>(p, k, u, ring, best, best_cost), ...);
+}
 
 // An F32Shape, or -1: the kernel that this product had otherwise (`ring`: the ring kernel, after `repacked` bytes were
 // written and read if there are any; else the FMA kernel).
@@ -791,15 +1044,7 @@ int choose_f32_kernel(const AxhipGemmParams &p, bool ring, double repacked) {
     int best = -1;
     float best_cost = 0.0f;
     if (ring) best_cost = f32_ring_tile(p).cost + (repacked > 0.0 ? 4.7f + 2.1e-7f * static_cast<float>(repacked) : 0.0f);
-    for (int i = 0; i < F32_SHAPES; ++i) {
-        const F32Kernel &h = F32_KERNELS[i];
-        const int64_t rows = (p.m + F32_GEOMETRY[i].tm - 1) / F32_GEOMETRY[i].tm, cols = (p.n + F32_GEOMETRY[i].tn - 1) / F32_GEOMETRY[i].tn;
-        if (!launch_fits(rows * cols + 7, 512)) continue; // (eight wavefronts a tile)
-        const float full = static_cast<float>(p.batch) * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
-        const float r = full <= 1.0f ? 1.0f : 0.5f * (std::ceil(full) + full);
-        const float cost = h.start + k * (h.per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
-        if ((best < 0 && !ring) || cost < best_cost) { best_cost = cost; best = i; }
-    }
+    consider_f32_kernels(p, k, u, ring, best, best_cost, std::make_index_sequence<F32_SHAPES>{});
     return best;
 }
 
@@ -962,7 +1207,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         if (rc) return rc;
     } else if (f32 && takes_f32_ring(p, a, b)) {
         // the fp32 MFMA, b along k or [k, n]
-        auto launch = [&](auto kernel, int tm_rows, int tn_cols, size_t lds_bytes) -> int {
+        auto launch = [&](auto kernel, int tm_rows, int tn_cols, int threads, size_t lds_bytes) -> int {
             static std::mutex mu;
             static std::set<const void *> configured;
             {
@@ -976,8 +1221,8 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
             const int64_t tiles_m = (p.m + tm_rows - 1) / tm_rows, tiles_n = (p.n + tn_cols - 1) / tn_cols;
             const bool by_rows = !p.trans_b || tiles_m >= tiles_n;
             const int64_t across = by_rows ? tiles_n : tiles_m, size = by_rows ? p.m : p.n;
-            AXHIP_REQUIRE(launch_fits(across + 7, 512), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
-            const int64_t strip = products_per_launch(across, 512) * (by_rows ? tm_rows : tn_cols);
+            AXHIP_REQUIRE(launch_fits(across + 7, threads), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: too many tiles");
+            const int64_t strip = products_per_launch(across, threads) * (by_rows ? tm_rows : tn_cols);
             for (int64_t at = 0; at < size; at += strip) {
                 GemmArgs part = g;
                 (by_rows ? part.M : part.N) = std::min(strip, size - at);
@@ -988,24 +1233,19 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
                 if (g.residual) part.residual = static_cast<const char *>(g.residual) + in_c;
                 if (g.bias && !by_rows) part.bias = static_cast<const char *>(g.bias) + 4 * at;
                 const int rows = static_cast<int>((part.M + tm_rows - 1) / tm_rows), cols = static_cast<int>((part.N + tn_cols - 1) / tn_cols);
-                launch_products(part, static_cast<int64_t>(rows) * cols, 512, 4, [&](const GemmArgs &some, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds_bytes, s, some, rows, cols); });
+                launch_products(part, static_cast<int64_t>(rows) * cols, threads, 4, [&](const GemmArgs &some, unsigned grid) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds_bytes, s, some, rows, cols); });
             }
             return AXHIP_OK;
         };
         int rc2;
         switch (f32_ring_tile(p).tile) {
-#define AXHIP_RING(TM, TN, S, TURNS) \
-    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, S, false, TURNS>, TM, TN, S * (TM + TN) * BIG_ROWB) \
-                    : launch(gemm_mfma_f32_ring_kernel<TM, TN, S, true, TURNS>, TM, TN, S * (TM + TN) * BIG_ROWB)
-        // (two accumulators in turn on the one work-group of a CU, where nothing else fills the pipe meanwhile; elsewhere their
-        // registers cost a second work-group its place: 2048^3 145 us instead of 134 on 64 x 128 tiles, and 128 x 128 tiles
-        // 182 instead of 176 for 4096 x 4096 x 512)
-        case 0: AXHIP_RING(128, 128, 3, false); break;
-        case 1: AXHIP_RING(64, 128, 3, false); break;
-        default: // (one work-group per CU: a fourth stage hides the rest of a load's latency, 80 -> 76 us for k of 4096; more: three of them share a CU's LDS)
-            if ((p.m + 63) / 64 * ((p.n + 63) / 64) * p.batch <= 256) AXHIP_RING(64, 64, 4, true);
-            else AXHIP_RING(64, 64, 3, false);
-            break;
+#define AXHIP_RING(TM, TN, KF, LW, LDS) \
+    rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, KF, LW, false>, TM, TN, 64 * (4 + LW), LDS) : launch(gemm_mfma_f32_ring_kernel<TM, TN, KF, LW, true>, TM, TN, 64 * (4 + LW), LDS)
+        case RING_64x64: AXHIP_RING(64, 64, 0, 4, (ring_lds_bytes<64, 64>())); break;
+        case RING_64x128: AXHIP_RING(64, 128, 0, 4, (ring_lds_bytes<64, 128>())); break;
+        case RING_128x128_PARTS: AXHIP_RING(128, 128, 32, 4, (split_lds_bytes<128, 128, 32, 4>())); break;
+        case RING_64x128_PARTS: AXHIP_RING(64, 128, 64, 4, (split_lds_bytes<64, 128, 64, 4>())); break;
+        default: AXHIP_RING(64, 64, 64, 8, (split_lds_bytes<64, 64, 64, 8>())); break;
 #undef AXHIP_RING
         }
         if (rc2) return rc2;

@@ -1,6 +1,7 @@
 // fp32 products without shared LDS tiles: see the kernel's comment.
 #include "common.hpp"
 #include "gemm_f32.hpp"
+#include "gemm_f32_split.hpp"
 #include "gemm_tile_device.hpp"
 
 namespace axhip {
@@ -11,6 +12,11 @@ template <int N> struct __attribute__((packed, aligned(4))) Floats { float v[N];
 
 constexpr int F32_WAVES = 8;
 
+template <bool NN, bool SPLIT, int MI, int NJ, int P> constexpr int direct_lds_bytes() { // the stages or the sums (SPLIT: and a flag of each wavefront)
+    const int stages = F32_WAVES * P * 2 * (MI + (NN ? 0 : NJ)) * 1024, sum = F32_WAVES * MI * NJ * 1024;
+    return (stages > sum ? stages : sum) + (SPLIT ? 64 : 0);
+}
+
 // C = A B (b [N, K], or [K, N]: NN) on v_mfma_f32_16x16x4_f32: fp32 products and sums.  Work-group tile 16 MI x 16 NJ;
 // eight wavefronts take pieces of 32 P elements of k in turn and add their sums through LDS at the end; until then no
 // wavefront waits for another.
@@ -20,7 +26,11 @@ constexpr int F32_WAVES = 8;
 // side, they took four times the address cycles: 1024^3 28.5 us); b as [K, N] needs no stage and no transpose: which
 // column a lane contributes to which MFMA is free, so lane (l16, g) loads the NJ columns NJ l16 .. of rows 4 g .. 4 g + 3.
 // Bound by the matrix pipe at 64 x 64 and by latency below, where narrower tiles put more CUs to work.
-template <bool NN, int MI, int NJ, int P>
+// SPLIT: by products of bf16 parts (gemm_f32_split.hpp), each wavefront splitting what it multiplies.  That pays at 32 x 64, where
+// eight fragments' splitting, 1250 cycles, stands for 2048 of fp32 MFMAs (333 x 1280 x 1280 18.0 -> 15.1 us, 64 x 1280 x 5120 on
+// these tiles 54 -> 45); 32 x 32 and below have no more MFMAs than splitting to do (64 x 1280 x 5120 28.2 and 28.1, 512^3
+// 6.0 and 6.6), and the fragments of 64 x 64 do not fit the registers.
+template <bool NN, bool SPLIT, int MI, int NJ, int P>
 __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(const TileArgs g) {
     extern __shared__ __attribute__((aligned(1024))) float sums[];
     constexpr int W = F32_WAVES, TM = 16 * MI, TN = 16 * NJ, KP = 32 * P, U = 2 * P;
@@ -123,6 +133,47 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
         wave_lds_fence();
     };
 
+    auto multiply_parts = [&](const float (&xb)[NN ? U : 1][NJ][4]) {
+        wave_lds_fence();
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            auto whole_fragment = [&](int first, int tile) __attribute__((always_inline)) { // k = 32 p + 4 g4 .. + 3 and, 16 on, four more
+                float x[8];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const f32x4_t v = *reinterpret_cast<const f32x4_t *>(stage + (p * NS + first) * 1024 + (16 * tile + l16) * 128 + (((4 * u + g4) ^ ((l16 >> 1) & 7)) * 16));
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) x[4 * u + c] = v[c];
+                }
+                return split_fragment(x);
+            };
+            SplitFragment sb[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                if constexpr (NN) {
+                    float x[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] = xb[2 * p + e / 4][j][e % 4];
+                    sb[j] = split_fragment(x);
+                } else {
+                    sb[j] = whole_fragment(NA, j);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const SplitFragment sa = whole_fragment(0, i);
+                f32x4_t t[NJ];
+#pragma unroll
+                for (int n = 0; n < SPLIT_PRODUCTS; ++n)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) t[j] = split_mfma(sb[j].part[SPLIT_B[n]], sa.part[SPLIT_A[n]], n == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : t[j]);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] += t[j];
+            }
+        }
+        wave_lds_fence();
+    };
+
     const int whole = g.K / KP * KP;
     int k = wave * KP;
     if (k < whole) load(k);
@@ -140,40 +191,69 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
         to_stage();
         k += W * KP;
         if (k < whole) load(k);
-        multiply(xb);
+        if constexpr (SPLIT) multiply_parts(xb);
+        else multiply(xb);
     }
     if (whole < g.K && k == whole) { // this wavefront's turn
         load_last(k);
         to_stage();
-        multiply(fb);
+        if constexpr (SPLIT) multiply_parts(fb);
+        else multiply(fb);
     }
-    __syncthreads(); // the stages become the sums
-
-    // sums[wave][f][lane], four columns each: NN f = (i, e) columns NJ (4 g4 + e) + 0 .. (fewer than four tiles: the
-    // columns of several e side by side); else f = (i, j) columns 16 j + 4 g4 + 0 .. 3
     constexpr int F = MI * NJ;
+    auto total = [&](int x) { // this lane's four columns
+        f32x4_t v = *reinterpret_cast<const f32x4_t *>(&sums[x * 4]);
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+        for (int w = 1; w < W; ++w) v += *reinterpret_cast<const f32x4_t *>(&sums[(w * F * 64 + x) * 4]);
+        return v;
+    };
+    float scale = SPLIT_UNSCALE;
+    for (;;) {
+        __syncthreads(); // the stages become the sums
+
+        // sums[wave][f][lane], four columns each: NN f = (i, e) columns NJ (4 g4 + e) + 0 .. (fewer than four tiles: the
+        // columns of several e side by side); else f = (i, j) columns 16 j + 4 g4 + 0 .. 3
 #pragma unroll
-        for (int f = 0; f < NJ; ++f) {
-            f32x4_t v;
-            if constexpr (NN) {
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int x = 0; x < 4; ++x) v[x] = acc[i][(4 * f + x) % NJ][(4 * f + x) / NJ];
-            } else {
-                v = acc[i][f];
+            for (int f = 0; f < NJ; ++f) {
+                f32x4_t v;
+                if constexpr (NN) {
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = acc[i][(4 * f + x) % NJ][(4 * f + x) / NJ];
+                } else {
+                    v = acc[i][f];
+                }
+                *reinterpret_cast<f32x4_t *>(&sums[((wave * F + i * NJ + f) * 64 + lane) * 4]) = v;
             }
-            *reinterpret_cast<f32x4_t *>(&sums[((wave * F + i * NJ + f) * 64 + lane) * 4]) = v;
+        __syncthreads();
+        if (!SPLIT || scale == 1.0f) break;
+        bool failed = false;
+        for (int x = tid; x < F * 64; x += 64 * W) {
+            const f32x4_t v = total(x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) failed = failed || split_failed(v[e]);
         }
-    __syncthreads();
+        if (!work_group_any<W>(failed, reinterpret_cast<uint32_t *>(sums) + direct_lds_bytes<NN, SPLIT, MI, NJ, P>() / 4 - 16)) break;
+        scale = 1.0f; // again, with fp32 products
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int again = wave * KP; again < g.K; again += W * KP) {
+            load_last(again);
+            to_stage();
+            multiply(fb);
+        }
+    }
     float *C = static_cast<float *>(g.c) + bz * g.sc;
     const float *bias = static_cast<const float *>(g.bias), *res = g.residual ? static_cast<const float *>(g.residual) + bz * g.sc : nullptr;
     for (int x = tid; x < F * 64; x += 64 * W) {
         const int f = x / 64 % NJ, m = m0 + 16 * (x / 64 / NJ) + x % 16, xg = x % 64 / 16;
         if (m >= g.M) continue;
-        f32x4_t v = *reinterpret_cast<const f32x4_t *>(&sums[x * 4]);
-#pragma unroll
-        for (int w = 1; w < W; ++w) v += *reinterpret_cast<const f32x4_t *>(&sums[(w * F * 64 + x) * 4]);
+        f32x4_t v = total(x);
+        if constexpr (SPLIT) v *= scale;
         // columns col .. col + 3.  (NN: a lane whose columns were moved left to end with the rows owns those at and
         // behind the place it was moved from)
         const int col = n0 + (NN ? 4 * NJ * xg + 4 * f : 16 * f + 4 * xg);
@@ -217,9 +297,9 @@ __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(cons
     }
 }
 
-template <bool NN, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, hipStream_t s) {
-    constexpr int stages = F32_WAVES * P * 2 * (MI + (NN ? 0 : NJ)) * 1024, sum = F32_WAVES * MI * NJ * 1024, lds = stages > sum ? stages : sum;
-    const auto kernel = gemm_f32_direct_kernel<NN, MI, NJ, P>;
+template <bool NN, bool SPLIT, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, hipStream_t s) {
+    constexpr int lds = direct_lds_bytes<NN, SPLIT, MI, NJ, P>();
+    const auto kernel = gemm_f32_direct_kernel<NN, SPLIT, MI, NJ, P>;
     static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     AXHIP_CHECK_HIP(configured);
     const int64_t tiles = static_cast<int64_t>((g.M + 16 * MI - 1) / (16 * MI)) * ((g.N + 16 * NJ - 1) / (16 * NJ));
@@ -229,12 +309,12 @@ template <bool NN, int MI, int NJ, int P> int launch_kernel(const TileArgs &g, h
 }
 template <bool NN> int launch_shape(const TileArgs &g, int shape, hipStream_t s) {
     switch (shape) {
-    case F32_16x16: return launch_kernel<NN, 1, 1, 2>(g, s);
-    case F32_16x32: return launch_kernel<NN, 1, 2, 2>(g, s);
-    case F32_16x64: return launch_kernel<NN, 1, 4, 1>(g, s);
-    case F32_32x32: return launch_kernel<NN, 2, 2, 1>(g, s);
-    case F32_32x64: return launch_kernel<NN, 2, 4, 1>(g, s);
-    default: return launch_kernel<NN, 4, 4, 1>(g, s);
+    case F32_16x16: return launch_kernel<NN, false, 1, 1, 2>(g, s);
+    case F32_16x32: return launch_kernel<NN, false, 1, 2, 2>(g, s);
+    case F32_16x64: return launch_kernel<NN, false, 1, 4, 1>(g, s);
+    case F32_32x32: return launch_kernel<NN, false, 2, 2, 1>(g, s);
+    case F32_32x64: return launch_kernel<NN, true, 2, 4, 1>(g, s);
+    default: return launch_kernel<NN, false, 4, 4, 1>(g, s);
     }
 }
 } // namespace

@@ -494,3 +494,77 @@ def test_batches_are_dealt_over_all_xcds(dtype, nn, M, N, K, batch, shared):
         want = x @ w + bias.double() + res[b].double()
         magnitude = x.abs() @ w.abs() + bias.double().abs() + res[b].double().abs()
         assert bool(((c[b].double() - want).abs() <= (K + 2) * 2.0**-24 * magnitude + half_ulp * want.abs() + 2.0**-24).all())
+
+
+# k from 32 to 8192 on every tile that multiplies parts: 32 x 64 and 64 x 64 (few output tiles), 64 x 128 and 128 x 128, with rows,
+# columns and k that end inside a tile, a chunk and a pair of k-tiles
+PARTS = [(300, 1280, 1285, 1), (130, 1984, 2050, 1), (1024, 1020, 1023, 1), (1000, 1028, 1090, 1), (257, 4100, 700, 1), (513, 132, 995, 8), (2048, 2044, 225, 1), (1153, 129, 256, 16)]
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", PARTS)
+def test_f32_products_of_parts(nn, M, N, K, batch):
+    """Products by way of bf16 parts are no further from the exact ones than fp32 sums of 32 products and then one per
+    32 k: (36 + K / 32) half ulps of the sum of magnitudes, for inputs of both signs, of one sign, and so small that their
+    last parts would be below bf16's smallest normal number, had they not been scaled."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + 3 * N + K)
+    for kind in ("normal", "positive", "small"):
+        x, W = torch.empty((batch, M, K), device="cuda"), torch.empty((batch, K, N) if nn else (batch, N, K), device="cuda")
+        for t in (x, W):
+            t.uniform_(0.0, 1.0, generator=gen) if kind == "positive" else t.normal_(generator=gen)
+        if kind == "small":
+            x *= 2.0**-118
+            W *= 2.0**40
+        c = _f32_product(x, W, nn)
+        for b in range(0, batch, 5):
+            x64, w64 = x[b].double(), W[b].double() if nn else W[b].double().t().contiguous()
+            assert bool(((c[b].double() - x64 @ w64).abs() <= min(K + 2, 36 + K / 32) * 2.0**-24 * (x64.abs() @ w64.abs())).all()), kind
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", PARTS)
+def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch):
+    """Infinities, NaN and numbers near the largest, whose parts have none: the same places of the result are infinite or NaN as in
+    float64, and everything else keeps its bound, in the tiles that are computed again and in the others."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + 3 * N + K)
+    x, W = torch.empty((batch, M, K), device="cuda").normal_(generator=gen), torch.empty((batch, K, N) if nn else (batch, N, K), device="cuda").normal_(generator=gen)
+    last = batch - 1
+    x[0, 3, 5], x[last, M - 1, K - 1], x[0, 40, :] = float("inf"), float("nan"), 3.0e38
+    W[0] = W[0].abs() * 2.0**-20
+    W[last, 0, 0] = -float("inf") if batch > 1 else W[last, 0, 0]
+    c = _f32_product(x, W, nn)
+    for b in {0, last // 2, last}:
+        x64, w64 = x[b].double(), W[b].double() if nn else W[b].double().t().contiguous()
+        want = x64 @ w64
+        finite = torch.isfinite(want) & (want.abs() < 3.0e38)
+        beyond = want.abs() > 3.5e38
+        assert bool((torch.isnan(c[b]) == torch.isnan(want)).all())
+        assert bool((c[b][beyond].double() == torch.sign(want[beyond]) * float("inf")).all())
+        bound = min(K + 2, 36 + K / 32) * 2.0**-24 * torch.nan_to_num(x64, nan=0.0, posinf=0.0).abs() @ torch.nan_to_num(w64, neginf=0.0).abs()
+        assert bool(((c[b].double() - want).abs() <= bound)[finite].all())
+
+
+def _f32_product(x, W, nn):
+    import ctypes as C
+
+    import torch
+
+    from axiom_amd import capi
+
+    batch, M, K = x.shape
+    N = W.shape[2] if nn else W.shape[1]
+    c = torch.full((batch, M, N), 7.0, device="cuda")
+    p = capi.GemmParams()
+    p.dtype, p.m, p.n, p.k, p.batch, p.lda, p.ldb, p.ldc, p.trans_b = F32, M, N, K, batch, K, N if nn else K, N, int(not nn)
+    p.stride_a, p.stride_b, p.stride_c = M * K, K * N, M * N
+    torch.cuda.synchronize()
+    gh.sync()
+    capi.check(capi.lib().axhip_gemm(x.data_ptr(), W.data_ptr(), c.data_ptr(), C.byref(p), None))
+    gh.sync()
+    return c
