@@ -452,6 +452,8 @@ __device__ __forceinline__ int4_t make_rsrc(const void *base, int bytes) {
 // SPLIT = 2 (problems too small to give every SIMD two waves otherwise): the work-group's waves form two groups, which
 // take the same 32 * NW / 2 query rows and one part of the key tiles each, through K/V tile buffers of their own; the
 // second hands its accumulators, reference maximum and row sums to the first through LDS at the end.  A part may be empty.
+// With four waves a tile serves two, each of which issues twice the loads (60 cycles of its issue each) and which together
+// take 53 of the 64 bytes per clock a CU can; eight waves, four to a tile, spend what a work-group without the split does.
 // (Four parts of 32 rows: 6 heads of 1344 x 64 11.6 us instead of 12.2, 10 of 356 17.7 instead of 7.9.)
 // (Four K and four V tile buffers with counted waits, so that a tile is requested three steps before its use, made the
 // 4-wave head_dim-64 kernel 5 % slower on small problems: its step is not waiting for tiles.)
@@ -462,7 +464,7 @@ enum SdpaMask { MASK_NONE = 0, MASK_BYTES = 1, MASK_BITS = 2 };
 template <bool BF16, int MASK, int NW, int D, int SPLIT = 1, int PAD = 0>
 __global__ __launch_bounds__(64 * NW, NW == 4 && SPLIT * D < 256 ? 2 : 1) void sdpa_mfma_pipelined_kernel(const SdpaArgs a) {
     static_assert(D == 128 || D == 64, "head sizes with a direct-to-LDS pipeline");
-    static_assert(SPLIT == 1 || (SPLIT == 2 && NW == 4), "key split: two parts, whose tile buffers fit the LDS");
+    static_assert(SPLIT == 1 || SPLIT == 2, "key split: two parts, whose tile buffers fit the LDS");
     constexpr int NWH = NW / SPLIT;       // waves that share a key range
     constexpr int DE = PAD ? PAD : D;     // dims that are computed
     constexpr int KT = (DE + 15) / 16;    // k-steps of the score product
@@ -1909,7 +1911,8 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
 }
 
 template <bool BF16, int MASK, int D, int PAD> void launch_pipelined_as(const SdpaArgs &a, int nw, bool split, unsigned grid, hipStream_t s) {
-    if (nw == 8) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 1, PAD>), dim3(grid), dim3(512), 0, s, a);
+    if (nw == 8 && !split) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 1, PAD>), dim3(grid), dim3(512), 0, s, a);
+    else if (nw == 8) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 2, PAD>), dim3(grid), dim3(512), 0, s, a);
     else if (!split) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 4, D, 1, PAD>), dim3(grid), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 4, D, 2, PAD>), dim3(grid), dim3(256), 0, s, a);
 }
@@ -2104,7 +2107,11 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
             //    (16 heads of 1000 x 64: 14.7 -> 10.7 us; 24 of 260 7.7 -> 9.2); a causal problem has half the keys, so two
             //    rounds still profit (20 heads of 1500: 19.6 -> 14.4).  Beyond 64 dims the two sets of tiles take a CU's LDS
             //    to themselves: one round, and enough keys (8 heads of 500 x 128: 13.5 -> 12.3; of 128 7.7 -> 8.1).
-            //  * pingpong (128 dims, no mask), persistent with 256 rows, where every CU gets a block.
+            //  * key_split8, 128 rows in eight waves, so that every SIMD has two, where those blocks are one round and there are keys
+            //    enough (20 heads of 1500 x 64 23.5 -> 22.1 us, 6 of 2870 34.0 -> 28.5, 20 of 2112 x 2479 x 128 41.6 -> 36.9; 448 keys
+            //    9.7 -> 10.3), or a causal problem long enough that its last rows' blocks decide (16 heads of 3328 x 64 40.1 -> 34.6).
+            //  * pingpong (128 dims, no mask), persistent with 256 rows, where every CU gets a block -- but not a few blocks a second one
+            //    while 128 rows would be one round (30 heads of 2176: 111 us and 78 on pipelined4).
             //  * pipelined4, 128 rows and two work-groups per CU, else -- causal blocks in work-groups of their own, longest
             //    first: in pairs (i, n-1-i) of equal length half of the CUs had nothing to do (8 heads of 832 x 128: 28.0 -> 19.3).
             //  * pipelined8, 256 rows, where that is one round of work-groups and 128 rows would be a round and a part
@@ -2114,11 +2121,14 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
             const int keys = a.causal ? std::min(p.seq_q, p.seq_kv) : p.seq_kv;
             const bool small = p.head_dim <= 64 ? g64 <= (a.causal ? 512 : 256) : g64 <= 256 && (mask || keys >= 384);
             const bool split = p.seq_kv > BN && sdpa_key_split != 0 && (small || sdpa_key_split == 2);
-            const bool pingpong = p.head_dim == 128 && !mask && !split && p.seq_q > 128 && (a.causal ? g256 >= 256 : g128 > 256) && sdpa_pingpong && sdpa_d128_waves != 4;
-            const bool wide = !split && !pingpong && p.seq_q > 128 && sdpa_d128_waves != 4 &&
-                              (sdpa_d128_waves == 8 || (!a.causal && ((g128 > 256 && g256 <= 256) || (p.seq_q <= 192 && g256 >= 256))));
-            const unsigned g = static_cast<unsigned>(split ? g64 : wide || pingpong ? g256 : g128);
-            last_schedule = split ? "key_split" : wide ? "pipelined8" : "pipelined4";
+            const bool split8 = p.seq_kv > BN && sdpa_key_split < 0 && sdpa_d128_waves == 0 && !split &&
+                                (a.causal ? (keys >= 1200 && g128 <= 256) || (keys >= 2000 && g128 <= 448) : keys >= (p.head_dim <= 64 ? 800 : 1000) && g128 <= 256);
+            const bool pingpong = p.head_dim == 128 && !mask && !split && !split8 && p.seq_q > 128 && (a.causal ? g256 >= 256 : g128 > 256 && (g128 > 512 || g256 <= 256)) &&
+                                  sdpa_pingpong && sdpa_d128_waves != 4;
+            const bool wide = split8 || (!split && !pingpong && p.seq_q > 128 && sdpa_d128_waves != 4 &&
+                                         (sdpa_d128_waves == 8 || (!a.causal && ((g128 > 256 && g256 <= 256) || (p.seq_q <= 192 && g256 >= 256)))));
+            const unsigned g = static_cast<unsigned>(split ? g64 : split8 ? g128 : wide || pingpong ? g256 : g128);
+            last_schedule = split ? "key_split" : split8 ? "key_split8" : wide ? "pipelined8" : "pipelined4";
             if (pingpong) {
                 last_schedule = "pingpong";
                 // persistent work-groups, one per CU (a multiple of 8: a (batch, head) keeps its XCD)
@@ -2143,14 +2153,14 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
                     a.mask_plane[1] = mp.planes_h > 1 ? 1 : 0;
                     hipLaunchKernelGGL(sdpa_pack_mask_kernel, dim3(static_cast<unsigned>(mp.planes_b * mp.planes_h * mp.nb32)), dim3(256), 0, s, mask, a.ms[0], a.ms[1],
                                        mp.planes_h, p.seq_q, p.seq_kv, bits, range);
-                    if (bf) launch_pipelined<true, MASK_BITS>(a, nw, split, g, s);
-                    else launch_pipelined<false, MASK_BITS>(a, nw, split, g, s);
+                    if (bf) launch_pipelined<true, MASK_BITS>(a, nw, split || split8, g, s);
+                    else launch_pipelined<false, MASK_BITS>(a, nw, split || split8, g, s);
                 } else if (mask) {
-                    if (bf) launch_pipelined<true, MASK_BYTES>(a, nw, split, g, s);
-                    else launch_pipelined<false, MASK_BYTES>(a, nw, split, g, s);
+                    if (bf) launch_pipelined<true, MASK_BYTES>(a, nw, split || split8, g, s);
+                    else launch_pipelined<false, MASK_BYTES>(a, nw, split || split8, g, s);
                 } else {
-                    if (bf) launch_pipelined<true, MASK_NONE>(a, nw, split, g, s);
-                    else launch_pipelined<false, MASK_NONE>(a, nw, split, g, s);
+                    if (bf) launch_pipelined<true, MASK_NONE>(a, nw, split || split8, g, s);
+                    else launch_pipelined<false, MASK_NONE>(a, nw, split || split8, g, s);
                 }
             }
         }

@@ -644,3 +644,24 @@ def test_packed_masks_with_the_keys_split(dt, D, B, H, S, Skv, causal, planes, o
         qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
         want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, mask[min(b, planes[0] - 1), min(h, planes[1] - 1)])
         assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h)
+
+
+@pytest.mark.parametrize("dt,B,H,Sq,Skv,D,causal,masked", [
+    (F16, 2, 8, 1030, 803, 64, False, False), (BF16, 3, 6, 1000, 1001, 128, False, False), (F16, 1, 7, 2400, 1089, 80, False, False), (BF16, 1, 18, 961, 832, 40, False, False),
+    (BF16, 1, 9, 1985, 1985, 80, True, False), (F16, 1, 16, 2100, 2100, 64, True, False), (BF16, 2, 4, 2177, 1290, 128, True, False),
+    (BF16, 2, 8, 1100, 900, 64, False, True), (F16, 3, 6, 1024, 1100, 128, False, True)])
+def test_eight_waves_that_share_the_keys(dt, B, H, Sq, Skv, D, causal, masked):
+    """128 query rows whose key tiles the two halves of a work-group divide, one round of such work-groups: odd and even numbers of
+    tiles, ragged rows and keys, causal blocks of which one half has nothing, masks with and without the workspace for their bits."""
+    mask = None
+    if masked:
+        mask = (np.random.default_rng(Sq).random((1, 1, Sq, Skv)) < 0.3).astype(np.uint8)
+        mask[..., :7, :] = 1 # (rows that see nothing)
+    q, k, v = inputs(B, H, Sq, Skv, D, dt, seed=Sq + D)
+    for give in (True, False) if masked else (False,):
+        got, _, ran = sdpa_ws(q, k, v, dt, causal, mask, (0, 0), 1, give) if masked else sdpa_ws(q, k, v, dt, causal)
+        assert ran == b"key_split8"
+        for b, h in {(0, 0), (B - 1, H - 1), (B // 2, H // 2)}:
+            qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
+            want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, None if mask is None else mask[0, 0])
+            assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h, give)
