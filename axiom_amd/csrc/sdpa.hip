@@ -1910,6 +1910,52 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
     return m;
 }
 
+// fp32: waves per 32-row query block on sdpa_mfma_f32_kernel (1, 2 or 4), or 0 for sdpa_direct_f32_kernel.
+// The times are in us, start + max(block + key longest, work-groups / 256 (3 block + busy average)): a block of the longest row
+// alone on its CU, or what every CU has to do, where a few work-groups more than fit at once start a round of their own.  Fitted
+// to 320 problems of 64 .. 4096 rows, 6 .. 512 slices (mean error 8 - 12 %), 64 dims and more than those.
+struct F32Schedule { int waves, rows, step, per_cu; float start, block, key, busy, masked; };
+constexpr F32Schedule F32_SCHEDULES[2][4] = {
+    {{0, 16, 256, 2, 2.30f, 1.16f, 0.0085f, 0.0104f, 0.46f}, {4, 32, 128, 2, 2.54f, 1.23f, 0.0278f, 0.0207f, 0.28f},
+     {2, 64, 64, 2, 2.50f, 1.71f, 0.0448f, 0.0372f, 0.37f}, {1, 128, 64, 2, 2.00f, 2.15f, 0.0739f, 0.0875f, 0.52f}},
+    {{0, 16, 128, 2, 3.52f, 1.50f, 0.0179f, 0.0199f, 0.14f}, {4, 32, 128, 1, 3.38f, 2.85f, 0.0439f, 0.0454f, 0.14f},
+     {2, 64, 64, 1, 3.34f, 2.96f, 0.0753f, 0.0827f, 0.20f}, {1, 128, 64, 1, 4.28f, 1.10f, 0.1371f, 0.1853f, 0.23f}}};
+float f32_schedule_time(const AxhipSdpaParams &p, bool masked, const F32Schedule &f) {
+    const float slices = static_cast<float>(p.batch) * static_cast<float>(p.heads), m = masked ? 1.0f + f.masked : 1.0f;
+    const int blocks = (p.seq_q + f.rows - 1) / f.rows, longest = p.is_causal ? std::min(p.seq_kv, p.seq_q) : p.seq_kv;
+    const float groups = slices * static_cast<float>(blocks);
+    float average = static_cast<float>(p.seq_kv); // keys of a block
+    if (p.is_causal) {
+        const float growing = static_cast<float>(std::min(blocks, p.seq_kv / f.rows)), n = static_cast<float>(blocks);
+        average = (static_cast<float>(f.rows) * growing * (growing + 1.0f) * 0.5f + (n - growing) * average) / n;
+    }
+    float time = f.block + f.key * static_cast<float>((longest + f.step - 1) / f.step * f.step) * m;
+    if (groups > 256.0f) {
+        float rounds = groups * (1.0f / 256.0f);
+        if (!p.is_causal) rounds = f.per_cu == 1 ? std::ceil(rounds) : 0.5f * (2.0f * std::ceil(0.5f * rounds) + rounds);
+        time = std::max(time, rounds * (3.0f * f.block + f.busy * average * m));
+    }
+    return f.start + time;
+}
+int f32_schedule(const AxhipSdpaParams &p, bool masked) {
+    // By the blocks alone: the kernel without shared tiles up to one 16-row block per CU (8 heads of 512 rows of 64: 16.3 -> 9.5
+    // us, 8 of 333 x 1000 of 128: 51.5 -> 25.1), else the more waves to a block the fewer blocks there are for the 1024 SIMDs
+    const int64_t slices = static_cast<int64_t>(p.batch) * p.heads, blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * slices, blocks32 = static_cast<int64_t>((p.seq_q + 31) / 32) * slices;
+    const int usual = blocks16 <= 256 && p.head_dim > 32 ? 0 : blocks32 >= 1536 ? 3 : blocks32 >= 768 ? 2 : 1; // (of the table)
+    const F32Schedule *table = F32_SCHEDULES[p.head_dim > 64];
+    if (p.head_dim <= 32) return table[usual].waves;
+    // ... unless another one is to win an eighth by its time (30 heads of 258 x 80: 43 -> 22 us without shared tiles, 8 of 700 x 64 causal
+    // 22.2 -> 12.3, 40 of 260 x 128 44.9 -> 31.0 with two waves; the 320 problems 0.92 of the time, the worst 1.09)
+    int best = usual;
+    float least = 0.88f * f32_schedule_time(p, masked, table[usual]);
+    for (int i = 0; i < 4; ++i) {
+        if (i == usual || (table[i].waves == 0 && !launch_fits(blocks16, 64 * DIRECT_WAVES))) continue;
+        const float t = f32_schedule_time(p, masked, table[i]);
+        if (t < least) { least = t; best = i; }
+    }
+    return table[best].waves;
+}
+
 template <bool BF16, int MASK, int D, int PAD> void launch_pipelined_as(const SdpaArgs &a, int nw, bool split, unsigned grid, hipStream_t s) {
     if (nw == 8 && !split) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 1, PAD>), dim3(grid), dim3(512), 0, s, a);
     else if (nw == 8) hipLaunchKernelGGL((sdpa_mfma_pipelined_kernel<BF16, MASK, 8, D, 2, PAD>), dim3(grid), dim3(512), 0, s, a);
@@ -2168,20 +2214,12 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
         }
     } else if (kind == SdpaKind::MFMA_F32) {
         last_schedule = "mfma_f32";
-        // waves per 32-row query block, by how many such blocks there are for the 1024 SIMDs (thresholds from timings
-        // of 128 .. 1024 blocks: below 0.75 blocks per SIMD the four-way split wins by up to 2.7x, above 1.5 none is needed)
-        // Up to one 16-row block per CU the kernel without shared tiles is the faster one (8 heads of 512 rows of 64: 16.3 ->
-        // 9.5 us, causal 16.2 -> 9.6, masked 17.9 -> 13.0; 8 of 333 x 1000 of 128: 51.5 -> 25.1); with 512 blocks its reads
-        // of K and V by every block cost more than the idle CUs did (16 heads of 512: 16.6 and 19.6 us).
-        const int64_t blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * p.batch * p.heads;
-        if (blocks16 <= 256 && p.head_dim > 32 && sdpa_f32_split == 0) {
+        const int split = sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4 ? sdpa_f32_split : f32_schedule(p, mask != nullptr);
+        if (split == 0) {
             last_schedule = "direct";
             a.nqb = (p.seq_q + 15) / 16;
             return launch_sdpa_direct_f32(a, s);
         }
-        const int64_t blocks32 = static_cast<int64_t>((p.seq_q + 31) / 32) * p.batch * p.heads;
-        int split = blocks32 >= 1536 ? 1 : blocks32 >= 768 ? 2 : 4;
-        if (sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4) split = sdpa_f32_split;
         const int bmw = 128 / split;
         a.nqb = (p.seq_q + bmw - 1) / bmw;
         AXHIP_REQUIRE(launch_fits(static_cast<int64_t>(a.nqb) * p.batch * p.heads, 256), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");

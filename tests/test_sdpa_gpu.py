@@ -665,3 +665,19 @@ def test_eight_waves_that_share_the_keys(dt, B, H, Sq, Skv, D, causal, masked):
             qs, ks, vs = (axo.to_f32(t[b:b + 1, h:h + 1], dt) for t in (q, k, v))
             want = naive_attention64(qs, ks, vs, 1 / math.sqrt(D), causal, None if mask is None else mask[0, 0])
             assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h, give)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D,causal,masked,schedule", [
+    (5, 6, 258, 258, 80, False, False, b"direct"), (1, 8, 700, 700, 64, True, False, b"direct"), (5, 6, 258, 261, 128, False, True, b"direct"),
+    (2, 20, 260, 260, 128, False, False, b"mfma_f32"), (4, 12, 300, 300, 64, False, True, b"mfma_f32"), (16, 20, 64, 64, 100, True, False, b"mfma_f32"), (1, 9, 449, 1031, 96, True, False, b"direct")])
+def test_f32_schedules_by_their_time(B, H, Sq, Skv, D, causal, masked, schedule):
+    """More 16-row blocks than CUs without shared tiles, and blocks that two waves share instead of four: where the time of a schedule
+    decides instead of the number of blocks."""
+    from axiom_amd import capi
+
+    mask = (np.random.default_rng(Sq).random((Sq, Skv)) < 0.3).astype(np.uint8) if masked else None
+    q, k, v = inputs(B, H, Sq, Skv, D, F32, seed=Sq + D)
+    got, _ = gh.sdpa(q, k, v, F32, -1.0, causal, mask)
+    assert capi.lib().axhip_sdpa_last_schedule() == schedule
+    want = naive_attention64(q, k, v, 1 / math.sqrt(D), causal, mask)
+    assert np.max(np.abs(got - want)) < 1e-4
