@@ -114,8 +114,10 @@ struct TransposeArgs {
 };
 
 // The same for equal 2- or 4-byte element types, in whole 16-byte vectors on both sides (LG / SG = 16: extents, strides
-// and bases are multiples of a vector; 8: of half a vector, e.g. the 3000-byte rows of a [.., 1500] 16-bit array; ES: of
-// nothing -- vectors are unaligned, the last one of a row is fetched as the 16 bytes that end with it and shifted into
+// and bases are multiples of a vector; 8: of half a vector, e.g. the 3000-byte rows of a [.., 1500] 16-bit array -- one unaligned
+// access for each vector, only the half of one that a row may end with by itself: as two aligned halves each, the store pass wrote
+// every line twice and a load pass twice the addresses (bf16 [32, 1500, 1280] 59.4 -> 53.7 us, [32, 1500, 1500] 84 -> 67.6, [425, 868, 132]
+// 56.5 -> 42.6); ES: of nothing -- vectors are unaligned, the last one of a row is fetched as the 16 bytes that end with it and shifted into
 // place, and leaves in pieces).  Tiles of NV x NV vectors: 128 x 128 16-bit or 64 x 64 32-bit elements with NV = 16,
 // 256-byte runs on the read and on the write side.  A thread reads vectors along J, scatters their elements as 32-bit
 // words into a tile that is stored transposed (16-bit: two neighbouring rows of L packed into one word first), and the
@@ -129,9 +131,9 @@ __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs 
         if constexpr (LG == 16) {
             return n > 0 ? *reinterpret_cast<const uint4_t *>(at) : uint4_t{0, 0, 0, 0};
         } else if constexpr (LG == 8) {
+            if (n >= V) return vec_load<true>(reinterpret_cast<const uint4_t *>(at));
             const uint2_t lo = n > 0 ? *reinterpret_cast<const uint2_t *>(at) : uint2_t{0, 0};
-            const uint2_t hi = n > V / 2 ? *reinterpret_cast<const uint2_t *>(at + 8) : uint2_t{0, 0};
-            return uint4_t{lo.x, lo.y, hi.x, hi.y};
+            return uint4_t{lo.x, lo.y, 0, 0};
         } else {
             if (n <= 0) return uint4_t{0, 0, 0, 0};
             const int drop = n >= V ? 0 : V - static_cast<int>(n);
@@ -211,8 +213,8 @@ __global__ __launch_bounds__(256) void transpose_vec_kernel(const TransposeArgs 
         if constexpr (SG == 16) {
             if (l_left > 0) *reinterpret_cast<uint4_t *>(to) = v;
         } else if constexpr (SG == 8) {
-            if (l_left > 0) *reinterpret_cast<uint2_t *>(to) = uint2_t{v.x, v.y};
-            if (l_left > V / 2) *reinterpret_cast<uint2_t *>(to + 8) = uint2_t{v.z, v.w};
+            if (l_left >= V) vec_store<true>(reinterpret_cast<uint4_t *>(to), v);
+            else if (l_left > 0) *reinterpret_cast<uint2_t *>(to) = uint2_t{v.x, v.y};
         } else if (l_left >= V) {
             vec_store<true>(reinterpret_cast<uint4_t *>(to), v);
         } else if (l_left > 0) { // 8, 4 and 2 bytes
@@ -1630,7 +1632,7 @@ int axhip_strided_copy(const void *src, int32_t src_dtype, void *dst, int32_t ds
         if (whole && vec_tiles) {
             // Rows of the output that start inside a 128-byte line make neighbouring tiles write parts of the same lines:
             // such tiles go to one XCD, whose L2 puts the parts together, and are smaller, so that it still holds them
-            // (bf16 [32, 1500, 1280] 70.8 us in the other order, 60.9 with large tiles, 59.3 with small ones; fp32 130,
+            // (bf16 [32, 1500, 1280] 69.7 us in the other order, 56.4 with large tiles, 53.6 with small ones; fp32 130,
             // 113, 98).  Rows of whole lines take large tiles along a diagonal over all XCDs (bf16 [8, 4096, 4096] 96 us
             // against 117).  Extents of one large tile or less: small ones waste fewer lanes (bf16 [2000, 64, 130] 25 ->
             // 17 us), except that fp32's 32 elements are too few (fp32 [5000, 33, 65] 30 us against 40).
