@@ -1012,7 +1012,7 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 // products of m 9 .. 8192, n 64 .. 4096, k 64 .. 4096 (mean error 5 - 8 %); on average the one picked is
 // 2 % slower than the fastest, and 2.3 times as fast as the ring and FMA kernels, which had these products to themselves:
 // 99 x 1024 x 5120 104 -> 18 us, 186 x 640 x 958 35 -> 8, 48 x 384 x 2048 77 -> 6.3.  Large products with both operands
-// along k stay on the ring: 2048^3 134 us against 188.
+// along k stay on the ring: 2048^3 97 us against 188.
 struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
     {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f},
