@@ -1911,15 +1911,16 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
 }
 
 // fp32: waves per 32-row query block on sdpa_mfma_f32_kernel (1, 2 or 4), or 0 for sdpa_direct_f32_kernel.
-// The times are in us, start + max(block + key longest, work-groups / 256 (3 block + busy average)): a block of the longest row
-// alone on its CU, or what every CU has to do, where a few work-groups more than fit at once start a round of their own.  Fitted
-// to 320 problems of 64 .. 4096 rows, 6 .. 512 slices (mean error 8 - 12 %), 64 dims and more than those.
-struct F32Schedule { int waves, rows, step, per_cu; float start, block, key, busy, masked; };
+// The times are in us, start + max(block + key longest, rounds (round + busy average)): a block of the longest row alone on its CU,
+// or what every CU has to do, in whole rounds of 256 work-groups (two that share a CU take twice the time); causal blocks, unequal
+// as they are, go on without rounds and take `causal` more.  Fitted to 368 problems of 64 .. 4096 rows, 6 .. 512 slices (mean error
+// 6 - 11 %), 64 dims and more than those.
+struct F32Schedule { int waves, rows, step; float start, block, key, round, busy, causal, masked; };
 constexpr F32Schedule F32_SCHEDULES[2][4] = {
-    {{0, 16, 256, 2, 2.30f, 1.16f, 0.0085f, 0.0104f, 0.46f}, {4, 32, 128, 2, 2.54f, 1.23f, 0.0278f, 0.0207f, 0.28f},
-     {2, 64, 64, 2, 2.50f, 1.71f, 0.0448f, 0.0372f, 0.37f}, {1, 128, 64, 2, 2.00f, 2.15f, 0.0739f, 0.0875f, 0.52f}},
-    {{0, 16, 128, 2, 3.52f, 1.50f, 0.0179f, 0.0199f, 0.14f}, {4, 32, 128, 1, 3.38f, 2.85f, 0.0439f, 0.0454f, 0.14f},
-     {2, 64, 64, 1, 3.34f, 2.96f, 0.0753f, 0.0827f, 0.20f}, {1, 128, 64, 1, 4.28f, 1.10f, 0.1371f, 0.1853f, 0.23f}}};
+    {{0, 16, 256, 2.88f, 0.0f, 0.0101f, 3.26f, 0.0098f, 0.13f, 0.55f}, {4, 32, 128, 3.92f, 0.0f, 0.0263f, 3.26f, 0.0178f, 0.25f, 0.37f},
+     {2, 64, 64, 4.25f, 0.0f, 0.0435f, 3.73f, 0.0319f, 0.39f, 0.47f}, {1, 128, 64, 4.15f, 0.0f, 0.0736f, 5.25f, 0.0629f, 0.44f, 0.62f}},
+    {{0, 16, 128, 3.98f, 0.58f, 0.0194f, 4.03f, 0.0189f, 0.18f, 0.22f}, {4, 32, 128, 6.04f, 0.0f, 0.0441f, 7.09f, 0.0431f, 0.20f, 0.19f},
+     {2, 64, 64, 6.21f, 0.0f, 0.0751f, 7.31f, 0.0726f, 0.30f, 0.26f}, {1, 128, 64, 5.21f, 0.0f, 0.1378f, 8.10f, 0.1331f, 0.41f, 0.25f}}};
 float f32_schedule_time(const AxhipSdpaParams &p, bool masked, const F32Schedule &f) {
     const float slices = static_cast<float>(p.batch) * static_cast<float>(p.heads), m = masked ? 1.0f + f.masked : 1.0f;
     const int blocks = (p.seq_q + f.rows - 1) / f.rows, longest = p.is_causal ? std::min(p.seq_kv, p.seq_q) : p.seq_kv;
@@ -1931,9 +1932,8 @@ float f32_schedule_time(const AxhipSdpaParams &p, bool masked, const F32Schedule
     }
     float time = f.block + f.key * static_cast<float>((longest + f.step - 1) / f.step * f.step) * m;
     if (groups > 256.0f) {
-        float rounds = groups * (1.0f / 256.0f);
-        if (!p.is_causal) rounds = f.per_cu == 1 ? std::ceil(rounds) : 0.5f * (2.0f * std::ceil(0.5f * rounds) + rounds);
-        time = std::max(time, rounds * (3.0f * f.block + f.busy * average * m));
+        const float rounds = groups * (1.0f / 256.0f);
+        time = std::max(time, p.is_causal ? rounds * (f.round + f.busy * (1.0f + f.causal) * average * m) : std::ceil(rounds) * (f.round + f.busy * average * m));
     }
     return f.start + time;
 }
@@ -1943,9 +1943,9 @@ int f32_schedule(const AxhipSdpaParams &p, bool masked) {
     const int64_t slices = static_cast<int64_t>(p.batch) * p.heads, blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * slices, blocks32 = static_cast<int64_t>((p.seq_q + 31) / 32) * slices;
     const int usual = blocks16 <= 256 && p.head_dim > 32 ? 0 : blocks32 >= 1536 ? 3 : blocks32 >= 768 ? 2 : 1; // (of the table)
     const F32Schedule *table = F32_SCHEDULES[p.head_dim > 64];
-    if (p.head_dim <= 32) return table[usual].waves;
+    if (p.head_dim <= 32 || (p.is_causal && masked)) return table[usual].waves; // (no times of these)
     // ... unless another one is to win an eighth by its time (30 heads of 258 x 80: 43 -> 22 us without shared tiles, 8 of 700 x 64 causal
-    // 22.2 -> 12.3, 40 of 260 x 128 44.9 -> 31.0 with two waves; the 320 problems 0.92 of the time, the worst 1.09)
+    // 22.2 -> 12.3, 40 of 260 x 128 44.9 -> 31.0 with two waves; 220 other problems 0.93 of the time, the worst 1.02)
     int best = usual;
     float least = 0.88f * f32_schedule_time(p, masked, table[usual]);
     for (int i = 0; i < 4; ++i) {
