@@ -1015,8 +1015,8 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 // along k stay on the ring: 2048^3 97 us against 188.
 struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
-    {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f},
-    {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f}, {5.30f, 0.00701f, 0.00159f, 3.70f, 0.00106f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}};
+    {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f}, {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f},
+    {4.59f, 0.00939f, 0.00112f, 3.91f, 0.00138f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}, {5.30f, 0.00701f, 0.00159f, 3.70f, 0.00106f}};
 
 template <size_t I> void consider_f32_kernel(const AxhipGemmParams &p, float k, float u, bool ring, int &best, float &best_cost) {
     constexpr F32Kernel h = F32_KERNELS[I];

@@ -497,8 +497,8 @@ def test_batches_are_dealt_over_all_xcds(dtype, nn, M, N, K, batch, shared):
 
 
 # k from 32 to 8192 on every tile that multiplies parts: 32 x 64 and 64 x 64 (few output tiles), 64 x 128 and 128 x 128, with rows,
-# columns and k that end inside a tile, a chunk and a pair of k-tiles
-PARTS = [(300, 1280, 1285, 1), (130, 1984, 2050, 1), (1024, 1020, 1023, 1), (1000, 1028, 1090, 1), (257, 4100, 700, 1), (513, 132, 995, 8), (2048, 2044, 225, 1), (1153, 129, 256, 16)]
+# columns and k that end inside a tile, a chunk and a pair of k-tiles; the last is short enough for fp32 products on 32 x 64
+PARTS = [(300, 1280, 1285, 1), (130, 1984, 2050, 1), (1024, 1020, 1023, 1), (1000, 1028, 1090, 1), (257, 4100, 700, 1), (513, 132, 995, 8), (2048, 2044, 225, 1), (1153, 129, 256, 16), (64, 241, 145, 32)]
 
 
 @pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
