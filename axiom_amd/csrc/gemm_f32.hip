@@ -29,7 +29,7 @@ template <bool NN, bool SPLIT, int MI, int NJ, int P> constexpr int direct_lds_b
 // SPLIT: by products of bf16 parts (gemm_f32_split.hpp), each wavefront splitting what it multiplies.  That pays at 32 x 64, where
 // eight fragments' splitting, 1250 cycles, stands for 2048 of fp32 MFMAs (333 x 1280 x 1280 18.0 -> 15.1 us, 64 x 1280 x 5120 on
 // these tiles 54 -> 45), once there is k enough for its longer end (32 x (64 x 240 x 145) 6.5 us with fp32 products, 6.95 with parts; about equal at
-// k = 370); 32 x 32 and below have no more MFMAs than splitting to do (64 x 1280 x 5120 28.2 and 28.1, 512^3
+// k = 500); 32 x 32 and below have no more MFMAs than splitting to do (64 x 1280 x 5120 28.2 and 28.1, 512^3
 // 6.0 and 6.6), and the fragments of 64 x 64 do not fit the registers.
 template <bool NN, bool SPLIT, int MI, int NJ, int P>
 __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(const TileArgs g) {
