@@ -386,11 +386,9 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // 32 rows, 8 k at a time, is 512 bytes, 16 a row (the row XOR-ed so that what 32 lanes write at a time meets all banks).
 // The multiplying ones, one per SIMD, hold all fragments of 32 k and refill them under the MFMAs of blocks that need them no
 // more.  Barrier kt: k-tile kt is in LDS and k-tile kt - 1 has been read.
-// What bounds it: with few work-groups the splitting (a k-tile of 128 x 128 x 32 on 64 CUs 2470 cycles, 2040 without MFMAs,
-// of which the MFMAs are 1536), with all CUs at work the power limit (3400 of the same cycles).  64 x 64 has two loading wavefronts per
-// SIMD for that reason (1024^3 22.5 us with one, 19.4 with two), and 64 k at a time for half the barriers.  v_mfma_f32_16x16x32, which leaves
-// less room beside it, took 3 % less on full chips and 10 % more on others.
-// 1024^3 22.2 -> 19.3 us, 2048^3 135 -> 97, 4096 x 2000 x 1000 138 -> 105.
+// 64 x 64 has two loading wavefronts per SIMD (1024^3 22.5 us with one, 19.4 with two, of six products) and 64 k at a time for half the barriers.
+// v_mfma_f32_16x16x32, which leaves less room beside it, took 3 % less on full chips and 10 % more on others.
+// 1024^3 21.6 -> 21.0 us, 2048^3 133 -> 113, 4096 x 2000 x 1000 134 -> 118, 4096^3 1014 -> 832 (with six of the products, to fewer bits: 18.9, 94, 100, 697).
 template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: floats per k-tile; LW: loading wavefronts
     static constexpr int MI = TM / 64, NJ = TNR / 64, DEPTH = KF == 32 || LW == 8 ? 3 : 2;
     static constexpr int CHUNKS = KF / 4, ROWS = WAVE / CHUNKS * LW;      // 16-byte chunks of a row along k, rows that the loading wavefronts fetch at a time
@@ -505,39 +503,44 @@ template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: fl
         // KF = 32, four blocks: the fragments of one are dead long before the next k-tile needs them.  KF = 64: the halves of a k-tile in turn
         constexpr int SLOTS = KF / 32, BLOCKS = MI * NJ;
         static_assert(SLOTS == 1 ? MI == 2 && NJ == 2 : MI == 1, "blocks");
-        uint4_t fa[SLOTS][MI][2][3], fb[SLOTS][NJ][2][3];
-        int a_off[SLOTS][MI][2], b_off[SLOTS][NJ][2];
+        uint4_t fa[SLOTS][MI][2][2], fb[SLOTS][NJ][2][2], fa_last[MI][2], fb_last[NJ][2]; // (the last parts are used first: one set of registers for both halves)
+        auto frag_a = [&](int h, int i, int ks, int part) __attribute__((always_inline)) -> uint4_t & { return part == 2 ? fa_last[i][ks] : fa[h][i][ks][part & 1]; };
+        auto frag_b = [&](int h, int j, int ks, int part) __attribute__((always_inline)) -> uint4_t & { return part == 2 ? fb_last[j][ks] : fb[h][j][ks][part & 1]; };
+        // One offset for a block of 32 rows, from which those of the other k of a k-tile are made: at(r, kc + 4) = (at(r, kc) ^ 32) + 2048, at(r, kc + 2) =
+        // (at(r, kc) ^ 128) + 1024.  (The stage is in it before the XOR, so that all of them are not kept, in registers that the fragments need.)
+        int a_off[MI], b_off[NJ];
 #pragma unroll
-        for (int h = 0; h < SLOTS; ++h)
+        for (int i = 0; i < MI; ++i) a_off[i] = at(wm + 32 * i + l32, g2);
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-                for (int i = 0; i < MI; ++i) a_off[h][i][ks] = at(wm + 32 * i + l32, 4 * h + 2 * ks + g2);
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) b_off[h][j][ks] = 3 * PLANE_A + at(wn + 32 * j + l32, 4 * h + 2 * ks + g2);
-            }
-        auto read_a = [&](int h, const unsigned char *stage, int i, int n) __attribute__((always_inline)) { // n: 3 ks + part
-            fa[h][i][n / 3][n % 3] = *reinterpret_cast<const uint4_t *>(stage + a_off[h][i][n / 3] + n % 3 * PLANE_A);
+        for (int j = 0; j < NJ; ++j) b_off[j] = 3 * PLANE_A + at(wn + 32 * j + l32, g2);
+        static_assert(STAGEB % 512 == 0 && PLANE_A % 512 == 0, "the XOR is of the bits below 512");
+        auto read_a = [&](int h, int stage, int i, int n) __attribute__((always_inline)) { // n: 3 ks + part
+            frag_a(h, i, n / 3, n % 3) = *reinterpret_cast<const uint4_t *>(lds + (((stage + a_off[i]) ^ (h * 32 + n / 3 * 128)) + h * 2048 + n / 3 * 1024 + n % 3 * PLANE_A));
         };
-        auto read_b = [&](int h, const unsigned char *stage, int j, int n) __attribute__((always_inline)) {
-            fb[h][j][n / 3][n % 3] = *reinterpret_cast<const uint4_t *>(stage + b_off[h][j][n / 3] + n % 3 * PLANE_B);
+        auto read_b = [&](int h, int stage, int j, int n) __attribute__((always_inline)) {
+            frag_b(h, j, n / 3, n % 3) = *reinterpret_cast<const uint4_t *>(lds + (((stage + b_off[j]) ^ (h * 32 + n / 3 * 128)) + h * 2048 + n / 3 * 1024 + n % 3 * PLANE_B));
         };
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) sum[i][j] = float16_t{};
-        float16_t t[2] = {float16_t{}, float16_t{}};
-        // block (i, j) of 32 k: twelve MFMAs, behind MFMA x what `between` does; the block before is added to its sum meanwhile
+        float16_t first[2] = {float16_t{}, float16_t{}}, rest{};
+        // block (i, j) of 32 k: sixteen MFMAs, behind MFMA x what `between` does.  The products of first parts, then, in a chain of their own, the rest;
+        // under the next block's MFMAs the two are added up, and to the sum of their block (`before`)
         auto block = [&](int h, int i, int j, float16_t &before, auto between) __attribute__((always_inline)) {
             const int turn = BLOCKS > 1 ? (i * NJ + j) & 1 : h;
 #pragma unroll
-            for (int x = 0; x < 12; ++x) {
+            for (int x = 0; x < 2 * SPLIT_PRODUCTS; ++x) {
                 const int n = x / 2, ks = x % 2;
-                t[turn] = mfma(fa[h][i][ks][SPLIT_A[n]], fb[h][j][ks][SPLIT_B[n]], x == 0 ? float16_t{} : t[turn]);
+                if (x < 2) first[turn] = mfma(frag_a(h, i, ks, SPLIT_A[n]), frag_b(h, j, ks, SPLIT_B[n]), x == 0 ? float16_t{} : first[turn]);
+                else rest = mfma(frag_a(h, i, ks, SPLIT_A[n]), frag_b(h, j, ks, SPLIT_B[n]), x == 2 ? float16_t{} : rest);
                 __builtin_amdgcn_sched_barrier(0);
-                if (x >= 3 && x < 11) {
+                if (x < 2) {
 #pragma unroll
-                    for (int e = 2 * (x - 3); e < 2 * (x - 3) + 2; ++e) before[e] += t[turn ^ 1][e];
+                    for (int e = 8 * x; e < 8 * x + 8; ++e) first[turn ^ 1][e] += rest[e];
+                } else if (x >= 3 && x < 11) {
+#pragma unroll
+                    for (int e = 2 * (x - 3); e < 2 * (x - 3) + 2; ++e) before[e] += first[turn ^ 1][e];
                 }
                 between(x);
                 __builtin_amdgcn_sched_barrier(0);
@@ -547,11 +550,11 @@ template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: fl
         if constexpr (SLOTS == 1) {
 #pragma unroll
             for (int n = 0; n < 6; ++n) {
-                read_a(0, lds, 0, n);
-                read_b(0, lds, 0, n);
+                read_a(0, 0, 0, n);
+                read_b(0, 0, 0, n);
             }
             for (int kt = 0; kt < nk; ++kt) {
-                const unsigned char *cur = lds + (kt & 1) * STAGEB, *next = lds + ((kt & 1) ^ 1) * STAGEB;
+                const int cur = (kt & 1) * STAGEB, next = STAGEB - cur;
                 block(0, 0, 0, sum[1][1], [&](int x) __attribute__((always_inline)) {
                     if (x < 6) read_b(0, cur, 1, x);
                     else read_a(0, cur, 1, x - 6);
@@ -565,31 +568,34 @@ template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: fl
                     if (x < 6) read_b(0, next, 0, x);
                 });
             }
-            sum[1][1] += t[1];
+            sum[1][1] += first[1] + rest;
         } else {
             float16_t odd[NJ]; // the second halves' sums: two chains of K / 64 additions
 #pragma unroll
             for (int j = 0; j < NJ; ++j) odd[j] = float16_t{};
-            auto half = [&](int h, const unsigned char *stage) __attribute__((always_inline)) { // multiplies half h and reads the other one from `stage`
+            auto half = [&](int h, int stage) __attribute__((always_inline)) { // multiplies half h and reads the other one from `stage`
 #pragma unroll
                 for (int j = 0; j < NJ; ++j)
                     block(h, 0, j, j == 0 ? (h == 0 ? odd[NJ - 1] : sum[0][NJ - 1]) : (h == 0 ? sum[0][j - 1] : odd[j - 1]), [&](int x) __attribute__((always_inline)) {
-                        if (j == 0 && x < 6) read_a(h ^ 1, stage, 0, x);
-                        if (j == 0 && x < 6 * NJ) read_b(h ^ 1, stage, x / 6, x % 6);
+                        if (j == 0 && x < 4) read_a(h ^ 1, stage, 0, x / 2 * 3 + x % 2);
+                        if (j == 0 && x < 4 * NJ) read_b(h ^ 1, stage, x / 4, x % 4 / 2 * 3 + x % 2);
+                        // (behind their last use, of SPLIT_B by MFMA 7 and of SPLIT_A by MFMA 9)
+                        if (x == 8 || x == 9) read_b(h ^ 1, stage, j, (x - 8) * 3 + 2);
+                        if (j == NJ - 1 && (x == 10 || x == 11)) read_a(h ^ 1, stage, 0, (x - 10) * 3 + 2);
                     });
             };
 #pragma unroll
             for (int n = 0; n < 6; ++n) {
-                read_a(0, lds, 0, n);
+                read_a(0, 0, 0, n);
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) read_b(0, lds, j, n);
+                for (int j = 0; j < NJ; ++j) read_b(0, 0, j, n);
             }
             for (int kt = 0; kt < nk; ++kt) {
-                half(0, lds + (kt & 1) * STAGEB);
+                half(0, (kt & 1) * STAGEB);
                 __syncthreads(); // barrier kt + 1
-                half(1, lds + ((kt & 1) ^ 1) * STAGEB);
+                half(1, ((kt & 1) ^ 1) * STAGEB);
             }
-            odd[NJ - 1] += t[1];
+            odd[NJ - 1] += first[1] + rest;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) sum[0][j] += odd[j];
         }
@@ -609,10 +615,8 @@ __global__ __launch_bounds__(64 * (4 + LW), 1) void gemm_mfma_f32_ring_kernel(co
     constexpr int NLA = TM / 32, NLB = TNR / 32, NL = NLA + NLB; // loads of 1 KiB per wavefront and k-tile
     constexpr int RK = 32, S = RING_STAGES, STAGEB = (TM + TNR) * BIG_ROWB; // (fp32 products: floats per k-tile, stages)
     extern __shared__ __attribute__((aligned(1024))) unsigned char big_lds[];
-    const int tid = threadIdx.x, lane = tid % WAVE;
-    const int wavefront = __builtin_amdgcn_readfirstlane(tid / WAVE), wave = wavefront % 4;
+    const int wavefront = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), wave = wavefront % 4;
     const bool loader = wavefront >= 4;
-    const int l32 = lane % 32, g2 = lane / 32;
 
     int product;
     const int t = tile_of_work_group(tiles_m * tiles_n, g.batch, product);
@@ -641,9 +645,9 @@ __global__ __launch_bounds__(64 * (4 + LW), 1) void gemm_mfma_f32_ring_kernel(co
         using Split = SplitRing<TM, TNR, KF, LW, NN>;
         bool failed = false;
         if (loader) {
-            Split::load(g, A, B, rows_a, rows_b, big_lds, wavefront - 4, lane);
+            Split::load(g, A, B, rows_a, rows_b, big_lds, wavefront - 4, lane_again());
         } else {
-            Split::multiply(K, big_lds, wm, wn, lane, sum);
+            Split::multiply(K, big_lds, wm, wn, lane_again(), sum);
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -654,8 +658,9 @@ __global__ __launch_bounds__(64 * (4 + LW), 1) void gemm_mfma_f32_ring_kernel(co
                         sum[i][j][e] *= SPLIT_UNSCALE;
                     }
         }
-        fp32_products = work_group_any<4 + LW>(failed, reinterpret_cast<uint32_t *>(big_lds + split_lds_bytes<TM, TNR, KF, LW>() - 64));
+        fp32_products = work_group_any<4 + LW>(failed, reinterpret_cast<uint32_t *>(big_lds + split_lds_bytes<TM, TNR, KF, LW>() - 64), wavefront, lane_again());
     }
+    const int lane = KF == 0 ? static_cast<int>(threadIdx.x % WAVE) : lane_again(), l32 = lane % 32, g2 = lane / 32;
     if (fp32_products) {
     const int ld_r = 8 * wave + (lane >> 3);
     const int ld_k = 4 * ((lane & 7) ^ ((ld_r >> 1) & 7)); // this lane's chunk of a row along k: floats ld_k .. ld_k + 3 of the k-tile

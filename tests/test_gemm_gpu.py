@@ -526,6 +526,31 @@ def test_f32_products_of_parts(nn, M, N, K, batch):
 
 @pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
 @pytest.mark.parametrize("M,N,K,batch", PARTS)
+def test_f32_products_of_parts_with_one_product_to_an_output(nn, M, N, K, batch):
+    """Rows of x with a single entry: the result is one product, rounded once.  By parts the last addition rounds by half
+    an ulp and the seven before it, of numbers below 2^-5 where the result is 1 or more, by 2^-30 each at most: 0.5 + 7 / 128 ulp.  Among
+    random factors some whose second and third parts are as large as they get (0x1.01ffp0 squared is 2 ulp off without their products)."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + 3 * N + K)
+    x, W = torch.zeros((batch, M, K), device="cuda"), torch.empty((batch, K, N) if nn else (batch, N, K), device="cuda").normal_(generator=gen)
+    at = torch.randint(0, K, (batch, M, 1), device="cuda", generator=gen)
+    value = torch.empty((batch, M, 1), device="cuda").normal_(generator=gen)
+    hard = float.fromhex("0x1.01ffp0")
+    value[:, ::3] = hard
+    (W[:, :, ::3] if nn else W[:, ::3]).fill_(hard)
+    x.scatter_(2, at, value)
+    c = _f32_product(x, W, nn)
+    for b in range(0, batch, 5):
+        want = value[b].double() * (W[b].t() if not nn else W[b]).contiguous()[at[b, :, 0]].double()
+        nearest = want.float().abs()
+        ulp = (torch.nextafter(nearest, torch.full_like(nearest, float("inf"))) - nearest).double()
+        assert bool(((c[b].double() - want).abs() <= (0.5 + 7 / 128) * ulp).all())
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch", PARTS)
 def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch):
     """Infinities, NaN and numbers near the largest, whose parts have none: the same places of the result are infinite or NaN as in
     float64, and everything else keeps its bound, in the tiles that are computed again and in the others."""
