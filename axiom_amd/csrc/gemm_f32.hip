@@ -31,23 +31,6 @@ template <bool NN, bool SPLIT, int MI, int NJ, int P> constexpr int direct_lds_b
 // is k enough for its longer end (32 x (64 x 240 x 145) 6.5 us with fp32 products, 6.95 with parts); 32 x 32 and below have no more
 // MFMAs than splitting to do (64 x 1280 x 5120 28.2 and 28.1, 512^3 6.0 and 6.6, with six products), and the fragments of
 // 64 x 64 do not fit the registers.
-template <bool NN, bool SPLIT, int MI, int NJ, int P> constexpr int direct_lds_bytes() { // the stages or the sums (SPLIT: and a flag of each wavefront)
-    const int stages = F32_WAVES * P * 2 * (MI + (NN ? 0 : NJ)) * 1024, sum = F32_WAVES * MI * NJ * 1024;
-    return (stages > sum ? stages : sum) + (SPLIT ? 64 : 0);
-}
-
-// C = A B (b [N, K], or [K, N]: NN) on v_mfma_f32_16x16x4_f32: fp32 products and sums.  Work-group tile 16 MI x 16 NJ;
-// eight wavefronts take pieces of 32 P elements of k in turn and add their sums through LDS at the end; until then no
-// wavefront waits for another.
-// The fp32 matrix rate is a sixteenth of the 16-bit one, so an operand that comes from the caches for every tile costs
-// little next to the MFMAs it feeds.  Rows along k (a, and b as [N, K]) pass through a stage of LDS that is the
-// wavefront's own, so that they are loaded in whole 128-byte lines (as fragments, 16 bytes of each of 16 rows side by
-// side, they took four times the address cycles: 1024^3 28.5 us); b as [K, N] needs no stage and no transpose: which
-// column a lane contributes to which MFMA is free, so lane (l16, g) loads the NJ columns NJ l16 .. of rows 4 g .. 4 g + 3.
-// Bound by the matrix pipe at 64 x 64 and by latency below, where narrower tiles put more CUs to work.
-// SPLIT: by products of bf16 parts (gemm_f32_split.hpp), each wavefront splitting what it multiplies.  That pays at 32 x 64, where
-// eight fragments' splitting, 1250 cycles, stands for 2048 of fp32 MFMAs (333 x 1280 x 1280 18.1 -> 15.2 us), once there is k enough for its longer end (32 x (64 x 240 x 145) 6.5 us with fp32 products, 6.95 with parts); 32 x 32 and below have no more MFMAs than splitting to do (64 x 1280 x 5120 28.2 and 28.1, 512^3
-// 6.0 and 6.6, with six products), and the fragments of 64 x 64 do not fit the registers.
 template <bool NN, bool SPLIT, int MI, int NJ, int P>
 __global__ __launch_bounds__(64 * F32_WAVES, 2) void gemm_f32_direct_kernel(const TileArgs g) {
     extern __shared__ __attribute__((aligned(1024))) float sums[];
