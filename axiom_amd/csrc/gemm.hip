@@ -986,9 +986,9 @@ enum RingTile { RING_64x64, RING_64x128, RING_128x128_PARTS, RING_64x128_PARTS, 
 struct F32RingTile { int tm, tn, tk; float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32RingTile F32_RING_TILES[RING_TILES] = {{64, 64, 32, 4.25f, 0.0166f, 0.0f, 0.78f, 0.0f},
                                                     {64, 128, 32, 5.20f, 0.0320f, 0.0f, 1.66f, 0.0015f},
-                                                    {128, 128, 32, 8.20f, 0.0297f, 0.0063f, 7.52f, 0.0020f},
-                                                    {64, 128, 64, 6.67f, 0.0204f, 0.0027f, 5.80f, 0.0021f},
-                                                    {64, 64, 64, 4.80f, 0.0125f, 0.0020f, 4.00f, 0.0016f}};
+                                                    {128, 128, 32, 9.22f, 0.0271f, 0.0202f, 6.69f, 0.0f},
+                                                    {64, 128, 64, 6.93f, 0.0183f, 0.0100f, 5.17f, 0.0005f},
+                                                    {64, 64, 64, 4.85f, 0.0119f, 0.0041f, 3.32f, 0.0012f}};
 struct F32Ring { int tile; float cost; };
 // (one candidate; the candidates are a parameter of the template, as those of the 16-bit kernels are)
 template <size_t I> void consider_f32_ring_tile(const AxhipGemmParams &p, float odd, F32Ring &best) {
@@ -1014,15 +1014,17 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 }
 // The time of the kernels of gemm_f32.hip in us, as for the 16-bit ones above: start + k (per_k + (per_k_full +
 // per_k_odd) u) r + per_round (r - 1), per_k_odd for rows off the 16-byte grid.  Fitted with the ring kernel's to 260
-// products of m 9 .. 8192, n 64 .. 8192, k 64 .. 8192 (mean error 2 - 4 % of the ring's, 6 - 10 % of these); of 300 others the one picked is
-// 0.8 % slower than the fastest on average, and no more than 7 % (two of them 3 %) than what is picked without the tiles of parts;
+// products of m 9 .. 8192, n 64 .. 8192, k 64 .. 8192 (mean error 2 - 4 % of the ring's, 6 - 10 % of these), those of parts to
+// 400 with k from 32 (2 - 3 %).  Of 1200 products the one picked is 1.4 % slower than the fastest on average; they take 0.976 of the time that
+// they take without the tiles of parts, 16 of them 2 % more or longer and 8 of these 5 % (33 x 8192 x 8192, b along k, 79 -> 90 us, the worst;
+// 3264 x 1280 x 1536 100 -> 104);
 // 2.3 times as fast as the ring and FMA kernels, which had the small ones to themselves:
 // 99 x 1024 x 5120 104 -> 18 us, 186 x 640 x 958 35 -> 8, 48 x 384 x 2048 77 -> 6.3.  Large products with both operands
-// along k stay on the ring: 2048^3 97 us against 188.
+// along k stay on the ring: 2048^3 115 us against 188.
 struct F32Kernel { float start, per_k, per_k_full, per_round, per_k_odd; };
 constexpr F32Kernel F32_KERNELS[F32_SHAPES] = {
     {3.28f, 0.00144f, 0.00039f, 0.43f, 0.00063f}, {3.59f, 0.00249f, 0.00096f, 1.11f, 0.00074f}, {3.84f, 0.00524f, 0.00076f, 1.69f, 0.00091f}, {3.76f, 0.00472f, 0.00079f, 1.11f, 0.00138f},
-    {4.59f, 0.00939f, 0.00112f, 3.91f, 0.00138f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}, {5.70f, 0.00701f, 0.00159f, 4.30f, 0.00106f}};
+    {4.59f, 0.00939f, 0.00112f, 3.91f, 0.00138f}, {6.25f, 0.01761f, 0.00329f, 6.68f, 0.00394f}, {5.40f, 0.00618f, 0.00378f, 3.44f, 0.00093f}};
 
 template <size_t I> void consider_f32_kernel(const AxhipGemmParams &p, float k, float u, bool ring, int &best, float &best_cost) {
     constexpr F32Kernel h = F32_KERNELS[I];
