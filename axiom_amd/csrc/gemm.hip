@@ -1015,8 +1015,8 @@ bool takes_f32_ring(const AxhipGemmParams &p, const void *a, const void *b) {
 // The time of the kernels of gemm_f32.hip in us, as for the 16-bit ones above: start + k (per_k + (per_k_full +
 // per_k_odd) u) r + per_round (r - 1), per_k_odd for rows off the 16-byte grid.  Fitted with the ring kernel's to 260
 // products of m 9 .. 8192, n 64 .. 8192, k 64 .. 8192 (mean error 2 - 4 % of the ring's, 6 - 10 % of these), those of parts to
-// 400 with k from 32 (2 - 3 %).  Of 1200 products the one picked is 1.4 % slower than the fastest on average; they take 0.976 of the time that
-// they take without the tiles of parts, 16 of them 2 % more or longer and 8 of these 5 % (33 x 8192 x 8192, b along k, 79 -> 90 us, the worst;
+// 400 with k from 32 (2 - 3 %).  Of 1200 products the one picked is 1.3 % slower than the fastest on average; they take 0.976 of the time that
+// they take without the tiles of parts, 19 of them 2 % more or longer and 11 of these 5 % (33 x 8192 x 8192, b along k, 79 -> 90 us, the worst;
 // 3264 x 1280 x 1536 100 -> 104);
 // 2.3 times as fast as the ring and FMA kernels, which had the small ones to themselves:
 // 99 x 1024 x 5120 104 -> 18 us, 186 x 640 x 958 35 -> 8, 48 x 384 x 2048 77 -> 6.3.  Large products with both operands
@@ -1033,7 +1033,9 @@ template <size_t I> void consider_f32_kernel(const AxhipGemmParams &p, float k, 
     if (!launch_fits(static_cast<int64_t>(rows) * cols + 7, 512)) return; // (eight wavefronts a tile)
     const float full = static_cast<float>(p.batch) * static_cast<float>(rows) * static_cast<float>(cols) * (1.0f / 256.0f);
     const float r = full <= 1.0f ? 1.0f : 0.5f * (std::ceil(full) + full);
-    const float cost = h.start + k * (h.per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
+    // (b as [k, n]: the small tiles of fp32 products are slower, 78 x 4096 x 2048 27.3 us on 16 x 16 against 18.7 with b along k)
+    const float per_k = I <= F32_32x32 && !p.trans_b ? 1.05f * h.per_k : h.per_k;
+    const float cost = h.start + k * (per_k + (h.per_k_full + h.per_k_odd * u) * std::min(full, 1.0f)) * r + h.per_round * (r - 1.0f);
     if ((best < 0 && !ring) || cost < best_cost) { best_cost = cost; best = static_cast<int>(I); }
 }
 template <size_t... I> void consider_f32_kernels(const AxhipGemmParams &p, float k, float u, bool ring, int &best, float &best_cost, std::index_sequence<I...>) {
