@@ -1302,7 +1302,9 @@ template <int D> constexpr int sdpa_f32_lds_bytes() { return 2 * BN * ((D + 4) +
 // turn); their (reference maximum, denominator, O^T) states are merged through LDS at the end.  A wave's MFMAs form
 // one dependent chain over its keys, so short problems (few work-groups, e.g. one batch of 8 heads x 512 rows) are
 // bound by that chain's length rather than by the chip: splitting the keys shortens it SPLIT-fold.
-template <bool HAS_MASK, int D, int SPLIT>
+// So does it the sums' error: with fewer waves they are further off (8 x 32 heads of 128 x 64: 2.9e-7 with four, 3.0e-7 with two,
+// 3.4e-7 with one).  PARTED: a sub-tile's sums start at zero and are added to those before, 2.9e-7 with any number; it takes 2 - 6 % longer.
+template <bool HAS_MASK, int D, int SPLIT, bool PARTED>
 __global__ __launch_bounds__(256) void sdpa_mfma_f32_kernel(const SdpaArgs a) {
     static_assert(SPLIT == 1 || SPLIT == 2 || SPLIT == 4, "waves per query block");
     constexpr int KSTR = D + 4, VSTR = D + 8; // LDS row strides in floats
@@ -1510,19 +1512,38 @@ __global__ __launch_bounds__(256) void sdpa_mfma_f32_kernel(const SdpaArgs a) {
             for (int i = 0; i < 16; ++i) {
                 const float pexp = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][i], a.scale_log2e, -m_use));
                 s[u][i] = pexp;
-                l_run += pexp;
+                if constexpr (!PARTED) l_run += pexp;
             }
+        if constexpr (PARTED) {
+#pragma unroll
+            for (int u = 0; u < NSUB; ++u) {
+                float four[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) four[i] = (s[u][4 * i] + s[u][4 * i + 1]) + (s[u][4 * i + 2] + s[u][4 * i + 3]);
+                l_run += (four[0] + four[1]) + (four[2] + four[3]);
+            }
+        }
 
         // ---- O^T += V^T P^T: MFMA e of a sub-tile multiplies keys 8 (e / 4) + e % 4 (lower half-wave) and + 4 (upper)
+        auto v_of = [&](int u, int e, int dt) __attribute__((always_inline)) { return Vb[v_frag + (sub_kt(u) * 32 + 8 * (e / 4) + e % 4) * VSTR + 32 * dt]; };
+        if constexpr (PARTED) {
 #pragma unroll
-        for (int u = 0; u < NSUB; ++u)
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
+            for (int u = 0; u < NSUB; ++u)
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) {
-                    const float vf = Vb[v_frag + (sub_kt(u) * 32 + 8 * (e / 4) + e % 4) * VSTR + 32 * dt];
-                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf, s[u][e], oacc[dt], 0, 0, 0);
+                    float16_t part{};
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(v_of(u, e, dt), s[u][e], part, 0, 0, 0);
+                    oacc[dt] += part;
                 }
+        } else {
+#pragma unroll
+            for (int u = 0; u < NSUB; ++u)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(v_of(u, e, dt), s[u][e], oacc[dt], 0, 0, 0);
+        }
     };
 
     if constexpr (SPLIT < 4) {
@@ -1910,7 +1931,9 @@ MaskPlan mask_plan(const AxhipSdpaParams &p, bool has_mask) {
     return m;
 }
 
-// fp32: waves per 32-row query block on sdpa_mfma_f32_kernel (1, 2 or 4), or 0 for sdpa_direct_f32_kernel.
+// fp32: waves per 32-row query block on sdpa_mfma_f32_kernel (1, 2 or 4), or 0 for sdpa_direct_f32_kernel; whether their time decided that,
+// against what the number of blocks says, and for longer sums of a wave, which are then parted so as not to come out further off.
+struct F32Choice { int waves; bool by_time, parted; };
 // The times are in us, start + max(block + key longest, rounds (round + busy average)): a block of the longest row alone on its CU,
 // or what every CU has to do, in whole rounds of 256 work-groups (two that share a CU take twice the time); causal blocks, unequal
 // as they are, go on without rounds and take `causal` more.  Fitted to 368 problems of 64 .. 4096 rows, 6 .. 512 slices (mean error
@@ -1937,13 +1960,13 @@ float f32_schedule_time(const AxhipSdpaParams &p, bool masked, const F32Schedule
     }
     return f.start + time;
 }
-int f32_schedule(const AxhipSdpaParams &p, bool masked) {
+F32Choice f32_schedule(const AxhipSdpaParams &p, bool masked) {
     // By the blocks alone: the kernel without shared tiles up to one 16-row block per CU (8 heads of 512 rows of 64: 16.3 -> 9.5
     // us, 8 of 333 x 1000 of 128: 51.5 -> 25.1), else the more waves to a block the fewer blocks there are for the 1024 SIMDs
     const int64_t slices = static_cast<int64_t>(p.batch) * p.heads, blocks16 = static_cast<int64_t>((p.seq_q + 15) / 16) * slices, blocks32 = static_cast<int64_t>((p.seq_q + 31) / 32) * slices;
     const int usual = blocks16 <= 256 && p.head_dim > 32 ? 0 : blocks32 >= 1536 ? 3 : blocks32 >= 768 ? 2 : 1; // (of the table)
     const F32Schedule *table = F32_SCHEDULES[p.head_dim > 64];
-    if (p.head_dim <= 32 || (p.is_causal && masked)) return table[usual].waves; // (no times of these)
+    if (p.head_dim <= 32 || (p.is_causal && masked)) return {table[usual].waves, false, false}; // (no times of these)
     // ... unless another one is to win an eighth by its time (30 heads of 258 x 80: 43 -> 22 us without shared tiles, 8 of 700 x 64 causal
     // 22.2 -> 12.3, 40 of 260 x 128 44.9 -> 31.0 with two waves; 220 other problems 0.93 of the time, the worst 1.02)
     int best = usual;
@@ -1953,7 +1976,7 @@ int f32_schedule(const AxhipSdpaParams &p, bool masked) {
         const float t = f32_schedule_time(p, masked, table[i]);
         if (t < least) { least = t; best = i; }
     }
-    return table[best].waves;
+    return {table[best].waves, best != usual, best > usual};
 }
 
 template <bool BF16, int MASK, int D, int PAD> void launch_pipelined_as(const SdpaArgs &a, int nw, bool split, unsigned grid, hipStream_t s) {
@@ -1986,24 +2009,24 @@ template <bool BF16, int D> int launch_mfma(const SdpaArgs &a, hipStream_t s) {
     return AXHIP_OK;
 }
 
-template <int D, int SPLIT> int launch_mfma_f32(const SdpaArgs &a, hipStream_t s) {
+template <int D, int SPLIT, bool PARTED> int launch_mfma_f32(const SdpaArgs &a, hipStream_t s) {
     constexpr int lds = sdpa_f32_lds_bytes<D>();
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute(reinterpret_cast<const void *>(sdpa_mfma_f32_kernel<false, D, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        attr = hipFuncSetAttribute(reinterpret_cast<const void *>(sdpa_mfma_f32_kernel<false, D, SPLIT, PARTED>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (attr == hipSuccess)
-            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(sdpa_mfma_f32_kernel<true, D, SPLIT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(sdpa_mfma_f32_kernel<true, D, SPLIT, PARTED>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     });
     AXHIP_CHECK_HIP(attr);
     const unsigned grid = static_cast<unsigned>(a.nqb) * static_cast<unsigned>(a.B * a.H);
-    if (a.mask) hipLaunchKernelGGL((sdpa_mfma_f32_kernel<true, D, SPLIT>), dim3(grid), dim3(256), lds, s, a);
-    else hipLaunchKernelGGL((sdpa_mfma_f32_kernel<false, D, SPLIT>), dim3(grid), dim3(256), lds, s, a);
+    if (a.mask) hipLaunchKernelGGL((sdpa_mfma_f32_kernel<true, D, SPLIT, PARTED>), dim3(grid), dim3(256), lds, s, a);
+    else hipLaunchKernelGGL((sdpa_mfma_f32_kernel<false, D, SPLIT, PARTED>), dim3(grid), dim3(256), lds, s, a);
     return AXHIP_OK;
 }
 
-template <int D> int launch_mfma_f32_d(const SdpaArgs &a, int split, hipStream_t s) {
-    return split == 1 ? launch_mfma_f32<D, 1>(a, s) : split == 2 ? launch_mfma_f32<D, 2>(a, s) : launch_mfma_f32<D, 4>(a, s);
+template <int D, bool PARTED> int launch_mfma_f32_d(const SdpaArgs &a, int split, hipStream_t s) {
+    return split == 1 ? launch_mfma_f32<D, 1, PARTED>(a, s) : split == 2 ? launch_mfma_f32<D, 2, PARTED>(a, s) : launch_mfma_f32<D, 4, PARTED>(a, s);
 }
 
 } // namespace
@@ -2213,17 +2236,19 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o, cons
             break;
         }
     } else if (kind == SdpaKind::MFMA_F32) {
-        last_schedule = "mfma_f32";
-        const int split = sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4 ? sdpa_f32_split : f32_schedule(p, mask != nullptr);
-        if (split == 0) {
+        const bool forced = sdpa_f32_split == 1 || sdpa_f32_split == 2 || sdpa_f32_split == 4;
+        const F32Choice f = forced ? F32Choice{sdpa_f32_split, false, false} : f32_schedule(p, mask != nullptr);
+        if (f.waves == 0) {
             last_schedule = "direct";
             a.nqb = (p.seq_q + 15) / 16;
             return launch_sdpa_direct_f32(a, s);
         }
-        const int bmw = 128 / split;
+        last_schedule = !f.by_time ? "mfma_f32" : f.waves == 1 ? "mfma_f32_1" : f.waves == 2 ? "mfma_f32_2" : "mfma_f32_4";
+        const int bmw = 128 / f.waves;
         a.nqb = (p.seq_q + bmw - 1) / bmw;
         AXHIP_REQUIRE(launch_fits(static_cast<int64_t>(a.nqb) * p.batch * p.heads, 256), AXHIP_ERR_UNSUPPORTED, "axhip_sdpa_fwd: grid too large");
-        rc = p.head_dim <= 32 ? launch_mfma_f32_d<32>(a, split, s) : p.head_dim <= 64 ? launch_mfma_f32_d<64>(a, split, s) : launch_mfma_f32_d<128>(a, split, s);
+        if (f.parted) rc = p.head_dim <= 64 ? launch_mfma_f32_d<64, true>(a, f.waves, s) : launch_mfma_f32_d<128, true>(a, f.waves, s); // (more than 32 dims)
+        else rc = p.head_dim <= 32 ? launch_mfma_f32_d<32, false>(a, f.waves, s) : p.head_dim <= 64 ? launch_mfma_f32_d<64, false>(a, f.waves, s) : launch_mfma_f32_d<128, false>(a, f.waves, s);
         if (rc) return rc;
     } else {
         last_schedule = "generic";

@@ -132,8 +132,9 @@ int axhip_sdpa_fwd_ws(const void *q, const void *k, const void *v, void *o,
  * the process. */
 const char *axhip_sdpa_kernel_name(const AxhipSdpaParams *params_host);
 /* diagnostic: the schedule the calling thread's last axhip_sdpa_fwd launched ("pingpong", "pipelined8",
- * "pipelined4", "key_split", "key_split8", "decode_split", "direct", "register_staged", "mfma_f32", "generic", "empty"); several
- * schedules share one kernel name.  AXHIP_SDPA_PINGPONG=0 in the environment (read when the library loads)
+ * "pipelined4", "key_split", "key_split8", "decode_split", "direct", "register_staged", "mfma_f32", "generic", "empty"; several
+ * schedules share one kernel name; "mfma_f32_1", "_2" and "_4": fp32 with that many waves to 32 query rows where it
+ * is not their number that says so).  AXHIP_SDPA_PINGPONG=0 in the environment (read when the library loads)
  * sends "pingpong" problems to "pipelined4" or "pipelined8". */
 const char *axhip_sdpa_last_schedule(void);
 

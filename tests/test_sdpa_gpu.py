@@ -667,12 +667,18 @@ def test_eight_waves_that_share_the_keys(dt, B, H, Sq, Skv, D, causal, masked):
             assert np.max(np.abs(got[b:b + 1, h:h + 1] - want)) < 2e-2, (b, h, give)
 
 
-@pytest.mark.parametrize("B,H,Sq,Skv,D,causal,masked,schedule", [
-    (5, 6, 258, 258, 80, False, False, b"direct"), (1, 8, 700, 700, 64, True, False, b"direct"), (5, 6, 258, 261, 128, False, True, b"direct"),
-    (2, 20, 260, 260, 128, False, False, b"mfma_f32"), (4, 12, 300, 300, 64, False, True, b"mfma_f32"), (16, 20, 64, 64, 100, True, False, b"mfma_f32"), (1, 9, 449, 1031, 96, True, False, b"direct")])
-def test_f32_schedules_by_their_time(B, H, Sq, Skv, D, causal, masked, schedule):
-    """More 16-row blocks than CUs without shared tiles, and blocks that two waves share instead of four: where the time of a schedule
-    decides instead of the number of blocks."""
+@pytest.mark.parametrize("B,H,Sq,Skv,D,causal,masked,schedule,by_number", [
+    # four waves by the number of blocks: without shared tiles, two waves, one
+    (5, 6, 258, 258, 80, False, False, b"direct", 3.45e-7), (1, 8, 700, 700, 64, True, False, b"direct", 2.57e-7), (5, 6, 258, 261, 128, False, True, b"direct", 3.94e-7),
+    (1, 9, 449, 1031, 96, True, False, b"direct", 2.80e-7), (2, 20, 260, 260, 128, False, False, b"mfma_f32_2", 4.07e-7), (16, 20, 64, 64, 100, True, False, b"mfma_f32_2", 2.12e-7),
+    (11, 20, 65, 65, 64, False, False, b"mfma_f32_1", 2.69e-7),
+    # two by their number: one wave, four
+    (8, 32, 128, 128, 64, False, False, b"mfma_f32_1", 3.03e-7), (8, 32, 100, 100, 128, False, True, b"mfma_f32_1", 3.53e-7), (3, 20, 520, 520, 64, False, False, b"mfma_f32_4", 4.17e-7),
+    # one by their number: two, four
+    (16, 20, 130, 130, 64, False, False, b"mfma_f32_2", 3.44e-7), (16, 20, 160, 160, 64, True, False, b"mfma_f32_4", 2.22e-7)])
+def test_f32_schedules_by_their_time(B, H, Sq, Skv, D, causal, masked, schedule, by_number):
+    """Where the time of a schedule decides instead of the number of blocks: which one, and that its result is no further from the
+    exact one than that of the schedule by number (`by_number`: its relative error for these inputs, rounded up)."""
     from axiom_amd import capi
 
     mask = (np.random.default_rng(Sq).random((Sq, Skv)) < 0.3).astype(np.uint8) if masked else None
@@ -680,4 +686,5 @@ def test_f32_schedules_by_their_time(B, H, Sq, Skv, D, causal, masked, schedule)
     got, _ = gh.sdpa(q, k, v, F32, -1.0, causal, mask)
     assert capi.lib().axhip_sdpa_last_schedule() == schedule
     want = naive_attention64(q, k, v, 1 / math.sqrt(D), causal, mask)
+    assert np.linalg.norm(got - want) <= by_number * np.linalg.norm(want)
     assert np.max(np.abs(got - want)) < 1e-4
