@@ -120,6 +120,7 @@ def lib() -> C.CDLL:
                                          C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.c_void_p]
         l.axhip_fill.argtypes = [C.c_void_p, C.c_int32, C.c_double, C.c_int64, C.c_void_p]
         l.axhip_gemm.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(GemmParams), C.c_void_p]
+        l.axhip_gemm_last_kernel.restype = C.c_char_p
         l.axhip_gemm_workspace_bytes.restype = C.c_size_t
         l.axhip_gemm_workspace_bytes.argtypes = [C.POINTER(GemmParams)]
         l.axhip_gemm_ws.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(GemmParams), C.c_void_p, C.c_size_t, C.c_void_p]

@@ -875,6 +875,8 @@ size_t repack_bytes(const AxhipGemmParams &p) {
     if (r.b) n += CallScratch::rounded(static_cast<size_t>(p.stride_b == 0 ? 1 : p.batch) * p.n * r.kp * es);
     return n;
 }
+thread_local const char *last_kernel = "none";
+
 int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *params, CallScratch *scratch_in, void *workspace, size_t workspace_bytes, void *stream);
 } // namespace
 
@@ -888,6 +890,8 @@ extern "C" size_t axhip_gemm_workspace_bytes(const AxhipGemmParams *params) {
 extern "C" int axhip_gemm(const void *a, const void *b, void *c, const AxhipGemmParams *params, void *stream) {
     return gemm_impl(a, b, c, params, nullptr, nullptr, 0, stream);
 }
+
+extern "C" const char *axhip_gemm_last_kernel(void) { return last_kernel; }
 
 extern "C" int axhip_gemm_ws(const void *a, const void *b, void *c, const AxhipGemmParams *params, void *workspace, size_t workspace_bytes, void *stream) {
     return gemm_impl(a, b, c, params, nullptr, workspace, workspace_bytes, stream);
@@ -1100,6 +1104,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
     AXHIP_REQUIRE(p.epilogue_op == 0 || p.epilogue_op == AXHIP_OP_RELU || p.epilogue_op == AXHIP_OP_GELU || p.epilogue_op == AXHIP_OP_SILU ||
                       p.epilogue_op == AXHIP_OP_SIGMOID || p.epilogue_op == AXHIP_OP_TANH,
                   AXHIP_ERR_INVALID_ARG, "axhip_gemm: unsupported epilogue op %d", p.epilogue_op);
+    last_kernel = "empty";
     if (p.m == 0 || p.n == 0 || p.batch == 0) return AXHIP_OK;
     AXHIP_REQUIRE(a && b && c, AXHIP_ERR_INVALID_ARG, "axhip_gemm: NULL matrix");
     if (p.batch >= 65536) {
@@ -1208,11 +1213,15 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         const int rows_per_wave = forced_rows == 1 || forced_rows == 2 || forced_rows == 4 ? forced_rows : (p.m >= 2 && w_elems >= (int64_t(64) << 20)) ? 2 : 1;
         const unsigned blocks = static_cast<unsigned>((p.n + 4 * rows_per_wave - 1) / (4 * rows_per_wave));
         launch_skinny(k, static_cast<int>(p.m), rows_per_wave, blocks, s);
+        last_kernel = "skinny";
     } else if (const HalfKernel *k = half_kernel()) {
         const bool aligned = half_aligned(p, a, b), bf = p.dtype == AXHIP_DTYPE_BF16;
+        last_kernel = k->kind == HalfKernel::BIG256 ? "big" : k->kind == HalfKernel::TILE ? "tile" : "small";
         rc = k->kind == HalfKernel::BIG256 ? launch_big(g, bf, s) : launch_half(p, a, b, c, *k, aligned, bf, s);
         if (rc) return rc;
     } else if (f32_shape >= 0) {
+        static constexpr const char *names[F32_SHAPES] = {"f32_16x16", "f32_16x32", "f32_16x64", "f32_32x32", "f32_32x64", "f32_64x64", "f32_32x64_parts"};
+        last_kernel = names[f32_shape];
         rc = launch_f32_direct(tile_args(p, a, b, c), !p.trans_b, f32_shape, s);
         if (rc) return rc;
     } else if (f32 && takes_f32_ring(p, a, b)) {
@@ -1248,7 +1257,10 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
             return AXHIP_OK;
         };
         int rc2;
-        switch (f32_ring_tile(p).tile) {
+        static constexpr const char *names[RING_TILES] = {"ring_64x64", "ring_64x128", "ring_128x128_parts", "ring_64x128_parts", "ring_64x64_parts"};
+        const int tile = f32_ring_tile(p).tile;
+        last_kernel = names[tile];
+        switch (tile) {
 #define AXHIP_RING(TM, TN, KF, LW, LDS) \
     rc2 = p.trans_b ? launch(gemm_mfma_f32_ring_kernel<TM, TN, KF, LW, false>, TM, TN, 64 * (4 + LW), LDS) : launch(gemm_mfma_f32_ring_kernel<TM, TN, KF, LW, true>, TM, TN, 64 * (4 + LW), LDS)
         case RING_64x64: AXHIP_RING(64, 64, 0, 4, (ring_lds_bytes<64, 64>())); break;
@@ -1260,6 +1272,7 @@ int gemm_impl(const void *a, const void *b, void *c, const AxhipGemmParams *para
         }
         if (rc2) return rc2;
     } else {
+        last_kernel = "fma";
         dim3 grid(static_cast<unsigned>((p.n + 15) / 16), static_cast<unsigned>((p.m + 15) / 16), static_cast<unsigned>(p.batch));
         AXHIP_REQUIRE(grid.y < 65536, AXHIP_ERR_UNSUPPORTED, "axhip_gemm: m too large for the generic kernel");
         AXHIP_REQUIRE(launch_fits((p.n + 15) / 16, 16 * 16), AXHIP_ERR_UNSUPPORTED, "axhip_gemm: n too large for the generic kernel");

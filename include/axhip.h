@@ -459,6 +459,10 @@ int axhip_gemm(const void *a, const void *b, void *c, const AxhipGemmParams *par
 size_t axhip_gemm_workspace_bytes(const AxhipGemmParams *params_host);
 int axhip_gemm_ws(const void *a, const void *b, void *c, const AxhipGemmParams *params_host,
                   void *workspace, size_t workspace_bytes, void *stream);
+/* diagnostic: the kernel that the calling thread's last axhip_gemm or axhip_gemm_ws multiplied with: "skinny" (at most
+ * eight rows), "big", "tile", "small" (16 bits), "f32_16x16" .. "f32_64x64", "ring_64x64", "ring_64x128" (fp32, by work-group
+ * tile), the same with "_parts" (fp32 by products of bf16 parts), "fma", "empty". */
+const char *axhip_gemm_last_kernel(void);
 
 /* sizeof() of the parameter structs as this library was compiled, so that a
  * foreign-language binding can verify its own struct layout at load time:

@@ -269,7 +269,7 @@ def test_few_rows_too_far_apart_for_the_tiled_kernels(dt):
 
 
 def test_the_fp32_ring_adds_up_odd_and_even_numbers_of_k_tiles():
-    """Whole numbers, exact in every order of the sum: 64 x 64 tiles with one work-group per CU (two accumulators in turn) and
+    """Whole numbers, exact in every order of the sum: 64 x 64 tiles of fp32 products with one work-group per CU and
     with several, two to five k-tiles and a ragged last one, rows off the tile, with and without each epilogue step."""
     for M, N in ((1000, 980), (1500, 1284)):
         for K in (64, 96, 100, 128, 131, 160):
@@ -373,7 +373,7 @@ def test_f32_products_at_the_edges_of_tiles(nn, M, N, K, batch):
 
 @pytest.mark.parametrize("M,N,K,batch", [(2048, 2044, 132, 1), (1000, 1100, 260, 8), (1024, 1024, 1024, 1), (1300, 4000, 44, 3), (700, 2500, 1000, 1)])
 def test_f32_products_of_plain_matrices_on_the_ring(M, N, K, batch):
-    """a b with b stored [k, n] in whole vectors, sizes of the ring kernel's four tiles: k that ends inside a k-tile, rows
+    """a b with b stored [k, n] in whole vectors, sizes of several of the ring kernel's tiles: k that ends inside a k-tile, rows
     and columns inside a tile; b lies in front of NaNs.  The same bound as above."""
     import ctypes as C
 
@@ -496,37 +496,49 @@ def test_batches_are_dealt_over_all_xcds(dtype, nn, M, N, K, batch, shared):
         assert bool(((c[b].double() - want).abs() <= (K + 2) * 2.0**-24 * magnitude + half_ulp * want.abs() + 2.0**-24).all())
 
 
-# k from 32 to 8192 on every tile that multiplies parts: 32 x 64 and 64 x 64 (few output tiles), 64 x 128 and 128 x 128, with rows,
-# columns and k that end inside a tile, a chunk and a pair of k-tiles; the last is short enough for fp32 products on 32 x 64
-PARTS = [(300, 1280, 1285, 1), (130, 1984, 2050, 1), (1024, 1020, 1023, 1), (1000, 1028, 1090, 1), (257, 4100, 700, 1), (513, 132, 995, 8), (2048, 2044, 225, 1), (1153, 129, 256, 16), (64, 241, 145, 32)]
+# Every tile that multiplies parts, and four products that stay with fp32 ones: k-tiles (of 32 on
+# 128 x 128, of 64 on the other two rings) of every remainder by how many are on their way (three, two, three), k of every
+# remainder by 4, rows and columns inside a tile, columns off the 16-byte grid (b as [k, n]: the last tile moved left)
+PARTS = [(346, 2137, 98, 4, "ring_128x128_parts"), (206, 1581, 133, 8, "ring_128x128_parts"), (321, 1054, 163, 8, "ring_128x128_parts"), (2048, 2044, 225, 1, "ring_128x128_parts"),
+         (51, 2093, 244, 8, "ring_64x128_parts"), (103, 1073, 289, 8, "ring_64x128_parts"), (257, 4100, 700, 1, "ring_64x128_parts"), (1000, 1028, 1090, 1, "ring_64x128_parts"),
+         (817, 614, 354, 1, "ring_64x64_parts"), (291, 1665, 418, 1, "ring_64x64_parts"), (1845, 263, 493, 1, "ring_64x64_parts"), (867, 579, 628, 1, "ring_64x64_parts"),
+         (300, 1280, 1285, 1, "f32_32x64_parts"), (130, 1984, 2050, 1, "f32_32x64_parts"), (21, 1071, 690, 8, "f32_32x64_parts"), (1684, 165, 547, 1, "f32_32x64_parts"),
+         (1024, 1020, 1023, 1, "ring_64x64"), (513, 132, 995, 8, "ring_64x64"), (1153, 129, 256, 16, "ring_64x64"), (64, 241, 145, 32, "f32_32x64")]
 
 
 @pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
-@pytest.mark.parametrize("M,N,K,batch", PARTS)
-def test_f32_products_of_parts(nn, M, N, K, batch):
+@pytest.mark.parametrize("M,N,K,batch,kernel", PARTS)
+def test_f32_products_of_parts(nn, M, N, K, batch, kernel):
     """Products by way of bf16 parts are no further from the exact ones than fp32 sums of 32 products and then one per
-    32 k: (36 + K / 32) half ulps of the sum of magnitudes, for inputs of both signs, of one sign, and so small that their
-    last parts would be below bf16's smallest normal number, had they not been scaled."""
+    32 k: (36 + K / 32) half ulps of the sum of magnitudes, for inputs of both signs, of one sign, so small that their
+    last parts would be below bf16's smallest normal number, had they not been scaled, denormal ones, and some on either side of 2^112, from which
+    on there are no parts."""
     import torch
 
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M + 3 * N + K)
-    for kind in ("normal", "positive", "small"):
+    scales = {"small": (2.0**-118, 2.0**40), "denormal": (2.0**-70, 2.0**100), "large": (2.0**111, 2.0**-30)}
+    for kind in ("normal", "positive", *scales):
+        if kind == "denormal" and "parts" not in kernel:
+            continue
         x, W = torch.empty((batch, M, K), device="cuda"), torch.empty((batch, K, N) if nn else (batch, N, K), device="cuda")
         for t in (x, W):
             t.uniform_(0.0, 1.0, generator=gen) if kind == "positive" else t.normal_(generator=gen)
-        if kind == "small":
-            x *= 2.0**-118
-            W *= 2.0**40
-        c = _f32_product(x, W, nn)
+        if kind in scales:
+            x *= scales[kind][0]
+            W *= scales[kind][1]
+        if kind == "denormal":
+            x *= scales[kind][0]
+            assert bool((x.abs() < 2.0**-130).all()) and bool((x != 0).any())
+        c = _f32_product(x, W, nn, kernel)
         for b in range(0, batch, 5):
             x64, w64 = x[b].double(), W[b].double() if nn else W[b].double().t().contiguous()
             assert bool(((c[b].double() - x64 @ w64).abs() <= min(K + 2, 36 + K / 32) * 2.0**-24 * (x64.abs() @ w64.abs())).all()), kind
 
 
 @pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
-@pytest.mark.parametrize("M,N,K,batch", PARTS)
-def test_f32_products_of_parts_with_one_product_to_an_output(nn, M, N, K, batch):
+@pytest.mark.parametrize("M,N,K,batch,kernel", PARTS)
+def test_f32_products_of_parts_with_one_product_to_an_output(nn, M, N, K, batch, kernel):
     """Rows of x with a single entry: the result is one product, rounded once.  By parts the last addition rounds by half
     an ulp and the seven before it, of numbers below 2^-5 where the result is 1 or more, by 2^-30 each at most: 0.5 + 7 / 128 ulp.  Among
     random factors some whose second and third parts are as large as they get (0x1.01ffp0 squared is 2 ulp off without their products)."""
@@ -541,7 +553,7 @@ def test_f32_products_of_parts_with_one_product_to_an_output(nn, M, N, K, batch)
     value[:, ::3] = hard
     (W[:, :, ::3] if nn else W[:, ::3]).fill_(hard)
     x.scatter_(2, at, value)
-    c = _f32_product(x, W, nn)
+    c = _f32_product(x, W, nn, kernel)
     for b in range(0, batch, 5):
         want = value[b].double() * (W[b].t() if not nn else W[b]).contiguous()[at[b, :, 0]].double()
         nearest = want.float().abs()
@@ -549,9 +561,33 @@ def test_f32_products_of_parts_with_one_product_to_an_output(nn, M, N, K, batch)
         assert bool(((c[b].double() - want).abs() <= (0.5 + 7 / 128) * ulp).all())
 
 
+@pytest.mark.parametrize("again", [False, True], ids=["once", "again"])
 @pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
-@pytest.mark.parametrize("M,N,K,batch", PARTS)
-def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch):
+@pytest.mark.parametrize("M,N,K,batch,kernel", PARTS)
+def test_f32_products_of_parts_of_whole_numbers(nn, M, N, K, batch, kernel, again):
+    """Whole numbers with one to three parts, sums below 2^24: exact, with bias, residual and activation, also (`again`) where a tile is
+    computed a second time because one of its rows is infinite."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + 3 * N + K)
+    whole = lambda shape, to: torch.randint(-to, to + 1, shape, device="cuda", generator=gen).float()
+    for wide in ("x", "W"):
+        x, W = whole((batch, M, K), 900 if wide == "x" else 4), whole((batch, K, N) if nn else (batch, N, K), 4 if wide == "x" else 900)
+        (x if wide == "x" else W.transpose(1, 2) if nn else W)[..., 1:K:K // 3] += 2.0**17 + 1 # (at most four in each sum)
+        bias, residual = whole((N,), 9), whole((batch, M, N), 9)
+        if again:
+            x[batch // 2, M - 1, K - 2], (W[:, K - 2] if nn else W[:, :, K - 2])[...] = float("inf"), 1.0
+        c = _f32_product(x, W, nn, kernel, bias, residual, "relu")
+        for b in {0, batch // 2, batch - 1}:
+            want = (x[b].double() @ (W[b].double() if nn else W[b].double().t().contiguous()) + bias + residual[b]).clamp_min(0.0)
+            assert bool((want[torch.isfinite(want)] < 2.0**24).all()) and bool(torch.isinf(want[M - 1]).all()) == (again and b == batch // 2)
+            assert bool((c[b].double() == want).all()), (wide, b)
+
+
+@pytest.mark.parametrize("nn", [False, True], ids=["nt", "nn"])
+@pytest.mark.parametrize("M,N,K,batch,kernel", PARTS)
+def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch, kernel):
     """Infinities, NaN and numbers near the largest, whose parts have none: the same places of the result are infinite or NaN as in
     float64, and everything else keeps its bound, in the tiles that are computed again and in the others."""
     import torch
@@ -560,10 +596,10 @@ def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch):
     gen.manual_seed(M + 3 * N + K)
     x, W = torch.empty((batch, M, K), device="cuda").normal_(generator=gen), torch.empty((batch, K, N) if nn else (batch, N, K), device="cuda").normal_(generator=gen)
     last = batch - 1
-    x[0, 3, 5], x[last, M - 1, K - 1], x[0, 40, :] = float("inf"), float("nan"), 3.0e38
+    x[0, 3, 5], x[last, M - 1, K - 1], x[0, min(40, M - 2), :] = float("inf"), float("nan"), 3.0e38
     W[0] = W[0].abs() * 2.0**-20
     W[last, 0, 0] = -float("inf") if batch > 1 else W[last, 0, 0]
-    c = _f32_product(x, W, nn)
+    c = _f32_product(x, W, nn, kernel)
     for b in {0, last // 2, last}:
         x64, w64 = x[b].double(), W[b].double() if nn else W[b].double().t().contiguous()
         want = x64 @ w64
@@ -575,7 +611,7 @@ def test_f32_products_of_parts_that_are_not_finite(nn, M, N, K, batch):
         assert bool(((c[b].double() - want).abs() <= bound)[finite].all())
 
 
-def _f32_product(x, W, nn):
+def _f32_product(x, W, nn, kernel, bias=None, residual=None, act=None):
     import ctypes as C
 
     import torch
@@ -588,8 +624,10 @@ def _f32_product(x, W, nn):
     p = capi.GemmParams()
     p.dtype, p.m, p.n, p.k, p.batch, p.lda, p.ldb, p.ldc, p.trans_b = F32, M, N, K, batch, K, N if nn else K, N, int(not nn)
     p.stride_a, p.stride_b, p.stride_c = M * K, K * N, M * N
+    p.bias, p.residual, p.epilogue_op = None if bias is None else bias.data_ptr(), None if residual is None else residual.data_ptr(), 0 if act is None else capi.OP[act]
     torch.cuda.synchronize()
     gh.sync()
     capi.check(capi.lib().axhip_gemm(x.data_ptr(), W.data_ptr(), c.data_ptr(), C.byref(p), None))
     gh.sync()
+    assert capi.lib().axhip_gemm_last_kernel() == kernel.encode()
     return c
