@@ -373,8 +373,8 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // 64 x 64, one work-group a CU: 1024 cycles of MFMAs in 1310.  The values of a finished block then take bias, residual and
 // activation together: with a branch on the activation for each, 60 KB of code that every CU read anew, 4096 x 4096 x 512 + GELU
 // took 228 us instead of 176.
-// Products of parts (SplitRing) take its place wherever there is k enough; this form stays for short k, of whose tiles of
-// 64 x 64 three work-groups share a CU (8 x (2939 x 704 x 66) 44 us against 54), and for tiles whose parts have no finite sums.
+// Products of parts (SplitRing) take its place where their time is less, which takes k enough: of this form's tiles of 64 x 64 three
+// work-groups share a CU (8 x (2939 x 704 x 66) 41 us against 54 on parts, when those were six products).  Tiles whose parts have no finite sums run it, too.
 // Rows may start anywhere: the loads need 4-byte alignment.  The chunk that K ends in is fetched as the four floats that
 // end with the row and shifted into place in LDS by the lane that loaded it; chunks behind it, and k-tiles past the last,
 // are sent out of the descriptor's range and arrive as zeros.  NN rows that are no whole chunks: the last column tile is
@@ -386,9 +386,12 @@ __global__ __launch_bounds__(512, 1) void gemm_mfma_nt_256_kernel(const GemmArgs
 // 32 rows, 8 k at a time, is 512 bytes, 16 a row (the row XOR-ed so that what 32 lanes write at a time meets all banks).
 // The multiplying ones, one per SIMD, hold all fragments of 32 k and refill them under the MFMAs of blocks that need them no
 // more.  Barrier kt: k-tile kt is in LDS and k-tile kt - 1 has been read.
-// 64 x 64 has two loading wavefronts per SIMD (1024^3 22.5 us with one, 19.4 with two, of six products) and 64 k at a time for half the barriers.
+// What bounds it: VALU issue where CUs have one tile (1024^3: 30.6 k of 49.5 k cycles, beside 16.4 k of MFMAs, under each of which about five
+// of eight VALU slots are free), the matrix pipe under the power limit on a full chip (4096^3: 74 % busy).  So 64 x 64 has two loading
+// wavefronts per SIMD (1024^3 22.5 us with one, 19.4 with two, of six products) and 64 k at a time for half the barriers.
 // v_mfma_f32_16x16x32, which leaves less room beside it, took 3 % less on full chips and 10 % more on others.
-// 1024^3 21.6 -> 21.0 us, 2048^3 133 -> 113, 4096 x 2000 x 1000 134 -> 118, 4096^3 1014 -> 832 (with six of the products, to fewer bits: 18.9, 94, 100, 697).
+// With fp32 products and with these, us: 1024^3 21.6 and 21.0 (b as [k, n] 22.1 and 22.4), 2048^3 133 and 114, 4096 x 2000 x 1000 134 and
+// 118, 4096^3 1014 and 832.  (Six of the products, to fewer bits: 18.9, 95, 101, 697.)
 template <int TM, int TNR, int KF, int LW, bool NN> struct SplitRing { // KF: floats per k-tile; LW: loading wavefronts
     static constexpr int MI = TM / 64, NJ = TNR / 64, DEPTH = KF == 32 || LW == 8 ? 3 : 2;
     static constexpr int CHUNKS = KF / 4, ROWS = WAVE / CHUNKS * LW;      // 16-byte chunks of a row along k, rows that the loading wavefronts fetch at a time
